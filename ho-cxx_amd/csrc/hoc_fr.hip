@@ -236,227 +236,22 @@ __device__ __forceinline__ void second_order_core(const TabT<R>& T, const R (&u)
 }
 
 // ==========================================================================================
-// Trace kernel with fused vector pre-operations producing the traced field u:
-//   PRE_COPY   u = x
-//   PRE_CHEB0  u = r * dinv * coef (coef = 1/theta); writes x = d = u   (Chebyshev step from zero)
-//   PRE_PROL   u = x + Pc xc (bilinear from the corner vertices); writes x = u
-//   PRE_PUPD   u = z + beta * p; writes p = u                     (PCG direction; beta =
-//              scal[scal_idx], or with scal_idx < 0 scal[einst[element]]: per ensemble instance)
-// einst, iact (may be null): a block inside one ensemble instance whose flag in iact is 0
-// returns at once.
-// RA: the type of a (R, or float for the FP64 direction update of the mixed-precision solve,
-// whose V-cycle leaves z in FP32).
+// Face traces of a field.
 // ==========================================================================================
-template <int K, int PRE, class R, class RA = R>
-__global__ __launch_bounds__(kWG) void k_trace(int N, TabT<R> T, R* __restrict__ x, const RA* __restrict__ a,
-                                                const R* __restrict__ b, R* __restrict__ d, R coef,
-                                                const double* __restrict__ scal, int scal_idx, const int* __restrict__ active,
-                                                R* __restrict__ tr, const int32_t* __restrict__ ev,
-                                                const int32_t* __restrict__ einst, const int* __restrict__ iact) {
-  if (active && !*active) return;
+template <int K>
+__global__ __launch_bounds__(kWG) void k_trace(int N, Tab T, const double* __restrict__ x, double* __restrict__ tr) {
   constexpr int K2 = K * K;
-  __shared__ __align__(16) R lds[kWG * K2];  // one tile: two inputs are staged in turn
+  __shared__ __align__(16) double lds[kWG * K2];
   const int e0 = blockIdx.x * kWG;
-  if (iact) {  // a block inside one stopped ensemble instance
-    const int i0 = einst[e0];
-    if (i0 == einst[min(e0 + kWG, N) - 1] && !iact[i0]) return;
-  }
   const int el = e0 + threadIdx.x;
-  const bool live = el < N;
-  R u[K2];
-  R beta = 0;
-  if (PRE == PRE_PUPD) beta = (R)(scal_idx >= 0 ? scal[scal_idx] : live ? scal[einst[el]] : 0.);
-  R xc[4] = {0, 0, 0, 0};
-  if (PRE == PRE_PROL && live)
+  tile_load<K2>(x, lds, e0, N);
+  if (el >= N) return;
+  double u[K2];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) xc[c] = (R)a[ev[(size_t)el * 4 + c]];
-  RA* la = reinterpret_cast<RA*>(lds);  // sizeof(RA) <= sizeof(R): a fits the tile
-  if constexpr (PRE == PRE_COPY || PRE == PRE_PROL) tile_load<K2>((const R*)x, lds, e0, N);
-  else tile_load<K2>(a, la, e0, N);
-#pragma unroll
-  for (int m = 0; m < K2; ++m) {
-    const int li = threadIdx.x * K2 + m;
-    R v = (PRE == PRE_COPY || PRE == PRE_PROL) ? lds[li] : (R)la[li];
-    if (PRE == PRE_PROL) {
-      const int j = m / K, i = m % K;
-      v += q1w(T, 0, j, i) * xc[0] + q1w(T, 1, j, i) * xc[1] + q1w(T, 2, j, i) * xc[2] + q1w(T, 3, j, i) * xc[3];
-    }
-    u[m] = v;
-  }
-  if (PRE == PRE_CHEB0 || PRE == PRE_PUPD) {  // second input
-    __syncthreads();
-    tile_load<K2>(PRE == PRE_CHEB0 ? b : (const R*)x, lds, e0, N);
-#pragma unroll
-    for (int m = 0; m < K2; ++m) {
-      const R w = lds[threadIdx.x * K2 + m];
-      u[m] = PRE == PRE_CHEB0 ? u[m] * w * coef : u[m] + beta * w;
-    }
-  }
-  if (PRE == PRE_CHEB0 || PRE == PRE_PROL || PRE == PRE_PUPD) {
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < K2; ++m) lds[threadIdx.x * K2 + m] = u[m];
-    if (PRE == PRE_CHEB0) { tile_store<K2>(x, lds, e0, N); tile_store<K2>(d, lds, e0, N); }
-    else tile_store<K2>(x, lds, e0, N);
-  }
-  if (!live) return;
-  R bv[4][K], bg[4][K];
+  for (int m = 0; m < K2; ++m) u[m] = lds[threadIdx.x * K2 + m];
+  double bv[4][K], bg[4][K];
   traces<K>(T, u, bv, bg);
   store_traces<K>(tr, N, el, bv, bg);
-}
-
-// ==========================================================================================
-// Poisson operator As = -W * L (W = w_i w_j) applied matrix-free, with fused epilogues:
-//   EPI_STORE     y = As x; partial sums of x.y                    (PCG / probing)
-//   EPI_RESID     y = r - As x; partial sums of y.y and (y/W).(y/W) (initial residual)
-//   EPI_CHEB      res = r - As x; e = c1 d + c2 res dinv; x += e; y = e unless y is null;
-//                 optional partial r.x
-//   EPI_CHEBF     res = r - As x; e = c2 res dinv (c2 = 1/theta); x += e; y = e unless null
-//                 (first step from x != 0)
-//   (dinv = 1/diag(As), the Jacobi scaling of the Chebyshev smoother; d and y are distinct
-//   direction buffers, and the last step of a sweep passes y = null)
-//   EPI_RESTRICT  ec[el][a] = sum_ij q1w(a,ij) (r - As x)_ij        (Pc^T residual, per element)
-// ==========================================================================================
-template <int K, int EPI, bool AFF, class R>
-// Affine FP32 instances with K <= 5 are held to 128 VGPRs (4 waves per SIMD; their LDS tile
-// allows more), which they fit without spilling; the others keep the compiler's allocation.
-__global__ __launch_bounds__(kWG, (AFF && sizeof(R) == 4 && K <= 5) ? 4 : 1) void k_lap(int N, TabT<R> T, GeoT<R> G, R* __restrict__ x, const R* __restrict__ tr,
-                                              R* __restrict__ y, const R* __restrict__ r,
-                                              const R* __restrict__ dinv, R* __restrict__ d,
-                                              R c1, R c2, double* __restrict__ part,
-                                              const int* __restrict__ active, R* __restrict__ tr_out,
-                                              int* __restrict__ ran) {
-  const bool go = !active || *active;
-  if (ran && blockIdx.x == 0 && threadIdx.x == 0) *ran = go ? 1 : 0;  // timed launches: did it work?
-  if (!go) return;
-  constexpr int K2 = K * K;
-  __shared__ __align__(16) R lds[kWG * K2];
-  const int e0 = blockIdx.x * kWG;
-  if (G.iact) {  // a block inside one stopped ensemble instance
-    const int i0 = G.inst[e0];
-    if (i0 == G.inst[min(e0 + kWG, N) - 1] && !G.iact[i0]) return;
-  }
-  const int el = e0 + threadIdx.x;
-  const bool live = el < N;
-  R u[K2], ga[K2], gb[K2], gc[K2];
-  tile_load<K2>(x, lds, e0, N);
-#pragma unroll
-  for (int m = 0; m < K2; ++m) u[m] = live ? lds[threadIdx.x * K2 + m] : R(0);  // tail threads: no stale LDS
-  if (AFF) {  // metrics constant per element
-    const R a = live ? G.gel[(size_t)el * 3] : R(0), b = live ? G.gel[(size_t)el * 3 + 1] : R(0),
-            c = live ? G.gel[(size_t)el * 3 + 2] : R(0);
-#pragma unroll
-    for (int m = 0; m < K2; ++m) { ga[m] = a; gb[m] = b; gc[m] = c; }
-  } else {
-    __syncthreads();
-    tile_load<K2>(G.Ga, lds, e0, N);
-#pragma unroll
-    for (int m = 0; m < K2; ++m) ga[m] = lds[threadIdx.x * K2 + m];
-    __syncthreads();
-    tile_load<K2>(G.Gb, lds, e0, N);
-#pragma unroll
-    for (int m = 0; m < K2; ++m) gb[m] = lds[threadIdx.x * K2 + m];
-    __syncthreads();
-    tile_load<K2>(G.Gc, lds, e0, N);
-#pragma unroll
-    for (int m = 0; m < K2; ++m) gc[m] = lds[threadIdx.x * K2 + m];
-  }
-  R out[K2];
-  if (live) {
-    R bv[4][K], bg[4][K], cv[4][K], cg[4][K];
-    traces<K>(T, u, bv, bg);
-    faces2<K, AFF>(T, G, el, tr, G.sw_psi, static_cast<const R*>(nullptr), false, bv, bg, cv, cg);
-    second_order_core<K>(T, u, bv, cv, cg, ga, gb, gc, out);
-#pragma unroll
-    for (int j = 0; j < K; ++j)
-#pragma unroll
-      for (int i = 0; i < K; ++i) out[j * K + i] *= -(T.w[j] * T.w[i]);
-  } else {
-#pragma unroll
-    for (int m = 0; m < K2; ++m) out[m] = 0;
-  }
-  double p0 = 0., p1 = 0.;
-  if (EPI == EPI_STORE) {
-#pragma unroll
-    for (int m = 0; m < K2; ++m) p0 += u[m] * out[m];
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < K2; ++m) lds[threadIdx.x * K2 + m] = out[m];
-    tile_store<K2>(y, lds, e0, N);
-  } else {
-    __syncthreads();
-    tile_load<K2>(r, lds, e0, N);
-    R res[K2];
-#pragma unroll
-    for (int m = 0; m < K2; ++m) res[m] = lds[threadIdx.x * K2 + m] - out[m];
-    if (EPI == EPI_RESID) {
-#pragma unroll
-      for (int j = 0; j < K; ++j)
-#pragma unroll
-        for (int i = 0; i < K; ++i) {
-          const double v = res[j * K + i], uw = v / ((double)T.w[j] * T.w[i]);
-          p0 += v * v; p1 += uw * uw;
-        }
-      if (!live) { p0 = 0.; p1 = 0.; }
-      __syncthreads();
-#pragma unroll
-      for (int m = 0; m < K2; ++m) lds[threadIdx.x * K2 + m] = res[m];
-      tile_store<K2>(y, lds, e0, N);
-    } else if (EPI == EPI_RESTRICT) {
-      R s[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < K; ++j)
-#pragma unroll
-        for (int i = 0; i < K; ++i)
-#pragma unroll
-          for (int c = 0; c < 4; ++c) s[c] += q1w(T, c, j, i) * res[j * K + i];
-      if (live)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) y[(size_t)el * 4 + c] = s[c];
-    } else {  // Chebyshev updates
-      __syncthreads();
-      tile_load<K2>(dinv, lds, e0, N);
-      R dd[K2];
-#pragma unroll
-      for (int m = 0; m < K2; ++m) dd[m] = res[m] * lds[threadIdx.x * K2 + m];
-      if (EPI == EPI_CHEB) {
-        __syncthreads();
-        tile_load<K2>(d, lds, e0, N);
-#pragma unroll
-        for (int m = 0; m < K2; ++m) dd[m] = c1 * lds[threadIdx.x * K2 + m] + c2 * dd[m];
-      } else {
-#pragma unroll
-        for (int m = 0; m < K2; ++m) dd[m] *= c2;
-      }
-      if (y) {  // uniform: the direction for the next step of the sweep
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < K2; ++m) lds[threadIdx.x * K2 + m] = dd[m];
-        tile_store<K2>(y, lds, e0, N);
-      }
-#pragma unroll
-      for (int m = 0; m < K2; ++m) u[m] += dd[m];
-#pragma unroll
-      for (int m = 0; m < K2; ++m) lds[threadIdx.x * K2 + m] = u[m];
-      tile_store<K2>(x, lds, e0, N);
-      if (tr_out && live) {  // traces of the updated iterate for the next operator application
-        R bv[4][K], bg[4][K];
-        traces<K>(T, u, bv, bg);
-        store_traces<K>(tr_out, N, el, bv, bg);
-      }
-      if (part) {  // r . x (PCG's r.z after the last smoothing step)
-        tile_load<K2>(r, lds, e0, N);
-#pragma unroll
-        for (int m = 0; m < K2; ++m) p0 += lds[threadIdx.x * K2 + m] * u[m];
-        if (!live) p0 = 0.;
-      }
-    }
-  }
-  if (part) {
-    p0 = wave_sum(p0);
-    p1 = wave_sum(p1);
-    if (threadIdx.x == 0) { part[blockIdx.x] = p0; part[gridDim.x + blockIdx.x] = p1; }
-  }
 }
 
 // ==========================================================================================
@@ -1015,79 +810,9 @@ __global__ void k_hybrid_blend(size_t n, double* __restrict__ w, HybridDev H, do
 
 static inline int nblk(int N) { return (N + kWG - 1) / kWG; }
 
-template <class R>
-static hipError_t launch_trace_t(int K, int pre, int N, const TabT<R>& T, R* x, const R* a, const R* b, R* d,
-                                 double coef, const double* scal, int scal_idx, const int* active, R* tr, hipStream_t s,
-                                 const int32_t* ev, const int32_t* einst, const int* iact) {
-#define LT(P) hipLaunchKernelGGL((k_trace<KK, P, R>), dim3(nblk(N)), dim3(kWG), 0, s, N, T, x, a, b, d, (R)coef, scal, \
-                                 scal_idx, active, tr, ev, einst, iact)
-  HOC_K_SWITCH(K, {
-    switch (pre) {
-      case PRE_COPY: LT(PRE_COPY); break;
-      case PRE_CHEB0: LT(PRE_CHEB0); break;
-      case PRE_PROL: LT(PRE_PROL); break;
-      case PRE_PUPD: LT(PRE_PUPD); break;
-      default: return hipErrorInvalidValue;
-    }
-  });
-#undef LT
+hipError_t launch_trace(int K, int N, const Tab& T, const double* x, double* tr, hipStream_t s) {
+  HOC_K_SWITCH(K, hipLaunchKernelGGL((k_trace<KK>), dim3(nblk(N)), dim3(kWG), 0, s, N, T, x, tr));
   return hipGetLastError();
-}
-
-template <class R>
-static hipError_t launch_lap_t(int K, int epi, int N, const TabT<R>& T, const GeoT<R>& G, R* x, const R* tr, R* y,
-                               const R* r, const R* diag, R* d, double c1, double c2, double* part, const int* active,
-                               hipStream_t s, R* tr_out, int* ran) {
-#define LL(E)                                                                                                        \
-  do {                                                                                                               \
-    if (G.gel)                                                                                                       \
-      hipLaunchKernelGGL((k_lap<KK, E, true, R>), dim3(nblk(N)), dim3(kWG), 0, s, N, T, G, x, tr, y, r, diag, d,      \
-                         (R)c1, (R)c2, part, active, tr_out, ran);                                                   \
-    else                                                                                                             \
-      hipLaunchKernelGGL((k_lap<KK, E, false, R>), dim3(nblk(N)), dim3(kWG), 0, s, N, T, G, x, tr, y, r, diag, d,     \
-                         (R)c1, (R)c2, part, active, tr_out, ran);                                                   \
-  } while (0)
-  HOC_K_SWITCH(K, {
-    switch (epi) {
-      case EPI_STORE: LL(EPI_STORE); break;
-      case EPI_RESID: LL(EPI_RESID); break;
-      case EPI_CHEB: LL(EPI_CHEB); break;
-      case EPI_CHEBF: LL(EPI_CHEBF); break;
-      case EPI_RESTRICT: LL(EPI_RESTRICT); break;
-      default: return hipErrorInvalidValue;
-    }
-  });
-#undef LL
-  return hipGetLastError();
-}
-
-hipError_t launch_trace(int K, int pre, int N, const TabT<double>& T, double* x, const double* a, const double* b,
-                        double* d, double coef, const double* scal, int scal_idx, const int* active, double* tr,
-                        hipStream_t s, const int32_t* ev, const int32_t* einst, const int* iact) {
-  return launch_trace_t<double>(K, pre, N, T, x, a, b, d, coef, scal, scal_idx, active, tr, s, ev, einst, iact);
-}
-hipError_t launch_trace(int K, int pre, int N, const TabT<float>& T, float* x, const float* a, const float* b,
-                        float* d, double coef, const double* scal, int scal_idx, const int* active, float* tr,
-                        hipStream_t s, const int32_t* ev, const int32_t* einst, const int* iact) {
-  return launch_trace_t<float>(K, pre, N, T, x, a, b, d, coef, scal, scal_idx, active, tr, s, ev, einst, iact);
-}
-hipError_t launch_trace_pupd_f32z(int K, int N, const TabT<double>& T, double* p, const float* z, const double* scal,
-                                  int scal_idx, const int* active, double* tr, hipStream_t s, const int32_t* einst,
-                                  const int* iact) {
-  HOC_K_SWITCH(K, hipLaunchKernelGGL((k_trace<KK, PRE_PUPD, double, float>), dim3(nblk(N)), dim3(kWG), 0, s, N, T, p,
-                                     z, (const double*)nullptr, (double*)nullptr, 0., scal, scal_idx, active, tr,
-                                     (const int32_t*)nullptr, einst, iact));
-  return hipGetLastError();
-}
-hipError_t launch_lap(int K, int epi, int N, const TabT<double>& T, const GeoT<double>& G, double* x, const double* tr,
-                      double* y, const double* r, const double* diag, double* d, double c1, double c2, double* part,
-                      const int* active, hipStream_t s, double* tr_out, int* ran) {
-  return launch_lap_t<double>(K, epi, N, T, G, x, tr, y, r, diag, d, c1, c2, part, active, s, tr_out, ran);
-}
-hipError_t launch_lap(int K, int epi, int N, const TabT<float>& T, const GeoT<float>& G, float* x, const float* tr,
-                      float* y, const float* r, const float* diag, float* d, double c1, double c2, double* part,
-                      const int* active, hipStream_t s, float* tr_out, int* ran) {
-  return launch_lap_t<float>(K, epi, N, T, G, x, tr, y, r, diag, d, c1, c2, part, active, s, tr_out, ran);
 }
 
 hipError_t launch_rhs(int K, int N, const Tab& T, const Geo& G, const double* omega, const double* bcpsi, double* bs,

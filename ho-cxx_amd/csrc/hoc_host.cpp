@@ -200,6 +200,115 @@ void build_tables(int K, int lnod, Tables& t) {
   }
 }
 
+void solve_dense(int n, int m, double* a, double* b) {
+  for (int c = 0; c < n; ++c) {
+    int p = c;
+    for (int r = c + 1; r < n; ++r)
+      if (std::fabs(a[(size_t)r * n + c]) > std::fabs(a[(size_t)p * n + c])) p = r;
+    if (p != c) {
+      for (int j = 0; j < n; ++j) std::swap(a[(size_t)c * n + j], a[(size_t)p * n + j]);
+      for (int j = 0; j < m; ++j) std::swap(b[(size_t)c * m + j], b[(size_t)p * m + j]);
+    }
+    for (int r = 0; r < n; ++r) {
+      if (r == c) continue;
+      const double f = a[(size_t)r * n + c] / a[(size_t)c * n + c];
+      for (int j = c; j < n; ++j) a[(size_t)r * n + j] -= f * a[(size_t)c * n + j];
+      for (int j = 0; j < m; ++j) b[(size_t)r * m + j] -= f * b[(size_t)c * m + j];
+    }
+  }
+  for (int r = 0; r < n; ++r)
+    for (int j = 0; j < m; ++j) b[(size_t)r * m + j] /= a[(size_t)r * n + r];
+}
+
+void fine_tables(const Tables& t, FineTables& f) {
+  const int K = t.K;
+  for (int d = 0; d < K; ++d)
+    for (int k = 0; k < K; ++k) {
+      f.DD[d][k] = 0.;
+      for (int m = 0; m < K; ++m) f.DD[d][k] += t.D[d][m] * t.D[m][k];
+    }
+  f.m0 = f.m1 = 0.;
+  for (int k = 0; k < K; ++k) {
+    f.Dg[k] = 0.;
+    for (int d = 0; d < K; ++d) f.Dg[k] += t.grad[d][0] * t.D[d][k];
+    f.m0 += t.grad[k][0] * t.bb[k][0];
+    f.m1 += t.grad[k][0] * t.bb[k][1];
+  }
+  f.fdm.assign((size_t)9 * (K + K * K), 0.);
+  for (int code = 0; code < 9; ++code) {
+    const int kind[2] = {code / 3, code % 3};
+    // X[i][c]: -w_i times the line operator's response at point i to a unit value at point c of
+    // the same element, the neighbours zero
+    std::vector<double> X((size_t)K * K);
+    for (int c = 0; c < K; ++c) {
+      double dv[2], fl[2];  // common minus own value and common flux at the two ends
+      for (int b = 0; b < 2; ++b) {
+        const double v = t.bb[c][b], g = t.bgb[c][b], gp = t.gprime[b];
+        if (kind[b] == 0) {
+          dv[b] = -0.5 * v;
+          fl[b] = 0.5 * (g + dv[b] * gp) + 0.25 * v * t.gprime[1 - b];
+        } else if (kind[b] == 1) {
+          dv[b] = -v;
+          fl[b] = g - v * gp;
+        } else {
+          dv[b] = -g / gp;
+          fl[b] = 0.;
+        }
+      }
+      std::vector<double> gr(K);
+      for (int k = 0; k < K; ++k) gr[k] = t.D[c][k] + dv[0] * t.grad[k][0] + dv[1] * t.grad[k][1];
+      for (int b = 0; b < 2; ++b)
+        for (int k = 0; k < K; ++k) fl[b] -= gr[k] * t.bb[k][b];
+      for (int i = 0; i < K; ++i) {
+        double s = fl[0] * t.grad[i][0] + fl[1] * t.grad[i][1];
+        for (int k = 0; k < K; ++k) s += gr[k] * t.D[k][i];
+        X[(size_t)i * K + c] = -t.wgt[i] * s;
+      }
+    }
+    // cyclic Jacobi on W^-1/2 X W^-1/2
+    std::vector<double> A((size_t)K * K), V((size_t)K * K, 0.);
+    for (int i = 0; i < K; ++i) {
+      V[(size_t)i * K + i] = 1.;
+      for (int j = 0; j < K; ++j)
+        A[(size_t)i * K + j] = 0.5 * (X[(size_t)i * K + j] + X[(size_t)j * K + i]) / std::sqrt(t.wgt[i] * t.wgt[j]);
+    }
+    for (int sweep = 0; sweep < 60; ++sweep) {
+      double off = 0., dia = 0.;
+      for (int i = 0; i < K; ++i)
+        for (int j = 0; j < K; ++j) (i == j ? dia : off) += A[(size_t)i * K + j] * A[(size_t)i * K + j];
+      if (off <= 1e-34 * dia) break;
+      for (int p = 0; p < K; ++p)
+        for (int q = p + 1; q < K; ++q) {
+          const double apq = A[(size_t)p * K + q];
+          if (apq == 0.) continue;
+          const double th = (A[(size_t)q * K + q] - A[(size_t)p * K + p]) / (2. * apq);
+          const double tt = (th >= 0. ? 1. : -1.) / (std::fabs(th) + std::sqrt(th * th + 1.));
+          const double cs = 1. / std::sqrt(tt * tt + 1.), sn = tt * cs;
+          for (int k = 0; k < K; ++k) {
+            const double x = A[(size_t)k * K + p], y = A[(size_t)k * K + q];
+            A[(size_t)k * K + p] = cs * x - sn * y;
+            A[(size_t)k * K + q] = sn * x + cs * y;
+          }
+          for (int k = 0; k < K; ++k) {
+            const double x = A[(size_t)p * K + k], y = A[(size_t)q * K + k];
+            A[(size_t)p * K + k] = cs * x - sn * y;
+            A[(size_t)q * K + k] = sn * x + cs * y;
+          }
+          for (int k = 0; k < K; ++k) {
+            const double x = V[(size_t)k * K + p], y = V[(size_t)k * K + q];
+            V[(size_t)k * K + p] = cs * x - sn * y;
+            V[(size_t)k * K + q] = sn * x + cs * y;
+          }
+        }
+    }
+    double* o = &f.fdm[(size_t)code * (K + K * K)];
+    for (int i = 0; i < K; ++i) {
+      o[i] = A[(size_t)i * K + i];
+      for (int j = 0; j < K; ++j) o[K + j * K + i] = V[(size_t)j * K + i] / std::sqrt(t.wgt[j]);
+    }
+  }
+}
+
 namespace {
 // Gmsh quad node slot of tensor position (i along xi, j along eta) (src/Mesh.cpp:34-91).
 int t2g(int L, int i, int j) {

@@ -92,6 +92,19 @@ void write_vtk_nodes(const std::string& path, const Mesh& m, const double* nodes
 void write_samples(const std::string& path, int n, const double* xy, const double* vals);
 
 
+// Tables of the fine-level Poisson kernels: the second-derivative matrix DD[d][k] = sum_m D[d][m]
+// D[m][k], Dg = the derivative of the lower Radau correction's derivative g' at the points, m0 and
+// m1 = g' extrapolated to -1 and +1, and per pair of end kinds (lower * 3 + upper; 0 interior, 1
+// Dirichlet, 2 Neumann) the generalised eigenpairs X S = W S lam, S^T W S = 1 of the line
+// operator's own block X (the neighbours' metric taken equal): lam [K], then S [K][K].
+struct FineTables {
+  double DD[kMaxK][kMaxK], Dg[kMaxK], m0 = 0., m1 = 0.;
+  std::vector<double> fdm;  // [9][K + K K]
+};
+void fine_tables(const Tables& t, FineTables& f);
+// A X = B by Gauss elimination with partial pivoting (A n x n, B n x m, row-major); X replaces B.
+void solve_dense(int n, int m, double* a, double* b);
+
 struct Geometry {
   // volume, [el][j][i]
   std::vector<double> xxi, xeta, yxi, yeta, jac;

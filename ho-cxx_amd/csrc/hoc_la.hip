@@ -30,18 +30,14 @@ __device__ __forceinline__ void block_sum2(double& a, double& b) {
 // inverse weight 1/(w_j w_i) of that position is A.winv[m].
 struct DofSlot {
   int m, step, K2;
-  size_t el, estep;  // the element of the dof
   __device__ DofSlot(const VecArgs& A, size_t v0, size_t stride) {
     K2 = A.K * A.K;
     m = (int)(v0 % (size_t)K2);
     step = (int)(stride % (size_t)K2);
-    el = v0 / (size_t)K2;
-    estep = stride / (size_t)K2;
   }
   __device__ void next() {
     m += step;
-    el += estep;
-    if (m >= K2) { m -= K2; ++el; }
+    if (m >= K2) m -= K2;
   }
 };
 
@@ -57,15 +53,6 @@ __global__ void k_vec(int op, VecArgs A, size_t n, R* __restrict__ a, R* __restr
   DofSlot ds(A, v0, stride);
   for (size_t v = v0; v < n; v += stride, ds.next()) {
     switch (op) {
-      case VOP_PCG_UPD: {  // x += alpha p; r -= alpha q      a=x b=r c=p d=q
-        if (A.ialpha && A.ialpha[A.einst[ds.el]] == 0.) break;  // a stopped ensemble instance
-        const R al = (R)(A.ialpha ? A.ialpha[A.einst[ds.el]] : S[S_ALPHA]);
-        a[v] += al * c[v];
-        const R r = b[v] - al * d[v];
-        b[v] = r;
-        const double ru = r * A.winv[ds.m];
-        p0 += (double)r * r; p1 += ru * ru;
-      } break;
       case VOP_BICG_P: {   // p = r + beta (p - omega v)      a=p c=r d=v
         a[v] = c[v] + (R)S[S_BETA] * (a[v] - (R)S[S_OMEGA] * d[v]);
       } break;
@@ -323,15 +310,6 @@ __global__ void k_dense(int n, const R* __restrict__ Ainv, const R* __restrict__
   if (lane == 0) x[row] = s;
 }
 
-// y = -y / (w_j w_i) at every solution point (el K^2 + j K + i): As = -W A turned back into A.
-struct Weights6 { double w[6]; };
-__global__ void k_unweight(size_t n, int K, Weights6 W, double* __restrict__ y) {
-  const size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const int m = (int)(v % (size_t)(K * K));
-  y[v] = -y[v] / (W.w[m / K] * W.w[m % K]);
-}
-
 // ---- probing ---------------------------------------------------------------------------------
 // x[el][m] = (color[el] == c && (m == rs || rs < 0)) ? 1 : 0
 __global__ void k_probe_set(int N, int K2, const int32_t* __restrict__ color, int c, int rs, double* __restrict__ x) {
@@ -376,14 +354,8 @@ __global__ void k_q1_probe_accum(int N, int K, Tab T, int rs, const double* __re
 }
 
 // ---- mixed precision ---------------------------------------------------------------------------
-// FP64 Krylov method with the FP32 V-cycle as its preconditioner: the V-cycle's input
-// r32 = (float) r64, and its output z64 = (double) z32 with partials of r64 . z64 (slot 0; slot 1
-// zero) when part is set.
-__global__ void k_demote(size_t n, const double* __restrict__ r64, float* __restrict__ r32, const int* __restrict__ F) {
-  if (F && !F[F_ACTIVE]) return;
-  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x)
-    r32[v] = (float)r64[v];
-}
+// FP64 Krylov method with the FP32 V-cycle as its preconditioner: the V-cycle's output
+// z64 = (double) z32 with partials of r64 . z64 (slot 0; slot 1 zero) when part is set.
 __global__ void k_promote_dot(size_t n, const float* __restrict__ z32, double* __restrict__ z64,
                               const double* __restrict__ r64, double* __restrict__ part, const int* __restrict__ F) {
   if (F && !F[F_ACTIVE]) return;
@@ -1136,20 +1108,12 @@ template <class R>
 void q1_gather(hipStream_t s, int nv, const int32_t* vptr, const int32_t* vinc, const R* ec, R* rc, const int* F) {
   hipLaunchKernelGGL(k_q1_gather<R>, dim3((nv + 255) / 256), dim3(256), 0, s, nv, vptr, vinc, ec, rc, F);
 }
-void demote(hipStream_t s, size_t n, const double* r64, float* r32, const int* F) {
-  hipLaunchKernelGGL(k_demote, dim3(vec_grid(n)), dim3(256), 0, s, n, r64, r32, F);
-}
 void promote_dot(hipStream_t s, size_t n, const float* z32, double* z64, const double* r64, double* part,
                  const int* F) {
   hipLaunchKernelGGL(k_promote_dot, dim3(vec_grid(n)), dim3(256), 0, s, n, z32, z64, r64, part, F);
 }
 void inst_norms(hipStream_t s, const VecArgs& A, int n_inst, const int32_t* off, int K2, const double* b, double* out) {
   hipLaunchKernelGGL(k_inst_norms, dim3(n_inst), dim3(256), 0, s, A, off, K2, b, out);
-}
-void unweight(hipStream_t s, size_t n, int K, const double* w, double* y) {
-  Weights6 W{};
-  for (int i = 0; i < K && i < 6; ++i) W.w[i] = w[i];
-  if (n) hipLaunchKernelGGL(k_unweight, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, K, W, y);
 }
 void probe_set(hipStream_t s, int N, int K2, const int32_t* color, int c, int rs, double* x) {
   size_t n = (size_t)N * K2;

@@ -18,17 +18,13 @@ namespace hoc {
 enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_COUNT = 16 };
 enum { F_ACTIVE = 0, F_ITER, F_ZERO, F_HALF, F_MAXIT, F_SEQ, F_COUNT = 8 };
 enum { PH_BB = 0, PH_INIT, PH_RZ, PH_PQ, PH_UPD, PH_RHO, PH_ALPHA, PH_SNORM, PH_OMEGA, PH_RNORM };
-enum { VOP_PCG_UPD = 0, VOP_BICG_P, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
+enum { VOP_BICG_P = 0, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
 
 // K: points per direction of an element (1 for a plain vector); winv: device table of the
 // K*K inverse quadrature weights 1/(w_j w_i), indexed j K + i.
 struct VecArgs {
   int K;
   const double* winv;
-  // ensembles with a step length per instance: VOP_PCG_UPD takes alpha = ialpha[einst[element]]
-  // and skips the dofs of an instance whose alpha is 0 (stopped)
-  const double* ialpha = nullptr;
-  const int32_t* einst = nullptr;
 };
 
 int vec_grid(size_t n);
@@ -66,9 +62,8 @@ void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F);
 template <class R>
 void q1_gather(hipStream_t s, int nv, const int32_t* vptr, const int32_t* vinc, const R* ec, R* rc, const int* F);
 
-// The FP32 V-cycle inside the FP64 Krylov method: r32 = (float) r64; z64 = (double) z32 with
-// partials of r64 . z64 in part (vec_grid(n) blocks; may be null).
-void demote(hipStream_t s, size_t n, const double* r64, float* r32, const int* F);
+// The FP32 V-cycle inside the FP64 Krylov method: z64 = (double) z32 with partials of r64 . z64 in
+// part (vec_grid(n) blocks; may be null).
 void promote_dot(hipStream_t s, size_t n, const float* z32, double* z64, const double* r64, double* part,
                  const int* F);
 
@@ -174,9 +169,6 @@ void psi_combine(hipStream_t s, size_t n, int nterm, const double* a, const doub
 // Ensembles: out[i] = ||b_i / W||^2 over instance i's elements [off[i], off[i+1]) (K2 values
 // per element), one workgroup per instance (deterministic order).
 void inst_norms(hipStream_t s, const VecArgs& A, int n_inst, const int32_t* off, int K2, const double* b, double* out);
-
-// y = -y / (w[j] w[i]) at every solution point (v = el K^2 + j K + i); w: K host values (K <= 6).
-void unweight(hipStream_t s, size_t n, int K, const double* w, double* y);
 
 // Setup-time probing (FP64).
 void probe_set(hipStream_t s, int N, int K2, const int32_t* color, int c, int rs, double* x);

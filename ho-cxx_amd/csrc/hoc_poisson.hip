@@ -1,0 +1,717 @@
+// hoc_poisson.hip - the fine-level Poisson operator and smoother for gfx950.
+//
+// The operator is the second-order FR operator of src/HO_2D.cpp:1533-1804 (the diffusion term of
+// :2666-2831 with zero boundary values), applied matrix-free.
+//
+// Mapping: K lanes per element, fine_epw(K) elements per wavefront.  Lane k of an element works on
+// its row k (the xi line) and its column k (the eta line); rows become columns through a tile in
+// LDS that only its own wavefront touches, so no barrier separates the two halves.  On each of the
+// four faces lane k owns face point k, whose neighbour data is one line of the neighbour element
+// (value and inward derivative at the shared face), read straight from the field.  That read
+// comes from the L2 (the neighbour's line is in use by a nearby wavefront), where face traces
+// stored by the kernel before cost 640 bytes of HBM traffic per element and application against
+// the field's own 200 (K = 5, FP64); it also frees each application from a trace kernel.
+//
+// The smoother is the block Jacobi of the elements' own diagonal blocks, B, used as a damped
+// Richardson step; a V-cycle takes degree-d Chebyshev polynomials in B As as d such steps with the
+// roots as dampings.  A block of constant orthogonal metrics is W (x) a X + c Y (x) W with the
+// one-dimensional line operators X, Y, so B = (S (x) S) (a lam_i + c lam_j)^-1 (S (x) S)^T with
+// the generalised eigenvectors S of (X, W): 4 K^3 operations and no stored inverse (fast
+// diagonalisation, R. E. Lynch, J. R. Rice and D. H. Thomas, Numer. Math. 6 (1964) 185-199).  S
+// depends on what the two ends of the line are (interior, Dirichlet, Neumann: 9 tables); elsewhere
+// a and c are the element's mean metrics.
+#include "hoc_poisson.hpp"
+
+namespace hoc {
+
+namespace {
+
+// Blocks are dealt to the 8 XCDs in turn: block b works on part b % 8 of the elements, so the
+// elements an XCD works on at one time are neighbours and share its L2.
+__device__ __forceinline__ int xcd_block(int b, int nb) {
+  const int q = nb >> 3, r = nb & 7, x = b & 7, i = b >> 3;
+  return x * q + min(x, r) + i;
+}
+
+// Orders this wavefront's LDS writes before its reads (LDS serves one wavefront in order).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+template <int K>
+struct Lay {
+  static constexpr int EPW = fine_epw(K);
+  static constexpr int RS = (K & 1) ? K : K + 1;  // row stride in LDS (odd: rows on distinct banks)
+  static constexpr int ES = K * RS;
+  static constexpr int TILE = EPW * ES;
+};
+
+// Two values at any address aligned to one of them (one 16- or 8-byte load).
+template <class R> struct Two;
+template <> struct Two<double> { typedef double t __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct Two<float> { typedef float t __attribute__((ext_vector_type(2), aligned(4))); };
+
+template <int K, class V, class R>
+__device__ __forceinline__ void load_row(const V* __restrict__ g, R (&v)[K]) {
+#pragma unroll
+  for (int i = 0; i + 1 < K; i += 2) {
+    const typename Two<V>::t t = *reinterpret_cast<const typename Two<V>::t*>(g + i);
+    v[i] = (R)t.x;
+    v[i + 1] = (R)t.y;
+  }
+  if (K & 1) v[K - 1] = (R)g[K - 1];
+}
+template <int K, class V, class R>
+__device__ __forceinline__ void store_row(V* __restrict__ g, const R (&v)[K]) {
+#pragma unroll
+  for (int i = 0; i + 1 < K; i += 2) {
+    typename Two<V>::t t;
+    t.x = (V)v[i];
+    t.y = (V)v[i + 1];
+    *reinterpret_cast<typename Two<V>::t*>(g + i) = t;
+  }
+  if (K & 1) g[K - 1] = (V)v[K - 1];
+}
+
+// rows -> columns (and columns -> rows) of the wavefront's elements through its LDS tile
+template <int K, class R>
+__device__ __forceinline__ void rows_to_cols(R* t, int k, const R (&row)[K], R (&col)[K]) {
+  constexpr int RS = Lay<K>::RS;
+  wave_fence();
+#pragma unroll
+  for (int i = 0; i < K; ++i) t[k * RS + i] = row[i];
+  wave_fence();
+#pragma unroll
+  for (int j = 0; j < K; ++j) col[j] = t[j * RS + k];
+}
+template <int K, class R>
+__device__ __forceinline__ void cols_to_rows(R* t, int k, const R (&col)[K], R (&row)[K]) {
+  constexpr int RS = Lay<K>::RS;
+  wave_fence();
+#pragma unroll
+  for (int j = 0; j < K; ++j) t[j * RS + k] = col[j];
+  wave_fence();
+#pragma unroll
+  for (int i = 0; i < K; ++i) row[i] = t[k * RS + i];
+}
+
+template <int K, class R>
+__device__ __forceinline__ R pick(const R (&a)[6], int k) {
+  R v = a[0];
+#pragma unroll
+  for (int i = 1; i < K; ++i) v = k == i ? a[i] : v;
+  return v;
+}
+
+// One face point of a lane: the neighbour line's value v and inward derivative g at the shared
+// face; own and neighbour weights of the common flux (1/2, 1/2 inside; 1, 0 Dirichlet; 0, 0
+// Neumann), and what the common value minus the own value is.
+template <class R>
+struct Face {
+  R v = 0, g = 0;   // neighbour trace
+  R an = 0;         // neighbour's normal metric
+  int nb = -1;      // neighbour, or -1 - edge
+  int fn = 0;       // its face
+  int kk = 0;       // its point on that face
+  bool neu = false;
+};
+
+// The neighbour's point on its face fn that meets this element's point k of face f.
+template <int K>
+__device__ __forceinline__ int face_point(int f, int fn, int k) {
+  return ((f + fn - f / 2 - fn / 2 + 1) & 1) ? K - 1 - k : k;
+}
+
+// As u on the lane's row (without the weights -w_k w_i).  u: rows; uc: columns.
+template <int K, int GEO, class R>
+struct Op {
+  // One line of an element with constant orthogonal metrics: out = (a u'' + corrections) with the
+  // two faces L (lower) and U (upper).
+  static __device__ __forceinline__ void line(const FineTab<R>& T, R a, const R (&u)[K], const Face<R>& L,
+                                              const Face<R>& U, R (&out)[K]) {
+    R bl = 0, gl = 0, bu = 0, gu = 0;
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+      bl += u[m] * T.lv[m];
+      gl += u[m] * T.ld[m];
+      bu += u[K - 1 - m] * T.lv[m];
+      gu += u[K - 1 - m] * T.ld[m];
+    }
+    // common value minus own, and the common flux along the line
+    const R ig = R(1) / T.g0;
+    const R dl = L.nb >= 0 ? R(0.5) * (L.v - bl) : (L.neu ? gl * ig : -bl);
+    const R du = U.nb >= 0 ? R(0.5) * (U.v - bu) : (U.neu ? gu * ig : -bu);
+    R fl = (gl - dl * T.g0) * a, fu = -(gu - du * T.g0) * a;
+    if (L.nb >= 0) fl = R(0.5) * (fl - (L.g + dl * T.g0) * L.an);
+    if (U.nb >= 0) fu = R(0.5) * (fu + (U.g + du * T.g0) * U.an);
+    if (L.nb < 0 && L.neu) fl = 0;
+    if (U.nb < 0 && U.neu) fu = 0;
+    fl -= a * (gl + dl * T.m0 - du * T.m1);
+    fu -= a * (dl * T.m1 - gu - du * T.m0);
+    const R adl = a * dl, adu = a * du;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      R s = 0;
+#pragma unroll
+      for (int d = 0; d < K; ++d) s += u[d] * T.DD[d][i];
+      out[i] = a * s + (adl * T.Dg[i] + adu * T.Dg[K - 1 - i]) + (fl * T.gd[i] - fu * T.gd[K - 1 - i]);
+    }
+  }
+
+  static __device__ __forceinline__ void apply(const FineTab<R>& T, const FineGeo<R>& G, int el, int k, R* t, R* tf,
+                                               const R (&u)[K], const R (&uc)[K], const Face<R> (&F)[4],
+                                               R (&out)[K]) {
+    if constexpr (GEO == GEO_ORTHO) {
+      const R a = G.ac[(size_t)el * 2], c = G.ac[(size_t)el * 2 + 1];
+      R oc[K], orw[K];
+      line(T, c, uc, F[2], F[3], oc);
+      line(T, a, u, F[0], F[1], out);
+      cols_to_rows<K>(t, k, oc, orw);
+#pragma unroll
+      for (int i = 0; i < K; ++i) out[i] += orw[i];
+      return;
+    } else {
+      // common values: interior average, 0 on Dirichlet faces; Neumann faces from the K x K system
+      // (src/HO_2D.cpp:2872-2927) solved at setup
+      const R ig = R(1) / T.g0;
+      R bv[4], gi[4], cv[4], cg[4];
+      for (int f = 0; f < 4; ++f) { bv[f] = 0; gi[f] = 0; }
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        bv[0] += u[m] * T.lv[m];
+        gi[0] += u[m] * T.ld[m];
+        bv[1] += u[K - 1 - m] * T.lv[m];
+        gi[1] += u[K - 1 - m] * T.ld[m];
+        bv[2] += uc[m] * T.lv[m];
+        gi[2] += uc[m] * T.ld[m];
+        bv[3] += uc[K - 1 - m] * T.lv[m];
+        gi[3] += uc[K - 1 - m] * T.ld[m];
+      }
+      wave_fence();
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        cv[f] = F[f].nb >= 0 ? R(0.5) * (bv[f] + F[f].v) : R(0);
+        tf[f * K + k] = F[f].nb < 0 && F[f].neu ? bv[f] + gi[f] * ig : cv[f];
+      }
+      wave_fence();
+      R Dk[K];  // column k of the derivative matrix
+#pragma unroll
+      for (int d = 0; d < K; ++d) {
+        R v = T.D[d][0];
+#pragma unroll
+        for (int i = 1; i < K; ++i) v = k == i ? T.D[d][i] : v;
+        Dk[d] = v;
+      }
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const R so = (f & 1) ? R(1) : R(-1);
+        if (F[f].nb < 0 && F[f].neu) {
+          const R* q = G.qn + ((size_t)(-1 - F[f].nb) * K + k) * K;
+          R s = 0;
+#pragma unroll
+          for (int m = 0; m < K; ++m) s += q[m] * tf[f * K + m];
+          cv[f] = s;
+          cg[f] = 0;
+          continue;
+        }
+        R cr = 0;
+#pragma unroll
+        for (int d = 0; d < K; ++d) cr += tf[f * K + d] * Dk[d];
+        R fa, fb;
+        if (GEO == GEO_AFFINE) {
+          fa = G.gface[((size_t)el * 4 + f) * 2];
+          fb = G.gface[((size_t)el * 4 + f) * 2 + 1];
+        } else {
+          fa = G.fa[((size_t)el * 4 + f) * K + k];
+          fb = G.fb[((size_t)el * 4 + f) * K + k];
+        }
+        const R own = -so * (gi[f] - (cv[f] - bv[f]) * T.g0) * fa;
+        if (F[f].nb < 0) {
+          cg[f] = own;  // zero common value: no tangential part
+        } else {
+          const int fn = F[f].fn;
+          R fan = F[f].an, fbn;
+          if (GEO == GEO_AFFINE) fbn = G.gface[((size_t)F[f].nb * 4 + fn) * 2 + 1];
+          else fbn = G.fb[((size_t)F[f].nb * 4 + fn) * K + F[f].kk];
+          const bool rev = (f + fn - f / 2 - fn / 2 + 1) & 1;
+          const R sg = (((f + fn) & 1) ? R(1) : R(-1)) * (rev ? R(-1) : R(1));
+          cg[f] = R(0.5) * (own + so * (F[f].g - (cv[f] - F[f].v) * T.g0) * fan - cr * (fb + sg * fbn));
+        }
+      }
+      // corrected contravariant gradient, its corrected divergence (src/HO_2D.cpp:2771-2816)
+      R dx[K], de[K], der[K];
+      const R d0 = cv[0] - bv[0], d1 = cv[1] - bv[1], d2 = cv[2] - bv[2], d3 = cv[3] - bv[3];
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        R s = 0, s2 = 0;
+#pragma unroll
+        for (int d = 0; d < K; ++d) {
+          s += u[d] * T.D[d][i];
+          s2 += uc[d] * T.D[d][i];
+        }
+        dx[i] = s + d0 * T.gd[i] - d1 * T.gd[K - 1 - i];
+        de[i] = s2 + d2 * T.gd[i] - d3 * T.gd[K - 1 - i];
+      }
+      cols_to_rows<K>(t, k, de, der);
+      R ft[K], gt[K], gtc[K];
+      if (GEO == GEO_AFFINE) {
+        const R a = G.gel[(size_t)el * 3], b = G.gel[(size_t)el * 3 + 1], c = G.gel[(size_t)el * 3 + 2];
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          ft[i] = dx[i] * a - der[i] * b;
+          gt[i] = der[i] * c - dx[i] * b;
+        }
+      } else {
+        R ga[K], gb[K], gc[K];
+        const size_t q = ((size_t)el * K + k) * K;
+        load_row<K>(G.Ga + q, ga);
+        load_row<K>(G.Gb + q, gb);
+        load_row<K>(G.Gc + q, gc);
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          ft[i] = dx[i] * ga[i] - der[i] * gb[i];
+          gt[i] = der[i] * gc[i] - dx[i] * gb[i];
+        }
+      }
+      rows_to_cols<K>(t, k, gt, gtc);
+      R c0 = cg[0], c1 = cg[1], c2 = cg[2], c3 = cg[3];
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        c0 -= ft[m] * T.lv[m];
+        c1 -= ft[K - 1 - m] * T.lv[m];
+        c2 -= gtc[m] * T.lv[m];
+        c3 -= gtc[K - 1 - m] * T.lv[m];
+      }
+      R oc[K], orw[K];
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        R s = 0, s2 = 0;
+#pragma unroll
+        for (int d = 0; d < K; ++d) {
+          s += ft[d] * T.D[d][i];
+          s2 += gtc[d] * T.D[d][i];
+        }
+        out[i] = s + c0 * T.gd[i] - c1 * T.gd[K - 1 - i];
+        oc[i] = s2 + c2 * T.gd[i] - c3 * T.gd[K - 1 - i];
+      }
+      cols_to_rows<K>(t, k, oc, orw);
+#pragma unroll
+      for (int i = 0; i < K; ++i) out[i] += orw[i];
+    }
+  }
+};
+
+// r <- B r (rows): the element blocks' inverse by fast diagonalisation.
+template <int K, class R>
+__device__ __forceinline__ void block_inverse(const FineTab<R>& T, const FineGeo<R>& G, int el, int k, R* t, R (&r)[K]) {
+  const R a = G.ac[(size_t)el * 2], c = G.ac[(size_t)el * 2 + 1];
+  const int ft = G.ftype[el];
+  R s[K], q[K];
+  if (__all(ft == 0)) {  // every element of the wavefront interior: the tables are scalars
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      R v = 0;
+#pragma unroll
+      for (int j = 0; j < K; ++j) v += T.S[j][i] * r[j];
+      s[i] = v;
+    }
+    rows_to_cols<K>(t, k, s, q);
+    const R al = a * pick<K>(T.lam, k);
+#pragma unroll
+    for (int b = 0; b < K; ++b) {
+      R v = 0;
+#pragma unroll
+      for (int j = 0; j < K; ++j) v += T.S[j][b] * q[j];
+      s[b] = v / (al + c * T.lam[b]);
+    }
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      R v = 0;
+#pragma unroll
+      for (int b = 0; b < K; ++b) v += T.S[j][b] * s[b];
+      q[j] = v;
+    }
+    cols_to_rows<K>(t, k, q, s);
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      R v = 0;
+#pragma unroll
+      for (int j = 0; j < K; ++j) v += T.S[i][j] * s[j];
+      r[i] = v;
+    }
+    return;
+  }
+  const R* fx = G.fdm + (ft & 15) * (K + K * K);
+  const R* fy = G.fdm + (ft >> 4) * (K + K * K);
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    R v = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) v += fx[K + j * K + i] * r[j];
+    s[i] = v;
+  }
+  rows_to_cols<K>(t, k, s, q);
+  const R al = a * fx[k];
+#pragma unroll
+  for (int b = 0; b < K; ++b) {
+    R v = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) v += fy[K + j * K + b] * q[j];
+    s[b] = v / (al + c * fy[b]);
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    R v = 0;
+#pragma unroll
+    for (int b = 0; b < K; ++b) v += fy[K + j * K + b] * s[b];
+    q[j] = v;
+  }
+  cols_to_rows<K>(t, k, q, s);
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    R v = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) v += fx[K + i * K + j] * s[j];
+    r[i] = v;
+  }
+}
+
+// Block sums of two per-lane values; thread 0 writes them to part[blk] and part[nblk + blk].
+__device__ __forceinline__ void block_part(double a, double b, double* __restrict__ part, int blk, int nblk) {
+  __shared__ double sa[kFineThreads / 64], sb[kFineThreads / 64];
+  a = wave_sum(a);
+  b = wave_sum(b);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { sa[w] = a; sb[w] = b; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    part[blk] = sa[0] + sa[1] + sa[2] + sa[3];
+    part[nblk + blk] = sb[0] + sb[1] + sb[2] + sb[3];
+  }
+}
+
+template <int K, int GEO, int IN, int EPI, class R, class RZ>
+__global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> G, FineArgs<R> A) {
+  const bool go = !A.active || *A.active;
+  if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
+  if (!go) return;
+  constexpr int K2 = K * K, EPW = Lay<K>::EPW, ES = Lay<K>::ES;
+  constexpr int FS = GEO == GEO_ORTHO ? 0 : 4 * K;  // face values of one element
+  __shared__ R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
+  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int EPB = EPW * (kFineThreads / 64);
+  if (G.iact) {  // a block inside one stopped ensemble instance
+    const int i0 = G.inst[blk * EPB];
+    if (i0 == G.inst[min((blk + 1) * EPB, G.N) - 1] && !G.iact[i0]) return;
+  }
+  const int le = lane < EPW * K ? lane / K : EPW - 1;
+  const int k = lane < EPW * K ? lane - le * K : K - 1;
+  const int el0 = blk * EPB + wv * EPW + le;
+  const bool live = lane < EPW * K && el0 < G.N;
+  // lanes past the mesh follow its last element in a slot of their own, and the lanes past the last
+  // slot its last row: the same reads, so the same values in LDS; neither writes to memory
+  const int el = min(el0, G.N - 1);
+  R* t = lds + wv * (Lay<K>::TILE + EPW * FS) + le * ES;
+  R* tf = lds + wv * (Lay<K>::TILE + EPW * FS) + Lay<K>::TILE + le * FS;
+  const size_t row = ((size_t)el * K + k) * K;
+
+  // connectivity and every global read of the kernel, issued before the arithmetic
+  const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
+  const int nbf = G.nbf[el];
+  R u[K], z[K], b[K];
+  (void)z;
+  load_row<K>(A.x + row, u);
+  R beta = 0;
+  if constexpr (IN == IN_PUPD) {
+    load_row<K>(static_cast<const RZ*>(A.z) + row, z);
+    beta = (R)(A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]]);
+  }
+  if constexpr (EPI == EPI_RESID || EPI == EPI_SMOOTH || EPI == EPI_RESTRICT) load_row<K>(A.b + row, b);
+  R xo[4] = {0, 0, 0, 0};  // IN_PROL: own vertex values
+  if constexpr (IN == IN_PROL) {
+    const int4 v = *reinterpret_cast<const int4*>(G.ev + (size_t)el * 4);
+    xo[0] = A.xc[v.x]; xo[1] = A.xc[v.y]; xo[2] = A.xc[v.z]; xo[3] = A.xc[v.w];
+  }
+  // the four neighbours' lines through the lane's face points, from the shared face inward: all
+  // loads unconditional (a boundary face reads the element's own line and ignores it), so that
+  // their latencies overlap
+  Face<R> F[4];
+  const int nbs[4] = {nbr.x, nbr.y, nbr.z, nbr.w};
+  R l[4][K], pl[IN == IN_PUPD ? 4 : 1][K], cn[IN == IN_PROL ? 4 : 1][4];
+  (void)pl;
+  (void)cn;
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    const bool in = nbs[f] >= 0;
+    const int nb = in ? nbs[f] : el, fn = in ? (nbf >> (8 * f)) & 3 : f, kk = face_point<K>(f, fn, k), up = fn & 1;
+    const int start = fn < 2 ? kk * K + (up ? K - 1 : 0) : (up ? (K - 1) * K : 0) + kk;
+    const int step = fn < 2 ? (up ? -1 : 1) : (up ? -K : K);
+    const size_t o = (size_t)nb * K2 + start;
+    if constexpr (IN == IN_PUPD) {
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        l[f][m] = (R)(static_cast<const RZ*>(A.z) + o)[m * step];
+        pl[f][m] = (A.x + o)[m * step];
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < K; ++m) l[f][m] = (A.x + o)[m * step];
+    }
+    if constexpr (IN == IN_PROL) {
+      // vertex values at the corners of the shared face (along its parameter) and of the opposite one
+      const int4 vn = *reinterpret_cast<const int4*>(G.ev + (size_t)nb * 4);
+      cn[f][0] = A.xc[fn == 0 || fn == 2 ? vn.x : fn == 1 ? vn.y : vn.w];
+      cn[f][1] = A.xc[fn == 0 ? vn.w : fn == 2 ? vn.y : vn.z];
+      cn[f][2] = A.xc[fn == 0 ? vn.y : fn == 2 ? vn.w : vn.x];
+      cn[f][3] = A.xc[fn == 0 || fn == 2 ? vn.z : fn == 1 ? vn.w : vn.y];
+    }
+    F[f].nb = nbs[f];
+    F[f].fn = fn;
+    F[f].kk = kk;
+    if (GEO == GEO_ORTHO) F[f].an = G.ac[(size_t)nb * 2 + (fn >> 1)];
+    else if (GEO == GEO_AFFINE) F[f].an = G.gface[((size_t)nb * 4 + fn) * 2];
+    else F[f].an = G.fa[((size_t)nb * 4 + fn) * K + kk];
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    if (nbs[f] < 0) F[f].neu = G.sw[-1 - nbs[f]] != 0;
+    R v = 0, g = 0;
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+      if constexpr (IN == IN_PUPD) l[f][m] = beta != R(0) ? l[f][m] + beta * pl[f][m] : l[f][m];
+      v += l[f][m] * T.lv[m];
+      g += l[f][m] * T.ld[m];
+    }
+    if constexpr (IN == IN_PROL) {  // the neighbour's bilinear correction on that line
+      const R sk = R(0.5) * (R(1) + pick<K>(T.x, F[f].kk));
+      const R near = cn[f][0] + sk * (cn[f][1] - cn[f][0]), far = cn[f][2] + sk * (cn[f][3] - cn[f][2]);
+      v += near;
+      g += R(0.5) * (far - near);
+    }
+    F[f].v = v;
+    F[f].g = g;
+  }
+  if constexpr (IN == IN_PUPD) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) u[i] = beta != R(0) ? z[i] + beta * u[i] : z[i];
+    if (live) store_row<K>(A.pn + row, u);
+  }
+  if constexpr (IN == IN_PROL) {
+    const R sy = R(0.5) * (R(1) + pick<K>(T.x, k));
+    const R wl = xo[0] + sy * (xo[3] - xo[0]), wu = xo[1] + sy * (xo[2] - xo[1]);
+#pragma unroll
+    for (int i = 0; i < K; ++i) u[i] += wl + R(0.5) * (R(1) + T.x[i]) * (wu - wl);
+  }
+  R uc[K], out[K];
+  rows_to_cols<K>(t, k, u, uc);
+  Op<K, GEO, R>::apply(T, G, el, k, t, tf, u, uc, F, out);
+  double p0 = 0., p1 = 0.;
+  if constexpr (EPI == EPI_PLAIN) {
+    if (live) store_row<K>(A.y + row, out);
+    return;
+  }
+  const R wk = pick<K>(T.w, k);
+#pragma unroll
+  for (int i = 0; i < K; ++i) out[i] *= -(wk * T.w[i]);
+  if constexpr (EPI == EPI_STORE) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) p0 += (double)u[i] * (double)out[i];
+    if (live) store_row<K>(A.y + row, out);
+  } else {
+    R res[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) res[i] = b[i] - out[i];
+    if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        const double v = res[i], uw = v / ((double)wk * (double)T.w[i]);
+        p0 += v * v;
+        p1 += uw * uw;
+      }
+      if (live) store_row<K>(A.y + row, res);
+    } else if constexpr (EPI == EPI_RESTRICT) {
+      R s0 = 0, s1 = 0;  // the row's share of its west and east ends
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        s0 += R(0.5) * (R(1) - T.x[i]) * res[i];
+        s1 += R(0.5) * (R(1) + T.x[i]) * res[i];
+      }
+      wave_fence();
+      t[2 * k] = s0;
+      t[2 * k + 1] = s1;
+      wave_fence();
+#pragma unroll
+      for (int c = 0; c < (3 + K) / K; ++c) {
+        const int a = k + c * K;
+        if (a < 4) {
+          const int east = a == 1 || a == 2, north = a >= 2;
+          R s = 0;
+#pragma unroll
+          for (int j = 0; j < K; ++j) s += R(0.5) * (north ? R(1) + T.x[j] : R(1) - T.x[j]) * t[2 * j + east];
+          if (live) A.y[(size_t)el * 4 + a] = s;
+        }
+      }
+    } else {  // EPI_SMOOTH
+      block_inverse<K>(T, G, el, k, t, res);
+      const R om = (R)A.omega;
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        u[i] += om * res[i];
+        p0 += (double)b[i] * (double)u[i];
+      }
+      if (live) store_row<K>(A.y + row, u);
+    }
+  }
+  if (A.part) {
+    if (!live) p0 = p1 = 0.;
+    block_part(p0, p1, A.part, blk, gridDim.x);
+  }
+}
+
+template <int K, bool UPD, class R>
+__global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G, PreArgs<R> A) {
+  if (A.active && !*A.active) return;
+  constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES, EPB = EPW * (kFineThreads / 64);
+  __shared__ R lds[(kFineThreads / 64) * Lay<K>::TILE];
+  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (G.iact) {
+    const int i0 = G.inst[blk * EPB];
+    if (i0 == G.inst[min((blk + 1) * EPB, G.N) - 1] && !G.iact[i0]) return;
+  }
+  const int le = lane < EPW * K ? lane / K : EPW - 1;
+  const int k = lane < EPW * K ? lane - le * K : K - 1;
+  const int el0 = blk * EPB + wv * EPW + le;
+  const bool live = lane < EPW * K && el0 < G.N;
+  const int el = min(el0, G.N - 1);
+  R* t = lds + wv * Lay<K>::TILE + le * ES;
+  const size_t row = ((size_t)el * K + k) * K;
+  double r[K];
+  load_row<K>(A.r + row, r);
+  double p0 = 0., p1 = 0.;
+  if constexpr (UPD) {
+    double x[K], p[K], q[K];
+    load_row<K>(A.q + row, q);
+    load_row<K>(A.p + row, p);
+    load_row<K>(A.x + row, x);
+    const double al = A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]];
+    if (al != 0.) {
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        x[i] += al * p[i];
+        r[i] -= al * q[i];
+      }
+      if (live) {
+        store_row<K>(A.x + row, x);
+        store_row<K>(A.r + row, r);
+      }
+    }
+    const double wk = pick<K>(A.iw, k);
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const double uw = r[i] * (wk * A.iw[i]);
+      p0 += r[i] * r[i];
+      p1 += uw * uw;
+    }
+  }
+  R v[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) v[i] = (R)r[i];
+  if constexpr (sizeof(R) == 4) {
+    if (live) store_row<K>(A.r32 + row, v);
+  }
+  block_inverse<K>(T, G, el, k, t, v);
+  const R om = (R)A.omega;
+#pragma unroll
+  for (int i = 0; i < K; ++i) v[i] *= om;
+  if (live) store_row<K>(A.z + row, v);
+  if (UPD && A.part) {
+    if (!live) p0 = p1 = 0.;
+    block_part(p0, p1, A.part, blk, gridDim.x);
+  }
+}
+
+}  // namespace
+
+#define HOC_K_SWITCH(KV, ...)                      \
+  switch (KV) {                                    \
+    case 2: { constexpr int KK = 2; __VA_ARGS__; } break; \
+    case 3: { constexpr int KK = 3; __VA_ARGS__; } break; \
+    case 4: { constexpr int KK = 4; __VA_ARGS__; } break; \
+    case 5: { constexpr int KK = 5; __VA_ARGS__; } break; \
+    case 6: { constexpr int KK = 6; __VA_ARGS__; } break; \
+    default: return hipErrorInvalidValue;          \
+  }
+#define HOC_GEO_SWITCH(GV, ...)                             \
+  switch (GV) {                                             \
+    case GEO_ORTHO: { constexpr int GG = GEO_ORTHO; __VA_ARGS__; } break;   \
+    case GEO_AFFINE: { constexpr int GG = GEO_AFFINE; __VA_ARGS__; } break; \
+    case GEO_POINT: { constexpr int GG = GEO_POINT; __VA_ARGS__; } break;   \
+    default: return hipErrorInvalidValue;                   \
+  }
+
+template <int K, int GEO, int IN, int EPI, class R, class RZ>
+static void go_fine(const FineTab<R>& T, const FineGeo<R>& G, const FineArgs<R>& A, hipStream_t s) {
+  hipLaunchKernelGGL((k_fine<K, GEO, IN, EPI, R, RZ>), dim3(fine_blocks(K, G.N)), dim3(kFineThreads), 0, s, T, G, A);
+}
+
+template <int K, int GEO, class R>
+static hipError_t fine_kg(int in, int epi, const FineTab<R>& T, const FineGeo<R>& G, const FineArgs<R>& A,
+                          hipStream_t s) {
+  if (in == IN_X && epi == EPI_SMOOTH) go_fine<K, GEO, IN_X, EPI_SMOOTH, R, R>(T, G, A, s);
+  else if (in == IN_PROL && epi == EPI_SMOOTH) go_fine<K, GEO, IN_PROL, EPI_SMOOTH, R, R>(T, G, A, s);
+  else if (in == IN_X && epi == EPI_RESTRICT) go_fine<K, GEO, IN_X, EPI_RESTRICT, R, R>(T, G, A, s);
+  else if constexpr (sizeof(R) == 8) {
+    if (in == IN_X && epi == EPI_STORE) go_fine<K, GEO, IN_X, EPI_STORE, R, R>(T, G, A, s);
+    else if (in == IN_X && epi == EPI_RESID) go_fine<K, GEO, IN_X, EPI_RESID, R, R>(T, G, A, s);
+    else if (in == IN_X && epi == EPI_PLAIN) go_fine<K, GEO, IN_X, EPI_PLAIN, R, R>(T, G, A, s);
+    else if (in == IN_PUPD && epi == EPI_STORE) go_fine<K, GEO, IN_PUPD, EPI_STORE, R, R>(T, G, A, s);
+    else return hipErrorInvalidValue;
+  } else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<double>& T, const FineGeo<double>& G,
+                       const FineArgs<double>& A, hipStream_t s) {
+  HOC_K_SWITCH(K, HOC_GEO_SWITCH(geo, return (fine_kg<KK, GG, double>(in, epi, T, G, A, s))));
+  return hipErrorInvalidValue;
+}
+hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<float>& T, const FineGeo<float>& G,
+                       const FineArgs<float>& A, hipStream_t s) {
+  HOC_K_SWITCH(K, HOC_GEO_SWITCH(geo, return (fine_kg<KK, GG, float>(in, epi, T, G, A, s))));
+  return hipErrorInvalidValue;
+}
+hipError_t launch_fine_pupd_f32z(int K, int geo, const FineTab<double>& T, const FineGeo<double>& G,
+                                 const FineArgs<double>& A, hipStream_t s) {
+  HOC_K_SWITCH(K, HOC_GEO_SWITCH(geo, (go_fine<KK, GG, IN_PUPD, EPI_STORE, double, float>(T, G, A, s))));
+  return hipGetLastError();
+}
+
+template <class R>
+static hipError_t launch_pre_t(int K, const FineTab<R>& T, const FineGeo<R>& G, const PreArgs<R>& A, hipStream_t s) {
+  HOC_K_SWITCH(K, {
+    const dim3 grid(fine_blocks(KK, G.N)), block(kFineThreads);
+    if (A.q) hipLaunchKernelGGL((k_pre<KK, true, R>), grid, block, 0, s, T, G, A);
+    else hipLaunchKernelGGL((k_pre<KK, false, R>), grid, block, 0, s, T, G, A);
+  });
+  return hipGetLastError();
+}
+hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G, const PreArgs<double>& A,
+                      hipStream_t s) {
+  return launch_pre_t<double>(K, T, G, A, s);
+}
+hipError_t launch_pre(int K, const FineTab<float>& T, const FineGeo<float>& G, const PreArgs<float>& A,
+                      hipStream_t s) {
+  return launch_pre_t<float>(K, T, G, A, s);
+}
+
+}  // namespace hoc

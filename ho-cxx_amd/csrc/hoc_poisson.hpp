@@ -1,0 +1,112 @@
+// hoc_poisson.hpp - launchers of the fine-level Poisson kernels (hoc_poisson.hip).
+#pragma once
+
+#include "hoc_kernels.hpp"
+
+namespace hoc {
+
+// What a fine-operator kernel does with As u (As = -W A, W = w_i w_j):
+//   EPI_STORE     y = As u; partial sums of u.y
+//   EPI_RESID     y = b - As u; partial sums of y.y and (y/W).(y/W)
+//   EPI_SMOOTH    y = u + omega B (b - As u); optional partial sums of b.y
+//   EPI_RESTRICT  ec[el][a] = sum_ij q1w(a,ij) (b - As u)_ij      (Pc^T residual, per element)
+//   EPI_PLAIN     y = A u (the operator itself, unscaled)
+enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SMOOTH = 2, EPI_RESTRICT = 3, EPI_PLAIN = 4 };
+// The field u it is applied to:
+//   IN_X     u = x
+//   IN_PROL  u = x + Pc xc (bilinear from the corner vertices)
+//   IN_PUPD  u = z + beta p, written to pn (PCG's direction update)
+enum { IN_X = 0, IN_PROL = 1, IN_PUPD = 2 };
+// The geometry the kernels are instantiated for: elements with constant orthogonal metrics,
+// constant metrics, metrics per point.
+enum { GEO_ORTHO = 0, GEO_AFFINE = 1, GEO_POINT = 2 };
+
+constexpr int kFineThreads = 256;
+// Elements per wavefront: K lanes each, and a multiple of 4 so that a block's elements start on
+// a 16-byte boundary in every field.
+constexpr int fine_epw(int K) { return K == 2 ? 32 : K == 3 ? 20 : K == 4 ? 16 : K == 5 ? 12 : 10; }
+inline int fine_blocks(int K, int N) {
+  const int e = fine_epw(K) * (kFineThreads / 64);
+  return (N + e - 1) / e;
+}
+
+// Static data of the fine level in precision R.
+template <class R>
+struct FineGeo {
+  int N;
+  const R* ac;           // [N][2] mean metrics (g22/J, g11/J) over the element: B's scales, and the
+                         // metrics themselves where they are constant and orthogonal
+  const R* fdm;          // [9] per pair of end kinds: eigenvalues [K], eigenvectors [K][K]
+  const uint16_t* ftype; // [N] kinds of the west/east and south/north ends: 9-way codes tx + 16 ty
+  const R* gel;          // [N][3]    Ga, Gb, Gc of affine elements
+  const R* gface;        // [N][4][2] fa, fb of affine elements
+  const R *Ga, *Gb, *Gc; // [N][K2]
+  const R *fa, *fb;      // [N][4][K]
+  const R* qn;           // [E][K][K] Neumann common values from value + inward derivative / g'
+  const int32_t* nb;     // [N][4] neighbour or -1-edge
+  const int32_t* nbf;    // [N] the four neighbours' faces, one per byte
+  const int8_t* sw;      // [E] 0 Dirichlet / 1 Neumann
+  const int32_t* ev;     // [N][4] corner vertices
+  const int32_t* inst;   // [N] ensemble instance, or null
+  const int* iact;       // [instances] live flags (null: all): blocks of one stopped instance return
+};
+
+// 1-D tables of the fine-level kernels (kernel argument).
+template <class R>
+struct FineTab {
+  R D[6][6];    // l_m'(xi_k)
+  R DD[6][6];   // second-derivative matrix: sum_m D[d][m] D[m][k]
+  R lv[6], ld[6];  // l_m(-1), l_m'(-1) (the upper end by reflection)
+  R gd[6], Dg[6];  // lower Radau correction's derivative and its second derivative at xi_k
+  R m0, m1;     // that derivative extrapolated to -1 and +1
+  R g0;         // -g'(-1), the interface coefficient
+  R w[6], x[6]; // Gauss weights and points
+  R S[6][6], lam[6];  // eigenpairs of the line operator of an interior element
+};
+
+template <class R>
+struct FineArgs {
+  const R* x = nullptr;      // IN_X, IN_PROL: the field; IN_PUPD: p
+  const void* z = nullptr;   // IN_PUPD: z (R, or float for the mixed-precision direction update)
+  R* pn = nullptr;           // IN_PUPD: the new direction
+  const R* xc = nullptr;     // IN_PROL: vertex values
+  const R* b = nullptr;
+  R* y = nullptr;
+  double omega = 0.;
+  const double* scal = nullptr;  // IN_PUPD: beta = scal[scal_idx], scal_idx < 0: scal[inst[el]]
+  int scal_idx = 0;
+  double* part = nullptr;    // [fine_blocks] sums, then [fine_blocks] second sums
+  const int* active = nullptr;
+  int* ran = nullptr;        // set to 1 when the launch worked, 0 when active made it return at once
+};
+
+hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<double>& T, const FineGeo<double>& G,
+                       const FineArgs<double>& A, hipStream_t s);
+hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<float>& T, const FineGeo<float>& G,
+                       const FineArgs<float>& A, hipStream_t s);
+// IN_PUPD + EPI_STORE with z in FP32
+hipError_t launch_fine_pupd_f32z(int K, int geo, const FineTab<double>& T, const FineGeo<double>& G,
+                                 const FineArgs<double>& A, hipStream_t s);
+
+// First smoothing step from zero, z = omega B r, with PCG's vector update in front of it:
+//   q != null: x += alpha p, r -= alpha q first (alpha = scal[scal_idx], or scal[inst[el]] with
+//   scal_idx < 0, where elements of alpha = 0 keep x and r); partial sums of r.r and (r/W).(r/W).
+// FP32 V-cycle: r32 receives r in FP32.
+template <class R>
+struct PreArgs {
+  double *r = nullptr, *x = nullptr;
+  const double *p = nullptr, *q = nullptr;
+  R* z = nullptr;
+  R* r32 = nullptr;
+  double omega = 0.;
+  const double* scal = nullptr;
+  int scal_idx = 0;
+  double* part = nullptr;
+  const int* active = nullptr;
+  double iw[6] = {0., 0., 0., 0., 0., 0.};  // 1 / w_k
+};
+hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G, const PreArgs<double>& A,
+                      hipStream_t s);
+hipError_t launch_pre(int K, const FineTab<float>& T, const FineGeo<float>& G, const PreArgs<float>& A, hipStream_t s);
+
+}  // namespace hoc

@@ -4,7 +4,7 @@
 //   update_BCs(t)            k_update_bcs
 //   solve_Poisson            k_rhs, then PCG or BiCGSTAB on As = -W A (W = Gauss weights
 //                            w_i w_j, which makes As symmetric on affine meshes) with a
-//                            V-cycle: matrix-free fine level + Chebyshev(3) Jacobi
+//                            V-cycle: matrix-free fine level + Chebyshev(2) element-block
 //                            smoothing, continuous bilinear coarse space on the element
 //                            corners (Ac = Pc^T As Pc assembled from probes of As), then
 //                            smoothed aggregation below
@@ -31,59 +31,36 @@
 #include "hoc_host.hpp"
 #include "hoc_la.hpp"
 #include "hoc_out.hpp"
+#include "hoc_poisson.hpp"
 
 namespace hoc {
 
-// ---- scratch of the no-allocation operator apply (hoc_apply_laplacian_device) ---------------
-// The face traces of that entry point live in this library-wide array instead of a buffer of
-// the handle: every GPU the library runs on holds one copy of kNoAllocScratchBytes until the
-// process ends, shared by every handle on that GPU (calls that overlap on one GPU race on it).
-// Host code never passes the array's name to a kernel: it uses the per-device address that
-// noalloc_scratch_init() takes from hipGetSymbolAddress.
-constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
-static __device__ __align__(256) double scratch[kNoAllocScratchBytes / sizeof(double)];
-constexpr int kMaxDevices = 64;
-static std::mutex g_scratch_mu;
-static double* g_scratch_ptr[kMaxDevices] = {nullptr};
+// The largest mesh hoc_apply_laplacian_device takes: face traces (n_elem * 8 * K doubles) of this
+// many bytes, the entry point's documented limit.
+constexpr size_t kNoAllocMaxTraceBytes = size_t(64) << 20;
 
-// Once per device, with that device current: the device address of `scratch`.
-static void noalloc_scratch_init(int dev) {
-  if (dev < 0 || dev >= kMaxDevices) throw StatusError(HOC_EINVAL, "device ordinal out of range");
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (g_scratch_ptr[dev]) return;
-  void* p = nullptr;
-  HIPCHK(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-  if (!p) throw HipError("hipGetSymbolAddress returned a null address for the scratch array");
-  g_scratch_ptr[dev] = static_cast<double*>(p);
-}
-static double* noalloc_scratch(int dev) {
-  if (dev < 0 || dev >= kMaxDevices) return nullptr;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  return g_scratch_ptr[dev];
-}
-
-// Preconditioned-Krylov state in working precision R: the fine operator's tables and
-// metrics, the Krylov and smoother vectors, face traces and the V-cycle hierarchy.
-// FP64 (R = double) serves the plain solve, the outer residual of the mixed solve and
-// setup probing; FP32 (R = float) is the mixed solve's inner Krylov + V-cycle.
+// Fine-level state in working precision R: tables and metrics of the operator and its smoother,
+// the Krylov and smoother vectors, and the V-cycle hierarchy.  FP64 (R = double) serves the Krylov
+// method and setup probing; FP32 (R = float) is the mixed solve's V-cycle.
 template <class R>
 struct Prec {
-  TabT<R> T{};
-  GeoT<R> G{};
-  DBuf<R> Ga, Gb, Gc, fa, fb, fA, fB, fjac, fAn, gel, gface;  // FP32 copies (unused for FP64)
-  // dinv: 1 / diag(As); dch, dch2: Chebyshev directions (ping-pong)
-  DBuf<R> r, z, p, q, rh, v, ph, sh, t, x, dch, dch2, dinv, tr, tr2, ec, rc, xc;
+  FineTab<R> T{};
+  FineGeo<R> G{};
+  DBuf<R> Ga, Gb, Gc, fa, fb, gel, gface;  // FP32 copies (unused for FP64)
+  DBuf<R> ac, fdm, qn;
+  // PCG ping-pongs its direction between p and v; t: the smoother's second iterate
+  DBuf<R> r, z, p, q, rh, v, ph, sh, t, ec, rc, xc;
   std::vector<std::unique_ptr<DevLevel<R>>> lv;  // Q1 vertex level and the SA levels below
   DBuf<R> coarse_inv;
   int coarse_n = 0;
   int prof_off = 0;  // offset of this precision's entries in the live kernel profile
-  // set only while the iterations of a batched ensemble PCG are queued: element -> instance and
-  // the instances' live flags; fine-level blocks of a stopped instance then return at once
-  const int32_t* einst = nullptr;
+  // set only while the iterations of a batched ensemble PCG are queued: the instances' live flags;
+  // fine-level blocks of a stopped instance then return at once
   const int* iact = nullptr;
-  void alloc_vectors(size_t D, int N, int K) {
-    for (auto* f : {&r, &z, &p, &q, &rh, &v, &ph, &sh, &t, &x, &dch, &dch2, &dinv}) f->alloc(D);
-    tr.alloc((size_t)N * 8 * K); tr2.alloc((size_t)N * 8 * K);
+  // vectors of the Krylov method (krylov) and of the V-cycle alone (the FP32 state)
+  void alloc_vectors(size_t D, int N, bool krylov) {
+    for (auto* f : {&r, &z, &t}) f->alloc(D);
+    for (auto* f : {&p, &q, &rh, &v, &ph, &sh}) f->alloc(krylov ? D : 0);
     ec.alloc((size_t)N * 4);
   }
   void upload_levels(const AMGHost& H) {
@@ -155,11 +132,14 @@ struct Solver {
   int nparts = 0;
   int nv = 0;                             // Q1 coarse space: element-corner vertices
   DBuf<int32_t> d_ev, d_vptr, d_vinc;     // element -> 4 vertices; vertex -> (element*4+corner)
-  // Chebyshev smoother of degree cheb_m: step 0 scales by 1/theta, step k >= 1 uses
-  // d = cheb_c1[k] d + cheb_c2[k] D^-1 res
+  // Chebyshev smoother of degree cheb_m in B As (B: the element blocks' inverse) as damped
+  // Richardson steps x += cheb_w[k] B (r - As x)
   int cheb_m = 2;
-  double cheb_theta = 1., cheb_c1[kMaxCheb] = {0}, cheb_c2[kMaxCheb] = {0};
+  double cheb_w[kMaxCheb] = {0};
   double lam_max = 0.;
+  int geo_kind = GEO_POINT;          // what the fine-level kernels are instantiated for
+  DBuf<uint16_t> d_ftype;            // kinds of each element's line ends
+  DBuf<double> d_traces;             // face traces of psi for the velocity kernel
   int krylov = HOC_KRYLOV_BICGSTAB;
   // live kernel timing (hoc_profile_*)
   struct Prof {
@@ -213,7 +193,6 @@ struct Solver {
     HIPCHK(hipSetDevice(device));
     if (!stream) HIPCHK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     clear_graphs();
-    noalloc_scratch_init(device);
     connect(mesh);
     build_tables(cfg.K, mesh.lnod, tab);
     build_geometry(mesh, tab, geo);
@@ -300,6 +279,8 @@ struct Solver {
             d_nb, d_nbf, d_swpsi, d_swdiff, d_noslip, d_esign, nullptr};
     setup_instances();
     setup_hybrid();
+    P64.prof_off = 0;
+    setup_fine(P64, affine, Ga, Gb, Gc, fa, fb, gel, gface);
     const size_t EK = std::max<size_t>((size_t)E * K, 1);
     for (auto* b : {&b_psi, &b_diff, &b_nvel, &b_pvel, &b_vj, &b_vort, &b_adv}) b->alloc(EK);
     auto upl = [&](DBuf<double>& d, const std::vector<double>& h) { if (h.empty()) d.alloc(1); else d.upload(h); };
@@ -311,25 +292,14 @@ struct Solver {
     vel.alloc(2 * D); U.alloc(2 * D);
     trw.alloc((size_t)N * 8 * K); tru.alloc((size_t)N * 4 * K);
     mixed = cfg.precision == HOC_MIXED;
-    P64.T = T; P64.G = G; P64.prof_off = 0;
-    P64.alloc_vectors(D, N, K);
-    if (mixed) {  // FP32 tables and metrics of the inner solve's fine operator
-      Prec<float>& P = P32;
-      static_assert(2 * sizeof(TabT<float>) == sizeof(TabT<double>), "table layout");
-      float* Tf = reinterpret_cast<float*>(&P.T);
-      const double* Td = reinterpret_cast<const double*>(&T);
-      for (size_t i = 0; i < sizeof(T) / sizeof(double); ++i) Tf[i] = (float)Td[i];
-      P.Ga.upload_as(Ga); P.Gb.upload_as(Gb); P.Gc.upload_as(Gc);
-      P.fa.upload_as(fa); P.fb.upload_as(fb); P.fA.upload_as(geo.fA); P.fB.upload_as(geo.fB);
-      P.fjac.upload_as(geo.fjac); P.fAn.upload_as(geo.fAn);
-      if (affine) { P.gel.upload_as(gel); P.gface.upload_as(gface); }
-      P.G = GeoT<float>{N, E, nullptr, nullptr, nullptr, nullptr, nullptr, P.Ga, P.Gb, P.Gc, P.fa, P.fb, P.fA, P.fB,
-                        P.fjac, P.fAn, affine ? P.gel.p : nullptr, affine ? P.gface.p : nullptr, nullptr,
-                        d_nb, d_nbf, d_swpsi, d_swdiff, d_noslip, nullptr, nullptr};
-      P.prof_off = HOC_PROF_VARIANTS / 2;
-      P.alloc_vectors(D, N, K);
+    d_traces.alloc((size_t)N * 8 * K);
+    P64.alloc_vectors(D, N, true);
+    if (mixed) {  // FP32 tables and metrics of the V-cycle's fine operator
+      P32.prof_off = HOC_PROF_VARIANTS / 2;
+      setup_fine(P32, affine, Ga, Gb, Gc, fa, fb, gel, gface);
+      P32.alloc_vectors(D, N, false);
     }
-    nparts = std::max(lap_blocks(N), vec_grid(D));
+    nparts = std::max(std::max(lap_blocks(N), fine_blocks(K, N)), vec_grid(D));
     part.alloc(2 * (size_t)nparts);
     S.alloc(S_COUNT); F.alloc(F_COUNT);
     if (!mirror) {
@@ -356,22 +326,139 @@ struct Solver {
     setup_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
 
+  // Tables, metrics and connectivity of the fine-level kernels in the precision of P.
+  template <class R>
+  void setup_fine(Prec<R>& P, bool affine, const std::vector<double>& Ga, const std::vector<double>& Gb,
+                  const std::vector<double>& Gc, const std::vector<double>& fa, const std::vector<double>& fb,
+                  const std::vector<double>& gel, const std::vector<double>& gface) {
+    FineTables ft;
+    fine_tables(tab, ft);
+    FineTab<R>& F = P.T;
+    F = FineTab<R>{};
+    for (int i = 0; i < K; ++i) {
+      for (int j = 0; j < K; ++j) {
+        F.D[i][j] = (R)tab.D[i][j];
+        F.DD[i][j] = (R)ft.DD[i][j];
+        F.S[i][j] = (R)ft.fdm[K + i * K + j];
+      }
+      F.lam[i] = (R)ft.fdm[i];
+      F.lv[i] = (R)tab.bb[i][0];
+      F.ld[i] = (R)tab.bgb[i][0];
+      F.gd[i] = (R)tab.grad[i][0];
+      F.Dg[i] = (R)ft.Dg[i];
+      F.w[i] = (R)tab.wgt[i];
+      F.x[i] = (R)tab.sps[i];
+    }
+    F.m0 = (R)ft.m0; F.m1 = (R)ft.m1; F.g0 = (R)(-tab.gprime[0]);
+    P.fdm.upload_as(ft.fdm);
+    // orthogonal elements: the off-diagonal metric is rounding noise of the affine test's size
+    bool ortho = affine;
+    for (int e = 0; e < N && ortho; ++e) {
+      const double* g = &gel[(size_t)e * 3];
+      ortho = std::fabs(g[1]) <= 1e-12 * std::max(std::fabs(g[0]), std::fabs(g[2]));
+    }
+    geo_kind = ortho ? GEO_ORTHO : affine ? GEO_AFFINE : GEO_POINT;
+    std::vector<double> ac((size_t)N * 2);
+    for (int e = 0; e < N; ++e) {
+      double a = 0., c = 0.;
+      if (affine) {
+        a = gel[(size_t)e * 3];
+        c = gel[(size_t)e * 3 + 2];
+      } else {
+        for (int m = 0; m < K2; ++m) {  // quadrature means over the reference square
+          const double ww = 0.25 * tab.wgt[m / K] * tab.wgt[m % K];
+          a += ww * Ga[(size_t)e * K2 + m];
+          c += ww * Gc[(size_t)e * K2 + m];
+        }
+      }
+      ac[(size_t)e * 2] = a;
+      ac[(size_t)e * 2 + 1] = c;
+    }
+    P.ac.upload_as(ac);
+    if constexpr (std::is_same<R, double>::value) {
+      std::vector<uint16_t> types(N);
+      for (int e = 0; e < N; ++e) {
+        int kind[4];
+        for (int f = 0; f < 4; ++f) {
+          const int nb = mesh.nb[(size_t)e * 4 + f];
+          kind[f] = nb >= 0 ? 0 : bch.sw_psi[-1 - nb] ? 2 : 1;
+        }
+        types[e] = (uint16_t)((kind[0] * 3 + kind[1]) + 16 * (kind[2] * 3 + kind[3]));
+      }
+      d_ftype.upload(types);
+    }
+    // Neumann faces with tangential metrics: common values from the K x K system of
+    // src/HO_2D.cpp:2872-2927, inverted here
+    std::vector<double> qn;
+    if (geo_kind != GEO_ORTHO) {
+      qn.assign((size_t)std::max(E, 1) * K2, 0.);
+      for (int e = 0; e < E; ++e) {
+        if (!bch.sw_psi[e]) continue;
+        const int f = mesh.be_ijp[e];
+        const size_t q = ((size_t)mesh.be_elem[e] * 4 + f) * K;
+        const double gp = tab.gprime[f & 1];
+        std::vector<double> M((size_t)K2), rhs((size_t)K2, 0.);
+        for (int k = 0; k < K; ++k) {
+          for (int i = 0; i < K; ++i) M[(size_t)k * K + i] = -geo.fB[q + k] * tab.D[i][k];
+          M[(size_t)k * K + k] += geo.fA[q + k] * gp;
+          rhs[(size_t)k * K + k] = geo.fA[q + k] * gp;
+        }
+        solve_dense(K, K, M.data(), rhs.data());
+        std::copy(rhs.begin(), rhs.end(), qn.begin() + (size_t)e * K2);
+      }
+    }
+    P.qn.upload_as(qn);
+    FineGeo<R>& G2 = P.G;
+    G2 = FineGeo<R>{};
+    if constexpr (std::is_same<R, double>::value) {
+      G2.gel = G.gel; G2.gface = G.gface;
+      G2.Ga = G.Ga; G2.Gb = G.Gb; G2.Gc = G.Gc; G2.fa = G.fa; G2.fb = G.fb;
+    } else if (affine) {
+      P.gel.upload_as(gel); P.gface.upload_as(gface);
+      G2.gel = P.gel; G2.gface = P.gface;
+    } else {
+      P.Ga.upload_as(Ga); P.Gb.upload_as(Gb); P.Gc.upload_as(Gc); P.fa.upload_as(fa); P.fb.upload_as(fb);
+      G2.Ga = P.Ga; G2.Gb = P.Gb; G2.Gc = P.Gc; G2.fa = P.fa; G2.fb = P.fb;
+    }
+    G2.N = N;
+    G2.ac = P.ac; G2.fdm = P.fdm; G2.qn = P.qn; G2.ftype = d_ftype;
+    G2.nb = d_nb; G2.nbf = reinterpret_cast<const int32_t*>(d_nbf.p); G2.sw = d_swpsi;
+    G2.inst = G.inst;
+  }
+
   // Fine-level operator launch in precision R, bracketed by events when profiling.
   template <class R>
-  void lap(Prec<R>& P, int epi, R* x, R* y, const R* rr, const R* dg, R* d, double c1, double c2, double* partp,
-           const int* active, const R* tin = nullptr, R* tout = nullptr) {
+  void fine(Prec<R>& P, int in, int epi, FineArgs<R> A) {
     const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
     if (rec) HIPCHK(hipEventRecord(prof.e0[prof.n], stream));
-    GeoT<R> G = P.G;
-    if (P.iact) { G.inst = P.einst; G.iact = P.iact; }
-    HIPCHK(launch_lap(K, epi, N, P.T, G, x, tin ? tin : P.tr.p, y, rr, dg, d, c1, c2, partp, active, stream, tout,
-                      rec ? prof.ran.p + prof.n : nullptr));
-    if (rec) {
-      HIPCHK(hipEventRecord(prof.e1[prof.n], stream));
-      prof.var[prof.n] = P.prof_off + epi;
-      prof.nbytes[prof.n] = lap_bytes(epi, (double)sizeof(R), tout != nullptr, y != nullptr);
-      if (++prof.n == (int)prof.e0.size()) prof_flush();
-    }
+    P.G.iact = P.iact;
+    A.ran = rec ? prof.ran.p + prof.n : nullptr;
+    HIPCHK(launch_fine(K, geo_kind, in, epi, P.T, P.G, A, stream));
+    if (rec) prof_mark(P.prof_off + prof_variant(in, epi), lap_bytes(in, epi, (double)sizeof(R), (double)sizeof(R)));
+  }
+  void prof_mark(int variant, double bytes) {
+    HIPCHK(hipEventRecord(prof.e1[prof.n], stream));
+    prof.var[prof.n] = variant;
+    prof.nbytes[prof.n] = bytes;
+    if (++prof.n == (int)prof.e0.size()) prof_flush();
+  }
+  // Entry of the live kernel profile: apply, residual, smoothing step, first smoothing step after the
+  // coarse correction, restriction.
+  static int prof_variant(int in, int epi) {
+    return epi == EPI_RESID ? 1 : epi == EPI_SMOOTH ? (in == IN_PROL ? 3 : 2) : epi == EPI_RESTRICT ? 4 : 0;
+  }
+  // p = z + beta p and q = As p in one launch (z in FP32 from the mixed-precision V-cycle).
+  void direction_apply(Prec<double>& P, const void* z, bool z32, const double* p, double* pn, double* q,
+                       const double* scal, int scal_idx, double* partp, const int* active) {
+    FineArgs<double> A;
+    A.x = p; A.z = z; A.pn = pn; A.y = q; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = active;
+    if (!z32) { fine(P, IN_PUPD, EPI_STORE, A); return; }
+    const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
+    if (rec) HIPCHK(hipEventRecord(prof.e0[prof.n], stream));
+    P.G.iact = P.iact;
+    A.ran = rec ? prof.ran.p + prof.n : nullptr;
+    HIPCHK(launch_fine_pupd_f32z(K, geo_kind, P.T, P.G, A, stream));
+    if (rec) prof_mark(0, lap_bytes(IN_PUPD, EPI_STORE, 8., 4.));
   }
   // Only launches that worked count: a launch predicated off after convergence returns at once
   // and would book its algorithmic bytes against a near-zero duration.
@@ -390,32 +477,35 @@ struct Solver {
     }
     prof.n = 0;
   }
-  // Algorithmic HBM bytes of one fine-operator launch per epilogue, for values of vb bytes:
-  // the field, the neighbour face traces (value + derivative), metrics, connectivity, the
-  // epilogue's own vectors and (traces_out) the updated iterate's face traces, each read or
-  // written once; dir_out: a Chebyshev step stores its direction.
-  double lap_bytes(int epi, double vb = 8., bool traces_out = false, bool dir_out = true) const {
+  // Algorithmic HBM bytes of one fine-operator launch for values of vb bytes (z: zb): every field,
+  // metric and connectivity array once (the neighbours' lines are other wavefronts' own rows).
+  double lap_bytes(int in, int epi, double vb = 8., double zb = 8.) const {
     const double vec = (double)N * K2 * vb;
-    double b = vec                                   // x
-             + (double)N * 4 * 2 * K * vb            // neighbour traces
-             + (double)N * 4 * (4 + 1);              // nb, nbf
-    if (G.gel) b += (double)N * (3 + 8 + 8) * vb;    // affine: element + own/neighbour face metrics
-    else b += 3 * vec + (double)N * 4 * K * 2 * vb * 2;
+    double b = vec + (double)N * (4 * 4 + 4);          // x; nb, nbf
+    if (geo_kind == GEO_ORTHO) b += (double)N * 2 * vb;
+    else if (geo_kind == GEO_AFFINE) b += (double)N * (3 + 8) * vb;
+    else b += 3 * vec + (double)N * 4 * K * 2 * vb;
+    if (in == IN_PUPD) b += vec + (double)N * K2 * zb; // z, p out
+    if (in == IN_PROL) b += (double)N * 4 * 4 + (double)nv * vb;
     switch (epi) {
-      case EPI_STORE: b += vec; break;                        // y
-      case EPI_RESID: b += 2 * vec; break;                    // r, y
-      case EPI_CHEB: b += (dir_out ? 5 : 4) * vec; break;     // r, dinv, d, x out (+ direction out)
-      case EPI_CHEBF: b += (dir_out ? 4 : 3) * vec; break;    // r, dinv, x out (+ direction out)
-      case EPI_RESTRICT: b += vec + (double)N * 4 * vb; break;  // r, corner sums
+      case EPI_STORE: case EPI_PLAIN: b += vec; break;                      // y
+      case EPI_RESID: b += 2 * vec; break;                                  // b, y
+      case EPI_SMOOTH: b += 2 * vec + (double)N * (geo_kind == GEO_ORTHO ? 2. : 2. + 2 * vb); break;  // b, y; types, scales
+      case EPI_RESTRICT: b += vec + (double)N * 4 * vb; break;              // b, corner sums
     }
-    if (traces_out) b += (double)N * 4 * 2 * K * vb;
     return b;
   }
 
-  // As x into y (FP64 trace + apply); x is not modified.
-  void apply_As(double* x, double* y) {
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, x, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    lap<double>(P64, EPI_STORE, x, y, nullptr, nullptr, nullptr, 0., 0., nullptr, nullptr);
+  // y = As x, and y = b - As x with the partial sums of its norms when partp is set (FP64).
+  void apply_As(const double* x, double* y) {
+    FineArgs<double> A;
+    A.x = x; A.y = y;
+    fine(P64, IN_X, EPI_STORE, A);
+  }
+  void residual_As(const double* x, const double* b, double* y, double* partp) {
+    FineArgs<double> A;
+    A.x = x; A.b = b; A.y = y; A.part = partp;
+    fine(P64, IN_X, EPI_RESID, A);
   }
 
   // Stream-ordered copies that return when the data has arrived.
@@ -439,7 +529,7 @@ struct Solver {
       for (int rs = 0; rs < K2; ++rs) {
         probe_set(stream, N, K2, dcol1, c, rs, P64.z);
         apply_As(P64.z, P64.q);
-        probe_diag(stream, N, K2, dcol1, c, rs, P64.q, P64.dinv);
+        probe_diag(stream, N, K2, dcol1, c, rs, P64.q, P64.t);
       }
     // Continuous bilinear coarse space on the element corners: Pc interpolates vertex values
     // to every element's solution points; Ac = Pc^T As Pc is assembled from probes of As.
@@ -460,6 +550,8 @@ struct Solver {
         for (int a = 0; a < 4; ++a) vinc[pos[ev[(size_t)e * 4 + a]]++] = e * 4 + a;
     }
     d_ev.upload(ev); d_vptr.upload(vptr); d_vinc.upload(vinc);
+    P64.G.ev = d_ev;
+    P32.G.ev = d_ev;
     inst_coupled = false;  // an ensemble whose instances share a corner vertex
     if (n_inst > 1 && (int)inst_off.size() == n_inst + 1) {
       auto inst_of = [&](int e) { return std::upper_bound(inst_off.begin(), inst_off.end(), e) - inst_off.begin() - 1; };
@@ -513,25 +605,32 @@ struct Solver {
     build_sa_amg(A1, 768, H);
     if (mixed) P32.upload_levels(H);
     else P64.upload_levels(H);
-    // Chebyshev interval from lambda_max(D^-1 As) by power iteration
+    std::vector<double> hd(D);
+    d2h(hd.data(), P64.t.p, D * sizeof(double));
+    for (size_t i = 0; i < D; ++i)
+      if (!(hd[i] > 0.)) throw StatusError(HOC_EINVAL, "Poisson operator has a non-positive diagonal entry");
+    // Chebyshev interval from lambda_max(B As) by power iteration
     std::vector<double> hx(D);
     uint64_t st = 88172645463325252ull;
     for (size_t i = 0; i < D; ++i) { st ^= st << 13; st ^= st >> 7; st ^= st << 17; hx[i] = (double)(st % 2000001) / 1e6 - 1.; }
     h2d(P64.z.p, hx.data(), D * sizeof(double));
-    std::vector<double> hd(D), hy(D);
-    d2h(hd.data(), P64.dinv.p, D * sizeof(double));  // the diagonal, inverted below
-    for (size_t i = 0; i < D; ++i)
-      if (!(hd[i] > 0.)) throw StatusError(HOC_EINVAL, "Poisson operator has a non-positive diagonal entry");
     double lam = 0.;
+    const int vg = vec_grid(D);
     for (int it = 0; it < 30; ++it) {
+      // z <- B As z / lam: the norm over one step estimates lambda_max (B As is similar to a
+      // symmetric operator on affine meshes)
       apply_As(P64.z, P64.q);
-      d2h(hy.data(), P64.q.p, D * sizeof(double));
-      double nrm = 0., ray = 0., xx = 0.;
-      for (size_t i = 0; i < D; ++i) { hy[i] /= hd[i]; nrm += hy[i] * hy[i]; ray += hy[i] * hx[i]; xx += hx[i] * hx[i]; }
-      lam = ray / xx;
-      nrm = std::sqrt(nrm);
-      for (size_t i = 0; i < D; ++i) hx[i] = hy[i] / nrm;
-      h2d(P64.z.p, hx.data(), D * sizeof(double));
+      PreArgs<double> A = pre_args<double>(P64.q.p, P64.t.p, it > 0 ? 1. / lam : 1.);
+      HIPCHK(launch_pre(K, P64.T, P64.G, A, stream));
+      double nn[2] = {0., 0.};
+      for (int k = 0; k < 2; ++k) {
+        double* v = k == 0 ? P64.z.p : P64.t.p;
+        vec<double>(stream, VOP_DOT2, VA, D, v, v, v, v, nullptr, nullptr, nullptr, part);
+        finalize(stream, PH_BB, part, vg, S, F, 0);
+        d2h(&nn[k], S.p + S_BB, sizeof(double));
+      }
+      lam = (it > 0 ? lam : 1.) * std::sqrt(nn[1] / nn[0]);
+      std::swap(P64.z.p, P64.t.p);
     }
     lam_max = lam;
     // symmetry of As decides the Krylov method
@@ -550,26 +649,15 @@ struct Solver {
       for (size_t i = 0; i < D; ++i) { a += hx2[i] * hAx[i]; b += hx[i] * hAy[i]; na += std::fabs(hx2[i] * hAx[i]); nb += std::fabs(hx[i] * hAy[i]); }
       krylov = std::fabs(a - b) <= 1e-12 * std::max(na, nb) ? HOC_KRYLOV_PCG : HOC_KRYLOV_BICGSTAB;
     }
-    const double lmax = 1.1 * lam, lmin = lmax * (cfg.cheb_lower > 0. ? cfg.cheb_lower : 1. / 60.);
+    const double lmax = 1.1 * lam, lmin = lmax * (cfg.cheb_lower > 0. ? cfg.cheb_lower : 1. / 10.);
     const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
-    const double sigma = theta / delta;
-    // default degree 3; 4 for the FP32 cycle of a mixed-precision PCG, where the two extra operator
-    // applies cost less than the residual reduction they add.  BiCGSTAB (non-affine meshes) keeps 3
-    // in both precisions: there degree 4 did not pay at the cylinder, and at the step it made the
-    // two precisions stop after different iteration counts, moving the mixed fields away from the
-    // FP64 ones by more than the 1e-8 budget at a Krylov tolerance of 1e-12.
-    cheb_m = cfg.cheb_degree > 0 ? cfg.cheb_degree : (mixed && krylov == HOC_KRYLOV_PCG) ? 4 : 3;
-    cheb_theta = theta;
-    double rho = 1. / sigma;
-    for (int k = 1; k < cheb_m; ++k) {
-      const double rho_new = 1. / (2. * sigma - rho);
-      cheb_c1[k] = rho_new * rho;
-      cheb_c2[k] = 2. * rho_new / delta;
-      rho = rho_new;
-    }
-    for (size_t i = 0; i < D; ++i) hd[i] = 1. / hd[i];
-    h2d(P64.dinv.p, hd.data(), D * sizeof(double));
-    if (mixed) P32.dinv.upload_as(hd);
+    // Degree 2 by default: on the cavity (K = 5) degree 1 takes about twice the iterations and
+    // degree 3 no fewer, the coarse space limiting them from there on.  The dampings are the
+    // inverse roots of the Chebyshev polynomial on [lmin, lmax], large and small in turn.
+    cheb_m = cfg.cheb_degree > 0 ? cfg.cheb_degree : 2;
+    std::vector<double> root(cheb_m);
+    for (int k = 0; k < cheb_m; ++k) root[k] = theta + delta * std::cos(M_PI * (k + 0.5) / cheb_m);
+    for (int k = 0; k < cheb_m; ++k) cheb_w[k] = 1. / ((k & 1) ? root[cheb_m - 1 - k / 2] : root[k / 2]);
     HIPCHK(hipMemsetAsync(P64.z.p, 0, D * sizeof(double), stream));
     HIPCHK(hipStreamSynchronize(stream));
   }
@@ -581,61 +669,63 @@ struct Solver {
     csr_vcycle<R>(stream, P.lv, P.coarse_inv, P.coarse_n, l, f, u, Fp);
   }
 
-  // zout = V(rin); if part != nullptr, partials of rin.zout are left in part.
+  // The first smoothing step of a V-cycle, z = omega B r (see PreArgs).
   template <class R>
-  void vcycle(Prec<R>& P, const R* rin, R* zout, double* partp, const int* Fp) {
-    R* rr = const_cast<R*>(rin);
-    R* cur = P.tr.p;   // traces of the current iterate
-    R* nxt = P.tr2.p;
-    // pre-smoothing: Chebyshev(m) from zero
-    // directions ping-pong between dch and dch2; the last step of a sweep stores none
-    R* din = P.dch.p;
-    R* dout = P.dch2.p;
-    HIPCHK(launch_trace(K, PRE_CHEB0, N, P.T, zout, rr, P.dinv.p, din, 1. / cheb_theta, nullptr, 0, Fp, cur, stream,
-                        nullptr, P.einst, P.iact));
-    for (int k = 1; k < cheb_m; ++k) {
-      lap(P, EPI_CHEB, zout, k + 1 < cheb_m ? dout : (R*)nullptr, rr, P.dinv.p, din, cheb_c1[k], cheb_c2[k], nullptr,
-          Fp, cur, nxt);
+  PreArgs<R> pre_args(const double* r, R* z, double omega) const {
+    PreArgs<R> A;
+    A.r = const_cast<double*>(r);  // written only with the PCG update in front of the step
+    A.z = z;
+    A.omega = omega;
+    for (int k = 0; k < K; ++k) A.iw[k] = 1. / tab.wgt[k];
+    return A;
+  }
+  template <class R>
+  void vcycle_begin(Prec<R>& P, const double* rin, const int* Fp) {
+    PreArgs<R> A = pre_args<R>(rin, P.t.p, cheb_w[0]);
+    if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
+    A.active = Fp;
+    P.G.iact = P.iact;
+    HIPCHK(launch_pre(K, P.T, P.G, A, stream));
+  }
+  // The rest of the V-cycle for the residual rr after vcycle_begin has left its first iterate in
+  // P.t: the iterate ping-pongs between P.t and zout and ends in zout; if partp != nullptr,
+  // partials of rr.zout are left there.
+  template <class R>
+  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, const int* Fp) {
+    R *cur = P.t.p, *nxt = zout;
+    FineArgs<R> A;
+    A.b = rr;
+    A.active = Fp;
+    auto smooth = [&](int in, double omega, double* pp) {
+      A.x = cur; A.y = nxt; A.omega = omega; A.part = pp;
+      fine(P, in, EPI_SMOOTH, A);
       std::swap(cur, nxt);
-      std::swap(din, dout);
-    }
+    };
+    for (int k = 1; k < cheb_m; ++k) smooth(IN_X, cheb_w[k], nullptr);
     // restrict the residual to the corner vertices
-    lap(P, EPI_RESTRICT, zout, P.ec.p, rr, (const R*)nullptr, (R*)nullptr, 0., 0., nullptr, Fp, cur);
+    A.x = cur; A.y = P.ec.p; A.part = nullptr;
+    fine(P, IN_X, EPI_RESTRICT, A);
     q1_gather<R>(stream, nv, d_vptr, d_vinc, P.ec, P.rc, Fp);
     coarse_cycle(P, 0, P.rc.p, P.xc.p, Fp);
-    // prolongate and post-smooth: Chebyshev(m) from the corrected iterate
-    cur = P.tr.p; nxt = P.tr2.p;
-    HIPCHK(launch_trace(K, PRE_PROL, N, P.T, zout, P.xc.p, (const R*)nullptr, (R*)nullptr, 0., nullptr, 0, Fp, cur,
-                        stream, d_ev.p, P.einst, P.iact));
-    din = P.dch.p;
-    dout = P.dch2.p;
-    lap(P, EPI_CHEBF, zout, cheb_m > 1 ? din : (R*)nullptr, rr, P.dinv.p, (R*)nullptr, 0., 1. / cheb_theta,
-        cheb_m == 1 ? partp : nullptr, Fp, cur, cheb_m == 1 ? (R*)nullptr : nxt);
-    std::swap(cur, nxt);
-    for (int k = 1; k < cheb_m; ++k) {
-      const bool last = k == cheb_m - 1;
-      lap(P, EPI_CHEB, zout, last ? (R*)nullptr : dout, rr, P.dinv.p, din, cheb_c1[k], cheb_c2[k],
-          last ? partp : nullptr, Fp, cur, last ? (R*)nullptr : nxt);
-      std::swap(cur, nxt);
-      std::swap(din, dout);
-    }
+    // prolongate and post-smooth, the dampings in reverse: the cycle stays symmetric
+    A.xc = P.xc.p;
+    for (int k = cheb_m - 1; k >= 0; --k)
+      smooth(k == cheb_m - 1 ? IN_PROL : IN_X, cheb_w[k], k == 0 ? partp : nullptr);
   }
 
   // z = M r: the V-cycle in the precision of P; for the FP64 Krylov method of a mixed-precision
   // handle, the FP32 V-cycle between a demotion of r and a promotion of z.  With partp set, the
   // partials of r . z are left there; returns their count (0 when partp is null).
-  template <class R>
-  int precond(Prec<R>& P, const R* rin, R* zout, double* partp, const int* Fp) {
-    if constexpr (std::is_same<R, double>::value) {
-      if (mixed) {
-        demote(stream, D, rin, P32.r.p, Fp);
-        vcycle(P32, P32.r.p, P32.z.p, nullptr, Fp);
-        promote_dot(stream, D, P32.z.p, zout, rin, partp, Fp);
-        return partp ? vec_grid(D) : 0;
-      }
+  int precond(const double* rin, double* zout, double* partp, const int* Fp) {
+    if (mixed) {
+      vcycle_begin(P32, rin, Fp);
+      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp);
+      promote_dot(stream, D, P32.z.p, zout, rin, partp, Fp);
+      return partp ? vec_grid(D) : 0;
     }
-    vcycle(P, rin, zout, partp, Fp);
-    return partp ? lap_blocks(N) : 0;
+    vcycle_begin(P64, rin, Fp);
+    vcycle_rest(P64, rin, zout, partp, Fp);
+    return partp ? fine_blocks(K, N) : 0;
   }
 
   // Wait, lag iterations behind (none when final_wait), until the finalize kernel of the
@@ -697,76 +787,79 @@ struct Solver {
     }
     kgraphs.clear();
   }
-  // Before the first iteration.
-  template <class R>
-  void krylov_begin(Prec<R>& P, R* r) {
+  // Before the first iteration.  PCG: the first smoothing step of the first V-cycle (an iteration
+  // ends with the next one's); its direction needs no clearing, beta = 0 leaves the old one out.
+  void krylov_begin(double* r, const int* Fp) {
+    Prec<double>& P = P64;
     if (krylov == HOC_KRYLOV_PCG) {
-      HIPCHK(hipMemsetAsync(P.p.p, 0, D * sizeof(R), stream));
+      if (mixed) vcycle_begin(P32, r, Fp);
+      else vcycle_begin(P64, r, Fp);
     } else {
-      vec<R>(stream, VOP_COPY, VA, D, P.rh, nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr);
-      HIPCHK(hipMemsetAsync(P.p.p, 0, D * sizeof(R), stream));
-      HIPCHK(hipMemsetAsync(P.v.p, 0, D * sizeof(R), stream));
+      vec<double>(stream, VOP_COPY, VA, D, P.rh, nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr);
+      HIPCHK(hipMemsetAsync(P.p.p, 0, D * sizeof(double), stream));
+      HIPCHK(hipMemsetAsync(P.v.p, 0, D * sizeof(double), stream));
     }
   }
+  // PCG's update x += alpha p, r -= alpha q with the first smoothing step of the next V-cycle.
+  void pcg_update(double* x, double* r, const double* p, const double* scal, int scal_idx, double* partp,
+                  const int* Fp) {
+    auto go = [&](auto& P) {
+      using R = std::remove_reference_t<decltype(*P.t.p)>;
+      PreArgs<R> A = pre_args<R>(r, P.t.p, cheb_w[0]);
+      if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
+      A.x = x; A.p = p; A.q = P64.q.p; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = Fp;
+      P.G.iact = P.iact;
+      HIPCHK(launch_pre(K, P.T, P.G, A, stream));
+    };
+    if (mixed) go(P32);
+    else go(P64);
+  }
   // One iteration's launches.  seq >= 0: the end-of-iteration finalize publishes seq; seq < 0:
-  // it takes the next number from F[F_SEQ].
-  template <class R>
-  void krylov_iter(Prec<R>& P, R* x, R* r, double* Sp, int* Fp, int maxit, int seq) {
-    const int lb = lap_blocks(N);
+  // it takes the next number from F[F_SEQ].  odd: which of the two direction buffers is the old one.
+  void krylov_iter(double* x, double* r, double* Sp, int* Fp, int maxit, int seq, bool odd) {
+    Prec<double>& P = P64;
+    const int fb = fine_blocks(K, N);
     const int vg = vec_grid(D);
-    if constexpr (std::is_same<R, double>::value) {
-      if (ens_batched()) {
-        ens_iter(x, r, Sp, Fp, maxit, seq);
-        return;
-      }
+    double* pold = odd ? P.v.p : P.p.p;
+    double* pnew = odd ? P.p.p : P.v.p;
+    if (ens_batched()) {
+      ens_iter(x, r, pold, pnew, Sp, Fp, maxit, seq);
+      return;
     }
     if (krylov == HOC_KRYLOV_PCG) {
-      bool zf = false;  // z left in FP32 by the mixed-precision V-cycle
-      if constexpr (std::is_same<R, double>::value) {
-        if (mixed) {  // r.z from the FP32 V-cycle's last sweep; p = z + beta p reads z in FP32
-          demote(stream, D, r, P32.r.p, Fp);
-          vcycle(P32, P32.r.p, P32.z.p, part.p, Fp);
-          finalize(stream, PH_RZ, part, lb, Sp, Fp, maxit);
-          HIPCHK(launch_trace_pupd_f32z(K, N, P.T, P.p.p, P32.z.p, Sp, S_BETA, Fp, P.tr.p, stream));
-          zf = true;
-        }
+      // r.z from the V-cycle's last sweep; in mixed precision the direction update reads z in FP32
+      if (mixed) vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, part.p, Fp);
+      else vcycle_rest(P64, r, P.z.p, part.p, Fp);
+      finalize(stream, PH_RZ, part, fb, Sp, Fp, maxit);
+      direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, Sp, S_BETA, part.p, Fp);
+      finalize(stream, PH_PQ, part, fb, Sp, Fp, maxit);
+      pcg_update(x, r, pnew, Sp, S_ALPHA, part.p, Fp);
+      if (ens_pcg()) {  // every instance against its own right-hand side
+        seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p);
+        finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq, ens_rr.p, ens_bb.p, pseg.nseg);
+        return;
       }
-      if (!zf) {
-        const int np = precond(P, r, P.z.p, part.p, Fp);
-        finalize(stream, PH_RZ, part, np, Sp, Fp, maxit);
-        HIPCHK(launch_trace(K, PRE_PUPD, N, P.T, P.p.p, P.z.p, (const R*)nullptr, (R*)nullptr, 0., Sp, S_BETA, Fp,
-                            P.tr.p, stream));
-      }
-      lap(P, EPI_STORE, P.p.p, P.q.p, (const R*)nullptr, (const R*)nullptr, (R*)nullptr, 0., 0., part.p, Fp);
-      finalize(stream, PH_PQ, part, lb, Sp, Fp, maxit);
-      vec<R>(stream, VOP_PCG_UPD, VA, D, x, r, P.p, P.q, nullptr, Sp, Fp, part);
-      if constexpr (std::is_same<R, double>::value) {
-        if (ens_pcg()) {  // every instance against its own right-hand side
-          seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p);
-          finalize(stream, PH_UPD, part, vg, Sp, Fp, maxit, mirror_dev, seq, ens_rr.p, ens_bb.p, pseg.nseg);
-          return;
-        }
-      }
-      finalize(stream, PH_UPD, part, vg, Sp, Fp, maxit, mirror_dev, seq);
+      finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq);
     } else {
-      const R* none = nullptr;
-      vec<R>(stream, VOP_DOT2, VA, D, P.rh, P.rh, r, r, nullptr, Sp, Fp, part);
+      FineArgs<double> A;
+      A.active = Fp;
+      vec<double>(stream, VOP_DOT2, VA, D, P.rh, P.rh, r, r, nullptr, Sp, Fp, part);
       finalize(stream, PH_RHO, part, vg, Sp, Fp, maxit);
-      vec<R>(stream, VOP_BICG_P, VA, D, P.p, nullptr, r, P.v, nullptr, Sp, Fp, nullptr);
-      precond(P, P.p.p, P.ph.p, nullptr, Fp);
-      HIPCHK(launch_trace(K, PRE_COPY, N, P.T, P.ph.p, none, none, (R*)nullptr, 0., nullptr, 0, Fp, P.tr.p, stream));
-      lap(P, EPI_STORE, P.ph.p, P.v.p, none, none, (R*)nullptr, 0., 0., nullptr, Fp);
-      vec<R>(stream, VOP_DOT2, VA, D, P.rh, P.rh, P.v, P.v, nullptr, Sp, Fp, part);
+      vec<double>(stream, VOP_BICG_P, VA, D, P.p, nullptr, r, P.v, nullptr, Sp, Fp, nullptr);
+      precond(P.p.p, P.ph.p, nullptr, Fp);
+      A.x = P.ph.p; A.y = P.v.p;
+      fine(P, IN_X, EPI_STORE, A);
+      vec<double>(stream, VOP_DOT2, VA, D, P.rh, P.rh, P.v, P.v, nullptr, Sp, Fp, part);
       finalize(stream, PH_ALPHA, part, vg, Sp, Fp, maxit);
-      vec<R>(stream, VOP_BICG_S, VA, D, nullptr, r, nullptr, P.v, nullptr, Sp, Fp, part);
+      vec<double>(stream, VOP_BICG_S, VA, D, nullptr, r, nullptr, P.v, nullptr, Sp, Fp, part);
       finalize(stream, PH_SNORM, part, vg, Sp, Fp, maxit);
-      bicg_half<R>(stream, D, x, P.ph, Sp, Fp);
-      precond(P, r, P.sh.p, nullptr, Fp);  // gated by F_ACTIVE only; harmless when converged at the half step
-      HIPCHK(launch_trace(K, PRE_COPY, N, P.T, P.sh.p, none, none, (R*)nullptr, 0., nullptr, 0, Fp, P.tr.p, stream));
-      lap(P, EPI_STORE, P.sh.p, P.t.p, none, none, (R*)nullptr, 0., 0., nullptr, Fp);
-      vec<R>(stream, VOP_DOT2, VA, D, P.t, P.t, r, P.t, nullptr, Sp, Fp, part);
+      bicg_half<double>(stream, D, x, P.ph, Sp, Fp);
+      precond(r, P.sh.p, nullptr, Fp);  // gated by F_ACTIVE only; harmless when converged at the half step
+      A.x = P.sh.p; A.y = P.q.p;
+      fine(P, IN_X, EPI_STORE, A);
+      vec<double>(stream, VOP_DOT2, VA, D, P.q, P.q, r, P.q, nullptr, Sp, Fp, part);
       finalize(stream, PH_OMEGA, part, vg, Sp, Fp, maxit);
-      vec<R>(stream, VOP_BICG_X, VA, D, x, r, P.ph, P.sh, P.t, Sp, Fp, part);
+      vec<double>(stream, VOP_BICG_X, VA, D, x, r, P.ph, P.sh, P.q, Sp, Fp, part);
       finalize(stream, PH_RNORM, part, vg, Sp, Fp, maxit, mirror_dev, seq);
     }
   }
@@ -775,42 +868,26 @@ struct Solver {
   // stopping on its own test; while an instance is stopped, the fine-level kernels skip the
   // blocks that hold only its elements, and its x and r stay as they are.  The coarse levels run
   // over every instance: with no Q1 vertex shared between instances they stay block-diagonal.
-  void ens_iter(double* x, double* r, double* Sp, int* Fp, int maxit, int seq) {
+  void ens_iter(double* x, double* r, const double* pold, double* pnew, double* Sp, int* Fp, int maxit, int seq) {
     struct Mask {  // the masks hold for this iteration's launches only
       Solver& s;
-      explicit Mask(Solver& so) : s(so) {
-        s.P64.einst = s.P32.einst = s.d_inst.p;
-        s.P64.iact = s.P32.iact = s.ens_act.p;
-      }
-      ~Mask() {
-        s.P64.einst = s.P32.einst = nullptr;
-        s.P64.iact = s.P32.iact = nullptr;
-      }
+      explicit Mask(Solver& so) : s(so) { s.P64.iact = s.P32.iact = s.ens_act.p; }
+      ~Mask() { s.P64.iact = s.P32.iact = nullptr; }
     } mask(*this);
     Prec<double>& P = P64;
     const EnsKry E = ensk();
-    VecArgs va = VA;  // x += alpha_i p, r -= alpha_i q
-    va.ialpha = ens_alpha.p;
-    va.einst = d_inst.p;
     if (mixed) {
-      demote(stream, D, r, P32.r.p, Fp);
-      vcycle(P32, P32.r.p, P32.z.p, nullptr, Fp);
+      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp);
       seg_dot<float>(stream, pseg, r, P32.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-      finalize_ens(stream, ENS_RZ, E, Sp, Fp, maxit);
-      HIPCHK(launch_trace_pupd_f32z(K, N, P.T, P.p.p, P32.z.p, ens_beta.p, -1, Fp, P.tr.p, stream, d_inst.p,
-                                    ens_act.p));
     } else {
-      vcycle(P, r, P.z.p, nullptr, Fp);
+      vcycle_rest(P64, r, P.z.p, nullptr, Fp);
       seg_dot<double>(stream, pseg, r, P.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-      finalize_ens(stream, ENS_RZ, E, Sp, Fp, maxit);
-      HIPCHK(launch_trace(K, PRE_PUPD, N, P.T, P.p.p, P.z.p, nullptr, nullptr, 0., ens_beta.p, -1, Fp, P.tr.p, stream,
-                          nullptr, d_inst.p, ens_act.p));
     }
-    lap(P, EPI_STORE, P.p.p, P.q.p, (const double*)nullptr, (const double*)nullptr, (double*)nullptr, 0., 0., nullptr,
-        Fp);
-    seg_dot<double>(stream, pseg, P.p.p, P.q.p, Fp, ens_part.p, ens_in.p, ens_act.p);
+    finalize_ens(stream, ENS_RZ, E, Sp, Fp, maxit);
+    direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr, Fp);
+    seg_dot<double>(stream, pseg, pnew, P.q.p, Fp, ens_part.p, ens_in.p, ens_act.p);
     finalize_ens(stream, ENS_PQ, E, Sp, Fp, maxit);
-    vec<double>(stream, VOP_PCG_UPD, va, D, x, r, P.p, P.q, nullptr, Sp, Fp, nullptr);
+    pcg_update(x, r, pnew, ens_alpha.p, -1, nullptr, Fp);
     // ||r_i||^2 into ens_rr, where a stopped instance keeps its last value (its r no longer changes)
     seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p, ens_act.p);
     EnsKry Eu = E;
@@ -818,9 +895,9 @@ struct Solver {
     finalize_ens(stream, ENS_UPD, Eu, Sp, Fp, maxit, mirror_dev, seq);
   }
   // The instantiated graph of kGraphChunk iterations on these buffers (captured on first use).
-  template <class R>
-  hipGraphExec_t krylov_graph(Prec<R>& P, R* x, R* r, double* Sp, int* Fp, int maxit) {
-    const void* key[6] = {&P, x, r, Sp, Fp, mixed ? (const void*)&P32 : nullptr};
+  static_assert(kGraphChunk % 2 == 0, "the direction buffers return to their places after a chunk");
+  hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit) {
+    const void* key[6] = {&P64, x, r, Sp, Fp, mixed ? (const void*)&P32 : nullptr};
     for (auto& k : kgraphs)
       if (k.maxit == maxit && std::equal(key, key + 6, k.key)) return k.e;
     KGraph kg;
@@ -828,7 +905,7 @@ struct Solver {
     kg.maxit = maxit;
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
-      for (int i = 0; i < kGraphChunk; ++i) krylov_iter(P, x, r, Sp, Fp, maxit, -1);
+      for (int i = 0; i < kGraphChunk; ++i) krylov_iter(x, r, Sp, Fp, maxit, -1, i & 1);
     } catch (...) {
       hipGraph_t g = nullptr;
       (void)hipStreamEndCapture(stream, &g);
@@ -840,13 +917,12 @@ struct Solver {
     kgraphs.push_back(kg);
     return kg.e;
   }
-  template <class R>
-  void krylov_solve(Prec<R>& P, R* x, R* r, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
+  void krylov_solve(double* x, double* r, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
     const int maxit = maxit_dev;
     const int seq0 = seq_next;
-    krylov_begin(P, r);
+    krylov_begin(r, Fp);
     if (use_graphs && !prof.on) {
-      hipGraphExec_t ge = krylov_graph(P, x, r, Sp, Fp, maxit);
+      hipGraphExec_t ge = krylov_graph(x, r, Sp, Fp, maxit);
       set_int(stream, Fp + F_SEQ, seq_next - 1);
       for (int done = 0;;) {
         HIPCHK(hipGraphLaunch(ge, stream));
@@ -860,7 +936,7 @@ struct Solver {
     }
     for (int it = 0;; ++it) {
       const int seq = seq_next++;
-      krylov_iter(P, x, r, Sp, Fp, maxit, seq);
+      krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
       bool near = false;
       if (!poll(seq, seq0, it > maxit_host + 2, 1, &near) || it > maxit_host + 4) break;
       // the previous iteration ended within 8x of the tolerance: the one just queued is likely
@@ -888,8 +964,8 @@ struct Solver {
     auto run = [&](bool graph) {
       HIPCHK(hipMemsetAsync(psi.p, 0, D * sizeof(double), stream));
       outer_residual();
-      krylov_begin(P64, P64.r.p);
-      hipGraphExec_t ge = graph ? krylov_graph(P64, psi.p, P64.r.p, S.p, F.p, maxit) : nullptr;
+      krylov_begin(P64.r.p, F.p);
+      hipGraphExec_t ge = graph ? krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit) : nullptr;
       HIPCHK(hipStreamSynchronize(stream));
       const auto t0 = std::chrono::steady_clock::now();
       if (graph) {
@@ -897,7 +973,7 @@ struct Solver {
         for (int c = 0; c < 2; ++c) HIPCHK(hipGraphLaunch(ge, stream));
         seq_next += 2 * kGraphChunk;
       } else {
-        for (int i = 0; i < 2 * kGraphChunk; ++i) krylov_iter(P64, psi.p, P64.r.p, S.p, F.p, maxit, seq_next++);
+        for (int i = 0; i < 2 * kGraphChunk; ++i) krylov_iter(psi.p, P64.r.p, S.p, F.p, maxit, seq_next++, i & 1);
       }
       HIPCHK(hipStreamSynchronize(stream));
       return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -916,9 +992,8 @@ struct Solver {
   // FP64 residual r = bs - As psi with the reference's unscaled norm, and the solve's
   // convergence state in (S, F).
   void outer_residual() {
-    const int lb = lap_blocks(N);
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, psi.p, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    lap<double>(P64, EPI_RESID, psi.p, P64.r.p, bs.p, nullptr, nullptr, 0., 0., part.p, nullptr);
+    const int lb = fine_blocks(K, N);
+    residual_As(psi.p, bs.p, P64.r.p, part.p);
     if (ens_pcg()) {
       seg_norm2(stream, pseg, VA, P64.r.p, nullptr, ens_part.p, ens_rr.p);
       finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, ens_rr.p, ens_bb.p, pseg.nseg);
@@ -1126,8 +1201,7 @@ struct Solver {
     proj_alloc();
     if (P.nseg != pseg.nseg) { P.m = 0; return; }
     double* t = ptmp.p;
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, psi.p, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    lap<double>(P64, EPI_RESID, psi.p, t, b, nullptr, nullptr, 0., 0., nullptr, nullptr);  // t = b - As x0
+    residual_As(psi.p, b, t, nullptr);  // t = b - As x0
     const double* Y = proj_mr() ? P.AX.p : P.X.p;
     if (P.gcol_pending >= 0 && P.gcol_pending == P.m - 1) {  // Y^T t, Y^T b and the newest Gram column
       const int j = P.m - 1;
@@ -1222,8 +1296,7 @@ struct Solver {
     else
       proj_ortho(stream, D, pseg, j, proj_mr() ? 1 : 0, P.X.p, pcoef.p + j, kProjCoef, psi, b, xj, ppart,
                  gcol + j + 1, M * kProjLdg, P.W.p + (size_t)j * M, M * M, M);
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, xj, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    lap<double>(P64, EPI_STORE, xj, axj, nullptr, nullptr, nullptr, 0., 0., nullptr, nullptr);
+    apply_As(xj, axj);
     // its Gram column (Y_i . axj, i <= j) comes from the next projected solve's pass over Y
     // (proj_dots3), or from proj_flush_gcol when the basis is used otherwise first
     P.m = j + 1;
@@ -1320,7 +1393,7 @@ struct Solver {
     };
     // FP64: the FP64 V-cycle; mixed: the FP32 V-cycle (precond), the Krylov vectors, the operator
     // application and the stopping test in FP64 either way.
-    krylov_solve(P64, psi.p, P64.r.p, S.p, F.p, maxit, maxit);
+    krylov_solve(psi.p, P64.r.p, S.p, F.p, maxit, maxit);
     read_state(S, F);
     const int iters = hf[F_ITER], outer = 0;
     // statistics
@@ -1380,8 +1453,8 @@ struct Solver {
   void refresh_fields() {
     update_bcs(0.);
     poisson(w);
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, psi, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, P64.tr, w, vel, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
+    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
+    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, w, vel, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
   }
   // Node-averaged vorticity, psi and velocity into d_nodeout (save_smooth_vtk,
   // src/HO_2D.cpp:3369-3531).
@@ -1471,11 +1544,11 @@ struct Solver {
   void stage_body(const double* win, const StageOut& so) {
     poisson(win);
     if (capture_psi && rk_stage >= 0) dcopy(capture_psi + (size_t)rk_stage * D, psi, D);
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, psi, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
+    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
     // the Cartesian velocity is an output of the step's last stage only (what the getters and
     // writers read); intermediate RK stages need the contravariant fluxes U alone
     double* v_out = (so.next && !so.final_mode) ? nullptr : vel.p;
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, P64.tr, win, v_out, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
+    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, win, v_out, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
     HIPCHK(launch_stage(K, cfg.advection_type, N, T, G, B, win, U, trw, tru, re_inv, cfg.dt, I, so, stream));
   }
   void stage(const double* win, double c, const StageOut& so) {
@@ -1803,8 +1876,8 @@ struct Solver {
       update_bcs(c[st]);
       if (stage_psi) dcopy(psi, stage_psi + (size_t)st * D, D);
       else poisson(adj.ws[st]);
-      HIPCHK(launch_trace(K, PRE_COPY, N, T, psi, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-      HIPCHK(launch_velocity(K, N, T, G, B, psi, P64.tr, adj.ws[st], vel, adj.Us[st], adj.trws[st], adj.trus[st],
+      HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
+      HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, adj.ws[st], vel, adj.Us[st], adj.trws[st], adj.trus[st],
                              1. / (cfg.dt * re_inv), I, stream));
       StageOut so;
       so.k = kscratch;
@@ -2137,8 +2210,8 @@ struct Solver {
     h2d(adj.lam.p, lam_h, D * sizeof(double));
     update_bcs(0., t);
     poisson(adj.ws[0]);
-    HIPCHK(launch_trace(K, PRE_COPY, N, T, psi, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, P64.tr.p, stream));
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, P64.tr, adj.ws[0], vel, adj.Us[0], adj.trws[0], adj.trus[0],
+    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
+    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, adj.ws[0], vel, adj.Us[0], adj.trws[0], adj.trus[0],
                            1. / (cfg.dt * re_inv), I, stream));
     StageOut so;
     so.k = kscratch;
@@ -2674,19 +2747,21 @@ int hoc_stage_residual_vjp(hoc_t h, const double* omega, double t, const double*
   });
 }
 
+// y = A x on device buffers (distinct) in one launch on a stream.
+static void apply_plain(Solver& s, const double* x, double* y, hipStream_t st) {
+  hoc::FineArgs<double> A;
+  A.x = x;
+  A.y = y;
+  HIPCHK(hoc::launch_fine(s.K, s.geo_kind, hoc::IN_X, hoc::EPI_PLAIN, s.P64.T, s.P64.G, A, st));
+}
+
 int hoc_apply_laplacian(hoc_t h, const double* x, double* y) {
   return guarded(h, [&] {
     NEED_READY(h);
     Solver& s = h->s;
     s.h2d(s.P64.z.p, x, s.D * sizeof(double));
-    s.apply_As(s.P64.z, s.P64.q);
-    std::vector<double> hy(s.D);
-    s.d2h(hy.data(), s.P64.q.p, s.D * sizeof(double));
-    // As = -W A  =>  A x = -(As x) / W
-    for (size_t v = 0; v < s.D; ++v) {
-      const int m = (int)(v % s.K2);
-      y[v] = -hy[v] / (s.tab.wgt[m / s.K] * s.tab.wgt[m % s.K]);
-    }
+    apply_plain(s, s.P64.z.p, s.P64.q.p, s.stream);
+    s.d2h(y, s.P64.q.p, s.D * sizeof(double));
   });
 }
 
@@ -2696,21 +2771,13 @@ int hoc_apply_laplacian_device(hoc_t h, const double* x, double* y, void* stream
     Solver& s = h->s;
     if (!x || !y) throw hoc::StatusError(HOC_EINVAL, "null buffer");
     if (x == y) throw hoc::StatusError(HOC_EINVAL, "x and y must not alias");
-    const size_t need = (size_t)s.N * 8 * s.K * sizeof(double);  // face traces: 4 faces x (value, derivative) x K
-    if (need > hoc::kNoAllocScratchBytes)
-      throw hoc::StatusError(HOC_EINVAL, "mesh too large for the no-allocation apply: its face traces need " +
-                                             std::to_string(need) + " bytes, the scratch array holds " +
-                                             std::to_string(hoc::kNoAllocScratchBytes));
-    double* tr = hoc::noalloc_scratch(s.device);  // set at hoc_setup on this device
-    if (!tr) throw hoc::StatusError(HOC_ESTATE, "scratch array not set up on this device");
+    const size_t need = (size_t)s.N * 8 * s.K * sizeof(double);
+    if (need > hoc::kNoAllocMaxTraceBytes)
+      throw hoc::StatusError(HOC_EINVAL, "mesh too large for the no-allocation apply: its face traces would need " +
+                                             std::to_string(need) + " bytes, the limit is " +
+                                             std::to_string(hoc::kNoAllocMaxTraceBytes));
     HIPCHK(hipSetDevice(s.device));
-    hipStream_t st = stream ? static_cast<hipStream_t>(stream) : s.stream;
-    double* xm = const_cast<double*>(x);  // read only: PRE_COPY and EPI_STORE do not write x
-    HIPCHK(hoc::launch_trace(s.K, hoc::PRE_COPY, s.N, s.T, xm, nullptr, nullptr, nullptr, 0., nullptr, 0, nullptr, tr, st));
-    HIPCHK(hoc::launch_lap(s.K, hoc::EPI_STORE, s.N, s.P64.T, s.P64.G, xm, tr, y, nullptr, nullptr, nullptr, 0., 0.,
-                           nullptr, nullptr, st));
-    hoc::unweight(st, s.D, s.K, s.tab.wgt, y);  // As = -W A  =>  A x = -(As x) / W
-    HIPCHK(hipGetLastError());
+    apply_plain(s, x, y, stream ? static_cast<hipStream_t>(stream) : s.stream);
   });
 }
 
@@ -2731,7 +2798,7 @@ int hoc_stats_get(hoc_t h, hoc_stats* st) {
     st->total_iters = s.total_iters;
     st->n_solves = s.n_solves;
     st->setup_seconds = s.setup_seconds;
-    st->fine_op_bytes = s.ready ? s.lap_bytes(hoc::EPI_STORE) : 0.;
+    st->fine_op_bytes = s.ready ? s.lap_bytes(hoc::IN_X, hoc::EPI_STORE) : 0.;
   });
 }
 
@@ -2756,6 +2823,12 @@ int hoc_profile_enable(hoc_t h, int32_t on) {
   });
 }
 
+// Algorithmic bytes of a profile entry that has no launches yet.
+static double prof_bytes(const Solver& s, int variant, double vb) {
+  using namespace hoc;
+  const int in[5] = {IN_X, IN_X, IN_X, IN_PROL, IN_X}, epi[5] = {EPI_STORE, EPI_RESID, EPI_SMOOTH, EPI_SMOOTH, EPI_RESTRICT};
+  return s.lap_bytes(in[variant], epi[variant], vb, vb);
+}
 int hoc_profile_get(hoc_t h, hoc_kernel_profile* p) {
   return guarded(h, [&] {
     NEED_READY(h);
@@ -2770,7 +2843,7 @@ int hoc_profile_get(hoc_t h, hoc_kernel_profile* p) {
       p->total_ms[v] = s.prof.ms[v];
       const int half = HOC_PROF_VARIANTS / 2;
       p->bytes_per_launch[v] = s.prof.cnt[v] > 0 ? s.prof.bytes[v] / (double)s.prof.cnt[v]
-                                                 : (v < half ? s.lap_bytes(v, 8.) : s.lap_bytes(v - half, 4.));
+                                                 : prof_bytes(s, v < half ? v : v - half, v < half ? 8. : 4.);
       std::strncpy(p->names[v], names[v], sizeof(p->names[v]) - 1);
     }
     p->noop_launches = s.prof.skipped;

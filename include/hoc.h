@@ -54,8 +54,8 @@ typedef struct {
   int32_t device;                 /* HIP device ordinal                                  */
   int32_t fail_on_noconv;         /* nonzero: return HOC_ENOCONV when tol is not met     */
   double mixed_inner_tol;         /* unused (kept for layout); must lie in [0, 1)       */
-  int32_t cheb_degree;            /* fine-level Chebyshev smoother degree, pre and post
-                                     (0 = 3, or 4 with HOC_MIXED and PCG; at most 8)      */
+  int32_t cheb_degree;            /* degree of the fine-level Chebyshev smoother in B As, pre and
+                                     post (B: the element blocks' inverse; 0 = 2; at most 8) */
   int32_t psi_guess;              /* initial guess of the stage Poisson solves: 1 = the
                                      previous solution (the reference's warm start),
                                      2 = linear extrapolation in the stage time from the
@@ -69,8 +69,8 @@ typedef struct {
                                      correction in the span of 12 to 24 recent stage
                                      solutions: in the As-norm for a symmetric operator,
                                      least-squares residual otherwise  (0 = 5)            */
-  double cheb_lower;              /* smoothing interval [cheb_lower, 1.1] x lambda_max(D^-1 As)
-                                     (0 = 1/60)                                          */
+  double cheb_lower;              /* smoothing interval [cheb_lower, 1.1] x lambda_max(B As)
+                                     (0 = 1/10)                                          */
   int32_t launch_mode;            /* Krylov iterations: 0 = chosen at hoc_setup by timing
                                      both, 1 = kernels queued one by one, 2 = replays of a
                                      captured hipGraph of 4 iterations (same iterates)   */
@@ -217,13 +217,11 @@ int hoc_stage_residual(hoc_t h, const double* omega, double t, double* k);
 int hoc_apply_laplacian(hoc_t h, const double* x, double* y);
 /* No counterpart in the reference: hoc_apply_laplacian for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * x and y are device buffers of n_dofs doubles (distinct); the call allocates nothing: its
- * scratch (the face traces, n_elem * 8 * K doubles) is a library-wide device array of 64 MiB per
- * GPU, held until the process ends, and larger meshes are rejected with HOC_EINVAL.  The work is
- * queued on `stream` (a hipStream_t; NULL = the handle's stream) and the call returns without
- * waiting; the caller synchronizes that stream before reading y.  Every call on one GPU shares
- * the array, so calls that overlap on one GPU (from any handles or streams) race.  Needs
- * hoc_setup on the handle (which takes the array's address on its device). */
+ * x and y are device buffers of n_dofs doubles (distinct); the call is one kernel launch, allocates
+ * nothing and keeps no scratch, so calls on different buffers may overlap.  Meshes whose face traces
+ * (n_elem * 8 * K doubles) would exceed 64 MiB are rejected with HOC_EINVAL.  The work is queued on
+ * `stream` (a hipStream_t; NULL = the handle's stream) and the call returns without waiting; the
+ * caller synchronizes that stream before reading y.  Needs hoc_setup on the handle. */
 int hoc_apply_laplacian_device(hoc_t h, const double* x, double* y, void* stream);
 
 /* Boundary flux points and the tangential wall velocity.  Boundary arrays are [E][K] in the
