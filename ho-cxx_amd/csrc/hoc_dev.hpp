@@ -100,6 +100,70 @@ struct DevLevel {
   DBuf<R> M, f, u, t;
 };
 
+// The Q1 vertex level and below of the Poisson V-cycle (build_vhierarchy): per level the matrices
+// R~ and U in sliced ELL and the vector [f_l; u_{l+1}] they read; u_{l+1} is written into the tail.
+template <class R>
+struct DevSell {
+  int n = 0, lanes = 4;
+  DBuf<int32_t> off, col;
+  DBuf<R> val;
+  void upload(const CSR& A) {
+    try {
+      csr_check(A);
+    } catch (const std::invalid_argument& e) {
+      throw StatusError(HOC_EINVAL, std::string("level matrix: ") + e.what());
+    }
+    n = A.n;
+    lanes = sell_lanes(A);
+    std::vector<int32_t> o, c;
+    std::vector<double> v;
+    sell_pack(A, lanes, o, c, v);
+    off.upload(o);
+    col.upload(c);
+    val.upload_as(v);
+  }
+  void apply(hipStream_t s, const R* x, R* y, const int* F) const {
+    sell<R>(s, n, lanes, off.p, col.p, val.p, x, y, F);
+  }
+};
+template <class R>
+struct DevVLevel {
+  DevSell<R> Rt, U;
+  DBuf<R> fu;
+  int n = 0;
+};
+template <class R>
+struct DevVHierarchy {
+  std::vector<std::unique_ptr<DevVLevel<R>>> lv;
+  DBuf<R> inv, f;  // the coarsest level's dense inverse and right-hand side
+  int nc = 0;
+  int levels() const { return (int)lv.size() + (nc > 0 ? 1 : 0); }
+  // The coarsest inverse (FP64, row-major) is passed in ci.
+  void upload(const VHierarchy& H, const std::vector<double>& ci) {
+    lv.clear();
+    for (const VLevel& h : H.levels) {
+      auto L = std::make_unique<DevVLevel<R>>();
+      L->n = h.U.n;
+      L->Rt.upload(h.Rt);
+      L->U.upload(h.U);
+      L->fu.alloc(h.U.m);
+      lv.push_back(std::move(L));
+    }
+    nc = H.coarse.n;
+    inv.upload_as(ci);
+    f.alloc(nc);
+  }
+  // Where the finest level's right-hand side is read from.
+  R* rhs() { return lv.empty() ? f.p : lv[0]->fu.p; }
+  // u = V(rhs()): all launches predicated on the active flag Fp (may be null).
+  void cycle(hipStream_t s, R* u, const int* Fp) {
+    const size_t n = lv.size();
+    for (size_t l = 0; l < n; ++l) lv[l]->Rt.apply(s, lv[l]->fu, l + 1 < n ? lv[l + 1]->fu.p : f.p, Fp);
+    if (nc > 0) dense<R>(s, nc, inv, f, n ? lv[n - 1]->fu.p + lv[n - 1]->n : u, Fp);
+    for (size_t l = n; l-- > 0;) lv[l]->U.apply(s, lv[l]->fu, l ? lv[l - 1]->fu.p + lv[l - 1]->n : u, Fp);
+  }
+};
+
 // V(1,1) cycle with spai0 relaxation from a zero guess on a sparse hierarchy (level l and
 // below; the last level is solved with its dense inverse): u_l = V_l(f_l).  Every step is
 // out of place, so the cycle is a fixed linear operator.  All launches are predicated on

@@ -1,6 +1,7 @@
 // hoc_host.cpp - host-side setup for the MI355X hot path (see hoc_host.hpp).
 #include "hoc_host.hpp"
 
+#include <queue>
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -604,6 +605,248 @@ CSR matmul(const CSR& A, const CSR& B) {
 }
 }  // namespace
 
+void dense_inverse(const CSR& A, std::vector<double>& inv) {
+  const int n = A.n;
+  std::vector<double> a((size_t)n * n, 0.);
+  inv.assign((size_t)n * n, 0.);
+  for (int i = 0; i < n; ++i) {
+    inv[(size_t)i * n + i] = 1.;
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) a[(size_t)i * n + A.col[j]] += A.val[j];
+  }
+  for (int c = 0; c < n; ++c) {
+    int p = c;
+    for (int r = c + 1; r < n; ++r) if (std::fabs(a[(size_t)r * n + c]) > std::fabs(a[(size_t)p * n + c])) p = r;
+    if (a[(size_t)p * n + c] == 0.) continue;  // singular direction: leave it out of the inverse
+    if (p != c)
+      for (int j = 0; j < n; ++j) { std::swap(a[(size_t)p * n + j], a[(size_t)c * n + j]); std::swap(inv[(size_t)p * n + j], inv[(size_t)c * n + j]); }
+    const double d = 1. / a[(size_t)c * n + c];
+    for (int j = 0; j < n; ++j) { a[(size_t)c * n + j] *= d; inv[(size_t)c * n + j] *= d; }
+    for (int r = 0; r < n; ++r) {
+      if (r == c) continue;
+      const double f = a[(size_t)r * n + c];
+      if (f == 0.) continue;
+      for (int j = 0; j < n; ++j) { a[(size_t)r * n + j] -= f * a[(size_t)c * n + j]; inv[(size_t)r * n + j] -= f * inv[(size_t)c * n + j]; }
+    }
+  }
+}
+
+namespace {
+// A without the entries that are rounding noise of the assembly (a bilinear function has no jumps,
+// so the interface terms of its Galerkin products cancel to ~1e-17 of the diagonal).
+CSR drop_noise(const CSR& A) {
+  CSR B;
+  B.n = A.n; B.m = A.m;
+  B.ptr.assign(A.n + 1, 0);
+  std::vector<double> d(A.n, 0.);
+  for (int i = 0; i < A.n; ++i)
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) if (A.col[j] == i) d[i] += std::fabs(A.val[j]);
+  for (int i = 0; i < A.n; ++i) {
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j)
+      if (A.col[j] == i || A.val[j] * A.val[j] > 1e-24 * d[i] * d[A.col[j]]) {
+        B.col.push_back(A.col[j]);
+        B.val.push_back(A.val[j]);
+      }
+    B.ptr[i + 1] = (int)B.col.size();
+  }
+  return B;
+}
+// Strong couplings of row i: negative entries (against a positive diagonal) of at least a quarter
+// of the row's largest, and above 1e-3 of the diagonal (rows that the diagonal dominates, such as
+// penalised boundary vertices, need no coarse correction).
+void strong_couplings(const CSR& A, std::vector<int32_t>& ptr, std::vector<int32_t>& idx) {
+  ptr.assign(A.n + 1, 0);
+  idx.clear();
+  for (int i = 0; i < A.n; ++i) {
+    double dia = 0., mx = 0.;
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) {
+      if (A.col[j] == i) dia += A.val[j];
+      else mx = std::max(mx, -A.val[j]);
+    }
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j)
+      if (A.col[j] != i && A.val[j] < 0. && -A.val[j] >= 0.25 * mx && -A.val[j] > 1e-3 * std::fabs(dia))
+        idx.push_back(A.col[j]);
+    ptr[i + 1] = (int)idx.size();
+  }
+}
+// First pass of the Ruge-Stueben colouring: 1 coarse, 2 fine.  Rows by the number of undecided rows
+// they influence, larger first, then by index.
+void rs_colour(int n, const std::vector<int32_t>& sp, const std::vector<int32_t>& si, std::vector<uint8_t>& state) {
+  std::vector<int32_t> tp(n + 1, 0), ti(si.size());
+  for (int32_t c : si) tp[c + 1]++;
+  for (int i = 0; i < n; ++i) tp[i + 1] += tp[i];
+  {
+    std::vector<int32_t> pos(tp.begin(), tp.end() - 1);
+    for (int i = 0; i < n; ++i)
+      for (int j = sp[i]; j < sp[i + 1]; ++j) ti[pos[si[j]]++] = i;
+  }
+  state.assign(n, 0);
+  std::vector<int> lam(n);
+  std::priority_queue<std::pair<int, int>> q;  // (measure, -row); outdated entries are skipped
+  for (int i = 0; i < n; ++i) {
+    lam[i] = tp[i + 1] - tp[i];
+    if (lam[i] == 0 && sp[i + 1] == sp[i]) state[i] = 2;
+    else q.push({lam[i], -i});
+  }
+  while (!q.empty()) {
+    const auto [l, mi] = q.top();
+    q.pop();
+    const int i = -mi;
+    if (state[i] != 0 || l != lam[i]) continue;
+    if (l == 0) {  // influences nothing undecided: fine where it can be interpolated
+      bool c = false;
+      for (int j = sp[i]; j < sp[i + 1] && !c; ++j) c = state[si[j]] == 1;
+      state[i] = c ? 2 : 1;
+      continue;
+    }
+    state[i] = 1;
+    for (int j = tp[i]; j < tp[i + 1]; ++j) {
+      const int f = ti[j];
+      if (state[f] != 0) continue;
+      state[f] = 2;
+      for (int k = sp[f]; k < sp[f + 1]; ++k)
+        if (state[si[k]] == 0) q.push({++lam[si[k]], -si[k]});
+    }
+    for (int j = sp[i]; j < sp[i + 1]; ++j)
+      if (state[si[j]] == 0) q.push({--lam[si[j]], -si[j]});
+  }
+}
+}  // namespace
+
+void build_vhierarchy(const CSR& A0, int coarse_enough, VHierarchy& h) {
+  h.levels.clear();
+  h.coarse = CSR();
+  CSR A = drop_noise(A0);
+  while (A.n > coarse_enough) {
+    const int n = A.n;
+    std::vector<int32_t> sp, si;
+    strong_couplings(A, sp, si);
+    std::vector<uint8_t> state;
+    rs_colour(n, sp, si, state);
+    std::vector<int32_t> cid(n, -1);
+    int nc = 0;
+    for (int i = 0; i < n; ++i) if (state[i] == 1) cid[i] = nc++;
+    if (nc >= n) break;
+    std::vector<double> dia(n, 0.), M(n, 0.);
+    for (int i = 0; i < n; ++i) {
+      double s2 = 0.;
+      for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) {
+        if (A.col[j] == i) dia[i] += A.val[j];
+        s2 += A.val[j] * A.val[j];
+      }
+      M[i] = s2 > 0. ? dia[i] / s2 : 0.;
+    }
+    CSR P;  // direct interpolation
+    P.n = n; P.m = nc;
+    P.ptr.assign(n + 1, 0);
+    std::vector<int> mark(n, -1);
+    for (int i = 0; i < n; ++i) {
+      if (state[i] == 1) {
+        P.col.push_back(cid[i]);
+        P.val.push_back(1.);
+      } else {
+        for (int j = sp[i]; j < sp[i + 1]; ++j) if (state[si[j]] == 1) mark[si[j]] = i;
+        double neg = 0., pos = 0., sum = 0.;
+        for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) {
+          const int c = A.col[j];
+          if (c == i) continue;
+          (A.val[j] < 0. ? neg : pos) += A.val[j];
+          if (mark[c] == i) sum += A.val[j];
+        }
+        if (sum != 0.)
+          for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j)
+            if (A.col[j] != i && mark[A.col[j]] == i) {
+              P.col.push_back(cid[A.col[j]]);
+              P.val.push_back(-(neg / sum) * A.val[j] / (dia[i] + pos));
+            }
+      }
+      P.ptr[i + 1] = (int)P.col.size();
+    }
+    const CSR PT = transpose(P);
+    VLevel lv;
+    // R~ = P^T (I - A M): P^T - (P^T A) M
+    const CSR PA = matmul(PT, A);
+    auto axpy_rows = [](const CSR& X, const CSR& Y) {  // X - Y, rows sorted
+      CSR Z;
+      Z.n = X.n; Z.m = X.m;
+      Z.ptr.assign(X.n + 1, 0);
+      for (int i = 0; i < X.n; ++i) {
+        int a = X.ptr[i], b = Y.ptr[i];
+        while (a < X.ptr[i + 1] || b < Y.ptr[i + 1]) {
+          const int ca = a < X.ptr[i + 1] ? X.col[a] : INT32_MAX, cb = b < Y.ptr[i + 1] ? Y.col[b] : INT32_MAX;
+          Z.col.push_back(std::min(ca, cb));
+          Z.val.push_back((ca <= cb ? X.val[a] : 0.) - (cb <= ca ? Y.val[b] : 0.));
+          if (ca <= cb) ++a;
+          if (cb <= ca) ++b;
+        }
+        Z.ptr[i + 1] = (int)Z.col.size();
+      }
+      return Z;
+    };
+    auto sorted = [](CSR& X) {
+      std::vector<std::pair<int32_t, double>> r;
+      for (int i = 0; i < X.n; ++i) {
+        r.clear();
+        for (int j = X.ptr[i]; j < X.ptr[i + 1]; ++j) r.push_back({X.col[j], X.val[j]});
+        std::sort(r.begin(), r.end());
+        for (size_t k = 0; k < r.size(); ++k) { X.col[X.ptr[i] + k] = r[k].first; X.val[X.ptr[i] + k] = r[k].second; }
+      }
+    };
+    sorted(P);
+    CSR PAM = PA;
+    for (size_t j = 0; j < PAM.col.size(); ++j) PAM.val[j] *= M[PAM.col[j]];
+    lv.Rt = axpy_rows(PT, PAM);
+    CSR MAP = matmul(A, P);
+    CSR Ac = nc > 0 ? matmul(PT, MAP) : CSR();
+    for (int i = 0; i < n; ++i)
+      for (int j = MAP.ptr[i]; j < MAP.ptr[i + 1]; ++j) MAP.val[j] *= M[i];
+    const CSR Pt = axpy_rows(P, MAP);
+    CSR& U = lv.U;
+    U.n = n; U.m = n + nc;
+    U.ptr.assign(n + 1, 0);
+    for (int i = 0; i < n; ++i) {
+      for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) {
+        const int c = A.col[j];
+        U.col.push_back(c);
+        U.val.push_back((c == i ? 2. * M[i] : 0.) - M[i] * A.val[j] * M[c]);
+      }
+      for (int j = Pt.ptr[i]; j < Pt.ptr[i + 1]; ++j) {
+        U.col.push_back(n + Pt.col[j]);
+        U.val.push_back(Pt.val[j]);
+      }
+      U.ptr[i + 1] = (int)U.col.size();
+    }
+    h.levels.push_back(std::move(lv));
+    if (nc == 0) return;
+    A = drop_noise(Ac);
+  }
+  h.coarse = std::move(A);
+}
+
+int sell_lanes(const CSR& A) {
+  const double avg = A.n ? (double)A.col.size() / A.n : 0.;
+  int l = 4;
+  while (l < 16 && (size_t)A.n * l < 131072 && l < avg) l *= 2;
+  return l;
+}
+void sell_pack(const CSR& A, int lanes, std::vector<int32_t>& off, std::vector<int32_t>& col, std::vector<double>& val) {
+  const int R = 64 / lanes, ns = (A.n + R - 1) / R;
+  off.assign(ns + 1, 0);
+  for (int s = 0; s < ns; ++s) {
+    int w = 0;
+    for (int i = s * R; i < std::min(A.n, (s + 1) * R); ++i) w = std::max(w, A.ptr[i + 1] - A.ptr[i]);
+    off[s + 1] = off[s] + 64 * ((w + lanes - 1) / lanes);
+  }
+  col.assign(off[ns], 0);
+  val.assign(off[ns], 0.);
+  for (int i = 0; i < A.n; ++i)
+    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) {
+      const int k = j - A.ptr[i];
+      const size_t q = (size_t)off[i / R] + 64 * (k / lanes) + (i % R) * lanes + k % lanes;
+      col[q] = A.col[j];
+      val[q] = A.val[j];
+    }
+}
+
 void csr_check(const CSR& A) {
   if (A.n < 0 || A.m < 0 || (int64_t)A.ptr.size() != (int64_t)A.n + 1 || A.ptr[0] != 0 ||
       (size_t)A.ptr[A.n] != A.col.size() || A.col.size() != A.val.size())
@@ -724,29 +967,7 @@ void build_sa_amg(const CSR& A0, int coarse_enough, AMGHost& h) {
   AMGLevelHost last;
   last.A = A;
   h.levels.push_back(last);
-  // dense inverse of the coarsest matrix (Gauss-Jordan, partial pivoting)
-  const int n = A.n;
-  std::vector<double> a((size_t)n * n, 0.), inv((size_t)n * n, 0.);
-  for (int i = 0; i < n; ++i) {
-    inv[(size_t)i * n + i] = 1.;
-    for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) a[(size_t)i * n + A.col[j]] += A.val[j];
-  }
-  for (int c = 0; c < n; ++c) {
-    int p = c;
-    for (int r = c + 1; r < n; ++r) if (std::fabs(a[(size_t)r * n + c]) > std::fabs(a[(size_t)p * n + c])) p = r;
-    if (a[(size_t)p * n + c] == 0.) continue;  // singular direction: leave it out of the inverse
-    if (p != c)
-      for (int j = 0; j < n; ++j) { std::swap(a[(size_t)p * n + j], a[(size_t)c * n + j]); std::swap(inv[(size_t)p * n + j], inv[(size_t)c * n + j]); }
-    const double d = 1. / a[(size_t)c * n + c];
-    for (int j = 0; j < n; ++j) { a[(size_t)c * n + j] *= d; inv[(size_t)c * n + j] *= d; }
-    for (int r = 0; r < n; ++r) {
-      if (r == c) continue;
-      const double f = a[(size_t)r * n + c];
-      if (f == 0.) continue;
-      for (int j = 0; j < n; ++j) { a[(size_t)r * n + j] -= f * a[(size_t)c * n + j]; inv[(size_t)r * n + j] -= f * inv[(size_t)c * n + j]; }
-    }
-  }
-  h.coarse_inv = std::move(inv);
+  dense_inverse(A, h.coarse_inv);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -168,6 +168,33 @@ int proj_restart_basis(int m, int keep, const double* gcols, int ldg, double* g,
                        std::vector<double>& c);
 void build_sa_amg(const CSR& A, int coarse_enough, AMGHost& h);
 
+// V-cycle hierarchy of the Q1 vertex level and below: Ruge-Stueben coarsening with direct
+// interpolation (K. Stueben, J. Comput. Appl. Math. 128 (2001) 281-309), which on a mesh of quads
+// finds every second vertex in each direction and bilinear interpolation; V(1,1) with spai0
+// relaxation M.  A level's cycle is kept as two matrices, with P the interpolation:
+//   R~ = P^T (I - A M)                            f_{l+1} = R~ f_l
+//   U  = [ 2 M - M A M | (I - M A) P ]            u_l = U [f_l; u_{l+1}]
+// that is, relaxation from zero, residual and restriction in one product, and interpolation,
+// correction and the closing relaxation in one (u = M f + P u_c, then u + M (f - A u), multiplied
+// out).  coarse: the matrix of the last level, for a direct solve (n = 0: none).
+struct VLevel {
+  CSR Rt, U;
+};
+struct VHierarchy {
+  std::vector<VLevel> levels;
+  CSR coarse;
+};
+// Levels are added until at most coarse_enough unknowns are left.
+void build_vhierarchy(const CSR& A, int coarse_enough, VHierarchy& h);
+// Sliced ELL packing: wavefront s holds the rows [s R, (s + 1) R), R = 64 / lanes, `lanes` lanes a
+// row; its entries lie at off[s] + 64 g + lane for g below the slice's longest row in groups of
+// `lanes`.  Padding repeats column 0 with value 0.
+void sell_pack(const CSR& A, int lanes, std::vector<int32_t>& off, std::vector<int32_t>& col, std::vector<double>& val);
+// Lanes per row: enough to fill the device with a level's rows, at most about a row's length.
+int sell_lanes(const CSR& A);
+// Dense inverse (row-major) by Gauss-Jordan with partial pivoting; a singular direction is left out.
+void dense_inverse(const CSR& A, std::vector<double>& inv);
+
 // Throws std::invalid_argument unless A is a well-formed n x m CSR matrix (row pointers from
 // 0 to nnz, non-decreasing; every column index in [0, m)).
 void csr_check(const CSR& A);

@@ -286,13 +286,91 @@ __global__ void k_ell(int mode, int n, int w, const int32_t* __restrict__ col, c
   sparse_out(mode, i, s, x, f, y, M, xio);
 }
 
-// x = M f (spai0 from a zero guess)
-template <class R>
-__global__ void k_scale(int n, const R* __restrict__ M, const R* __restrict__ f, R* __restrict__ x,
-                        const int* __restrict__ F) {
-  if (F && !F[F_ACTIVE]) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = M[i] * f[i];
+// y = A x, A in sliced ELL (sell_pack): L lanes a row, 64 / L rows a wavefront, each wavefront's
+// loads contiguous and as many as its own longest row takes.
+template <int L, class R>
+__global__ __launch_bounds__(256) void k_sell(int n, const int32_t* __restrict__ off, const int32_t* __restrict__ col,
+                                              const R* __restrict__ val, const R* __restrict__ x, R* __restrict__ y,
+                                              const int* __restrict__ F) {
+  const int sl = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = sl * (64 / L) + lane / L;
+  if (sl * (64 / L) >= n || (F && !F[F_ACTIVE])) return;  // uniform over the wavefront
+  const int q0 = off[sl], q1 = off[sl + 1];
+  R s = 0;
+#pragma unroll 4
+  for (int q = q0 + lane; q < q1; q += 64) s += val[q] * x[col[q]];
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, L);
+  if (lane % L == 0 && row < n) y[row] = s;
+}
+
+// ---- dense inverse in place: Gauss-Jordan by blocks of kGJ columns, without pivoting (the caller
+// checks the result).  One block step at columns [c0, c0 + b):
+//   k_gj_diag: D = the diagonal block's inverse
+//   k_gj_panel: P = D A[c0.., :] outside the block's columns, D inside; C = A[:, c0..]
+//   k_gj_update: A[i, j] = P for the block's rows, else (j in the block ? 0 : A[i, j]) - C P
+constexpr int kGJ = 32;
+__global__ __launch_bounds__(kGJ * kGJ) void k_gj_diag(int n, int c0, int b, const double* __restrict__ A,
+                                                       double* __restrict__ D) {
+  __shared__ double a[kGJ][kGJ + 1];
+  const int r = threadIdx.x / kGJ, c = threadIdx.x % kGJ;
+  const bool in = r < b && c < b;
+  a[r][c] = in ? A[(size_t)(c0 + r) * n + c0 + c] : r == c ? 1. : 0.;
+  __syncthreads();
+  for (int k = 0; k < b; ++k) {
+    const double p = 1. / a[k][k], rk = a[r][k], kc = a[k][c], v = a[r][c];
+    __syncthreads();
+    if (r == k && c == k) a[r][c] = p;
+    else if (r == k) a[r][c] = kc * p;
+    else if (c == k) a[r][c] = -rk * p;
+    else a[r][c] = v - rk * kc * p;
+    __syncthreads();
+  }
+  D[r * kGJ + c] = a[r][c];
+}
+__global__ __launch_bounds__(256) void k_gj_panel(int n, int c0, int b, const double* __restrict__ A,
+                                                  const double* __restrict__ D, double* __restrict__ P,
+                                                  double* __restrict__ C) {
+  __shared__ double d[kGJ * kGJ];
+  for (int t = threadIdx.x; t < kGJ * kGJ; t += 256) d[t] = D[t];
+  __syncthreads();
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= n) return;
+  double v[kGJ];
+#pragma unroll
+  for (int k = 0; k < kGJ; ++k) v[k] = k < b ? A[(size_t)(c0 + k) * n + j] : 0.;
+  const bool in = j >= c0 && j < c0 + b;
+  for (int r = 0; r < kGJ; ++r) {
+    double s = 0.;
+#pragma unroll
+    for (int k = 0; k < kGJ; ++k) s += d[r * kGJ + k] * v[k];
+    P[(size_t)r * n + j] = r < b ? (in ? d[r * kGJ + j - c0] : s) : 0.;
+    C[(size_t)j * kGJ + r] = r < b ? A[(size_t)j * n + c0 + r] : 0.;
+  }
+}
+__global__ __launch_bounds__(256) void k_gj_update(int n, int c0, int b, double* __restrict__ A,
+                                                   const double* __restrict__ P, const double* __restrict__ C) {
+  __shared__ double cs[kGJ][kGJ + 1], ps[kGJ][kGJ];
+  const int i0 = blockIdx.y * kGJ, j0 = blockIdx.x * kGJ;
+  for (int t = threadIdx.x; t < kGJ * kGJ; t += 256) {
+    const int r = t / kGJ, c = t % kGJ;
+    cs[r][c] = i0 + r < n ? C[(size_t)(i0 + r) * kGJ + c] : 0.;
+    ps[r][c] = j0 + c < n ? P[(size_t)r * n + j0 + c] : 0.;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < kGJ * kGJ; t += 256) {
+    const int r = t / kGJ, c = t % kGJ, i = i0 + r, j = j0 + c;
+    if (i >= n || j >= n) continue;
+    double* a = A + (size_t)i * n + j;
+    if (i >= c0 && i < c0 + b) {
+      *a = P[(size_t)(i - c0) * n + j];
+      continue;
+    }
+    double s = (j >= c0 && j < c0 + b) ? 0. : *a;
+#pragma unroll
+    for (int k = 0; k < kGJ; ++k) s -= cs[r][k] * ps[k][c];
+    *a = s;
+  }
 }
 
 // Coarsest level: x = Ainv f (dense, row-major), one wavefront per row.
@@ -1097,8 +1175,27 @@ int csr_lanes(int n, size_t nnz) {
   return avg >= 24 ? 16 : avg >= 12 ? 8 : avg >= 6 ? 4 : avg >= 3 ? 2 : 1;
 }
 template <class R>
-void scale(hipStream_t s, int n, const R* M, const R* f, R* x, const int* F) {
-  hipLaunchKernelGGL(k_scale<R>, dim3((n + 255) / 256), dim3(256), 0, s, n, M, f, x, F);
+void sell(hipStream_t s, int n, int lanes, const int32_t* off, const int32_t* col, const R* val, const R* x, R* y,
+          const int* F) {
+  if (n <= 0) return;
+  const int slices = (n + 64 / lanes - 1) / (64 / lanes);
+  const dim3 grid((slices + 3) / 4), block(256);
+  switch (lanes) {
+    case 4: hipLaunchKernelGGL((k_sell<4, R>), grid, block, 0, s, n, off, col, val, x, y, F); break;
+    case 8: hipLaunchKernelGGL((k_sell<8, R>), grid, block, 0, s, n, off, col, val, x, y, F); break;
+    default: hipLaunchKernelGGL((k_sell<16, R>), grid, block, 0, s, n, off, col, val, x, y, F); break;
+  }
+}
+size_t dense_invert_work(int n) { return (size_t)kGJ * kGJ + 2 * (size_t)n * kGJ; }
+void dense_invert(hipStream_t s, int n, double* A, double* work) {
+  double *D = work, *P = D + kGJ * kGJ, *C = P + (size_t)n * kGJ;
+  const int nt = (n + kGJ - 1) / kGJ;
+  for (int c0 = 0; c0 < n; c0 += kGJ) {
+    const int b = std::min(kGJ, n - c0);
+    hipLaunchKernelGGL(k_gj_diag, dim3(1), dim3(kGJ * kGJ), 0, s, n, c0, b, A, D);
+    hipLaunchKernelGGL(k_gj_panel, dim3((n + 255) / 256), dim3(256), 0, s, n, c0, b, A, D, P, C);
+    hipLaunchKernelGGL(k_gj_update, dim3(nt, nt), dim3(256), 0, s, n, c0, b, A, P, C);
+  }
 }
 template <class R>
 void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F) {
@@ -1135,7 +1232,7 @@ void q1_probe_accum(hipStream_t s, int N, int K, const Tab& T, int rs, const dou
                        const R*, R*, const int*, int);                                                                 \
   template void ell<R>(hipStream_t, int, int, int, int, const int32_t*, const R*, const R*, const R*, R*, const R*,  \
                        R*, const int*);                                                                        \
-  template void scale<R>(hipStream_t, int, const R*, const R*, R*, const int*);                                       \
+  template void sell<R>(hipStream_t, int, int, const int32_t*, const int32_t*, const R*, const R*, R*, const int*);    \
   template void dense<R>(hipStream_t, int, const R*, const R*, R*, const int*);                                       \
   template void q1_gather<R>(hipStream_t, int, const int32_t*, const int32_t*, const R*, R*, const int*);
 HOC_LA_INST(double)

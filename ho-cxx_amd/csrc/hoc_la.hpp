@@ -55,8 +55,13 @@ int csr_lanes(int n, size_t nnz);  // lanes per row suited to a matrix's average
 template <class R>
 void ell(hipStream_t s, int mode, int n, int w, int lanes, const int32_t* col, const R* val, const R* x, const R* f,
          R* y, const R* M, R* xio, const int* F);
+// y = A x, A packed by sell_pack (lanes 4, 8 or 16).
 template <class R>
-void scale(hipStream_t s, int n, const R* M, const R* f, R* x, const int* F);
+void sell(hipStream_t s, int n, int lanes, const int32_t* off, const int32_t* col, const R* val, const R* x, R* y,
+          const int* F);
+// A (n x n, row-major) replaced by its inverse (Gauss-Jordan without pivoting); work: dense_invert_work(n).
+size_t dense_invert_work(int n);
+void dense_invert(hipStream_t s, int n, double* A, double* work);
 template <class R>
 void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F);
 template <class R>

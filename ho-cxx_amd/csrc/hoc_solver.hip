@@ -7,7 +7,7 @@
 //                            V-cycle: matrix-free fine level + Chebyshev(2) element-block
 //                            smoothing, continuous bilinear coarse space on the element
 //                            corners (Ac = Pc^T As Pc assembled from probes of As), then
-//                            smoothed aggregation below
+//                            Ruge-Stueben coarsening below
 //   velocity, wall vorticity k_trace + k_velocity
 //   diffusion + advection    k_stage (fused with k = dt (adv + diff) and the RK update)
 #include <hip/hip_runtime.h>
@@ -49,10 +49,8 @@ struct Prec {
   DBuf<R> Ga, Gb, Gc, fa, fb, gel, gface;  // FP32 copies (unused for FP64)
   DBuf<R> ac, fdm, qn;
   // PCG ping-pongs its direction between p and v; t: the smoother's second iterate
-  DBuf<R> r, z, p, q, rh, v, ph, sh, t, ec, rc, xc;
-  std::vector<std::unique_ptr<DevLevel<R>>> lv;  // Q1 vertex level and the SA levels below
-  DBuf<R> coarse_inv;
-  int coarse_n = 0;
+  DBuf<R> r, z, p, q, rh, v, ph, sh, t, ec, xc;
+  DevVHierarchy<R> lv;  // Q1 vertex level and below
   int prof_off = 0;  // offset of this precision's entries in the live kernel profile
   // set only while the iterations of a batched ensemble PCG are queued: the instances' live flags;
   // fine-level blocks of a stopped instance then return at once
@@ -62,24 +60,6 @@ struct Prec {
     for (auto* f : {&r, &z, &t}) f->alloc(D);
     for (auto* f : {&p, &q, &rh, &v, &ph, &sh}) f->alloc(krylov ? D : 0);
     ec.alloc((size_t)N * 4);
-  }
-  void upload_levels(const AMGHost& H) {
-    lv.clear();
-    for (size_t l = 0; l < H.levels.size(); ++l) {
-      auto L = std::make_unique<DevLevel<R>>();
-      L->A.upload(H.levels[l].A);
-      if (l + 1 < H.levels.size()) {
-        L->P.upload(H.levels[l].P);
-        L->Rs.upload(H.levels[l].R);
-        L->M.upload_as(H.levels[l].Minv);
-      }
-      const int n = H.levels[l].A.n;
-      L->f.alloc(n); L->u.alloc(n); L->t.alloc(n);
-      lv.push_back(std::move(L));
-    }
-    coarse_n = H.levels.back().A.n;
-    coarse_inv.upload_as(H.coarse_inv);
-    rc.alloc(H.levels[0].A.n); xc.alloc(H.levels[0].A.n);
   }
 };
 
@@ -518,7 +498,7 @@ struct Solver {
     HIPCHK(hipStreamSynchronize(stream));
   }
 
-  // Fine-level diagonal and element-level operator by probing, then SA below it.
+  // Fine-level diagonal and the Q1 operator by probing, then the levels below it.
   void build_hierarchy() {
     std::vector<int32_t> col1, col2;
     const int nc1 = color_elements(mesh, 1, col1);
@@ -599,12 +579,12 @@ struct Solver {
       for (auto& pr : rows[r0]) { A1.col.push_back(pr.first); A1.val.push_back(pr.second); }
       A1.ptr[r0 + 1] = (int)A1.col.size();
     }
-    // Aggregation stops at <= 768 unknowns, solved by a dense inverse: one launch reading
-    // at most 4.7 MB replaces a level's four sparse launches (each latency-bound at ~5 us).
-    AMGHost H;
-    build_sa_amg(A1, 768, H);
-    if (mixed) P32.upload_levels(H);
-    else P64.upload_levels(H);
+    VHierarchy H;
+    build_vhierarchy(A1, kCoarseDense, H);
+    std::vector<double> ci;
+    coarse_inverse(H.coarse, ci);
+    if (mixed) { P32.lv.upload(H, ci); P32.xc.alloc(nv); }
+    else { P64.lv.upload(H, ci); P64.xc.alloc(nv); }
     std::vector<double> hd(D);
     d2h(hd.data(), P64.t.p, D * sizeof(double));
     for (size_t i = 0; i < D; ++i)
@@ -663,10 +643,35 @@ struct Solver {
   }
 
   // ---------------------------------------------------------------------------------------
-  // V-cycle on the Q1 vertex level and below: u_l = V_l(f_l)
-  template <class R>
-  void coarse_cycle(Prec<R>& P, size_t l, const R* f, R* u, const int* Fp) {
-    csr_vcycle<R>(stream, P.lv, P.coarse_inv, P.coarse_n, l, f, u, Fp);
+  // Coarsening stops at this many unknowns, solved by their dense inverse: one launch in place of
+  // two per level below.
+  static constexpr int kCoarseDense = 1200;
+  // The dense inverse of the coarsest matrix, by the GPU's unpivoted elimination; a result that does
+  // not reproduce a vector to 1e-6 is replaced by the host's pivoted one.
+  void coarse_inverse(const CSR& A, std::vector<double>& ci) {
+    const int n = A.n;
+    ci.assign((size_t)n * n, 0.);
+    if (n == 0) return;
+    for (int i = 0; i < n; ++i)
+      for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) ci[(size_t)i * n + A.col[j]] += A.val[j];
+    DBuf<double> d, wk;
+    d.upload(ci);
+    wk.alloc(dense_invert_work(n));
+    dense_invert(stream, n, d, wk);
+    HIPCHK(hipGetLastError());
+    d2h(ci.data(), d.p, ci.size() * sizeof(double));
+    std::vector<double> x(n), b(n, 0.);
+    for (int i = 0; i < n; ++i) x[i] = 1. + std::sin(1.7 * i);
+    for (int i = 0; i < n; ++i)
+      for (int j = A.ptr[i]; j < A.ptr[i + 1]; ++j) b[i] += A.val[j] * x[A.col[j]];
+    double e = 0., xx = 0.;
+    for (int i = 0; i < n; ++i) {
+      double y = 0.;
+      for (int j = 0; j < n; ++j) y += ci[(size_t)i * n + j] * b[j];
+      e += (y - x[i]) * (y - x[i]);
+      xx += x[i] * x[i];
+    }
+    if (!(e <= 1e-12 * xx)) dense_inverse(A, ci);
   }
 
   // The first smoothing step of a V-cycle, z = omega B r (see PreArgs).
@@ -705,8 +710,8 @@ struct Solver {
     // restrict the residual to the corner vertices
     A.x = cur; A.y = P.ec.p; A.part = nullptr;
     fine(P, IN_X, EPI_RESTRICT, A);
-    q1_gather<R>(stream, nv, d_vptr, d_vinc, P.ec, P.rc, Fp);
-    coarse_cycle(P, 0, P.rc.p, P.xc.p, Fp);
+    q1_gather<R>(stream, nv, d_vptr, d_vinc, P.ec, P.lv.rhs(), Fp);
+    P.lv.cycle(stream, P.xc.p, Fp);
     // prolongate and post-smooth, the dampings in reverse: the cycle stays symmetric
     A.xc = P.xc.p;
     for (int k = cheb_m - 1; k >= 0; --k)
@@ -2786,7 +2791,7 @@ int hoc_stats_get(hoc_t h, hoc_stats* st) {
     Solver& s = h->s;
     std::memset(st, 0, sizeof(*st));
     st->n_elem = s.N; st->n_dofs = (int64_t)s.D; st->n_bedges = s.E;
-    st->n_levels = (int32_t)(s.mixed ? s.P32.lv.size() : s.P64.lv.size()) + 1;
+    st->n_levels = (int32_t)(s.mixed ? s.P32.lv.levels() : s.P64.lv.levels()) + 1;
     st->last_refinements = s.last_outer;
     st->precision = s.cfg.precision;
     st->n_nodes = s.mesh.n_nodes;
