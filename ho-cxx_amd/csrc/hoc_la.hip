@@ -98,32 +98,65 @@ __global__ void k_zero_if_flag(size_t n, R* __restrict__ x, const int* __restric
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x) x[v] = 0;
 }
 
-// Scalar logic of the Krylov solvers.  pa: np partials of q0 then np of q1.  With mirror
-// set (pinned host memory), thread 0 finally publishes seq * 4 + near * 2 + (active flag) there
-// with a system-scope store, whether or not the phase ran, so the host can follow the iterations
-// without a copy (the host reads only this word, so the store needs no ordering); near: still
-// active with the residual within 8x of the tolerance, so the next iteration may be the last.
+// Scalar logic of the Krylov solvers.  pa: np partials of q0 then np of q1; pbb (PH_INIT, may be
+// null): npbb partials of ||b||^2, summed into S[S_BB] first.  With mirror set (pinned host memory),
+// thread 0 finally publishes the solve's results (MirrorState) and, after a system-scope fence, the
+// status word seq * 4 + near * 2 + (active flag), whether or not the phase ran, so the host can
+// follow the iterations and take the results without a copy; near: still active with the residual
+// within 8x of the tolerance, so the next iteration may be the last.
+__device__ void publish(MirrorState* __restrict__ mirror, int seq, bool near, const double* __restrict__ S,
+                        const int* __restrict__ F) {
+  mirror->bb = S[S_BB];
+  mirror->rr = S[S_RR];
+  mirror->iter = F[F_ITER];
+  mirror->zero = F[F_ZERO];
+  __threadfence_system();
+  __hip_atomic_store(&mirror->status, seq * 4 + (near ? 2 : 0) + (F[F_ACTIVE] ? 1 : 0), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
 __device__ void finalize_phase(int phase, double a, double b, double* __restrict__ S, int* __restrict__ F,
                                int maxiter, const double* __restrict__ irr, const double* __restrict__ ibb,
                                int ninst);
-__global__ void k_finalize(int phase, const double* __restrict__ pa, int np, double* __restrict__ S,
-                           int* __restrict__ F, int maxiter, int* __restrict__ mirror, int seq,
-                           const double* __restrict__ irr, const double* __restrict__ ibb, int ninst) {
+constexpr int kFinThreads = 1024;  // the partials' loads in flight bound the kernel: 5461 pairs took
+                                   // 9.4 us with 256 threads
+__global__ __launch_bounds__(kFinThreads) void k_finalize(int phase, const double* __restrict__ pa, int np,
+                                                          const double* __restrict__ pbb, int npbb,
+                                                          double* __restrict__ S, int* __restrict__ F, int maxiter,
+                                                          MirrorState* __restrict__ mirror, int seq,
+                                                          const double* __restrict__ irr,
+                                                          const double* __restrict__ ibb, int ninst) {
   const bool live = phase == PH_INIT || phase == PH_BB || F[F_ACTIVE];
   const bool half = live && phase >= PH_OMEGA && F[F_HALF];  // BiCGSTAB converged at the half step
   if (live && !half) {  // uniform over the block
-    double a = 0., b = 0.;
-    for (int i = threadIdx.x; i < np; i += blockDim.x) { a += pa[i]; b += pa[np + i]; }
-    block_sum2(a, b);
-    if (threadIdx.x == 0) finalize_phase(phase, a, b, S, F, maxiter >= 0 ? maxiter : F[F_MAXIT], irr, ibb, ninst);
+    double a = 0., b = 0., c = 0.;
+    const bool second = phase == PH_INIT || phase == PH_UPD || phase >= PH_SNORM;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < np; i += kFinThreads) {
+      a += pa[i];
+      if (second) b += pa[np + i];
+    }
+    if (pbb)
+#pragma unroll 4
+      for (int i = threadIdx.x; i < npbb; i += kFinThreads) c += pbb[i];
+    __shared__ double sa[kFinThreads / 64], sb[kFinThreads / 64], sc[kFinThreads / 64];
+    a = wsum(a);
+    b = wsum(b);
+    c = wsum(c);
+    if ((threadIdx.x & 63) == 0) { sa[threadIdx.x >> 6] = a; sb[threadIdx.x >> 6] = b; sc[threadIdx.x >> 6] = c; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      a = b = c = 0.;
+      for (int w = 0; w < kFinThreads / 64; ++w) { a += sa[w]; b += sb[w]; c += sc[w]; }
+      if (pbb) S[S_BB] = c;
+      finalize_phase(phase, a, b, S, F, maxiter >= 0 ? maxiter : F[F_MAXIT], irr, ibb, ninst);
+    }
   } else if (half && phase == PH_RNORM && threadIdx.x == 0) {
     F[F_ACTIVE] = 0;
   }
   if (mirror && threadIdx.x == 0) {
     const int sq = seq >= 0 ? seq : ++F[F_SEQ];
-    const int act = F[F_ACTIVE] ? 1 : 0;
-    const int near = act && (irr ? S[S_IMAX] <= 64. : S[S_RR] <= 64. * S[S_TOL2] * S[S_BB]);  // within 8x of the tolerance
-    __hip_atomic_store(mirror, sq * 4 + near * 2 + act, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const bool near = F[F_ACTIVE] && (irr ? S[S_IMAX] <= 64. : S[S_RR] <= 64. * S[S_TOL2] * S[S_BB]);
+    publish(mirror, sq, near, S, F);
   }
 }
 __global__ void k_set_int(int* __restrict__ p, int v) { *p = v; }
@@ -373,19 +406,27 @@ __global__ __launch_bounds__(256) void k_gj_update(int n, int c0, int b, double*
   }
 }
 
-// Coarsest level: x = Ainv f (dense, row-major), one wavefront per row.
-template <class R>
-__global__ void k_dense(int n, const R* __restrict__ Ainv, const R* __restrict__ f, R* __restrict__ x,
-                        const int* __restrict__ F) {
+// Coarsest level: x = Ainv f (dense, row-major), T threads a row, so that the loads of a row of up
+// to 1200 are a few per thread: one wavefront a row took 9.5 us at 1024 rows.
+template <int T, class R>
+__global__ __launch_bounds__(T) void k_dense(int n, const R* __restrict__ Ainv, const R* __restrict__ f,
+                                             R* __restrict__ x, const int* __restrict__ F) {
   if (F && !F[F_ACTIVE]) return;
-  const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= n) return;
+  const R* a = Ainv + (size_t)blockIdx.x * n;
   R s = 0;
-  for (int j = lane; j < n; j += 64) s += Ainv[(size_t)row * n + j] * f[j];
+#pragma unroll 8
+  for (int j = threadIdx.x; j < n; j += T) s += a[j] * f[j];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) x[row] = s;
+  if constexpr (T > 64) {
+    __shared__ R red[T / 64];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = 0;
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) s += red[w];
+  }
+  if (threadIdx.x == 0) x[blockIdx.x] = s;
 }
 
 // ---- probing ---------------------------------------------------------------------------------
@@ -654,9 +695,10 @@ __global__ __launch_bounds__(256) void k_proj_dots3(size_t n, ProjSeg S, const d
   block_sums<3 * M>(s, part + (size_t)blockIdx.x * 3 * M);
 }
 // out[s * ostride + k] = sum of part[b * nv + k] over the blocks b of segment s (grid: nv x nseg),
-// strided partial sums, then a fixed-order tree
+// strided partial sums, then a fixed-order tree; sums k >= n1 go to out2[s * ostride2 + k - n1]
 __global__ __launch_bounds__(256) void k_proj_fin(ProjSeg S, int nv, const double* __restrict__ part,
-                                                  double* __restrict__ out, int ostride) {
+                                                  double* __restrict__ out, int ostride, int n1,
+                                                  double* __restrict__ out2, int ostride2) {
   const int k = blockIdx.x, sg = blockIdx.y;
   double s = 0.;
   for (int b = S.bbeg[sg] + threadIdx.x; b < S.bbeg[sg + 1]; b += 256) s += part[(size_t)b * nv + k];
@@ -664,7 +706,11 @@ __global__ __launch_bounds__(256) void k_proj_fin(ProjSeg S, int nv, const doubl
   __shared__ double red[4];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) out[(size_t)sg * ostride + k] = red[0] + red[1] + red[2] + red[3];
+  if (threadIdx.x == 0) {
+    s = red[0] + red[1] + red[2] + red[3];
+    if (k < n1) out[(size_t)sg * ostride + k] = s;
+    else out2[(size_t)sg * ostride2 + k - n1] = s;
+  }
 }
 // out += sum_j c_j X_j, c of the block's segment at c + s cstride
 template <int M>
@@ -803,8 +849,13 @@ __global__ __launch_bounds__(256) void k_proj_reseed(size_t n, ProjSeg S, int kk
 // (left in the span of the others), or whose Cholesky pivot falls below 1e-8 G_jj, is left out.
 // v[0, m) and v[m, 2m) become G^-1 v on the kept vectors and 0 on the others: Cholesky by one
 // wavefront, lane i holding row i of L in registers (m <= kProjMax <= 64); each column of L is
-// broadcast by lane shuffles, and L goes to LDS once for the back substitution, which reads it
-// by columns.
+// broadcast by lane reads (scalar registers; shuffles through the LDS unit took 25 us at m = 24), and
+// L goes to LDS once for the back substitution, which reads it by columns.
+__device__ __forceinline__ double lane_bcast(double v, int lane) {  // lane: a compile-time constant
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
 __global__ __launch_bounds__(64) void k_proj_solve(int m, const double* __restrict__ Gall, int ldg, int gstride,
                                                    double* __restrict__ vall, int vstride) {
   constexpr int MX = kProjMax;
@@ -820,35 +871,33 @@ __global__ __launch_bounds__(64) void k_proj_solve(int m, const double* __restri
   const double gd = row ? G[(size_t)i * ldg + i] : 0.;
   int ok = row && gd > 1e-24 * fabs(G[(size_t)i * ldg + i + 1]) && gd > 0.;
   double y0 = row ? v[i] : 0., y1 = row ? v[m + i] : 0.;
+  double il = 0.;  // lane j: 1 / L_jj
 #pragma unroll
   for (int j = 0; j < MX; ++j) {  // right-looking: column j, then the trailing rows
-    const double d = __shfl(a[j], j);
-    const bool okj = j < m && __shfl(ok, j) && d > 1e-8 * __shfl(gd, j);  // the same on every lane
-    if (okj) {
-      const double l = sqrt(d);
-      if (i == j) a[j] = l;
-      else if (i > j && ok) a[j] /= l;
+    if (j < m) {                  // uniform
+      const double d = lane_bcast(a[j], j);
+      const bool okj = __builtin_amdgcn_readlane(ok, j) && d > 1e-8 * lane_bcast(gd, j);  // the same on every lane
+      if (okj) {
+        const double ij = 1. / sqrt(d);
+        if (i == j) il = ij;
+        else if (i > j && ok) a[j] *= ij;
 #pragma unroll
-      for (int k = j + 1; k < MX; ++k) {
-        const double lkj = __shfl(a[j], k);
-        const int okk = __shfl(ok, k);
-        if (k < m && k <= i && i > j && ok && okk) a[k] -= a[j] * lkj;
-      }
-    } else if (i == j) {
-      ok = 0;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < MX; ++j) {  // L y = v
-    const double ljj = __shfl(a[j], j);
-    const double y0j = __shfl(y0, j) / ljj, y1j = __shfl(y1, j) / ljj;
-    if (j < m && __shfl(ok, j)) {
-      if (i == j) {
-        y0 = y0j;
-        y1 = y1j;
-      } else if (i > j && ok) {
-        y0 -= a[j] * y0j;
-        y1 -= a[j] * y1j;
+        for (int k = j + 1; k < MX; ++k) {
+          const double lkj = lane_bcast(a[j], k);
+          const int okk = __builtin_amdgcn_readlane(ok, k);
+          if (k < m && k <= i && i > j && ok && okk) a[k] -= a[j] * lkj;
+        }
+        // L y = v, column j
+        const double y0j = lane_bcast(y0, j) * ij, y1j = lane_bcast(y1, j) * ij;
+        if (i == j) {
+          y0 = y0j;
+          y1 = y1j;
+        } else if (i > j && ok) {
+          y0 -= a[j] * y0j;
+          y1 -= a[j] * y1j;
+        }
+      } else if (i == j) {
+        ok = 0;
       }
     }
   }
@@ -857,17 +906,19 @@ __global__ __launch_bounds__(64) void k_proj_solve(int m, const double* __restri
     for (int k = 0; k < MX; ++k) Ls[i][k] = a[k];
   }
   __syncthreads();
-  for (int j = m - 1; j >= 0; --j) {  // L^T x = y
-    if (!__shfl(ok, j)) continue;
-    const double ljj = Ls[j][j];
-    const double x0 = __shfl(y0, j) / ljj, x1 = __shfl(y1, j) / ljj;
-    if (i == j) {
-      y0 = x0;
-      y1 = x1;
-    } else if (i < j && ok) {
-      const double lji = Ls[j][i];
-      y0 -= lji * x0;
-      y1 -= lji * x1;
+#pragma unroll
+  for (int j = MX - 1; j >= 0; --j) {  // L^T x = y
+    if (j < m && __builtin_amdgcn_readlane(ok, j)) {
+      const double ij = lane_bcast(il, j);
+      const double x0 = lane_bcast(y0, j) * ij, x1 = lane_bcast(y1, j) * ij;
+      if (i == j) {
+        y0 = x0;
+        y1 = x1;
+      } else if (i < j && ok) {
+        const double lji = Ls[j][i];
+        y0 -= lji * x0;
+        y1 -= lji * x1;
+      }
     }
   }
   if (row) {
@@ -919,7 +970,7 @@ void proj_dots2(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* 
     constexpr int M = decltype(Mc)::value;
     hipLaunchKernelGGL(k_proj_dots2<M>, dim3(S.nb), dim3(256), 0, s, n, S, Y, t, b, part);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(2 * m, S.nseg), dim3(256), 0, s, S, 2 * m, part, out, ostride);
+  hipLaunchKernelGGL(k_proj_fin, dim3(2 * m, S.nseg), dim3(256), 0, s, S, 2 * m, part, out, ostride, 2 * m, nullptr, 0);
 }
 void proj_dots3(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* ax, const double* t,
                 const double* b, double* part, double* out, int ostride, double* gcol, int gstride) {
@@ -928,8 +979,7 @@ void proj_dots3(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* 
     constexpr int M = decltype(Mc)::value;
     hipLaunchKernelGGL(k_proj_dots3<M>, dim3(S.nb), dim3(256), 0, s, n, S, Y, ax, t, b, part);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(2 * m, S.nseg), dim3(256), 0, s, S, 3 * m, part, out, ostride);
-  hipLaunchKernelGGL(k_proj_fin, dim3(m, S.nseg), dim3(256), 0, s, S, 3 * m, part + 2 * m, gcol, gstride);
+  hipLaunchKernelGGL(k_proj_fin, dim3(3 * m, S.nseg), dim3(256), 0, s, S, 3 * m, part, out, ostride, 2 * m, gcol, gstride);
 }
 void proj_solve(hipStream_t s, const ProjSeg& S, int m, const double* G, int ldg, int gstride, double* v,
                 int vstride) {
@@ -950,7 +1000,7 @@ void proj_append(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const
   if (m < 0 || m > kProjMax || n == 0 || ldw > 256) return;
   hipLaunchKernelGGL(k_proj_append, dim3(S.nb), dim3(256), 0, s, n, S, m, mr, e, estride, psi, b, x, part, wcol,
                      wstride, ldw);
-  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride);
+  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride, 1, nullptr, 0);
 }
 void proj_ortho(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* X, const double* e,
                 int estride, const double* psi, const double* b, double* x, double* part, double* n0, int n0stride,
@@ -961,7 +1011,7 @@ void proj_ortho(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const 
     hipLaunchKernelGGL(k_proj_ortho<M>, dim3(S.nb), dim3(256), 0, s, n, S, mr, X, e, estride, psi, b, x, part, wcol,
                        wstride, ldw);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride);
+  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride, 1, nullptr, 0);
 }
 void proj_gcol(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* Y, const double* x,
                const double* ax, double* part, double* gcol, int gstride) {
@@ -969,7 +1019,7 @@ void proj_gcol(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const d
   proj_dispatch<0>(m, [&](auto Mc) {
     constexpr int M = decltype(Mc)::value;
     hipLaunchKernelGGL(k_proj_gcol<M>, dim3(S.nb), dim3(256), 0, s, n, S, mr, Y, x, ax, part);
-    hipLaunchKernelGGL(k_proj_fin, dim3(M + 1, S.nseg), dim3(256), 0, s, S, M + 1, part, gcol, gstride);
+    hipLaunchKernelGGL(k_proj_fin, dim3(M + 1, S.nseg), dim3(256), 0, s, S, M + 1, part, gcol, gstride, M + 1, nullptr, 0);
   });
 }
 void proj_gram(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* AX, double* part,
@@ -979,7 +1029,7 @@ void proj_gram(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y
     constexpr int M = decltype(Mc)::value;
     hipLaunchKernelGGL(k_proj_gram<M>, dim3(S.nb), dim3(256), 0, s, n, S, Y, AX, part);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(m * m, S.nseg), dim3(256), 0, s, S, m * m, part, out, m * m);
+  hipLaunchKernelGGL(k_proj_fin, dim3(m * m, S.nseg), dim3(256), 0, s, S, m * m, part, out, m * m, m * m, nullptr, 0);
 }
 void proj_reseed(hipStream_t s, size_t n, const ProjSeg& S, int m, int kk, const double* C, int cstride, double* X,
                  double* AX) {
@@ -1047,8 +1097,8 @@ template void seg_dot<float>(hipStream_t, const ProjSeg&, const double*, const f
 // One block: thread t handles instances t, t + 256, ..; the block then reduces "any active", the
 // largest residual ratio of the active instances and the sum of the residual norms.
 __global__ __launch_bounds__(256) void k_finalize_ens(int phase, EnsKry E, double* __restrict__ S,
-                                                      int* __restrict__ F, int maxiter, int* __restrict__ mirror,
-                                                      int seq) {
+                                                      int* __restrict__ F, int maxiter,
+                                                      MirrorState* __restrict__ mirror, int seq) {
   const bool live = phase == ENS_INIT || F[F_ACTIVE];
   __shared__ int sany[256];
   __shared__ double smax[256], ssum[256];
@@ -1126,12 +1176,11 @@ __global__ __launch_bounds__(256) void k_finalize_ens(int phase, EnsKry E, doubl
   }
   if (mirror) {
     const int sq = seq >= 0 ? seq : ++F[F_SEQ];
-    const int act = F[F_ACTIVE] ? 1 : 0;
-    const int near = act && S[S_IMAX] <= 64.;
-    __hip_atomic_store(mirror, sq * 4 + near * 2 + act, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    publish(mirror, sq, F[F_ACTIVE] && S[S_IMAX] <= 64., S, F);
   }
 }
-void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter, int* mirror, int seq) {
+void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter, MirrorState* mirror,
+                  int seq) {
   hipLaunchKernelGGL(k_finalize_ens, dim3(1), dim3(256), 0, s, phase, E, S, F, maxiter, mirror, seq);
 }
 void psi_predict(hipStream_t s, size_t n, double f, int extrap, double* psi, double* prev) {
@@ -1143,10 +1192,10 @@ void zero_if_flag(hipStream_t s, size_t n, R* x, const int* F) {
   hipLaunchKernelGGL(k_zero_if_flag<R>, dim3(vec_grid(n)), dim3(256), 0, s, n, x, F);
 }
 void set_int(hipStream_t s, int* p, int v) { hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, p, v); }
-void finalize(hipStream_t s, int phase, const double* part, int np, double* S, int* F, int maxiter, int* mirror,
-              int seq, const double* irr, const double* ibb, int ninst) {
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, phase, part, np, S, F, maxiter, mirror, seq, irr, ibb,
-                     ninst);
+void finalize(hipStream_t s, int phase, const double* part, int np, double* S, int* F, int maxiter, MirrorState* mirror,
+              int seq, const double* irr, const double* ibb, int ninst, const double* pbb, int npbb) {
+  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinThreads), 0, s, phase, part, np, pbb, npbb, S, F, maxiter, mirror,
+                     seq, irr, ibb, ninst);
 }
 template <class R>
 void csr(hipStream_t s, int mode, int n, const int32_t* ptr, const int32_t* col, const R* val, const R* x, const R* f,
@@ -1199,7 +1248,8 @@ void dense_invert(hipStream_t s, int n, double* A, double* work) {
 }
 template <class R>
 void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F) {
-  hipLaunchKernelGGL(k_dense<R>, dim3((n + 3) / 4), dim3(256), 0, s, n, Ainv, f, x, F);
+  if (n <= 256) hipLaunchKernelGGL((k_dense<64, R>), dim3(n), dim3(64), 0, s, n, Ainv, f, x, F);
+  else hipLaunchKernelGGL((k_dense<256, R>), dim3(n), dim3(256), 0, s, n, Ainv, f, x, F);
 }
 template <class R>
 void q1_gather(hipStream_t s, int nv, const int32_t* vptr, const int32_t* vinc, const R* ec, R* rc, const int* F) {

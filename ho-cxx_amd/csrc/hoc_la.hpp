@@ -15,10 +15,18 @@ namespace hoc {
 
 // Device scalar slots (double) and flags (int) of the Krylov solvers.
 // F_MAXIT: iteration budget read by finalize kernels launched with maxiter < 0.
-enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_COUNT = 16 };
+enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_RZN, S_COUNT = 16 };
 enum { F_ACTIVE = 0, F_ITER, F_ZERO, F_HALF, F_MAXIT, F_SEQ, F_COUNT = 8 };
 enum { PH_BB = 0, PH_INIT, PH_RZ, PH_PQ, PH_UPD, PH_RHO, PH_ALPHA, PH_SNORM, PH_OMEGA, PH_RNORM };
 enum { VOP_BICG_P = 0, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
+
+// What a solve's finalize kernels leave in pinned host memory: the status word, and the results of
+// the solve so far (stored before the status, ordered by a system-scope fence).
+struct MirrorState {
+  int status;
+  int iter, zero;
+  double bb, rr;
+};
 
 // K: points per direction of an element (1 for a plain vector); winv: device table of the
 // K*K inverse quadrature weights 1/(w_j w_i), indexed j K + i.
@@ -35,17 +43,19 @@ template <class R>
 void bicg_half(hipStream_t s, size_t n, R* x, const R* ph, const double* S, int* F);
 template <class R>
 void zero_if_flag(hipStream_t s, size_t n, R* x, const int* F);
-// mirror (optional): pinned host int that receives seq * 4 + near * 2 + (active flag) when the
-// kernel ends (near: active with the residual within 8x of the tolerance);
+// mirror (optional): pinned host state that receives the solve's results and the status word
+// seq * 4 + near * 2 + (active flag) when the kernel ends (near: active with the residual within 8x
+// of the tolerance);
 // seq < 0: the next number of the device counter F[F_SEQ] (incremented) instead of seq.
+// pbb (PH_INIT): npbb partials of ||b||^2 for S[S_BB], which PH_BB would otherwise have set.
 // maxiter < 0: the budget is read from F[F_MAXIT].
 // irr, ibb (optional, ninst values): per-instance squared residual and right-hand-side norms of
 // an ensemble; PH_INIT and PH_UPD then continue while some instance has irr > tol^2 ibb (tol^2 =
 // S[S_TOL2]; an instance with ibb = 0 is held to the largest ibb), and S[S_IMAX] keeps the
 // largest irr / (tol^2 ibb).
 void finalize(hipStream_t s, int phase, const double* part, int np, double* S, int* F, int maxiter,
-              int* mirror = nullptr, int seq = 0, const double* irr = nullptr, const double* ibb = nullptr,
-              int ninst = 0);
+              MirrorState* mirror = nullptr, int seq = 0, const double* irr = nullptr, const double* ibb = nullptr,
+              int ninst = 0, const double* pbb = nullptr, int npbb = 0);
 // *p = v, in stream order (a kernel: usable where a memset or copy may not be recorded).
 void set_int(hipStream_t s, int* p, int v);
 template <class R>
@@ -149,8 +159,8 @@ enum { ENS_INIT = 0, ENS_RZ, ENS_PQ, ENS_UPD };
 // instance); ENS_PQ: alpha_i; ENS_UPD: the instances' tests, the iteration count, F_ACTIVE =
 // any instance active within maxiter, S[S_RR] = sum ||r_i||^2, S[S_IMAX], and the status word as
 // finalize publishes it.  An instance with bb_i = 0 is held to the largest bb.
-void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter, int* mirror = nullptr,
-                  int seq = 0);
+void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter,
+                  MirrorState* mirror = nullptr, int seq = 0);
 // out[s] = sum over segment s of a . b (a FP64, b FP64 or FP32); skipped when F's active flag is
 // clear (F may be null), and out[s] left as it is for a segment whose flag in iact (may be null)
 // is 0.  part: S.nb values.

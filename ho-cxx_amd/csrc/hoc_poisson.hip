@@ -398,9 +398,21 @@ __device__ __forceinline__ void block_part(double a, double b, double* __restric
   }
 }
 
+// The sum of np partials, the same in every thread of every block.
+__device__ __forceinline__ double sum_parts(const double* __restrict__ part, int np) {
+  __shared__ double sp[kFineThreads / 64];
+  double s = 0.;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < np; i += kFineThreads) s += part[i];
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) sp[threadIdx.x >> 6] = s;
+  __syncthreads();
+  return sp[0] + sp[1] + sp[2] + sp[3];
+}
+
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> G, FineArgs<R> A) {
-  const bool go = !A.active || *A.active;
+  const bool go = !A.active || A.active[F_ACTIVE];
   if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
   if (!go) return;
   constexpr int K2 = K * K, EPW = Lay<K>::EPW, ES = Lay<K>::ES;
@@ -433,7 +445,21 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   R beta = 0;
   if constexpr (IN == IN_PUPD) {
     load_row<K>(static_cast<const RZ*>(A.z) + row, z);
-    beta = (R)(A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]]);
+    if (A.rz) {
+      const double rz = sum_parts(A.rz, A.np), be = A.active[F_ITER] > 0 ? rz / A.scal[S_RZ] : 0.;
+      const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+      if (!(rz > 0.) || !isfinite(rz)) {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
+        if (first) A.active[F_ACTIVE] = 0;
+        return;
+      }
+      if (first) {
+        A.scal[S_RZN] = rz;
+        A.scal[S_BETA] = be;
+      }
+      beta = (R)be;
+    } else {
+      beta = (R)(A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]]);
+    }
   }
   if constexpr (EPI == EPI_RESID || EPI == EPI_SMOOTH || EPI == EPI_RESTRICT) load_row<K>(A.b + row, b);
   R xo[4] = {0, 0, 0, 0};  // IN_PROL: own vertex values
@@ -579,7 +605,8 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
 
 template <int K, bool UPD, class R>
 __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G, PreArgs<R> A) {
-  if (A.active && !*A.active) return;
+  if (!UPD && !A.zero && A.active && !A.active[F_ACTIVE]) return;
+  if (UPD && A.active && !A.active[F_ACTIVE]) return;
   constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES, EPB = EPW * (kFineThreads / 64);
   __shared__ R lds[(kFineThreads / 64) * Lay<K>::TILE];
   const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -595,6 +622,13 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
   const int el = min(el0, G.N - 1);
   R* t = lds + wv * Lay<K>::TILE + le * ES;
   const size_t row = ((size_t)el * K + k) * K;
+  if (!UPD && A.zero) {  // a zero right-hand side: x = 0, as the reference's solver returns
+    if (*A.zero && live) {
+      const double z[K] = {};
+      store_row<K>(A.x + row, z);
+    }
+    if (A.active && !A.active[F_ACTIVE]) return;
+  }
   double r[K];
   load_row<K>(A.r + row, r);
   double p0 = 0., p1 = 0.;
@@ -603,7 +637,23 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
     load_row<K>(A.q + row, q);
     load_row<K>(A.p + row, p);
     load_row<K>(A.x + row, x);
-    const double al = A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]];
+    double al;
+    if (A.pq) {
+      const double pq = sum_parts(A.pq, A.np), rz = A.scal[S_RZN];
+      al = rz / pq;
+      const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+      if (!(pq > 0.) || !isfinite(al)) {
+        if (first) A.active[F_ACTIVE] = 0;
+        return;
+      }
+      if (first) {
+        A.scal[S_PQ] = pq;
+        A.scal[S_ALPHA] = al;
+        A.scal[S_RZ] = rz;
+      }
+    } else {
+      al = A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]];
+    }
     if (al != 0.) {
 #pragma unroll
       for (int i = 0; i < K; ++i) {

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "hoc_kernels.hpp"
+#include "hoc_la.hpp"
 
 namespace hoc {
 
@@ -25,6 +26,9 @@ constexpr int kFineThreads = 256;
 // Elements per wavefront: K lanes each, and a multiple of 4 so that a block's elements start on
 // a 16-byte boundary in every field.
 constexpr int fine_epw(int K) { return K == 2 ? 32 : K == 3 ? 20 : K == 4 ? 16 : K == 5 ? 12 : 10; }
+// Up to this many partials every block of the next kernel sums them itself, which saves a launch
+// (4.4 us in a chain of dependent kernels) for about 1 us; above, a finalize kernel does.
+constexpr int kInlineParts = 1024;
 inline int fine_blocks(int K, int N) {
   const int e = fine_epw(K) * (kFineThreads / 64);
   return (N + e - 1) / e;
@@ -73,10 +77,14 @@ struct FineArgs {
   const R* b = nullptr;
   R* y = nullptr;
   double omega = 0.;
-  const double* scal = nullptr;  // IN_PUPD: beta = scal[scal_idx], scal_idx < 0: scal[inst[el]]
+  double* scal = nullptr;  // IN_PUPD: beta = scal[scal_idx], scal_idx < 0: scal[inst[el]]
   int scal_idx = 0;
+  // IN_PUPD, small meshes: r.z as np partials, summed by every block; block 0 leaves the new r.z and
+  // beta in scal (S_RZN, S_BETA) and clears active on a breakdown
+  const double* rz = nullptr;
+  int np = 0;
   double* part = nullptr;    // [fine_blocks] sums, then [fine_blocks] second sums
-  const int* active = nullptr;
+  int* active = nullptr;     // the Krylov flags F (may be null)
   int* ran = nullptr;        // set to 1 when the launch worked, 0 when active made it return at once
 };
 
@@ -99,10 +107,15 @@ struct PreArgs {
   R* z = nullptr;
   R* r32 = nullptr;
   double omega = 0.;
-  const double* scal = nullptr;
+  double* scal = nullptr;
   int scal_idx = 0;
+  // small meshes: p.q as np partials, summed by every block (alpha = scal[S_RZN] / p.q); block 0
+  // leaves alpha and r.z in scal and clears active on a breakdown
+  const double* pq = nullptr;
+  int np = 0;
   double* part = nullptr;
-  const int* active = nullptr;
+  int* active = nullptr;     // the Krylov flags F (may be null)
+  const int* zero = nullptr; // q == null: x is set to zero where this flag is set
   double iw[6] = {0., 0., 0., 0., 0., 0.};  // 1 / w_k
 };
 hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G, const PreArgs<double>& A,

@@ -102,12 +102,12 @@ struct Solver {
   // state (the mixed-precision V-cycle); S/F = scalars and flags of the Krylov solve.
   Prec<double> P64;
   Prec<float> P32;
-  DBuf<double> part, S;
+  DBuf<double> part, part2, S;  // part2: p.q partials, and ||b||^2's before the first residual
   DBuf<int> F;
-  // Krylov progress published by the end-of-iteration finalize kernel (seq * 4 + near * 2 + active), in
-  // pinned coherent host memory; seq counts iterations over the handle's lifetime.
-  int* mirror = nullptr;
-  int* mirror_dev = nullptr;
+  // Krylov progress and results published by the end-of-iteration finalize kernel, in pinned coherent
+  // host memory; the status' sequence number counts iterations over the handle's lifetime.
+  MirrorState* mirror = nullptr;
+  MirrorState* mirror_dev = nullptr;
   int seq_next = 0;
   int nparts = 0;
   int nv = 0;                             // Q1 coarse space: element-corner vertices
@@ -281,10 +281,11 @@ struct Solver {
     }
     nparts = std::max(std::max(lap_blocks(N), fine_blocks(K, N)), vec_grid(D));
     part.alloc(2 * (size_t)nparts);
+    part2.alloc(2 * (size_t)nparts);
     S.alloc(S_COUNT); F.alloc(F_COUNT);
     if (!mirror) {
-      HIPCHK(hipHostMalloc((void**)&mirror, 64, hipHostMallocCoherent | hipHostMallocMapped));
-      __atomic_store_n(mirror, -2, __ATOMIC_RELEASE);
+      HIPCHK(hipHostMalloc((void**)&mirror, sizeof(MirrorState), hipHostMallocCoherent | hipHostMallocMapped));
+      __atomic_store_n(&mirror->status, -2, __ATOMIC_RELEASE);
       HIPCHK(hipHostGetDevicePointer((void**)&mirror_dev, mirror, 0));
     }
     build_hierarchy();
@@ -298,6 +299,8 @@ struct Solver {
     ensure_segments();  // (the timed iterations of an ensemble run its per-instance test)
     tune_launch_mode();
     invalidate_guess();
+    const double tol2 = cfg.tol * cfg.tol;
+    h2d(S.p + S_TOL2, &tol2, sizeof(double));
     time = 0.;
     smooth_ready = false;
     n_sp = 0;
@@ -429,9 +432,11 @@ struct Solver {
   }
   // p = z + beta p and q = As p in one launch (z in FP32 from the mixed-precision V-cycle).
   void direction_apply(Prec<double>& P, const void* z, bool z32, const double* p, double* pn, double* q,
-                       const double* scal, int scal_idx, double* partp, const int* active) {
+                       double* scal, int scal_idx, const double* rz, double* partp,
+                       int* active) {
     FineArgs<double> A;
     A.x = p; A.z = z; A.pn = pn; A.y = q; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = active;
+    A.rz = rz; A.np = rz ? fine_blocks(K, N) : 0;
     if (!z32) { fine(P, IN_PUPD, EPI_STORE, A); return; }
     const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
     if (rec) HIPCHK(hipEventRecord(prof.e0[prof.n], stream));
@@ -684,9 +689,11 @@ struct Solver {
     for (int k = 0; k < K; ++k) A.iw[k] = 1. / tab.wgt[k];
     return A;
   }
+  // xz (may be null): set to zero first when the right-hand side is zero.
   template <class R>
-  void vcycle_begin(Prec<R>& P, const double* rin, const int* Fp) {
+  void vcycle_begin(Prec<R>& P, const double* rin, int* Fp, double* xz = nullptr) {
     PreArgs<R> A = pre_args<R>(rin, P.t.p, cheb_w[0]);
+    if (xz) { A.x = xz; A.zero = Fp + F_ZERO; }
     if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
     A.active = Fp;
     P.G.iact = P.iact;
@@ -696,7 +703,7 @@ struct Solver {
   // P.t: the iterate ping-pongs between P.t and zout and ends in zout; if partp != nullptr,
   // partials of rr.zout are left there.
   template <class R>
-  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, const int* Fp) {
+  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, int* Fp) {
     R *cur = P.t.p, *nxt = zout;
     FineArgs<R> A;
     A.b = rr;
@@ -721,7 +728,7 @@ struct Solver {
   // z = M r: the V-cycle in the precision of P; for the FP64 Krylov method of a mixed-precision
   // handle, the FP32 V-cycle between a demotion of r and a promotion of z.  With partp set, the
   // partials of r . z are left there; returns their count (0 when partp is null).
-  int precond(const double* rin, double* zout, double* partp, const int* Fp) {
+  int precond(const double* rin, double* zout, double* partp, int* Fp) {
     if (mixed) {
       vcycle_begin(P32, rin, Fp);
       vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp);
@@ -743,7 +750,7 @@ struct Solver {
     if (near) *near = false;
     if (target < seq_first) return true;
     for (unsigned spin = 1;; ++spin) {
-      const int v = __atomic_load_n(mirror, __ATOMIC_ACQUIRE);
+      const int v = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
       if ((v >> 2) >= target) {
         if (near) *near = (v & 2) != 0;
         return (v & 1) != 0;
@@ -751,7 +758,7 @@ struct Solver {
       if ((spin & 4095) == 0) {
         const hipError_t q = hipStreamQuery(stream);
         if (q == hipSuccess) {
-          const int v2 = __atomic_load_n(mirror, __ATOMIC_ACQUIRE);
+          const int v2 = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
           if ((v2 >> 2) >= target) {
             if (near) *near = (v2 & 2) != 0;
             return (v2 & 1) != 0;
@@ -769,18 +776,19 @@ struct Solver {
   // maxit bounds the host loop; maxit_dev is the device budget (< 0: Fp[F_MAXIT]).
   //
   // Launch modes.  Direct: the host queues each iteration's kernels and waits for the status of
-  // the iteration before the last one it queued.  Graph: a hipGraph holding kGraphChunk
-  // iterations, captured once per set of buffers, is replayed; its end-of-iteration finalize
-  // kernels number themselves from the device counter F[F_SEQ], and the host waits one chunk
-  // behind.  The kernels and their order are the same, so both modes give the same iterates;
-  // graphs pay where the host's launch cost exceeds the kernels' run time (small meshes), and
-  // setup chooses by timing both (launch_mode 0).
-  static constexpr int kGraphChunk = 4;
+  // the iteration before the last one it queued.  Graph: the same with an iteration's kernels as one
+  // captured hipGraph (one per order of the two direction buffers and set of buffers); the captured
+  // end-of-iteration finalize takes its number from the device counter F[F_SEQ].  The kernels and
+  // their order are the same, so both modes give the same iterates; graphs pay where the host's
+  // launch cost exceeds the kernels' run time (small meshes), and setup chooses by timing both
+  // (launch_mode 0).
+  static constexpr int kTuneIters = 8;
   struct KGraph {
     hipGraph_t g = nullptr;
     hipGraphExec_t e = nullptr;
     const void* key[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     int maxit = 0;
+    bool odd = false;
   };
   std::vector<KGraph> kgraphs;
   bool use_graphs = false;
@@ -794,25 +802,27 @@ struct Solver {
   }
   // Before the first iteration.  PCG: the first smoothing step of the first V-cycle (an iteration
   // ends with the next one's); its direction needs no clearing, beta = 0 leaves the old one out.
-  void krylov_begin(double* r, const int* Fp) {
+  void krylov_begin(double* x, double* r, int* Fp) {
     Prec<double>& P = P64;
     if (krylov == HOC_KRYLOV_PCG) {
-      if (mixed) vcycle_begin(P32, r, Fp);
-      else vcycle_begin(P64, r, Fp);
+      if (mixed) vcycle_begin(P32, r, Fp, x);
+      else vcycle_begin(P64, r, Fp, x);
     } else {
+      zero_if_flag<double>(stream, D, x, Fp);
       vec<double>(stream, VOP_COPY, VA, D, P.rh, nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr);
       HIPCHK(hipMemsetAsync(P.p.p, 0, D * sizeof(double), stream));
       HIPCHK(hipMemsetAsync(P.v.p, 0, D * sizeof(double), stream));
     }
   }
   // PCG's update x += alpha p, r -= alpha q with the first smoothing step of the next V-cycle.
-  void pcg_update(double* x, double* r, const double* p, const double* scal, int scal_idx, double* partp,
-                  const int* Fp) {
+  void pcg_update(double* x, double* r, const double* p, double* scal, int scal_idx, const double* pq, double* partp,
+                  int* Fp) {
     auto go = [&](auto& P) {
       using R = std::remove_reference_t<decltype(*P.t.p)>;
       PreArgs<R> A = pre_args<R>(r, P.t.p, cheb_w[0]);
       if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
       A.x = x; A.p = p; A.q = P64.q.p; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = Fp;
+      A.pq = pq; A.np = pq ? fine_blocks(K, N) : 0;
       P.G.iact = P.iact;
       HIPCHK(launch_pre(K, P.T, P.G, A, stream));
     };
@@ -835,10 +845,12 @@ struct Solver {
       // r.z from the V-cycle's last sweep; in mixed precision the direction update reads z in FP32
       if (mixed) vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, part.p, Fp);
       else vcycle_rest(P64, r, P.z.p, part.p, Fp);
-      finalize(stream, PH_RZ, part, fb, Sp, Fp, maxit);
-      direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, Sp, S_BETA, part.p, Fp);
-      finalize(stream, PH_PQ, part, fb, Sp, Fp, maxit);
-      pcg_update(x, r, pnew, Sp, S_ALPHA, part.p, Fp);
+      const bool inl = fb <= kInlineParts;  // the next kernel sums the partials itself
+      if (!inl) finalize(stream, PH_RZ, part, fb, Sp, Fp, maxit);
+      direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, Sp, S_BETA,
+                      inl ? part.p : nullptr, part2.p, Fp);
+      if (!inl) finalize(stream, PH_PQ, part2, fb, Sp, Fp, maxit);
+      pcg_update(x, r, pnew, Sp, S_ALPHA, inl ? part2.p : nullptr, part.p, Fp);
       if (ens_pcg()) {  // every instance against its own right-hand side
         seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p);
         finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq, ens_rr.p, ens_bb.p, pseg.nseg);
@@ -889,28 +901,29 @@ struct Solver {
       seg_dot<double>(stream, pseg, r, P.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
     }
     finalize_ens(stream, ENS_RZ, E, Sp, Fp, maxit);
-    direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr, Fp);
+    direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr, nullptr,
+                    Fp);
     seg_dot<double>(stream, pseg, pnew, P.q.p, Fp, ens_part.p, ens_in.p, ens_act.p);
     finalize_ens(stream, ENS_PQ, E, Sp, Fp, maxit);
-    pcg_update(x, r, pnew, ens_alpha.p, -1, nullptr, Fp);
+    pcg_update(x, r, pnew, ens_alpha.p, -1, nullptr, nullptr, Fp);
     // ||r_i||^2 into ens_rr, where a stopped instance keeps its last value (its r no longer changes)
     seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p, ens_act.p);
     EnsKry Eu = E;
     Eu.in = ens_rr.p;
     finalize_ens(stream, ENS_UPD, Eu, Sp, Fp, maxit, mirror_dev, seq);
   }
-  // The instantiated graph of kGraphChunk iterations on these buffers (captured on first use).
-  static_assert(kGraphChunk % 2 == 0, "the direction buffers return to their places after a chunk");
-  hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit) {
+  // The instantiated graph of one iteration on these buffers (captured on first use).
+  hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit, bool odd) {
     const void* key[6] = {&P64, x, r, Sp, Fp, mixed ? (const void*)&P32 : nullptr};
     for (auto& k : kgraphs)
-      if (k.maxit == maxit && std::equal(key, key + 6, k.key)) return k.e;
+      if (k.maxit == maxit && k.odd == odd && std::equal(key, key + 6, k.key)) return k.e;
     KGraph kg;
     std::copy(key, key + 6, kg.key);
     kg.maxit = maxit;
+    kg.odd = odd;
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
-      for (int i = 0; i < kGraphChunk; ++i) krylov_iter(x, r, Sp, Fp, maxit, -1, i & 1);
+      krylov_iter(x, r, Sp, Fp, maxit, -1, odd);
     } catch (...) {
       hipGraph_t g = nullptr;
       (void)hipStreamEndCapture(stream, &g);
@@ -925,23 +938,17 @@ struct Solver {
   void krylov_solve(double* x, double* r, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
     const int maxit = maxit_dev;
     const int seq0 = seq_next;
-    krylov_begin(r, Fp);
-    if (use_graphs && !prof.on) {
-      hipGraphExec_t ge = krylov_graph(x, r, Sp, Fp, maxit);
+    krylov_begin(x, r, Fp);
+    const bool graphs = use_graphs && !prof.on;
+    hipGraphExec_t ge[2] = {nullptr, nullptr};
+    if (graphs) {
+      for (int k = 0; k < 2; ++k) ge[k] = krylov_graph(x, r, Sp, Fp, maxit, k == 1);
       set_int(stream, Fp + F_SEQ, seq_next - 1);
-      for (int done = 0;;) {
-        HIPCHK(hipGraphLaunch(ge, stream));
-        const int last = seq_next + kGraphChunk - 1;
-        seq_next += kGraphChunk;
-        done += kGraphChunk;
-        const bool fin = done > maxit_host + 2;
-        if (!poll(last, seq0, fin, kGraphChunk) || done > maxit_host + 4) break;
-      }
-      return;
     }
     for (int it = 0;; ++it) {
       const int seq = seq_next++;
-      krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
+      if (graphs) HIPCHK(hipGraphLaunch(ge[it & 1], stream));
+      else krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
       bool near = false;
       if (!poll(seq, seq0, it > maxit_host + 2, 1, &near) || it > maxit_host + 4) break;
       // the previous iteration ended within 8x of the tolerance: the one just queued is likely
@@ -950,9 +957,9 @@ struct Solver {
     }
   }
 
-  // Launch mode (launch_mode 0): the same 2 kGraphChunk iterations of a solve on a random
-  // right-hand side, queued directly and replayed from the captured graph; graphs are used when
-  // they take under 85% of the direct time.  The solve's state is reset afterwards.
+  // Launch mode (launch_mode 0): the same kTuneIters iterations of a solve on a random right-hand
+  // side, queued directly and replayed from the captured graphs; graphs are used when they take under
+  // 85% of the direct time.  The solve's state is reset afterwards.
   void tune_launch_mode() {
     clear_graphs();
     use_graphs = cfg.launch_mode == 2;
@@ -965,20 +972,19 @@ struct Solver {
     const double sv[2] = {1., 0.};  // S_BB = 1, S_TOL2 = 0: every tuning iteration stays active
     h2d(S.p + S_BB, &sv[0], sizeof(double));
     h2d(S.p + S_TOL2, &sv[1], sizeof(double));
-    const int maxit = std::max(cfg.maxiter, 4 * kGraphChunk);
+    const int maxit = std::max(cfg.maxiter, 2 * kTuneIters);
     auto run = [&](bool graph) {
       HIPCHK(hipMemsetAsync(psi.p, 0, D * sizeof(double), stream));
-      outer_residual();
-      krylov_begin(P64.r.p, F.p);
-      hipGraphExec_t ge = graph ? krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit) : nullptr;
+      outer_residual(nullptr);
+      krylov_begin(psi.p, P64.r.p, F.p);
+      hipGraphExec_t ge[2] = {nullptr, nullptr};
+      for (int k = 0; k < 2 && graph; ++k) ge[k] = krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit, k == 1);
       HIPCHK(hipStreamSynchronize(stream));
       const auto t0 = std::chrono::steady_clock::now();
-      if (graph) {
-        set_int(stream, F.p + F_SEQ, seq_next - 1);
-        for (int c = 0; c < 2; ++c) HIPCHK(hipGraphLaunch(ge, stream));
-        seq_next += 2 * kGraphChunk;
-      } else {
-        for (int i = 0; i < 2 * kGraphChunk; ++i) krylov_iter(psi.p, P64.r.p, S.p, F.p, maxit, seq_next++, i & 1);
+      if (graph) set_int(stream, F.p + F_SEQ, seq_next - 1);
+      for (int i = 0; i < kTuneIters; ++i, ++seq_next) {
+        if (graph) HIPCHK(hipGraphLaunch(ge[i & 1], stream));
+        else krylov_iter(psi.p, P64.r.p, S.p, F.p, maxit, seq_next, i & 1);
       }
       HIPCHK(hipStreamSynchronize(stream));
       return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -996,19 +1002,21 @@ struct Solver {
 
   // FP64 residual r = bs - As psi with the reference's unscaled norm, and the solve's
   // convergence state in (S, F).
-  void outer_residual() {
+  // pbb (may be null): lap_blocks(N) partials of ||b||^2 for S[S_BB].
+  void outer_residual(const double* pbb) {
     const int lb = fine_blocks(K, N);
     residual_As(psi.p, bs.p, P64.r.p, part.p);
     if (ens_pcg()) {
       seg_norm2(stream, pseg, VA, P64.r.p, nullptr, ens_part.p, ens_rr.p);
-      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, ens_rr.p, ens_bb.p, pseg.nseg);
+      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, ens_rr.p, ens_bb.p, pseg.nseg, pbb,
+               lap_blocks(N));
       if (ens_batched()) {
         EnsKry E = ensk();
         E.in = ens_rr.p;
         finalize_ens(stream, ENS_INIT, E, S, F, cfg.maxiter);
       }
     } else {
-      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter);
+      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, nullptr, nullptr, 0, pbb, lap_blocks(N));
     }
   }
 
@@ -1359,19 +1367,18 @@ struct Solver {
 
   void poisson(const double* omega) {
     guess_before_solve();
-    const int lb = lap_blocks(N);
     const int maxit = cfg.maxiter;
-    const double tol2 = cfg.tol * cfg.tol;
-    HIPCHK(hipMemcpyAsync(S.p + S_TOL2, &tol2, sizeof(double), hipMemcpyHostToDevice, stream));
-    HIPCHK(launch_rhs(K, N, T, G, omega, rhs_bc ? rhs_bc : b_psi.p, bs, part, stream));
+    HIPCHK(launch_rhs(K, N, T, G, omega, rhs_bc ? rhs_bc : b_psi.p, bs, part2, stream));
     const bool proj = proj_on() && (!std::isnan(stage_tau) || proj_force);
     if (proj) proj_before(bs);
-    finalize(stream, PH_BB, part, lb, S, F, maxit);
+    bool have_bb = false;
     if (ens_pcg()) {
       // PCG: the iterations continue while some instance has ||r_i|| > tol ||b_i||
       ensure_segments();
       seg_norm2(stream, pseg, VA, bs, nullptr, ens_part.p, ens_bb.p);
     } else if (n_inst > 1) {
+      finalize(stream, PH_BB, part2, lap_blocks(N), S, F, maxit);
+      have_bb = true;
       // BiCGSTAB: ||b - A psi|| <= tol min_i ||b_i|| bounds every instance's own relative residual
       // (instances with a zero right-hand side are left out of the minimum)
       inst_norms(stream, VA, n_inst, d_ioff, K2, bs, d_inorm);
@@ -1383,36 +1390,29 @@ struct Solver {
       double mx = 0., mn = HUGE_VAL;
       for (double v : bi) mx = std::max(mx, v);
       for (double v : bi) if (v > 1e-30 * mx) mn = std::min(mn, v);
+      const double tol2 = cfg.tol * cfg.tol;
       const double t2 = (bb > 0. && mn < HUGE_VAL) ? tol2 * mn / bb : tol2;
       HIPCHK(hipMemcpyAsync(S.p + S_TOL2, &t2, sizeof(double), hipMemcpyHostToDevice, stream));
       HIPCHK(hipStreamSynchronize(stream));
     }
-    outer_residual();
-    zero_if_flag<double>(stream, D, psi, F);
-    double hs[S_COUNT];
-    int hf[F_COUNT];
-    auto read_state = [&](const double* Sp, const int* Fp) {
-      HIPCHK(hipMemcpyAsync(hs, Sp, sizeof(hs), hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipMemcpyAsync(hf, Fp, sizeof(hf), hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipStreamSynchronize(stream));
-    };
+    outer_residual(have_bb ? nullptr : part2.p);
     // FP64: the FP64 V-cycle; mixed: the FP32 V-cycle (precond), the Krylov vectors, the operator
-    // application and the stopping test in FP64 either way.
+    // application and the stopping test in FP64 either way.  The results arrive with the status of
+    // the last iteration, so the stream goes on without a copy or a wait for it to drain.
     krylov_solve(psi.p, P64.r.p, S.p, F.p, maxit, maxit);
-    read_state(S, F);
-    const int iters = hf[F_ITER], outer = 0;
+    const MirrorState res = *mirror;
     // statistics
-    last_iters = iters;
-    last_outer = outer;
-    if (!std::isfinite(hs[S_BB]) || !std::isfinite(hs[S_RR])) {
+    last_iters = res.iter;
+    last_outer = 0;
+    if (!std::isfinite(res.bb) || !std::isfinite(res.rr)) {
       last_rel = std::nan("");
       throw StatusError(HOC_ENAN, "NaN/Inf in the Poisson right-hand side or residual");
     }
-    last_rel = hs[S_BB] > 0. ? std::sqrt(hs[S_RR] / hs[S_BB]) : 0.;
-    if (hf[F_ZERO]) last_rel = 0.;
+    last_rel = res.bb > 0. ? std::sqrt(res.rr / res.bb) : 0.;
+    if (res.zero) last_rel = 0.;
     total_iters += last_iters;
     ++n_solves;
-    if (proj && !hf[F_ZERO]) proj_after(bs);
+    if (proj && !res.zero) proj_after(bs);
     guess_after_solve();
     if (!std::isfinite(last_rel)) throw StatusError(HOC_ENAN, "NaN/Inf in the Poisson solve");
     if (cfg.fail_on_noconv && last_rel > cfg.tol)

@@ -73,7 +73,7 @@ typedef struct {
                                      (0 = 1/10)                                          */
   int32_t launch_mode;            /* Krylov iterations: 0 = chosen at hoc_setup by timing
                                      both, 1 = kernels queued one by one, 2 = replays of a
-                                     captured hipGraph of 4 iterations (same iterates)   */
+                                     captured hipGraph of an iteration (same iterates)   */
 } hoc_config;
 
 typedef struct {
