@@ -103,12 +103,36 @@ __device__ __forceinline__ void cols_to_rows(R* t, int k, const R (&col)[K], R (
   for (int i = 0; i < K; ++i) row[i] = t[k * RS + i];
 }
 
+// Even and odd parts of a line, and back.
 template <int K, class R>
-__device__ __forceinline__ R pick(const R (&a)[6], int k) {
-  R v = a[0];
+__device__ __forceinline__ void split(const R (&u)[K], R (&e)[3], R (&o)[3]) {
 #pragma unroll
-  for (int i = 1; i < K; ++i) v = k == i ? a[i] : v;
-  return v;
+  for (int i = 0; i < K / 2; ++i) {
+    e[i] = u[i] + u[K - 1 - i];
+    o[i] = u[i] - u[K - 1 - i];
+  }
+  if (K & 1) e[K / 2] = u[K / 2];
+}
+template <int K, class R>
+__device__ __forceinline__ void join(const R (&e)[3], const R (&o)[3], R (&u)[K]) {
+#pragma unroll
+  for (int i = 0; i < K / 2; ++i) {
+    u[i] = e[i] + o[i];
+    u[K - 1 - i] = e[i] - o[i];
+  }
+  if (K & 1) u[K / 2] = e[K / 2];
+}
+
+// 1 / x for the smoother's scales, x > 0 and normal: the hardware estimate and two Newton steps (to
+// within an ulp or two; the quotient's exact rounding takes twice the instructions).
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.), r, r);
+  return fma(fma(-x, r, 1.), r, r);
+}
+__device__ __forceinline__ float recip(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.f), r, r);
 }
 
 // One face point of a lane: the neighbour line's value v and inward derivative g at the shared
@@ -137,33 +161,42 @@ struct Op {
   // two faces L (lower) and U (upper).
   static __device__ __forceinline__ void line(const FineTab<R>& T, R a, const R (&u)[K], const Face<R>& L,
                                               const Face<R>& U, R (&out)[K]) {
-    R bl = 0, gl = 0, bu = 0, gu = 0;
+    constexpr int HE = (K + 1) / 2, HO = K / 2;
+    R e[3], o[3];
+    split<K>(u, e, o);
+    R ve = 0, vo = 0, ge = 0, go = 0;
 #pragma unroll
-    for (int m = 0; m < K; ++m) {
-      bl += u[m] * T.lv[m];
-      gl += u[m] * T.ld[m];
-      bu += u[K - 1 - m] * T.lv[m];
-      gu += u[K - 1 - m] * T.ld[m];
-    }
+    for (int i = 0; i < HE; ++i) { ve += e[i] * T.lvE[i]; ge += e[i] * T.ldE[i]; }
+#pragma unroll
+    for (int i = 0; i < HO; ++i) { vo += o[i] * T.lvO[i]; go += o[i] * T.ldO[i]; }
+    const R bl = ve + vo, bu = ve - vo, gl = ge + go, gu = ge - go;
     // common value minus own, and the common flux along the line
-    const R ig = R(1) / T.g0;
-    const R dl = L.nb >= 0 ? R(0.5) * (L.v - bl) : (L.neu ? gl * ig : -bl);
-    const R du = U.nb >= 0 ? R(0.5) * (U.v - bu) : (U.neu ? gu * ig : -bu);
-    R fl = (gl - dl * T.g0) * a, fu = -(gu - du * T.g0) * a;
-    if (L.nb >= 0) fl = R(0.5) * (fl - (L.g + dl * T.g0) * L.an);
-    if (U.nb >= 0) fu = R(0.5) * (fu + (U.g + du * T.g0) * U.an);
-    if (L.nb < 0 && L.neu) fl = 0;
-    if (U.nb < 0 && U.neu) fu = 0;
+    R dl = R(0.5) * (L.v - bl), du = R(0.5) * (U.v - bu);
+    if (L.nb < 0) dl = L.neu ? gl * T.ig0 : -bl;
+    if (U.nb < 0) du = U.neu ? gu * T.ig0 : -bu;
+    const R tl = (gl - dl * T.g0) * a, tu = (gu - du * T.g0) * a;  // own inward fluxes
+    R fl = R(0.5) * (tl - (L.g + dl * T.g0) * L.an), fu = R(0.5) * ((U.g + du * T.g0) * U.an - tu);
+    if (L.nb < 0) fl = L.neu ? R(0) : tl;
+    if (U.nb < 0) fu = U.neu ? R(0) : -tu;
     fl -= a * (gl + dl * T.m0 - du * T.m1);
     fu -= a * (dl * T.m1 - gu - du * T.m0);
-    const R adl = a * dl, adu = a * du;
+    const R se = a * (dl + du), so = a * (dl - du), ce = fl - fu, co = fl + fu;
+    R re[3], ro[3];
 #pragma unroll
-    for (int i = 0; i < K; ++i) {
-      R s = 0;
+    for (int i = 0; i < HE; ++i) {
+      R t = 0;
 #pragma unroll
-      for (int d = 0; d < K; ++d) s += u[d] * T.DD[d][i];
-      out[i] = a * s + (adl * T.Dg[i] + adu * T.Dg[K - 1 - i]) + (fl * T.gd[i] - fu * T.gd[K - 1 - i]);
+      for (int d = 0; d < HE; ++d) t += e[d] * T.DDE[d][i];
+      re[i] = a * t + (se * T.DgE[i] + ce * T.gdE[i]);
     }
+#pragma unroll
+    for (int i = 0; i < HO; ++i) {
+      R t = 0;
+#pragma unroll
+      for (int d = 0; d < HO; ++d) t += o[d] * T.DDO[d][i];
+      ro[i] = a * t + (so * T.DgO[i] + co * T.gdO[i]);
+    }
+    join<K>(re, ro, out);
   }
 
   static __device__ __forceinline__ void apply(const FineTab<R>& T, const FineGeo<R>& G, int el, int k, R* t, R* tf,
@@ -181,7 +214,6 @@ struct Op {
     } else {
       // common values: interior average, 0 on Dirichlet faces; Neumann faces from the K x K system
       // (src/HO_2D.cpp:2872-2927) solved at setup
-      const R ig = R(1) / T.g0;
       R bv[4], gi[4], cv[4], cg[4];
       for (int f = 0; f < 4; ++f) { bv[f] = 0; gi[f] = 0; }
 #pragma unroll
@@ -199,7 +231,7 @@ struct Op {
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         cv[f] = F[f].nb >= 0 ? R(0.5) * (bv[f] + F[f].v) : R(0);
-        tf[f * K + k] = F[f].nb < 0 && F[f].neu ? bv[f] + gi[f] * ig : cv[f];
+        tf[f * K + k] = F[f].nb < 0 && F[f].neu ? bv[f] + gi[f] * T.ig0 : cv[f];
       }
       wave_fence();
       R Dk[K];  // column k of the derivative matrix
@@ -309,44 +341,59 @@ struct Op {
   }
 };
 
-// r <- B r (rows): the element blocks' inverse by fast diagonalisation.
+// r <- B r (rows): the element blocks' inverse by fast diagonalisation.  lamk: T.lam of the lane.
 template <int K, class R>
-__device__ __forceinline__ void block_inverse(const FineTab<R>& T, const FineGeo<R>& G, int el, int k, R* t, R (&r)[K]) {
+__device__ __forceinline__ void block_inverse(const FineTab<R>& T, const FineGeo<R>& G, int el, int k, R lamk, R* t,
+                                              R (&r)[K]) {
   const R a = G.ac[(size_t)el * 2], c = G.ac[(size_t)el * 2 + 1];
   const int ft = G.ftype[el];
   R s[K], q[K];
-  if (__all(ft == 0)) {  // every element of the wavefront interior: the tables are scalars
+  if (__all(ft == 0)) {  // every element of the wavefront interior: even and odd eigenvectors
+    constexpr int HE = (K + 1) / 2, HO = K / 2;
+    R e[3], o[3];
+    auto forward = [&](const R (&in)[K], R (&out)[K]) {
+      split<K>(in, e, o);
 #pragma unroll
-    for (int i = 0; i < K; ++i) {
-      R v = 0;
+      for (int b = 0; b < HE; ++b) {
+        R v = 0;
 #pragma unroll
-      for (int j = 0; j < K; ++j) v += T.S[j][i] * r[j];
-      s[i] = v;
-    }
+        for (int i = 0; i < HE; ++i) v += T.SE[i][b] * e[i];
+        out[b] = v;
+      }
+#pragma unroll
+      for (int b = 0; b < HO; ++b) {
+        R v = 0;
+#pragma unroll
+        for (int i = 0; i < HO; ++i) v += T.SO[i][b] * o[i];
+        out[HE + b] = v;
+      }
+    };
+    auto backward = [&](const R (&in)[K], R (&out)[K]) {
+#pragma unroll
+      for (int i = 0; i < HE; ++i) {
+        R v = 0;
+#pragma unroll
+        for (int b = 0; b < HE; ++b) v += T.SE[i][b] * in[b];
+        e[i] = v;
+      }
+#pragma unroll
+      for (int i = 0; i < HO; ++i) {
+        R v = 0;
+#pragma unroll
+        for (int b = 0; b < HO; ++b) v += T.SO[i][b] * in[HE + b];
+        o[i] = v;
+      }
+      join<K>(e, o, out);
+    };
+    forward(r, s);
     rows_to_cols<K>(t, k, s, q);
-    const R al = a * pick<K>(T.lam, k);
+    const R al = a * lamk;
+    forward(q, s);
 #pragma unroll
-    for (int b = 0; b < K; ++b) {
-      R v = 0;
-#pragma unroll
-      for (int j = 0; j < K; ++j) v += T.S[j][b] * q[j];
-      s[b] = v / (al + c * T.lam[b]);
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      R v = 0;
-#pragma unroll
-      for (int b = 0; b < K; ++b) v += T.S[j][b] * s[b];
-      q[j] = v;
-    }
+    for (int b = 0; b < K; ++b) s[b] *= recip(al + c * T.lam[b]);
+    backward(s, q);
     cols_to_rows<K>(t, k, q, s);
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      R v = 0;
-#pragma unroll
-      for (int j = 0; j < K; ++j) v += T.S[i][j] * s[j];
-      r[i] = v;
-    }
+    backward(s, r);
     return;
   }
   const R* fx = G.fdm + (ft & 15) * (K + K * K);
@@ -365,7 +412,7 @@ __device__ __forceinline__ void block_inverse(const FineTab<R>& T, const FineGeo
     R v = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j) v += fy[K + j * K + b] * q[j];
-    s[b] = v / (al + c * fy[b]);
+    s[b] = v * recip(al + c * fy[b]);
   }
 #pragma unroll
   for (int j = 0; j < K; ++j) {
@@ -435,13 +482,19 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   R* t = lds + wv * (Lay<K>::TILE + EPW * FS) + le * ES;
   R* tf = lds + wv * (Lay<K>::TILE + EPW * FS) + Lay<K>::TILE + le * FS;
   const size_t row = ((size_t)el * K + k) * K;
+  const R wk = G.lane[4 * k], xk = G.lane[4 * k + 1], lamk = G.lane[4 * k + 2];
+  (void)wk;
+  (void)xk;
+  (void)lamk;
 
   // connectivity and every global read of the kernel, issued before the arithmetic
   const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
   const int nbf = G.nbf[el];
   R u[K], z[K], b[K];
   (void)z;
-  load_row<K>(A.x + row, u);
+  // a solve's first direction is z: the old one, of another solve, is not read
+  const bool first_dir = IN == IN_PUPD && A.active[F_ITER] == 0;
+  if (!first_dir) load_row<K>(A.x + row, u);
   R beta = 0;
   if constexpr (IN == IN_PUPD) {
     load_row<K>(static_cast<const RZ*>(A.z) + row, z);
@@ -467,9 +520,10 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     const int4 v = *reinterpret_cast<const int4*>(G.ev + (size_t)el * 4);
     xo[0] = A.xc[v.x]; xo[1] = A.xc[v.y]; xo[2] = A.xc[v.z]; xo[3] = A.xc[v.w];
   }
-  // the four neighbours' lines through the lane's face points, from the shared face inward: all
+  // The four neighbours' lines through the lane's face points, from the shared face inward: all
   // loads unconditional (a boundary face reads the element's own line and ignores it), so that
-  // their latencies overlap
+  // their latencies overlap.  Where every neighbour of the wavefront across a face meets it with
+  // its opposite face (meshes numbered and oriented alike), the line's stride is a constant.
   Face<R> F[4];
   const int nbs[4] = {nbr.x, nbr.y, nbr.z, nbr.w};
   R l[4][K], pl[IN == IN_PUPD ? 4 : 1][K], cn[IN == IN_PROL ? 4 : 1][4];
@@ -478,19 +532,46 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     const bool in = nbs[f] >= 0;
-    const int nb = in ? nbs[f] : el, fn = in ? (nbf >> (8 * f)) & 3 : f, kk = face_point<K>(f, fn, k), up = fn & 1;
-    const int start = fn < 2 ? kk * K + (up ? K - 1 : 0) : (up ? (K - 1) * K : 0) + kk;
-    const int step = fn < 2 ? (up ? -1 : 1) : (up ? -K : K);
-    const size_t o = (size_t)nb * K2 + start;
-    if constexpr (IN == IN_PUPD) {
+    const int nb = in ? nbs[f] : el, fn = in ? (nbf >> (8 * f)) & 3 : f ^ 1;
+    F[f].nb = nbs[f];
+    if (__all(fn == (f ^ 1))) {
+      const size_t o = (size_t)nb * K2;
+      auto line = [&](const auto* g, R (&v)[K]) {
+        if (f < 2) {
+          R w[K];
+          load_row<K>(g + o + k * K, w);
 #pragma unroll
-      for (int m = 0; m < K; ++m) {
-        l[f][m] = (R)(static_cast<const RZ*>(A.z) + o)[m * step];
-        pl[f][m] = (A.x + o)[m * step];
+          for (int m = 0; m < K; ++m) v[m] = f == 0 ? w[K - 1 - m] : w[m];
+        } else {
+#pragma unroll
+          for (int m = 0; m < K; ++m) v[m] = (R)g[o + k + (f == 2 ? (K - 1 - m) * K : m * K)];
+        }
+      };
+      if constexpr (IN == IN_PUPD) {
+        line(static_cast<const RZ*>(A.z), l[f]);
+        if (!first_dir) line(A.x, pl[f]);
+      } else {
+        line(A.x, l[f]);
       }
+      F[f].fn = f ^ 1;
+      F[f].kk = k;
     } else {
+      const int kk = face_point<K>(f, fn, k), up = fn & 1;
+      const int start = fn < 2 ? kk * K + (up ? K - 1 : 0) : (up ? (K - 1) * K : 0) + kk;
+      const int step = fn < 2 ? (up ? -1 : 1) : (up ? -K : K);
+      const size_t o = (size_t)nb * K2 + start;
+      if constexpr (IN == IN_PUPD) {
 #pragma unroll
-      for (int m = 0; m < K; ++m) l[f][m] = (A.x + o)[m * step];
+        for (int m = 0; m < K; ++m) l[f][m] = (R)(static_cast<const RZ*>(A.z) + o)[m * step];
+        if (!first_dir)
+#pragma unroll
+          for (int m = 0; m < K; ++m) pl[f][m] = (A.x + o)[m * step];
+      } else {
+#pragma unroll
+        for (int m = 0; m < K; ++m) l[f][m] = (A.x + o)[m * step];
+      }
+      F[f].fn = fn;
+      F[f].kk = kk;
     }
     if constexpr (IN == IN_PROL) {
       // vertex values at the corners of the shared face (along its parameter) and of the opposite one
@@ -500,25 +581,25 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
       cn[f][2] = A.xc[fn == 0 ? vn.y : fn == 2 ? vn.w : vn.x];
       cn[f][3] = A.xc[fn == 0 || fn == 2 ? vn.z : fn == 1 ? vn.w : vn.y];
     }
-    F[f].nb = nbs[f];
-    F[f].fn = fn;
-    F[f].kk = kk;
     if (GEO == GEO_ORTHO) F[f].an = G.ac[(size_t)nb * 2 + (fn >> 1)];
     else if (GEO == GEO_AFFINE) F[f].an = G.gface[((size_t)nb * 4 + fn) * 2];
-    else F[f].an = G.fa[((size_t)nb * 4 + fn) * K + kk];
+    else F[f].an = G.fa[((size_t)nb * 4 + fn) * K + F[f].kk];
   }
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     if (nbs[f] < 0) F[f].neu = G.sw[-1 - nbs[f]] != 0;
+    if constexpr (IN == IN_PUPD)
+      if (!first_dir)
+#pragma unroll
+        for (int m = 0; m < K; ++m) l[f][m] += beta * pl[f][m];
     R v = 0, g = 0;
 #pragma unroll
     for (int m = 0; m < K; ++m) {
-      if constexpr (IN == IN_PUPD) l[f][m] = beta != R(0) ? l[f][m] + beta * pl[f][m] : l[f][m];
       v += l[f][m] * T.lv[m];
       g += l[f][m] * T.ld[m];
     }
     if constexpr (IN == IN_PROL) {  // the neighbour's bilinear correction on that line
-      const R sk = R(0.5) * (R(1) + pick<K>(T.x, F[f].kk));
+      const R sk = R(0.5) * (R(1) + G.lane[4 * F[f].kk + 1]);
       const R near = cn[f][0] + sk * (cn[f][1] - cn[f][0]), far = cn[f][2] + sk * (cn[f][3] - cn[f][2]);
       v += near;
       g += R(0.5) * (far - near);
@@ -527,12 +608,17 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     F[f].g = g;
   }
   if constexpr (IN == IN_PUPD) {
+    if (first_dir) {
 #pragma unroll
-    for (int i = 0; i < K; ++i) u[i] = beta != R(0) ? z[i] + beta * u[i] : z[i];
+      for (int i = 0; i < K; ++i) u[i] = z[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < K; ++i) u[i] = z[i] + beta * u[i];
+    }
     if (live) store_row<K>(A.pn + row, u);
   }
   if constexpr (IN == IN_PROL) {
-    const R sy = R(0.5) * (R(1) + pick<K>(T.x, k));
+    const R sy = R(0.5) * (R(1) + xk);
     const R wl = xo[0] + sy * (xo[3] - xo[0]), wu = xo[1] + sy * (xo[2] - xo[1]);
 #pragma unroll
     for (int i = 0; i < K; ++i) u[i] += wl + R(0.5) * (R(1) + T.x[i]) * (wu - wl);
@@ -545,7 +631,6 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     if (live) store_row<K>(A.y + row, out);
     return;
   }
-  const R wk = pick<K>(T.w, k);
 #pragma unroll
   for (int i = 0; i < K; ++i) out[i] *= -(wk * T.w[i]);
   if constexpr (EPI == EPI_STORE) {
@@ -587,7 +672,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
         }
       }
     } else {  // EPI_SMOOTH
-      block_inverse<K>(T, G, el, k, t, res);
+      block_inverse<K>(T, G, el, k, lamk, t, res);
       const R om = (R)A.omega;
 #pragma unroll
       for (int i = 0; i < K; ++i) {
@@ -665,7 +750,7 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
         store_row<K>(A.r + row, r);
       }
     }
-    const double wk = pick<K>(A.iw, k);
+    const double wk = A.iwl[k];
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const double uw = r[i] * (wk * A.iw[i]);
@@ -679,7 +764,7 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
   if constexpr (sizeof(R) == 4) {
     if (live) store_row<K>(A.r32 + row, v);
   }
-  block_inverse<K>(T, G, el, k, t, v);
+  block_inverse<K>(T, G, el, k, G.lane[4 * k + 2], t, v);
   const R om = (R)A.omega;
 #pragma unroll
   for (int i = 0; i < K; ++i) v[i] *= om;

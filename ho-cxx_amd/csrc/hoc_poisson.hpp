@@ -41,6 +41,7 @@ struct FineGeo {
   const R* ac;           // [N][2] mean metrics (g22/J, g11/J) over the element: B's scales, and the
                          // metrics themselves where they are constant and orthogonal
   const R* fdm;          // [9] per pair of end kinds: eigenvalues [K], eigenvectors [K][K]
+  const R* lane;         // [K][4] weight, point and interior eigenvalue of a lane
   const uint16_t* ftype; // [N] kinds of the west/east and south/north ends: 9-way codes tx + 16 ty
   const R* gel;          // [N][3]    Ga, Gb, Gc of affine elements
   const R* gface;        // [N][4][2] fa, fb of affine elements
@@ -55,17 +56,21 @@ struct FineGeo {
   const int* iact;       // [instances] live flags (null: all): blocks of one stopped instance return
 };
 
-// 1-D tables of the fine-level kernels (kernel argument).
+// 1-D tables of the fine-level kernels (kernel argument).  The Gauss points are symmetric, so the
+// line operators are applied to a line's even and odd parts, e_i = u_i + u_{K-1-i} (the middle value
+// itself) and o_i = u_i - u_{K-1-i}: about half the products and half the constants, which then
+// stay in scalar registers.
 template <class R>
 struct FineTab {
-  R D[6][6];    // l_m'(xi_k)
-  R DD[6][6];   // second-derivative matrix: sum_m D[d][m] D[m][k]
   R lv[6], ld[6];  // l_m(-1), l_m'(-1) (the upper end by reflection)
-  R gd[6], Dg[6];  // lower Radau correction's derivative and its second derivative at xi_k
-  R m0, m1;     // that derivative extrapolated to -1 and +1
-  R g0;         // -g'(-1), the interface coefficient
-  R w[6], x[6]; // Gauss weights and points
-  R S[6][6], lam[6];  // eigenpairs of the line operator of an interior element
+  R lvE[3], lvO[3], ldE[3], ldO[3];      // the same on the even and odd parts
+  R DDE[3][3], DDO[3][3];                // second derivative: [in][out]
+  R gdE[3], gdO[3], DgE[3], DgO[3];      // lower Radau correction's derivative, and its derivative
+  R m0, m1;        // that correction's derivative extrapolated to -1 and +1
+  R g0, ig0;       // -g'(-1), the interface coefficient, and its inverse
+  R w[6], x[6];    // Gauss weights and points
+  R SE[3][3], SO[3][3], lam[6];  // eigenpairs of an interior element's line operator, even ones first
+  R D[6][6], gd[6];  // l_m'(xi_k), the correction's derivative (elements with tangential metrics)
 };
 
 template <class R>
@@ -117,6 +122,7 @@ struct PreArgs {
   int* active = nullptr;     // the Krylov flags F (may be null)
   const int* zero = nullptr; // q == null: x is set to zero where this flag is set
   double iw[6] = {0., 0., 0., 0., 0., 0.};  // 1 / w_k
+  const double* iwl = nullptr;              // the same on the device, for the lane's own
 };
 hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G, const PreArgs<double>& A,
                       hipStream_t s);

@@ -47,7 +47,7 @@ struct Prec {
   FineTab<R> T{};
   FineGeo<R> G{};
   DBuf<R> Ga, Gb, Gc, fa, fb, gel, gface;  // FP32 copies (unused for FP64)
-  DBuf<R> ac, fdm, qn;
+  DBuf<R> ac, fdm, qn, lane;
   // PCG ping-pongs its direction between p and v; t: the smoother's second iterate
   DBuf<R> r, z, p, q, rh, v, ph, sh, t, ec, xc;
   DevVHierarchy<R> lv;  // Q1 vertex level and below
@@ -82,6 +82,7 @@ struct Solver {
   double time = 0., re_inv = 0.;
   Tab T{};
   VecArgs VA{};
+  DBuf<double> d_iw;    // 1/w_k
   DBuf<double> d_winv;  // 1/(w_j w_i), the inverse quadrature weights VA.winv points at
   bool mixed = false;
 
@@ -202,6 +203,9 @@ struct Solver {
       for (int j = 0; j < K; ++j)
         for (int i = 0; i < K; ++i) wi[(size_t)j * K + i] = 1. / (tab.wgt[j] * tab.wgt[i]);
       d_winv.upload(wi);
+      std::vector<double> iw(K);
+      for (int k = 0; k < K; ++k) iw[k] = 1. / tab.wgt[k];
+      d_iw.upload(iw);
       VA.K = K;
       VA.winv = d_winv.p;
     }
@@ -318,21 +322,48 @@ struct Solver {
     fine_tables(tab, ft);
     FineTab<R>& F = P.T;
     F = FineTab<R>{};
+    const int HE = (K + 1) / 2, HO = K / 2;
+    auto even = [&](const double* v, int i) { return 2 * i + 1 == K ? v[i] : 0.5 * (v[i] + v[K - 1 - i]); };
+    auto odd = [&](const double* v, int i) { return 0.5 * (v[i] - v[K - 1 - i]); };
+    double lv[kMaxK], ld[kMaxK], gd[kMaxK];
     for (int i = 0; i < K; ++i) {
-      for (int j = 0; j < K; ++j) {
-        F.D[i][j] = (R)tab.D[i][j];
-        F.DD[i][j] = (R)ft.DD[i][j];
-        F.S[i][j] = (R)ft.fdm[K + i * K + j];
-      }
-      F.lam[i] = (R)ft.fdm[i];
-      F.lv[i] = (R)tab.bb[i][0];
-      F.ld[i] = (R)tab.bgb[i][0];
-      F.gd[i] = (R)tab.grad[i][0];
-      F.Dg[i] = (R)ft.Dg[i];
+      lv[i] = tab.bb[i][0];
+      ld[i] = tab.bgb[i][0];
+      gd[i] = tab.grad[i][0];
+      F.lv[i] = (R)lv[i];
+      F.ld[i] = (R)ld[i];
+      F.gd[i] = (R)gd[i];
       F.w[i] = (R)tab.wgt[i];
       F.x[i] = (R)tab.sps[i];
+      for (int j = 0; j < K; ++j) F.D[i][j] = (R)tab.D[i][j];
     }
-    F.m0 = (R)ft.m0; F.m1 = (R)ft.m1; F.g0 = (R)(-tab.gprime[0]);
+    for (int i = 0; i < HE; ++i) {
+      F.lvE[i] = (R)even(lv, i); F.ldE[i] = (R)even(ld, i); F.gdE[i] = (R)even(gd, i); F.DgE[i] = (R)even(ft.Dg, i);
+      for (int d = 0; d < HE; ++d) F.DDE[d][i] = (R)even(ft.DD[d], i);
+    }
+    for (int i = 0; i < HO; ++i) {
+      F.lvO[i] = (R)odd(lv, i); F.ldO[i] = (R)odd(ld, i); F.gdO[i] = (R)odd(gd, i); F.DgO[i] = (R)odd(ft.Dg, i);
+      for (int d = 0; d < HO; ++d) F.DDO[d][i] = (R)odd(ft.DD[d], i);
+    }
+    // interior eigenvectors, even ones first (the line operator commutes with the reflection)
+    for (int q = 0, ne = 0, no = 0; q < K; ++q) {
+      double v[kMaxK], se = 0., so = 0.;
+      for (int i = 0; i < K; ++i) v[i] = ft.fdm[K + i * K + q];
+      for (int i = 0; i < HO; ++i) { se += std::fabs(v[i] + v[K - 1 - i]); so += std::fabs(v[i] - v[K - 1 - i]); }
+      if (se >= so && ne < HE) {
+        F.lam[ne] = (R)ft.fdm[q];
+        for (int i = 0; i < HE; ++i) F.SE[i][ne] = (R)even(v, i);
+        ++ne;
+      } else {
+        F.lam[HE + no] = (R)ft.fdm[q];
+        for (int i = 0; i < HO; ++i) F.SO[i][no] = (R)odd(v, i);
+        ++no;
+      }
+    }
+    F.m0 = (R)ft.m0; F.m1 = (R)ft.m1; F.g0 = (R)(-tab.gprime[0]); F.ig0 = (R)(-1. / tab.gprime[0]);
+    std::vector<R> lane((size_t)4 * K, R(0));
+    for (int k = 0; k < K; ++k) { lane[4 * k] = F.w[k]; lane[4 * k + 1] = F.x[k]; lane[4 * k + 2] = F.lam[k]; }
+    P.lane.upload(lane);
     P.fdm.upload_as(ft.fdm);
     // orthogonal elements: the off-diagonal metric is rounding noise of the affine test's size
     bool ortho = affine;
@@ -404,7 +435,7 @@ struct Solver {
       G2.Ga = P.Ga; G2.Gb = P.Gb; G2.Gc = P.Gc; G2.fa = P.fa; G2.fb = P.fb;
     }
     G2.N = N;
-    G2.ac = P.ac; G2.fdm = P.fdm; G2.qn = P.qn; G2.ftype = d_ftype;
+    G2.ac = P.ac; G2.fdm = P.fdm; G2.lane = P.lane; G2.qn = P.qn; G2.ftype = d_ftype;
     G2.nb = d_nb; G2.nbf = reinterpret_cast<const int32_t*>(d_nbf.p); G2.sw = d_swpsi;
     G2.inst = G.inst;
   }
@@ -687,6 +718,7 @@ struct Solver {
     A.z = z;
     A.omega = omega;
     for (int k = 0; k < K; ++k) A.iw[k] = 1. / tab.wgt[k];
+    A.iwl = d_iw;
     return A;
   }
   // xz (may be null): set to zero first when the right-hand side is zero.
