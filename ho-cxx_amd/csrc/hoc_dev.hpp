@@ -153,6 +153,8 @@ struct DevVHierarchy {
     inv.upload_as(ci);
     f.alloc(nc);
   }
+  // Whether the dense inverse is of the finest level itself.
+  bool dense_only() const { return lv.empty() && nc > 0; }
   // Where the finest level's right-hand side is read from.
   R* rhs() { return lv.empty() ? f.p : lv[0]->fu.p; }
   // u = V(rhs()): all launches predicated on the active flag Fp (may be null).

@@ -1,5 +1,6 @@
 // hoc_la.hip - vector, reduction, CSR and probing kernels of the Poisson solver.
 #include "hoc_la.hpp"
+#include "hoc_status.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -100,20 +101,7 @@ __global__ void k_zero_if_flag(size_t n, R* __restrict__ x, const int* __restric
 
 // Scalar logic of the Krylov solvers.  pa: np partials of q0 then np of q1; pbb (PH_INIT, may be
 // null): npbb partials of ||b||^2, summed into S[S_BB] first.  With mirror set (pinned host memory),
-// thread 0 finally publishes the solve's results (MirrorState) and, after a system-scope fence, the
-// status word seq * 4 + near * 2 + (active flag), whether or not the phase ran, so the host can
-// follow the iterations and take the results without a copy; near: still active with the residual
-// within 8x of the tolerance, so the next iteration may be the last.
-__device__ void publish(MirrorState* __restrict__ mirror, int seq, bool near, const double* __restrict__ S,
-                        const int* __restrict__ F) {
-  mirror->bb = S[S_BB];
-  mirror->rr = S[S_RR];
-  mirror->iter = F[F_ITER];
-  mirror->zero = F[F_ZERO];
-  __threadfence_system();
-  __hip_atomic_store(&mirror->status, seq * 4 + (near ? 2 : 0) + (F[F_ACTIVE] ? 1 : 0), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_SYSTEM);
-}
+// thread 0 finally publishes the state, whether or not the phase ran.
 __device__ void finalize_phase(int phase, double a, double b, double* __restrict__ S, int* __restrict__ F,
                                int maxiter, const double* __restrict__ irr, const double* __restrict__ ibb,
                                int ninst);
@@ -155,7 +143,7 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(int phase, const doubl
   }
   if (mirror && threadIdx.x == 0) {
     const int sq = seq >= 0 ? seq : ++F[F_SEQ];
-    const bool near = F[F_ACTIVE] && (irr ? S[S_IMAX] <= 64. : S[S_RR] <= 64. * S[S_TOL2] * S[S_BB]);
+    const bool near = F[F_ACTIVE] && (irr ? S[S_IMAX] <= 64. : likely_last(S));
     publish(mirror, sq, near, S, F);
   }
 }
@@ -163,6 +151,14 @@ __global__ void k_set_int(int* __restrict__ p, int v) { *p = v; }
 __device__ void finalize_phase(int phase, double a, double b, double* __restrict__ S, int* __restrict__ F,
                                int maxiter, const double* __restrict__ irr, const double* __restrict__ ibb,
                                int ninst) {
+  if ((phase == PH_UPD && !irr) || phase >= PH_BHALF) {
+    check_phase(phase, a, b, S, F, maxiter);
+    if (phase == PH_BNEXT && F[F_ACTIVE]) {
+      S[S_BETA] = (a / S[S_RHO]) * (S[S_ALPHA] / S[S_OMEGA]);
+      S[S_RHO] = S[S_RHON] = a;
+    }
+    return;
+  }
   const double tol2bb = S[S_TOL2] * S[S_BB];
   // the convergence test of PH_INIT / PH_UPD: the joint residual, or every instance's own
   bool above = b > tol2bb;
@@ -179,14 +175,14 @@ __device__ void finalize_phase(int phase, double a, double b, double* __restrict
   switch (phase) {
     case PH_BB: S[S_BB] = a; break;
     case PH_INIT: {
-      S[S_RR] = b;
+      S[S_RR] = S[S_RRL] = S[S_PRED] = b;
       const double tiny = 2. * 2.220446049250313e-16;
       const bool zero = S[S_BB] < tiny * tiny;
       F[F_ZERO] = zero;
       F[F_ITER] = 0;
       F[F_HALF] = 0;
       F[F_ACTIVE] = (!zero && above && maxiter > 0) ? 1 : 0;
-      S[S_RZ] = 0.; S[S_RHO] = 1.; S[S_ALPHA] = 1.; S[S_OMEGA] = 1.; S[S_BETA] = 0.;
+      S[S_RZ] = 0.; S[S_RHO] = S[S_RHON] = a; S[S_ALPHA] = 1.; S[S_OMEGA] = 1.; S[S_BETA] = 0.;
     } break;
     case PH_RZ: {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
       if (!(a > 0.) || !isfinite(a)) { F[F_ACTIVE] = 0; break; }
@@ -447,14 +443,47 @@ __global__ void k_probe_diag(int N, int K2, const int32_t* __restrict__ color, i
 // ---- Q1 coarse space ---------------------------------------------------------------------------
 // rc[v] = sum over the (element, corner) incidences of vertex v of ec[element][corner]
 template <class R>
-__global__ void k_q1_gather(int nv, const int32_t* __restrict__ vptr, const int32_t* __restrict__ vinc,
-                            const R* __restrict__ ec, R* __restrict__ rc, const int* __restrict__ F) {
-  if (F && !F[F_ACTIVE]) return;
+__global__ void k_q1_gather(int nv, int w, const int32_t* __restrict__ inc, const R* __restrict__ ec,
+                            R* __restrict__ rc, const int* __restrict__ F) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nv) return;
+  if ((F && !F[F_ACTIVE]) || v >= nv) return;
   R s = 0;
-  for (int k = vptr[v]; k < vptr[v + 1]; ++k) s += ec[vinc[k]];
+#pragma unroll 4
+  for (int c = 0; c < w; ++c) s += ec[inc[(size_t)c * nv + v]];
   rc[v] = s;
+}
+
+// The coarsest level where it is the vertex space itself: the gather of the corner sums and the
+// product with the inverse in one launch.  A wavefront takes one row, C values a lane in registers
+// before the block has gathered the right-hand side into LDS, so the row is in flight meanwhile.
+// Every block gathers the whole right-hand side (4 n values from the L2); a launch costs more.
+template <int C, class R>
+__global__ __launch_bounds__(256) void k_dense_gather(int n, const R* __restrict__ Ainv, int w,
+                                                      const int32_t* __restrict__ inc, const R* __restrict__ ec,
+                                                      R* __restrict__ x, const int* __restrict__ F) {
+  __shared__ R f[64 * C];
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const R* a = Ainv + (size_t)min(row, n - 1) * n;
+  if (F && !F[F_ACTIVE]) return;
+  R v[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) v[c] = lane + 64 * c < n ? a[lane + 64 * c] : R(0);
+#pragma unroll
+  for (int q = 0; q < (64 * C + 255) / 256; ++q) {
+    const int i = threadIdx.x + 256 * q;
+    R s = 0;
+    if (i < n)
+#pragma unroll 4
+      for (int c = 0; c < w; ++c) s += ec[inc[(size_t)c * n + i]];
+    if (i < 64 * C) f[i] = s;
+  }
+  __syncthreads();
+  R s = 0;
+#pragma unroll
+  for (int c = 0; c < C; ++c) s += v[c] * f[lane + 64 * c];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if (lane == 0 && row < n) x[row] = s;
 }
 // For a probe y = As x (x = unit vector at local dof rs of every element of one colour),
 // M[f][a][b] += (sum_ij q1w(a,ij) y[f][ij]) * q1w(b, rs): the Galerkin block between the
@@ -1252,8 +1281,14 @@ void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F) 
   else hipLaunchKernelGGL((k_dense<256, R>), dim3(n), dim3(256), 0, s, n, Ainv, f, x, F);
 }
 template <class R>
-void q1_gather(hipStream_t s, int nv, const int32_t* vptr, const int32_t* vinc, const R* ec, R* rc, const int* F) {
-  hipLaunchKernelGGL(k_q1_gather<R>, dim3((nv + 255) / 256), dim3(256), 0, s, nv, vptr, vinc, ec, rc, F);
+void q1_gather(hipStream_t s, int nv, int w, const int32_t* inc, const R* ec, R* rc, const int* F) {
+  hipLaunchKernelGGL(k_q1_gather<R>, dim3((nv + 255) / 256), dim3(256), 0, s, nv, w, inc, ec, rc, F);
+}
+template <class R>
+void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc, const R* ec, R* x, const int* F) {
+  const dim3 grid((n + 3) / 4), block(256);
+  if (n <= 320) hipLaunchKernelGGL((k_dense_gather<5, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
+  else hipLaunchKernelGGL((k_dense_gather<kDenseGather / 64, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
 }
 void promote_dot(hipStream_t s, size_t n, const float* z32, double* z64, const double* r64, double* part,
                  const int* F) {
@@ -1284,7 +1319,8 @@ void q1_probe_accum(hipStream_t s, int N, int K, const Tab& T, int rs, const dou
                        R*, const int*);                                                                        \
   template void sell<R>(hipStream_t, int, int, const int32_t*, const int32_t*, const R*, const R*, R*, const int*);    \
   template void dense<R>(hipStream_t, int, const R*, const R*, R*, const int*);                                       \
-  template void q1_gather<R>(hipStream_t, int, const int32_t*, const int32_t*, const R*, R*, const int*);
+  template void q1_gather<R>(hipStream_t, int, int, const int32_t*, const R*, R*, const int*);                          \
+  template void dense_gather<R>(hipStream_t, int, const R*, int, const int32_t*, const R*, R*, const int*);
 HOC_LA_INST(double)
 HOC_LA_INST(float)
 #undef HOC_LA_INST

@@ -15,9 +15,9 @@ namespace hoc {
 
 // Device scalar slots (double) and flags (int) of the Krylov solvers.
 // F_MAXIT: iteration budget read by finalize kernels launched with maxiter < 0.
-enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_RZN, S_COUNT = 16 };
+enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_RZN, S_RHON, S_RRL, S_PRED, S_COUNT = 16 };
 enum { F_ACTIVE = 0, F_ITER, F_ZERO, F_HALF, F_MAXIT, F_SEQ, F_COUNT = 8 };
-enum { PH_BB = 0, PH_INIT, PH_RZ, PH_PQ, PH_UPD, PH_RHO, PH_ALPHA, PH_SNORM, PH_OMEGA, PH_RNORM };
+enum { PH_BB = 0, PH_INIT, PH_RZ, PH_PQ, PH_UPD, PH_RHO, PH_ALPHA, PH_SNORM, PH_OMEGA, PH_RNORM, PH_BHALF, PH_BNEXT };
 enum { VOP_BICG_P = 0, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
 
 // What a solve's finalize kernels leave in pinned host memory: the status word, and the results of
@@ -44,8 +44,7 @@ void bicg_half(hipStream_t s, size_t n, R* x, const R* ph, const double* S, int*
 template <class R>
 void zero_if_flag(hipStream_t s, size_t n, R* x, const int* F);
 // mirror (optional): pinned host state that receives the solve's results and the status word
-// seq * 4 + near * 2 + (active flag) when the kernel ends (near: active with the residual within 8x
-// of the tolerance);
+// seq * 4 + near * 2 + (active flag) when the kernel ends (near: likely_last);
 // seq < 0: the next number of the device counter F[F_SEQ] (incremented) instead of seq.
 // pbb (PH_INIT): npbb partials of ||b||^2 for S[S_BB], which PH_BB would otherwise have set.
 // maxiter < 0: the budget is read from F[F_MAXIT].
@@ -74,8 +73,13 @@ size_t dense_invert_work(int n);
 void dense_invert(hipStream_t s, int n, double* A, double* work);
 template <class R>
 void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F);
+// rc[v] = sum of the element corners at vertex v: ec[inc[c nv + v]], c < w (padding names a zero).
 template <class R>
-void q1_gather(hipStream_t s, int nv, const int32_t* vptr, const int32_t* vinc, const R* ec, R* rc, const int* F);
+void q1_gather(hipStream_t s, int nv, int w, const int32_t* inc, const R* ec, R* rc, const int* F);
+// x = Ainv q1_gather(ec) in one launch (n = nv <= kDenseGather).
+constexpr int kDenseGather = 1216;
+template <class R>
+void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc, const R* ec, R* x, const int* F);
 
 // The FP32 V-cycle inside the FP64 Krylov method: z64 = (double) z32 with partials of r64 . z64 in
 // part (vec_grid(n) blocks; may be null).

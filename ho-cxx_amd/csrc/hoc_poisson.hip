@@ -22,6 +22,8 @@
 // a and c are the element's mean metrics.
 #include "hoc_poisson.hpp"
 
+#include "hoc_status.hpp"
+
 namespace hoc {
 
 namespace {
@@ -457,21 +459,58 @@ __device__ __forceinline__ double sum_parts(const double* __restrict__ part, int
   return sp[0] + sp[1] + sp[2] + sp[3];
 }
 
+// sums of the first and of the second halves of 2 np partials, for thread 0 of the block
+__device__ __forceinline__ void sum_pairs(const double* __restrict__ part, int np, double& a, double& b) {
+  __shared__ double sa[kFineThreads / 64], sb[kFineThreads / 64];
+  a = b = 0.;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < np; i += kFineThreads) {
+    a += part[i];
+    b += part[np + i];
+  }
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if ((threadIdx.x & 63) == 0) { sa[threadIdx.x >> 6] = a; sb[threadIdx.x >> 6] = b; }
+  __syncthreads();
+  a = sa[0] + sa[1] + sa[2] + sa[3];
+  b = sb[0] + sb[1] + sb[2] + sb[3];
+}
+
+// The end of the iteration before, in a block of its own (FineArgs::chk_part): a launch of one
+// block would hold the stream for 4.4 us.  The kernel's other blocks may or may not see the flag
+// that it clears: what they write is not used then.
+template <class A>
+__device__ void check_block(const A& a) {
+  int* F = a.active;
+  const bool live = F[F_ACTIVE] != 0;  // uniform over the block
+  double u = 0., v = 0.;
+  if (live) sum_pairs(a.chk_part, a.chk_np, u, v);
+  if (threadIdx.x) return;
+  double* S = a.scal;
+  if (live) check_phase(a.chk_phase, u, v, S, F, a.chk_maxit >= 0 ? a.chk_maxit : F[F_MAXIT]);
+  if (!a.chk_mirror) return;
+  const int seq = a.chk_seq >= 0 ? a.chk_seq : ++F[F_SEQ];
+  publish(a.chk_mirror, seq, F[F_ACTIVE] && likely_last(S), S, F);
+}
+
+// Makes a loaded value due here, so that its load is issued before the branch that follows (on the
+// flag of the solve, loaded at the same time) and not after it.
+__device__ __forceinline__ void due(int v) { asm volatile("" ::"v"(v)); }
+
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> G, FineArgs<R> A) {
-  const bool go = !A.active || A.active[F_ACTIVE];
-  if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
-  if (!go) return;
+  constexpr bool CHK = IN == IN_X && EPI == EPI_SMOOTH;
+  const int nblk = CHK && A.chk_part ? (int)gridDim.x - 1 : (int)gridDim.x;
+  if (CHK && (int)blockIdx.x == nblk) {
+    check_block(A);
+    return;
+  }
   constexpr int K2 = K * K, EPW = Lay<K>::EPW, ES = Lay<K>::ES;
   constexpr int FS = GEO == GEO_ORTHO ? 0 : 4 * K;  // face values of one element
   __shared__ R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  const int blk = xcd_block(blockIdx.x, nblk);
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int EPB = EPW * (kFineThreads / 64);
-  if (G.iact) {  // a block inside one stopped ensemble instance
-    const int i0 = G.inst[blk * EPB];
-    if (i0 == G.inst[min((blk + 1) * EPB, G.N) - 1] && !G.iact[i0]) return;
-  }
   const int le = lane < EPW * K ? lane / K : EPW - 1;
   const int k = lane < EPW * K ? lane - le * K : K - 1;
   const int el0 = blk * EPB + wv * EPW + le;
@@ -479,6 +518,16 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   // lanes past the mesh follow its last element in a slot of their own, and the lanes past the last
   // slot its last row: the same reads, so the same values in LDS; neither writes to memory
   const int el = min(el0, G.N - 1);
+  const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
+  const int nbf = G.nbf[el];
+  const bool go = !A.active || A.active[F_ACTIVE];
+  due(nbr.x); due(nbr.y); due(nbr.z); due(nbr.w); due(nbf);
+  if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
+  if (!go) return;
+  if (G.iact) {  // a block inside one stopped ensemble instance
+    const int i0 = G.inst[blk * EPB];
+    if (i0 == G.inst[min((blk + 1) * EPB, G.N) - 1] && !G.iact[i0]) return;
+  }
   R* t = lds + wv * (Lay<K>::TILE + EPW * FS) + le * ES;
   R* tf = lds + wv * (Lay<K>::TILE + EPW * FS) + Lay<K>::TILE + le * FS;
   const size_t row = ((size_t)el * K + k) * K;
@@ -487,9 +536,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   (void)xk;
   (void)lamk;
 
-  // connectivity and every global read of the kernel, issued before the arithmetic
-  const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
-  const int nbf = G.nbf[el];
+  // every global read of the kernel, issued before the arithmetic
   R u[K], z[K], b[K];
   (void)z;
   // a solve's first direction is z: the old one, of another solve, is not read
@@ -498,23 +545,9 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   R beta = 0;
   if constexpr (IN == IN_PUPD) {
     load_row<K>(static_cast<const RZ*>(A.z) + row, z);
-    if (A.rz) {
-      const double rz = sum_parts(A.rz, A.np), be = A.active[F_ITER] > 0 ? rz / A.scal[S_RZ] : 0.;
-      const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-      if (!(rz > 0.) || !isfinite(rz)) {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
-        if (first) A.active[F_ACTIVE] = 0;
-        return;
-      }
-      if (first) {
-        A.scal[S_RZN] = rz;
-        A.scal[S_BETA] = be;
-      }
-      beta = (R)be;
-    } else {
-      beta = (R)(A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]]);
-    }
+    if (!A.rz) beta = (R)(A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]]);
   }
-  if constexpr (EPI == EPI_RESID || EPI == EPI_SMOOTH || EPI == EPI_RESTRICT) load_row<K>(A.b + row, b);
+  if constexpr (EPI == EPI_RESID || EPI == EPI_SMOOTH || EPI == EPI_RESTRICT || EPI == EPI_DOTS) load_row<K>(A.b + row, b);
   R xo[4] = {0, 0, 0, 0};  // IN_PROL: own vertex values
   if constexpr (IN == IN_PROL) {
     const int4 v = *reinterpret_cast<const int4*>(G.ev + (size_t)el * 4);
@@ -585,6 +618,21 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     else if (GEO == GEO_AFFINE) F[f].an = G.gface[((size_t)nb * 4 + fn) * 2];
     else F[f].an = G.fa[((size_t)nb * 4 + fn) * K + F[f].kk];
   }
+  if constexpr (IN == IN_PUPD) {
+    if (A.rz) {  // behind the loads: the sum takes longer than they do
+      const double rz = sum_parts(A.rz, A.np), be = A.active[F_ITER] > 0 ? rz / A.scal[S_RZ] : 0.;
+      const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+      if (!(rz > 0.) || !isfinite(rz)) {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
+        if (first) A.active[F_ACTIVE] = 0;
+        return;
+      }
+      if (first) {
+        A.scal[S_RZN] = rz;
+        A.scal[S_BETA] = be;
+      }
+      beta = (R)be;
+    }
+  }
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     if (nbs[f] < 0) F[f].neu = G.sw[-1 - nbs[f]] != 0;
@@ -633,7 +681,14 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   }
 #pragma unroll
   for (int i = 0; i < K; ++i) out[i] *= -(wk * T.w[i]);
-  if constexpr (EPI == EPI_STORE) {
+  if constexpr (EPI == EPI_DOTS) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      p0 += (double)b[i] * (double)out[i];
+      p1 += (double)out[i] * (double)out[i];
+    }
+    if (live) store_row<K>(A.y + row, out);
+  } else if constexpr (EPI == EPI_STORE) {
 #pragma unroll
     for (int i = 0; i < K; ++i) p0 += (double)u[i] * (double)out[i];
     if (live) store_row<K>(A.y + row, out);
@@ -684,14 +739,14 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   }
   if (A.part) {
     if (!live) p0 = p1 = 0.;
-    block_part(p0, p1, A.part, blk, gridDim.x);
+    block_part(p0, p1, A.part, blk, nblk);
   }
 }
 
-template <int K, bool UPD, class R>
+template <int K, int UPD, class R>
 __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G, PreArgs<R> A) {
-  if (!UPD && !A.zero && A.active && !A.active[F_ACTIVE]) return;
-  if (UPD && A.active && !A.active[F_ACTIVE]) return;
+  constexpr bool XR = UPD == PRE_XR, ZERO = UPD == PRE_NONE || UPD == PRE_BICG0;
+  if (!(ZERO && A.zero) && A.active && !A.active[F_ACTIVE]) return;
   constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES, EPB = EPW * (kFineThreads / 64);
   __shared__ R lds[(kFineThreads / 64) * Lay<K>::TILE];
   const int blk = xcd_block(blockIdx.x, gridDim.x);
@@ -707,7 +762,7 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
   const int el = min(el0, G.N - 1);
   R* t = lds + wv * Lay<K>::TILE + le * ES;
   const size_t row = ((size_t)el * K + k) * K;
-  if (!UPD && A.zero) {  // a zero right-hand side: x = 0, as the reference's solver returns
+  if (ZERO && A.zero) {  // a zero right-hand side: x = 0, as the reference's solver returns
     if (*A.zero && live) {
       const double z[K] = {};
       store_row<K>(A.x + row, z);
@@ -717,24 +772,24 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
   double r[K];
   load_row<K>(A.r + row, r);
   double p0 = 0., p1 = 0.;
-  if constexpr (UPD) {
+  if constexpr (XR) {
     double x[K], p[K], q[K];
     load_row<K>(A.q + row, q);
     load_row<K>(A.p + row, p);
     load_row<K>(A.x + row, x);
     double al;
     if (A.pq) {
-      const double pq = sum_parts(A.pq, A.np), rz = A.scal[S_RZN];
-      al = rz / pq;
+      const double pq = sum_parts(A.pq, A.np), num = A.scal[A.num];
+      al = num / pq;
       const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-      if (!(pq > 0.) || !isfinite(al)) {
+      if (pq == 0. || (A.spd && !(pq > 0.)) || !isfinite(al)) {
         if (first) A.active[F_ACTIVE] = 0;
         return;
       }
       if (first) {
         A.scal[S_PQ] = pq;
         A.scal[S_ALPHA] = al;
-        A.scal[S_RZ] = rz;
+        A.scal[A.keep] = num;
       }
     } else {
       al = A.scal_idx >= 0 ? A.scal[A.scal_idx] : A.scal[G.inst[el]];
@@ -758,6 +813,32 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
       p1 += uw * uw;
     }
   }
+  if constexpr (UPD == PRE_BICGP) {
+    double p[K], q[K];
+    load_row<K>(A.q + row, q);
+    load_row<K>(A.p + row, p);
+    const double om = A.scal[S_OMEGA];
+    double be;
+    if (A.pq) {
+      const double rho = sum_parts(A.pq, A.np);
+      be = (rho / A.scal[S_RHO]) * (A.scal[S_ALPHA] / om);
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        A.scal[S_RHON] = rho;
+        A.scal[S_BETA] = be;
+      }
+    } else {
+      be = A.scal[S_BETA];
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i) r[i] += be * (p[i] - om * q[i]);
+    if (live) store_row<K>(A.pw + row, r);
+  }
+  if constexpr (UPD == PRE_BICG0) {
+    if (live) {
+      store_row<K>(A.pw + row, r);
+      store_row<K>(A.rh + row, r);
+    }
+  }
   R v[K];
 #pragma unroll
   for (int i = 0; i < K; ++i) v[i] = (R)r[i];
@@ -769,10 +850,55 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
 #pragma unroll
   for (int i = 0; i < K; ++i) v[i] *= om;
   if (live) store_row<K>(A.z + row, v);
-  if (UPD && A.part) {
+  if (XR && A.part) {
     if (!live) p0 = p1 = 0.;
     block_part(p0, p1, A.part, blk, gridDim.x);
   }
+}
+
+// Element rows over the lanes as in the kernels around it, so that its partial sums are as many.
+template <int K>
+__global__ __launch_bounds__(kFineThreads) void k_bicg_x(int N, BicgArgs A) {
+  if (!A.active[F_ACTIVE]) return;
+  constexpr int EPW = Lay<K>::EPW, EPB = EPW * (kFineThreads / 64);
+  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int le = min(lane / K, EPW - 1), k = lane - le * K, el0 = blk * EPB + wv * EPW + le;
+  const bool live = k < K && el0 < N;
+  const size_t row = ((size_t)min(el0, N - 1) * K + min(k, K - 1)) * K;
+  double x[K], r[K], sh[K], t[K], rh[K];
+  load_row<K>(A.t + row, t);
+  load_row<K>(A.r + row, r);
+  load_row<K>(A.sh + row, sh);
+  load_row<K>(A.x + row, x);
+  load_row<K>(A.rh + row, rh);
+  double om;
+  if (A.ts) {
+    double ts, tt;
+    sum_pairs(A.ts, A.np, ts, tt);
+    om = tt != 0. ? ts / tt : 0.;
+    if (!isfinite(om)) om = 0.;
+    if (blockIdx.x == 0 && threadIdx.x == 0) A.scal[S_OMEGA] = om;
+  } else {
+    om = A.scal[S_OMEGA];
+  }
+  double p0 = 0., p1 = 0.;
+  const double wk = A.iwl[min(k, K - 1)];
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    x[i] += om * sh[i];
+    r[i] -= om * t[i];
+    const double uw = r[i] * (wk * A.iw[i]);
+    p0 += rh[i] * r[i];
+    p1 += uw * uw;
+  }
+  if (live) {
+    store_row<K>(A.x + row, x);
+    store_row<K>(A.r + row, r);
+  } else {
+    p0 = p1 = 0.;
+  }
+  block_part(p0, p1, A.part, blk, gridDim.x);
 }
 
 }  // namespace
@@ -796,7 +922,8 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
 
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 static void go_fine(const FineTab<R>& T, const FineGeo<R>& G, const FineArgs<R>& A, hipStream_t s) {
-  hipLaunchKernelGGL((k_fine<K, GEO, IN, EPI, R, RZ>), dim3(fine_blocks(K, G.N)), dim3(kFineThreads), 0, s, T, G, A);
+  hipLaunchKernelGGL((k_fine<K, GEO, IN, EPI, R, RZ>), dim3(fine_blocks(K, G.N) + (A.chk_part ? 1 : 0)),
+                     dim3(kFineThreads), 0, s, T, G, A);
 }
 
 template <int K, int GEO, class R>
@@ -809,6 +936,7 @@ static hipError_t fine_kg(int in, int epi, const FineTab<R>& T, const FineGeo<R>
     if (in == IN_X && epi == EPI_STORE) go_fine<K, GEO, IN_X, EPI_STORE, R, R>(T, G, A, s);
     else if (in == IN_X && epi == EPI_RESID) go_fine<K, GEO, IN_X, EPI_RESID, R, R>(T, G, A, s);
     else if (in == IN_X && epi == EPI_PLAIN) go_fine<K, GEO, IN_X, EPI_PLAIN, R, R>(T, G, A, s);
+    else if (in == IN_X && epi == EPI_DOTS) go_fine<K, GEO, IN_X, EPI_DOTS, R, R>(T, G, A, s);
     else if (in == IN_PUPD && epi == EPI_STORE) go_fine<K, GEO, IN_PUPD, EPI_STORE, R, R>(T, G, A, s);
     else return hipErrorInvalidValue;
   } else return hipErrorInvalidValue;
@@ -835,8 +963,13 @@ template <class R>
 static hipError_t launch_pre_t(int K, const FineTab<R>& T, const FineGeo<R>& G, const PreArgs<R>& A, hipStream_t s) {
   HOC_K_SWITCH(K, {
     const dim3 grid(fine_blocks(KK, G.N)), block(kFineThreads);
-    if (A.q) hipLaunchKernelGGL((k_pre<KK, true, R>), grid, block, 0, s, T, G, A);
-    else hipLaunchKernelGGL((k_pre<KK, false, R>), grid, block, 0, s, T, G, A);
+    switch (A.up) {
+      case PRE_NONE: hipLaunchKernelGGL((k_pre<KK, PRE_NONE, R>), grid, block, 0, s, T, G, A); break;
+      case PRE_XR: hipLaunchKernelGGL((k_pre<KK, PRE_XR, R>), grid, block, 0, s, T, G, A); break;
+      case PRE_BICGP: hipLaunchKernelGGL((k_pre<KK, PRE_BICGP, R>), grid, block, 0, s, T, G, A); break;
+      case PRE_BICG0: hipLaunchKernelGGL((k_pre<KK, PRE_BICG0, R>), grid, block, 0, s, T, G, A); break;
+      default: return hipErrorInvalidValue;
+    }
   });
   return hipGetLastError();
 }
@@ -847,6 +980,10 @@ hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G,
 hipError_t launch_pre(int K, const FineTab<float>& T, const FineGeo<float>& G, const PreArgs<float>& A,
                       hipStream_t s) {
   return launch_pre_t<float>(K, T, G, A, s);
+}
+hipError_t launch_bicg_x(int K, int N, const BicgArgs& A, hipStream_t s) {
+  HOC_K_SWITCH(K, hipLaunchKernelGGL((k_bicg_x<KK>), dim3(fine_blocks(KK, N)), dim3(kFineThreads), 0, s, N, A));
+  return hipGetLastError();
 }
 
 }  // namespace hoc

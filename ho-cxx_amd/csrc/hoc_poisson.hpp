@@ -12,7 +12,8 @@ namespace hoc {
 //   EPI_SMOOTH    y = u + omega B (b - As u); optional partial sums of b.y
 //   EPI_RESTRICT  ec[el][a] = sum_ij q1w(a,ij) (b - As u)_ij      (Pc^T residual, per element)
 //   EPI_PLAIN     y = A u (the operator itself, unscaled)
-enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SMOOTH = 2, EPI_RESTRICT = 3, EPI_PLAIN = 4 };
+//   EPI_DOTS      y = As u; partial sums of b.y and y.y
+enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SMOOTH = 2, EPI_RESTRICT = 3, EPI_PLAIN = 4, EPI_DOTS = 5 };
 // The field u it is applied to:
 //   IN_X     u = x
 //   IN_PROL  u = x + Pc xc (bilinear from the corner vertices)
@@ -91,6 +92,11 @@ struct FineArgs {
   double* part = nullptr;    // [fine_blocks] sums, then [fine_blocks] second sums
   int* active = nullptr;     // the Krylov flags F (may be null)
   int* ran = nullptr;        // set to 1 when the launch worked, 0 when active made it return at once
+  // EPI_SMOOTH of IN_X: one block more, which tests np pairs of partial norms that an earlier kernel
+  // left (phase: check_phase) and publishes the state; the other blocks do not wait for it
+  const double* chk_part = nullptr;
+  int chk_np = 0, chk_phase = 0, chk_maxit = 0, chk_seq = 0;
+  MirrorState* chk_mirror = nullptr;  // null: tested, not published
 };
 
 hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<double>& T, const FineGeo<double>& G,
@@ -101,10 +107,14 @@ hipError_t launch_fine(int K, int geo, int in, int epi, const FineTab<float>& T,
 hipError_t launch_fine_pupd_f32z(int K, int geo, const FineTab<double>& T, const FineGeo<double>& G,
                                  const FineArgs<double>& A, hipStream_t s);
 
-// First smoothing step from zero, z = omega B r, with PCG's vector update in front of it:
-//   q != null: x += alpha p, r -= alpha q first (alpha = scal[scal_idx], or scal[inst[el]] with
-//   scal_idx < 0, where elements of alpha = 0 keep x and r); partial sums of r.r and (r/W).(r/W).
-// FP32 V-cycle: r32 receives r in FP32.
+// First smoothing step from zero, z = omega B r, with a Krylov update in front of it (up):
+//   PRE_NONE
+//   PRE_XR      x += alpha p, r -= alpha q; alpha = scal[scal_idx], or scal[inst[el]] with scal_idx < 0,
+//               where elements of alpha = 0 keep x and r; partial sums of r.r and (r/W).(r/W)
+//   PRE_BICGP   p = r + beta (p - omega_k q), z = omega B p, with BiCGSTAB's beta and omega_k from scal
+//   PRE_BICG0   the same before the first iteration: p = r, and rh = r
+// FP32 V-cycle: r32 receives the residual that the cycle is for in FP32.
+enum { PRE_NONE = 0, PRE_XR = 1, PRE_BICGP = 2, PRE_BICG0 = 3 };
 template <class R>
 struct PreArgs {
   double *r = nullptr, *x = nullptr;
@@ -114,18 +124,39 @@ struct PreArgs {
   double omega = 0.;
   double* scal = nullptr;
   int scal_idx = 0;
-  // small meshes: p.q as np partials, summed by every block (alpha = scal[S_RZN] / p.q); block 0
-  // leaves alpha and r.z in scal and clears active on a breakdown
+  int up = PRE_NONE;
+  double *pw = nullptr, *rh = nullptr;  // PRE_BICGP, PRE_BICG0: the direction, the shadow residual
+  // small meshes: a dot product as np partials, summed by every block.  PRE_XR: the denominator of
+  // alpha (numerator scal[num]); block 0 leaves alpha and the numerator (in scal[keep]) behind and
+  // clears active on a breakdown (spd: also where the sum is negative).  PRE_BICGP: rh.r, from which
+  // block 0 leaves beta and scal[S_RHON]; a breakdown is left to the test of the iteration.
   const double* pq = nullptr;
-  int np = 0;
+  int np = 0, num = 0, keep = 0;
+  bool spd = true;
   double* part = nullptr;
   int* active = nullptr;     // the Krylov flags F (may be null)
-  const int* zero = nullptr; // q == null: x is set to zero where this flag is set
+  const int* zero = nullptr; // PRE_NONE, PRE_BICG0: x is set to zero where this flag is set
   double iw[6] = {0., 0., 0., 0., 0., 0.};  // 1 / w_k
   const double* iwl = nullptr;              // the same on the device, for the lane's own
 };
 hipError_t launch_pre(int K, const FineTab<double>& T, const FineGeo<double>& G, const PreArgs<double>& A,
                       hipStream_t s);
 hipError_t launch_pre(int K, const FineTab<float>& T, const FineGeo<float>& G, const PreArgs<float>& A, hipStream_t s);
+
+// End of a BiCGSTAB iteration: x += omega sh, r -= omega t; partial sums of rh.r and (r/W).(r/W).
+// omega = scal[S_OMEGA]; with ts set, from np pairs of partials of (t.s, t.t), summed by every block,
+// and left in scal by block 0.
+struct BicgArgs {
+  double *x = nullptr, *r = nullptr;
+  const double *sh = nullptr, *t = nullptr, *rh = nullptr;
+  double* scal = nullptr;
+  const double* ts = nullptr;
+  int np = 0;
+  double* part = nullptr;
+  const int* active = nullptr;
+  double iw[6] = {0., 0., 0., 0., 0., 0.};
+  const double* iwl = nullptr;
+};
+hipError_t launch_bicg_x(int K, int N, const BicgArgs& A, hipStream_t s);
 
 }  // namespace hoc

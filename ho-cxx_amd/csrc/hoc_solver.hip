@@ -59,7 +59,7 @@ struct Prec {
   void alloc_vectors(size_t D, int N, bool krylov) {
     for (auto* f : {&r, &z, &t}) f->alloc(D);
     for (auto* f : {&p, &q, &rh, &v, &ph, &sh}) f->alloc(krylov ? D : 0);
-    ec.alloc((size_t)N * 4);
+    ec.alloc((size_t)N * 4 + 1);  // and a zero for the gather's padding (setup)
   }
 };
 
@@ -112,7 +112,8 @@ struct Solver {
   int seq_next = 0;
   int nparts = 0;
   int nv = 0;                             // Q1 coarse space: element-corner vertices
-  DBuf<int32_t> d_ev, d_vptr, d_vinc;     // element -> 4 vertices; vertex -> (element*4+corner)
+  DBuf<int32_t> d_ev, d_vinc;             // element -> 4 vertices; vertex -> (element*4+corner), k_q1_gather
+  int vdeg = 0;                           // largest number of elements at a vertex
   // Chebyshev smoother of degree cheb_m in B As (B: the element blocks' inverse) as damped
   // Richardson steps x += cheb_w[k] B (r - As x)
   int cheb_m = 2;
@@ -505,7 +506,7 @@ struct Solver {
     if (in == IN_PROL) b += (double)N * 4 * 4 + (double)nv * vb;
     switch (epi) {
       case EPI_STORE: case EPI_PLAIN: b += vec; break;                      // y
-      case EPI_RESID: b += 2 * vec; break;                                  // b, y
+      case EPI_RESID: case EPI_DOTS: b += 2 * vec; break;                   // b, y
       case EPI_SMOOTH: b += 2 * vec + (double)N * (geo_kind == GEO_ORTHO ? 2. : 2. + 2 * vb); break;  // b, y; types, scales
       case EPI_RESTRICT: b += vec + (double)N * 4 * vb; break;              // b, corner sums
     }
@@ -565,7 +566,12 @@ struct Solver {
       for (int e = 0; e < N; ++e)
         for (int a = 0; a < 4; ++a) vinc[pos[ev[(size_t)e * 4 + a]]++] = e * 4 + a;
     }
-    d_ev.upload(ev); d_vptr.upload(vptr); d_vinc.upload(vinc);
+    vdeg = 0;
+    for (int v = 0; v < nv; ++v) vdeg = std::max(vdeg, vptr[v + 1] - vptr[v]);
+    std::vector<int32_t> inc((size_t)vdeg * nv, N * 4);
+    for (int v = 0; v < nv; ++v)
+      for (int k = vptr[v]; k < vptr[v + 1]; ++k) inc[(size_t)(k - vptr[v]) * nv + v] = vinc[k];
+    d_ev.upload(ev); d_vinc.upload(inc);
     P64.G.ev = d_ev;
     P32.G.ev = d_ev;
     inst_coupled = false;  // an ensemble whose instances share a corner vertex
@@ -721,21 +727,20 @@ struct Solver {
     A.iwl = d_iw;
     return A;
   }
-  // xz (may be null): set to zero first when the right-hand side is zero.
+  // The test of an iteration's end by the second smoothing step of the next V-cycle (FineArgs).
+  struct Check {
+    const double* part;
+    int np, phase, maxit, seq;
+    MirrorState* mirror;
+    double* S;
+  };
+  enum { WHOLE = 0, HEAD, REST };
+  // The rest of the V-cycle for the residual rr after its first smoothing step has left the first
+  // iterate in P.t: the iterate ping-pongs between P.t and zout and ends in zout; if partp != nullptr,
+  // partials of rr.zout are left there.  HEAD: the second smoothing step only; REST: what follows it.
   template <class R>
-  void vcycle_begin(Prec<R>& P, const double* rin, int* Fp, double* xz = nullptr) {
-    PreArgs<R> A = pre_args<R>(rin, P.t.p, cheb_w[0]);
-    if (xz) { A.x = xz; A.zero = Fp + F_ZERO; }
-    if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
-    A.active = Fp;
-    P.G.iact = P.iact;
-    HIPCHK(launch_pre(K, P.T, P.G, A, stream));
-  }
-  // The rest of the V-cycle for the residual rr after vcycle_begin has left its first iterate in
-  // P.t: the iterate ping-pongs between P.t and zout and ends in zout; if partp != nullptr,
-  // partials of rr.zout are left there.
-  template <class R>
-  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, int* Fp) {
+  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, int* Fp, int part_of = WHOLE,
+                   const Check* chk = nullptr) {
     R *cur = P.t.p, *nxt = zout;
     FineArgs<R> A;
     A.b = rr;
@@ -745,31 +750,40 @@ struct Solver {
       fine(P, in, EPI_SMOOTH, A);
       std::swap(cur, nxt);
     };
-    for (int k = 1; k < cheb_m; ++k) smooth(IN_X, cheb_w[k], nullptr);
+    for (int k = 1; k < cheb_m; ++k) {
+      if (k == 1 && chk) {
+        A.chk_part = chk->part; A.chk_np = chk->np; A.chk_phase = chk->phase; A.chk_maxit = chk->maxit;
+        A.chk_seq = chk->seq; A.chk_mirror = chk->mirror; A.scal = chk->S;
+      }
+      if (k > 1 || part_of != REST) smooth(IN_X, cheb_w[k], nullptr);
+      else std::swap(cur, nxt);
+      A.chk_part = nullptr;
+      if (part_of == HEAD) return;
+    }
     // restrict the residual to the corner vertices
     A.x = cur; A.y = P.ec.p; A.part = nullptr;
     fine(P, IN_X, EPI_RESTRICT, A);
-    q1_gather<R>(stream, nv, d_vptr, d_vinc, P.ec, P.lv.rhs(), Fp);
-    P.lv.cycle(stream, P.xc.p, Fp);
+    if (P.lv.dense_only() && nv <= kDenseGather) {
+      dense_gather<R>(stream, nv, P.lv.inv, vdeg, d_vinc, P.ec, P.xc.p, Fp);
+    } else {
+      q1_gather<R>(stream, nv, vdeg, d_vinc, P.ec, P.lv.rhs(), Fp);
+      P.lv.cycle(stream, P.xc.p, Fp);
+    }
     // prolongate and post-smooth, the dampings in reverse: the cycle stays symmetric
     A.xc = P.xc.p;
     for (int k = cheb_m - 1; k >= 0; --k)
       smooth(k == cheb_m - 1 ? IN_PROL : IN_X, cheb_w[k], k == 0 ? partp : nullptr);
   }
 
-  // z = M r: the V-cycle in the precision of P; for the FP64 Krylov method of a mixed-precision
-  // handle, the FP32 V-cycle between a demotion of r and a promotion of z.  With partp set, the
-  // partials of r . z are left there; returns their count (0 when partp is null).
-  int precond(const double* rin, double* zout, double* partp, int* Fp) {
+  // z = M r, begun by a first smoothing step (krylov_pre): the rest of the V-cycle in
+  // its precision, for a mixed-precision handle with a promotion of z at the end.
+  void precond_rest(const double* rin, double* zout, int* Fp, int part_of, const Check* chk) {
     if (mixed) {
-      vcycle_begin(P32, rin, Fp);
-      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp);
-      promote_dot(stream, D, P32.z.p, zout, rin, partp, Fp);
-      return partp ? vec_grid(D) : 0;
+      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp, part_of, chk);
+      if (part_of != HEAD) promote_dot(stream, D, P32.z.p, zout, rin, nullptr, Fp);
+    } else {
+      vcycle_rest(P64, rin, zout, nullptr, Fp, part_of, chk);
     }
-    vcycle_begin(P64, rin, Fp);
-    vcycle_rest(P64, rin, zout, partp, Fp);
-    return partp ? fine_blocks(K, N) : 0;
   }
 
   // Wait, lag iterations behind (none when final_wait), until the finalize kernel of the
@@ -807,20 +821,25 @@ struct Solver {
   // right-preconditioned BiCGSTAB.  Every kernel is predicated on Fp's active flag.
   // maxit bounds the host loop; maxit_dev is the device budget (< 0: Fp[F_MAXIT]).
   //
-  // Launch modes.  Direct: the host queues each iteration's kernels and waits for the status of
-  // the iteration before the last one it queued.  Graph: the same with an iteration's kernels as one
-  // captured hipGraph (one per order of the two direction buffers and set of buffers); the captured
-  // end-of-iteration finalize takes its number from the device counter F[F_SEQ].  The kernels and
-  // their order are the same, so both modes give the same iterates; graphs pay where the host's
-  // launch cost exceeds the kernels' run time (small meshes), and setup chooses by timing both
-  // (launch_mode 0).
+  // Launches.  An iteration is queued in two pieces, up to its test (krylov_iter) and the rest of the
+  // next one's V-cycle (krylov_tail), and the host reads the status in between.  What bounds small
+  // meshes is the chain of dependent launches, 5 to 6 us each: every vector update, dot product and
+  // test rides on a kernel that needs its result or on the one that made its operands (32 x 32
+  // elements, K = 4: 9 launches and 50.3 us a PCG iteration with the test and the vertices' gather as
+  // launches of their own, now 7 and 42.0; BiCGSTAB on 384 x 64 elements, K = 5: 43 launches and 256 us,
+  // now 33 and 213).
+  // Direct mode launches the kernels, graph mode the pieces as captured hipGraphs (two for the
+  // iteration, by which of the direction buffers is the old one), whose test takes its number from the
+  // device counter F[F_SEQ].  The kernels and their order are the same, so both modes give the same
+  // iterates; graphs pay where the host's launch cost exceeds the kernels' run time, and setup chooses
+  // by timing both (launch_mode 0).
   static constexpr int kTuneIters = 8;
   struct KGraph {
     hipGraph_t g = nullptr;
     hipGraphExec_t e = nullptr;
     const void* key[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     int maxit = 0;
-    bool odd = false;
+    int piece = 0;  // 0, 1: krylov_iter (odd 0, 1); 2: krylov_tail
   };
   std::vector<KGraph> kgraphs;
   bool use_graphs = false;
@@ -832,130 +851,167 @@ struct Solver {
     }
     kgraphs.clear();
   }
-  // Before the first iteration.  PCG: the first smoothing step of the first V-cycle (an iteration
-  // ends with the next one's); its direction needs no clearing, beta = 0 leaves the old one out.
-  void krylov_begin(double* x, double* r, int* Fp) {
-    Prec<double>& P = P64;
-    if (krylov == HOC_KRYLOV_PCG) {
-      if (mixed) vcycle_begin(P32, r, Fp, x);
-      else vcycle_begin(P64, r, Fp, x);
-    } else {
-      zero_if_flag<double>(stream, D, x, Fp);
-      vec<double>(stream, VOP_COPY, VA, D, P.rh, nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr);
-      HIPCHK(hipMemsetAsync(P.p.p, 0, D * sizeof(double), stream));
-      HIPCHK(hipMemsetAsync(P.v.p, 0, D * sizeof(double), stream));
-    }
-  }
-  // PCG's update x += alpha p, r -= alpha q with the first smoothing step of the next V-cycle.
-  void pcg_update(double* x, double* r, const double* p, double* scal, int scal_idx, const double* pq, double* partp,
-                  int* Fp) {
+  // Whether the blocks of the kernels sum the partials of the kernel before themselves, and the
+  // iteration's test rides on the next smoothing step.  Past kInlineParts partials every block's
+  // sum costs more than the finalize launch that it saves.
+  bool inline_sums() const { return fine_blocks(K, N) <= kInlineParts; }
+  bool inline_check() const { return inline_sums() && cheb_m > 1 && !ens_pcg(); }
+  // The first smoothing step of a V-cycle behind a Krylov update.
+  template <class Set>
+  void krylov_pre(const double* r, Set&& set) {
     auto go = [&](auto& P) {
       using R = std::remove_reference_t<decltype(*P.t.p)>;
       PreArgs<R> A = pre_args<R>(r, P.t.p, cheb_w[0]);
       if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
-      A.x = x; A.p = p; A.q = P64.q.p; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = Fp;
-      A.pq = pq; A.np = pq ? fine_blocks(K, N) : 0;
+      set(A);
       P.G.iact = P.iact;
       HIPCHK(launch_pre(K, P.T, P.G, A, stream));
     };
     if (mixed) go(P32);
     else go(P64);
   }
-  // One iteration's launches.  seq >= 0: the end-of-iteration finalize publishes seq; seq < 0:
-  // it takes the next number from F[F_SEQ].  odd: which of the two direction buffers is the old one.
+  // Before the first iteration: its V-cycle (an iteration ends with the next one's).  The first
+  // direction needs no clearing, beta = 0 leaves the old one out.
+  void krylov_begin(double* x, double* r, double* Sp, int* Fp, int maxit) {
+    if (krylov == HOC_KRYLOV_PCG) {
+      krylov_pre(r, [&](auto& A) { A.x = x; A.zero = Fp + F_ZERO; A.active = Fp; });
+    } else {
+      krylov_pre(r, [&](auto& A) {
+        A.up = PRE_BICG0; A.x = x; A.zero = Fp + F_ZERO; A.pw = P64.p; A.rh = P64.rh; A.active = Fp;
+      });
+    }
+    krylov_vcycle(r, Sp, Fp, maxit, WHOLE, nullptr);
+  }
+  // The V-cycle of the next iteration, or a part of it, after its first smoothing step.
+  void krylov_vcycle(double* r, double* Sp, int* Fp, int maxit, int part_of, const Check* chk) {
+    Prec<double>& P = P64;
+    if (krylov != HOC_KRYLOV_PCG) {
+      precond_rest(P.p.p, P.ph.p, Fp, part_of, chk);
+      return;
+    }
+    if (ens_batched()) {
+      EnsMask mask(*this);
+      vcycle_pcg(r, nullptr, Fp, part_of, chk);
+      if (part_of == HEAD) return;
+      if (mixed) seg_dot<float>(stream, pseg, r, P32.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
+      else seg_dot<double>(stream, pseg, r, P.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
+      finalize_ens(stream, ENS_RZ, ensk(), Sp, Fp, maxit);
+      return;
+    }
+    // r.z from the V-cycle's last sweep; in mixed precision the direction update reads z in FP32
+    vcycle_pcg(r, part.p, Fp, part_of, chk);
+    if (part_of != HEAD && !inline_sums()) finalize(stream, PH_RZ, part, fine_blocks(K, N), Sp, Fp, maxit);
+  }
+  void vcycle_pcg(double* r, double* partp, int* Fp, int part_of, const Check* chk) {
+    if (mixed) vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, partp, Fp, part_of, chk);
+    else vcycle_rest(P64, r, P64.z.p, partp, Fp, part_of, chk);
+  }
+  // One iteration up to its test and the publication of its status (seq >= 0: as seq; seq < 0: as the
+  // next number of F[F_SEQ]); with inline_check() that takes the second smoothing step of the next
+  // V-cycle along.  krylov_tail: the rest of that V-cycle.  odd: which of the two direction buffers of
+  // PCG is the old one.
   void krylov_iter(double* x, double* r, double* Sp, int* Fp, int maxit, int seq, bool odd) {
     Prec<double>& P = P64;
     const int fb = fine_blocks(K, N);
-    const int vg = vec_grid(D);
+    const bool inl = inline_sums(), ichk = inline_check();
     double* pold = odd ? P.v.p : P.p.p;
     double* pnew = odd ? P.p.p : P.v.p;
     if (ens_batched()) {
       ens_iter(x, r, pold, pnew, Sp, Fp, maxit, seq);
       return;
     }
+    Check chk{part.p, fb, PH_UPD, maxit, seq, mirror_dev, Sp};
     if (krylov == HOC_KRYLOV_PCG) {
-      // r.z from the V-cycle's last sweep; in mixed precision the direction update reads z in FP32
-      if (mixed) vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, part.p, Fp);
-      else vcycle_rest(P64, r, P.z.p, part.p, Fp);
-      const bool inl = fb <= kInlineParts;  // the next kernel sums the partials itself
-      if (!inl) finalize(stream, PH_RZ, part, fb, Sp, Fp, maxit);
       direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, Sp, S_BETA,
                       inl ? part.p : nullptr, part2.p, Fp);
       if (!inl) finalize(stream, PH_PQ, part2, fb, Sp, Fp, maxit);
-      pcg_update(x, r, pnew, Sp, S_ALPHA, inl ? part2.p : nullptr, part.p, Fp);
+      krylov_pre(r, [&](auto& A) {
+        A.up = PRE_XR; A.x = x; A.p = pnew; A.q = P.q; A.scal = Sp; A.scal_idx = S_ALPHA; A.part = part; A.active = Fp;
+        if (inl) { A.pq = part2; A.np = fb; A.num = S_RZN; A.keep = S_RZ; }
+      });
       if (ens_pcg()) {  // every instance against its own right-hand side
         seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p);
         finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq, ens_rr.p, ens_bb.p, pseg.nseg);
-        return;
+      } else if (!ichk) {
+        finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq);
       }
-      finalize(stream, PH_UPD, part, fb, Sp, Fp, maxit, mirror_dev, seq);
     } else {
+      // BiCGSTAB, right-preconditioned: v = As M p, alpha = rho / rh.v, s = r - alpha v, t = As M s,
+      // omega = t.s / t.t; every vector update rides on the kernel that needs its result
       FineArgs<double> A;
       A.active = Fp;
-      vec<double>(stream, VOP_DOT2, VA, D, P.rh, P.rh, r, r, nullptr, Sp, Fp, part);
-      finalize(stream, PH_RHO, part, vg, Sp, Fp, maxit);
-      vec<double>(stream, VOP_BICG_P, VA, D, P.p, nullptr, r, P.v, nullptr, Sp, Fp, nullptr);
-      precond(P.p.p, P.ph.p, nullptr, Fp);
-      A.x = P.ph.p; A.y = P.v.p;
-      fine(P, IN_X, EPI_STORE, A);
-      vec<double>(stream, VOP_DOT2, VA, D, P.rh, P.rh, P.v, P.v, nullptr, Sp, Fp, part);
-      finalize(stream, PH_ALPHA, part, vg, Sp, Fp, maxit);
-      vec<double>(stream, VOP_BICG_S, VA, D, nullptr, r, nullptr, P.v, nullptr, Sp, Fp, part);
-      finalize(stream, PH_SNORM, part, vg, Sp, Fp, maxit);
-      bicg_half<double>(stream, D, x, P.ph, Sp, Fp);
-      precond(r, P.sh.p, nullptr, Fp);  // gated by F_ACTIVE only; harmless when converged at the half step
-      A.x = P.sh.p; A.y = P.q.p;
-      fine(P, IN_X, EPI_STORE, A);
-      vec<double>(stream, VOP_DOT2, VA, D, P.q, P.q, r, P.q, nullptr, Sp, Fp, part);
-      finalize(stream, PH_OMEGA, part, vg, Sp, Fp, maxit);
-      vec<double>(stream, VOP_BICG_X, VA, D, x, r, P.ph, P.sh, P.q, Sp, Fp, part);
-      finalize(stream, PH_RNORM, part, vg, Sp, Fp, maxit, mirror_dev, seq);
+      A.x = P.ph.p; A.y = P.v.p; A.b = P.rh.p; A.part = part2;
+      fine(P, IN_X, EPI_DOTS, A);
+      if (!inl) finalize(stream, PH_ALPHA, part2, fb, Sp, Fp, maxit);
+      krylov_pre(r, [&](auto& B) {
+        B.up = PRE_XR; B.x = x; B.p = P.ph; B.q = P.v; B.scal = Sp; B.scal_idx = S_ALPHA; B.part = part; B.active = Fp;
+        B.spd = false;
+        if (inl) { B.pq = part2; B.np = fb; B.num = S_RHON; B.keep = S_RHO; }
+      });
+      const Check half{part.p, fb, PH_BHALF, maxit, 0, nullptr, Sp};
+      if (!ichk) finalize(stream, PH_BHALF, part, fb, Sp, Fp, maxit);
+      precond_rest(r, P.sh.p, Fp, WHOLE, ichk ? &half : nullptr);
+      A.x = P.sh.p; A.y = P.q.p; A.b = r; A.part = part2;
+      fine(P, IN_X, EPI_DOTS, A);
+      if (!inl) finalize(stream, PH_OMEGA, part2, fb, Sp, Fp, maxit);
+      BicgArgs B;
+      B.x = x; B.r = r; B.sh = P.sh; B.t = P.q; B.rh = P.rh; B.scal = Sp; B.part = part; B.active = Fp;
+      if (inl) { B.ts = part2; B.np = fb; }
+      for (int k = 0; k < K; ++k) B.iw[k] = 1. / tab.wgt[k];
+      B.iwl = d_iw;
+      HIPCHK(launch_bicg_x(K, N, B, stream));
+      if (!ichk) finalize(stream, PH_BNEXT, part, fb, Sp, Fp, maxit, mirror_dev, seq);
+      chk.phase = PH_BNEXT;
+      krylov_pre(r, [&](auto& C) {
+        C.up = PRE_BICGP; C.p = P.p; C.pw = P.p; C.q = P.v; C.scal = Sp; C.active = Fp;
+        if (ichk) { C.pq = part; C.np = fb; }  // else PH_BNEXT has left beta
+      });
     }
+    if (ichk) krylov_vcycle(r, Sp, Fp, maxit, HEAD, &chk);
   }
+  void krylov_tail(double* r, double* Sp, int* Fp, int maxit) {
+    krylov_vcycle(r, Sp, Fp, maxit, inline_check() ? REST : WHOLE, nullptr);
+  }
+  struct EnsMask {  // the masks hold for the launches in its scope only
+    Solver& s;
+    explicit EnsMask(Solver& so) : s(so) { s.P64.iact = s.P32.iact = s.ens_act.p; }
+    ~EnsMask() { s.P64.iact = s.P32.iact = nullptr; }
+  };
   // One iteration of the batched ensemble PCG (ens_batched): PCG with a step length and a
   // direction coefficient per instance (r_i.z_i, p_i.q_i and ||r_i|| by segment), each instance
   // stopping on its own test; while an instance is stopped, the fine-level kernels skip the
   // blocks that hold only its elements, and its x and r stay as they are.  The coarse levels run
   // over every instance: with no Q1 vertex shared between instances they stay block-diagonal.
   void ens_iter(double* x, double* r, const double* pold, double* pnew, double* Sp, int* Fp, int maxit, int seq) {
-    struct Mask {  // the masks hold for this iteration's launches only
-      Solver& s;
-      explicit Mask(Solver& so) : s(so) { s.P64.iact = s.P32.iact = s.ens_act.p; }
-      ~Mask() { s.P64.iact = s.P32.iact = nullptr; }
-    } mask(*this);
+    EnsMask mask(*this);
     Prec<double>& P = P64;
     const EnsKry E = ensk();
-    if (mixed) {
-      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp);
-      seg_dot<float>(stream, pseg, r, P32.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-    } else {
-      vcycle_rest(P64, r, P.z.p, nullptr, Fp);
-      seg_dot<double>(stream, pseg, r, P.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-    }
-    finalize_ens(stream, ENS_RZ, E, Sp, Fp, maxit);
     direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr, nullptr,
                     Fp);
     seg_dot<double>(stream, pseg, pnew, P.q.p, Fp, ens_part.p, ens_in.p, ens_act.p);
     finalize_ens(stream, ENS_PQ, E, Sp, Fp, maxit);
-    pcg_update(x, r, pnew, ens_alpha.p, -1, nullptr, nullptr, Fp);
+    krylov_pre(r, [&](auto& A) {
+      A.up = PRE_XR; A.x = x; A.p = pnew; A.q = P.q; A.scal = ens_alpha; A.scal_idx = -1; A.active = Fp;
+    });
     // ||r_i||^2 into ens_rr, where a stopped instance keeps its last value (its r no longer changes)
     seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p, ens_act.p);
     EnsKry Eu = E;
     Eu.in = ens_rr.p;
     finalize_ens(stream, ENS_UPD, Eu, Sp, Fp, maxit, mirror_dev, seq);
   }
-  // The instantiated graph of one iteration on these buffers (captured on first use).
-  hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit, bool odd) {
+  // The instantiated graph of a piece of an iteration on these buffers (captured on first use).
+  hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit, int piece) {
     const void* key[6] = {&P64, x, r, Sp, Fp, mixed ? (const void*)&P32 : nullptr};
     for (auto& k : kgraphs)
-      if (k.maxit == maxit && k.odd == odd && std::equal(key, key + 6, k.key)) return k.e;
+      if (k.maxit == maxit && k.piece == piece && std::equal(key, key + 6, k.key)) return k.e;
     KGraph kg;
     std::copy(key, key + 6, kg.key);
     kg.maxit = maxit;
-    kg.odd = odd;
+    kg.piece = piece;
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
-      krylov_iter(x, r, Sp, Fp, maxit, -1, odd);
+      if (piece < 2) krylov_iter(x, r, Sp, Fp, maxit, -1, piece);
+      else krylov_tail(r, Sp, Fp, maxit);
     } catch (...) {
       hipGraph_t g = nullptr;
       (void)hipStreamEndCapture(stream, &g);
@@ -970,22 +1026,26 @@ struct Solver {
   void krylov_solve(double* x, double* r, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
     const int maxit = maxit_dev;
     const int seq0 = seq_next;
-    krylov_begin(x, r, Fp);
+    krylov_begin(x, r, Sp, Fp, maxit);
     const bool graphs = use_graphs && !prof.on;
-    hipGraphExec_t ge[2] = {nullptr, nullptr};
+    hipGraphExec_t ge[3] = {nullptr, nullptr, nullptr};
     if (graphs) {
-      for (int k = 0; k < 2; ++k) ge[k] = krylov_graph(x, r, Sp, Fp, maxit, k == 1);
+      for (int k = 0; k < 3; ++k) ge[k] = krylov_graph(x, r, Sp, Fp, maxit, k);
       set_int(stream, Fp + F_SEQ, seq_next - 1);
     }
+    // The host runs ahead by an iteration up to its test: while it waits for the status of the one
+    // before, the rest of a V-cycle and that iteration are queued.  Where that status says that the
+    // iteration is likely the last (near), its own is waited for before the next V-cycle is queued,
+    // which would run predicated off.
     for (int it = 0;; ++it) {
       const int seq = seq_next++;
       if (graphs) HIPCHK(hipGraphLaunch(ge[it & 1], stream));
       else krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
       bool near = false;
       if (!poll(seq, seq0, it > maxit_host + 2, 1, &near) || it > maxit_host + 4) break;
-      // the previous iteration ended within 8x of the tolerance: the one just queued is likely
-      // the last, so wait for it instead of queuing one that would run predicated off
       if (near && !poll(seq, seq0, true)) break;
+      if (graphs) HIPCHK(hipGraphLaunch(ge[2], stream));
+      else krylov_tail(r, Sp, Fp, maxit);
     }
   }
 
@@ -1008,15 +1068,20 @@ struct Solver {
     auto run = [&](bool graph) {
       HIPCHK(hipMemsetAsync(psi.p, 0, D * sizeof(double), stream));
       outer_residual(nullptr);
-      krylov_begin(psi.p, P64.r.p, F.p);
-      hipGraphExec_t ge[2] = {nullptr, nullptr};
-      for (int k = 0; k < 2 && graph; ++k) ge[k] = krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit, k == 1);
+      krylov_begin(psi.p, P64.r.p, S.p, F.p, maxit);
+      hipGraphExec_t ge[3] = {nullptr, nullptr, nullptr};
+      for (int k = 0; k < 3 && graph; ++k) ge[k] = krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit, k);
       HIPCHK(hipStreamSynchronize(stream));
       const auto t0 = std::chrono::steady_clock::now();
       if (graph) set_int(stream, F.p + F_SEQ, seq_next - 1);
       for (int i = 0; i < kTuneIters; ++i, ++seq_next) {
-        if (graph) HIPCHK(hipGraphLaunch(ge[i & 1], stream));
-        else krylov_iter(psi.p, P64.r.p, S.p, F.p, maxit, seq_next, i & 1);
+        if (graph) {
+          HIPCHK(hipGraphLaunch(ge[i & 1], stream));
+          HIPCHK(hipGraphLaunch(ge[2], stream));
+        } else {
+          krylov_iter(psi.p, P64.r.p, S.p, F.p, maxit, seq_next, i & 1);
+          krylov_tail(P64.r.p, S.p, F.p, maxit);
+        }
       }
       HIPCHK(hipStreamSynchronize(stream));
       return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
