@@ -10,17 +10,18 @@ constexpr int kTB = 256;
 inline unsigned grid(size_t n) { return (unsigned)((n + kTB - 1) / kTB); }
 
 // seeds: one thread per (value, probe)
-__global__ void k_adj_seed(size_t D, int K2, const int32_t* __restrict__ color, int c, double* __restrict__ x) {
+__global__ void k_adj_seed(size_t D, int K2, const int32_t* __restrict__ color, int u0, double* __restrict__ x) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int b = blockIdx.y;
   if (i >= D) return;
   const size_t e = i / K2;
-  x[(size_t)b * D + i] = (color[e] == c && (int)(i - e * K2) == b) ? 1. : 0.;
+  const int u = b / K2, m = b - u * K2;
+  x[(size_t)b * D + i] = (color[e] == u0 + u && (int)(i - e * K2) == m) ? 1. : 0.;
 }
 
 // traces of the seeds (the traces of src/HO_2D.cpp:2695-2713 of a unit value at (j0, i0)):
 // faces 0/1 (xi = -1/+1) carry l_i0 and l_i0' at eta point j0, faces 2/3 l_j0 and l_j0' at xi point i0
-__global__ void k_adj_seed_tr(int N, int K, const int32_t* __restrict__ color, int c, Tab T, double* __restrict__ tr) {
+__global__ void k_adj_seed_tr(int N, int K, const int32_t* __restrict__ color, int u0, Tab T, double* __restrict__ tr) {
   const size_t TR = (size_t)4 * N * 2 * K;
   const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // plane f, element e, slot kk
   const int b = blockIdx.y;
@@ -28,11 +29,11 @@ __global__ void k_adj_seed_tr(int N, int K, const int32_t* __restrict__ color, i
   const int f = (int)(q / ((size_t)N * 2 * K));
   const size_t rem = q - (size_t)f * N * 2 * K;
   const int e = (int)(rem / (2 * K)), kk = (int)(rem - (size_t)e * 2 * K);
-  const int j0 = b / K, i0 = b % K;
+  const int u = b / (K * K), m = b - u * K * K, j0 = m / K, i0 = m % K;
   const int pos = f < 2 ? j0 : i0, idx = f < 2 ? i0 : j0, ib = f & 1;
   const int k = kk < K ? kk : kk - K;
   double v = 0.;
-  if (color[e] == c && k == pos) v = kk < K ? T.bb[idx][ib] : T.bgb[idx][ib];
+  if (color[e] == u0 + u && k == pos) v = kk < K ? T.bb[idx][ib] : T.bgb[idx][ib];
   tr[(size_t)b * TR + q] = v;
 }
 
@@ -56,31 +57,33 @@ __global__ __launch_bounds__(kDotEl) void k_adj_dot(int N, int K2, const double*
   p[(size_t)b * N + e0 + threadIdx.x] = s;
 }
 
-// one thread per (member of the colour, dof): members = the colour's element list
-__global__ void k_adj_gather(int N, int K2, int nmem, const int32_t* __restrict__ members,
+// one thread per (element, component, dof)
+__global__ void k_adj_gather(int N, int K2, int ncomp, int u0, int nu, const int32_t* __restrict__ color,
                              const int32_t* __restrict__ rptr, const int32_t* __restrict__ ridx,
-                             const double* __restrict__ p, double* __restrict__ out, int ostride, int ooff) {
+                             const double* __restrict__ p, double* __restrict__ out) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)nmem * K2) return;
-  const int k = (int)(t / K2), m = (int)(t - (size_t)k * K2);
-  const int e = members[k];
-  const double* pm = p + (size_t)m * N;
+  const int R = ncomp * K2;
+  if (t >= (size_t)N * R) return;
+  const int e = (int)(t / R), r = (int)(t - (size_t)e * R), comp = r / K2, m = r - comp * K2;
+  const int u = color[e] * ncomp + comp - u0;
+  if (u < 0 || u >= nu) return;
+  const double* pm = p + ((size_t)u * K2 + m) * N;
   double s = 0.;
   for (int j = rptr[e]; j < rptr[e + 1]; ++j) s += pm[ridx[j]];
-  out[(size_t)e * ostride + ooff + m] = s;
+  out[t] = s;
 }
 
 // U seeds and their normal traces (k_velocity's: faces 0/1 from U1 along xi at eta point j,
 // faces 2/3 from U2 along eta at xi point i)
-__global__ void k_adj_seed_u(int N, int K, const int32_t* __restrict__ color, int c, int comp, Tab T,
+__global__ void k_adj_seed_u(int N, int K, const int32_t* __restrict__ color, int u0, Tab T,
                              double* __restrict__ U, double* __restrict__ tru) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int b = blockIdx.y;
-  const int K2 = K * K, j0 = b / K, i0 = b % K;
+  const int K2 = K * K, u = b / K2, m = b - u * K2, c = (u0 + u) >> 1, comp = (u0 + u) & 1, j0 = m / K, i0 = m % K;
   const size_t NU = (size_t)N * 2 * K2, TU = (size_t)4 * N * K;
   if (t < NU) {  // U values
     const int e = (int)(t / (2 * K2)), o = (int)(t - (size_t)e * 2 * K2);
-    U[(size_t)b * NU + t] = (color[e] == c && o == comp * K2 + b) ? 1. : 0.;
+    U[(size_t)b * NU + t] = (color[e] == c && o == comp * K2 + m) ? 1. : 0.;
   } else if (t < NU + TU) {  // normal traces
     const size_t q = t - NU;
     const int f = (int)(q / ((size_t)N * K));
@@ -211,14 +214,14 @@ __global__ void k_adj_wj(size_t D, int K, Wts W, const double* __restrict__ jac,
 
 }  // namespace
 
-hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int c, const Tab& T, double* x, double* tr,
-                                 hipStream_t s) {
+hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* x,
+                                 double* tr, hipStream_t s) {
   const int K2 = K * K;
   const size_t D = (size_t)N * K2;
   if (D == 0) return hipSuccess;
   if (K > kMaxKd) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_adj_seed, dim3(grid(D), K2), dim3(kTB), 0, s, D, K2, color, c, x);
-  hipLaunchKernelGGL(k_adj_seed_tr, dim3(grid((size_t)4 * N * 2 * K), K2), dim3(kTB), 0, s, N, K, color, c, T, tr);
+  hipLaunchKernelGGL(k_adj_seed, dim3(grid(D), nu * K2), dim3(kTB), 0, s, D, K2, color, u0, x);
+  hipLaunchKernelGGL(k_adj_seed_tr, dim3(grid((size_t)4 * N * 2 * K), nu * K2), dim3(kTB), 0, s, N, K, color, u0, T, tr);
   return hipGetLastError();
 }
 
@@ -229,21 +232,21 @@ hipError_t launch_adj_dot_batch(int N, int K2, int nb, const double* lam, const 
   return hipGetLastError();
 }
 
-hipError_t launch_adj_gather_batch(int N, int K2, int nmem, const int32_t* members, const int32_t* rptr,
-                                   const int32_t* ridx, const double* p, double* out, int ostride, int ooff,
+hipError_t launch_adj_gather_batch(int N, int K2, int ncomp, int u0, int nu, const int32_t* color,
+                                   const int32_t* rptr, const int32_t* ridx, const double* p, double* out,
                                    hipStream_t s) {
-  if (nmem == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_adj_gather, dim3(grid((size_t)nmem * K2)), dim3(kTB), 0, s, N, K2, nmem, members, rptr, ridx,
-                     p, out, ostride, ooff);
+  if (N == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_adj_gather, dim3(grid((size_t)N * ncomp * K2)), dim3(kTB), 0, s, N, K2, ncomp, u0, nu, color,
+                     rptr, ridx, p, out);
   return hipGetLastError();
 }
 
-hipError_t launch_adj_seed_u_batch(int N, int K, const int32_t* color, int c, int comp, const Tab& T, double* U,
+hipError_t launch_adj_seed_u_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* U,
                                    double* tru, hipStream_t s) {
   if (N == 0) return hipSuccess;
-  if (K > kMaxKd || comp < 0 || comp > 1) return hipErrorInvalidValue;
+  if (K > kMaxKd) return hipErrorInvalidValue;
   const size_t n = (size_t)N * 2 * K * K + (size_t)4 * N * K;
-  hipLaunchKernelGGL(k_adj_seed_u, dim3(grid(n), K * K), dim3(kTB), 0, s, N, K, color, c, comp, T, U, tru);
+  hipLaunchKernelGGL(k_adj_seed_u, dim3(grid(n), nu * K * K), dim3(kTB), 0, s, N, K, color, u0, T, U, tru);
   return hipGetLastError();
 }
 

@@ -6,27 +6,31 @@
 // of any output element, the product y = J seed holds, at every element e, the column of its
 // one colour-c ring member.  Then (J^T lam)[i][m] = sum over the elements e whose ring holds i
 // of lam_e . y_e, a gather over i's ring of the per-element products p_e = lam_e . y_e.  The
-// K^2 probes of a colour run as one batch (probe b at offset b * the array size).
+// probes run in batches (probe b at offset b * the array size).
 #pragma once
 
 #include "hoc_kernels.hpp"
 
 namespace hoc {
 
-// K^2 probes of colour c: x[b] = unit seed at local dof b of the colour-c elements ([K2][N][K2])
-// and tr[b] its face traces in the trace-plane layout ([K2][4][N][2K])
-hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int c, const Tab& T, double* x, double* tr,
-                                 hipStream_t s);
+// Probes come in units of K^2: of the vorticity, unit c seeds the colour-c elements; of the velocity,
+// unit 2 c + comp component comp of theirs.  A batch holds the units [u0, u0 + nu), probe m of unit u
+// at (u - u0) K^2 + m: one launch of the stage for many colours, where one colour's probes leave the
+// chip empty (24 x 24 elements, K = 4: 144 blocks and 14 us for a launch of 16 probes).
+// Vorticity: x[b] = unit seed at local dof m ([.][N][K2]) and tr[b] its face traces in the trace-plane
+// layout ([.][4][N][2K])
+hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* x,
+                                 double* tr, hipStream_t s);
 // p[b][e] = sum_r lam[e][r] y[b][e][r], b < nb
 hipError_t launch_adj_dot_batch(int N, int K2, int nb, const double* lam, const double* y, double* p, hipStream_t s);
-// out[i][ooff + m] (row stride ostride) = sum over e in ring(i) of p[m][e], for the nmem elements
-// i of a colour (members; ring as CSR)
-hipError_t launch_adj_gather_batch(int N, int K2, int nmem, const int32_t* members, const int32_t* rptr,
-                                   const int32_t* ridx, const double* p, double* out, int ostride, int ooff,
+// out[i][comp K2 + m] (ncomp K2 values a row) = sum over e in ring(i) of p[b][e], for the elements i and
+// components comp < ncomp whose unit is in the batch (ring as CSR)
+hipError_t launch_adj_gather_batch(int N, int K2, int ncomp, int u0, int nu, const int32_t* color,
+                                   const int32_t* rptr, const int32_t* ridx, const double* p, double* out,
                                    hipStream_t s);
-// K^2 probes of colour c on velocity component comp of U ([N][2][K2]): U[b] = unit seed at local dof b
-// of component comp of the colour-c elements, tru[b] its contravariant normal traces ([4][N][K])
-hipError_t launch_adj_seed_u_batch(int N, int K, const int32_t* color, int c, int comp, const Tab& T, double* U,
+// Velocity: U[b] = unit seed at local dof m of component comp of U ([.][N][2][K2]), tru[b] its
+// contravariant normal traces ([.][4][N][K])
+hipError_t launch_adj_seed_u_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* U,
                                    double* tru, hipStream_t s);
 // Assembly of the (state-independent) velocity map psi -> U from K^2 probes of colour c
 // (dU [K2][N][2K2]): Mv[e][slot][m][o] = dU[m][e][o] for the slot (0 self, 1 + f neighbour across

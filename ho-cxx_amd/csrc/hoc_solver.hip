@@ -1794,12 +1794,12 @@ struct Solver {
     bool init = false;
     int nc1 = 0;
     DBuf<int32_t> col1, r1p, r1i, own_el;
-    DBuf<int32_t> members;            // elements sorted by colour, colour c at [moff[c], moff[c + 1])
-    std::vector<int> moff;
+    int ub = 1;                       // probe units (hoc_adj.hpp) of a batch
+    bool seeds_kept = false;          // every unit fits one batch: its seeds are written once, by the setup
     DBuf<int8_t> own_f;
     DBuf<double> ws[4], Us[4], trws[4], trus[4];  // recorded stages of one step
     DBuf<int8_t> sig[4];
-    // probe batches (nb = max(K^2, 4K) probes): seeds and their traces, products, velocities
+    // probe batches (ub K^2 probes, at least 4K): seeds and their traces, products, velocities
     DBuf<double> seed, seed_tr, y, p, dU, dvel, dtrw, dtru, lin_diff, lin_vj, pvel_seed;
     DBuf<double> zero_d, zero_tr, zero_e, lin_nvel, lin_vort, lin_adv;
     DBuf<double> lam, xbar, psibar, z, fake, wbar, kbar[4], pvbar;
@@ -1902,22 +1902,18 @@ struct Solver {
     rings(1, p1, i1);
     adj.col1.upload(c1);
     adj.r1p.upload(p1); adj.r1i.upload(i1);
-    {
-      std::vector<int32_t> mem;
-      adj.moff.assign(1, 0);
-      for (int c = 0; c < adj.nc1; ++c) {
-        for (int e = 0; e < N; ++e)
-          if (c1[e] == c) mem.push_back(e);
-        adj.moff.push_back((int)mem.size());
-      }
-      adj.members.upload(mem);
-    }
     std::vector<int32_t> oe(std::max(E, 1), 0);
     std::vector<int8_t> of(std::max(E, 1), -1);
     for (int e = 0; e < E; ++e) { oe[e] = mesh.be_elem[e]; of[e] = mesh.be_ijp[e]; }
     adj.own_el.upload(oe); adj.own_f.upload(of);
     const size_t TR = (size_t)4 * N * 2 * K, TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
-    const size_t NB = std::max(K2, 4 * K);
+    // Units per batch: as many as 256 MiB hold (one, whatever it takes, on meshes whose single units
+    // fill the chip): batches of all 14 take 24 x 24 elements, K = 4, from 95 launches a stage to 14.
+    const double unit = 8. * K2 * (4. * (double)D + (double)TR + (double)TU);
+    adj.ub = (int)std::min(std::max(268435456. / unit, 1.), 2. * adj.nc1);
+    adj.seeds_kept = adj.ub == 2 * adj.nc1;
+    const size_t NB1 = std::max(K2, 4 * K), NB = std::max<size_t>((size_t)adj.ub * K2, NB1);
+    const size_t NBw = std::max<size_t>((size_t)std::min(adj.ub, adj.nc1) * K2, NB1);  // vorticity units alone
     for (int s4 = 0; s4 < 4; ++s4) {
       adj.ws[s4].alloc(D); adj.Us[s4].alloc(2 * D); adj.trws[s4].alloc(TR); adj.trus[s4].alloc(TU);
       adj.sig[s4].alloc((size_t)4 * N * K); adj.kbar[s4].alloc(D);
@@ -1927,10 +1923,10 @@ struct Solver {
       b->alloc(D);
     adj.save_vel.alloc(2 * D);
     adj.zero_tr.alloc(TR);
-    adj.seed.alloc(NB * D); adj.y.alloc(NB * D); adj.seed_tr.alloc(NB * TR); adj.dtrw.alloc(NB * TR);
-    adj.dU.alloc(NB * 2 * D); adj.dvel.alloc(NB * 2 * D); adj.dtru.alloc(NB * TU);
+    adj.seed.alloc(NBw * D); adj.y.alloc(NB * D); adj.seed_tr.alloc(NBw * TR); adj.dtrw.alloc(NB1 * TR);
+    adj.dU.alloc(NB * 2 * D); adj.dvel.alloc(NB1 * 2 * D); adj.dtru.alloc(NB * TU);
     adj.p.alloc(NB * std::max(N, 1));
-    adj.lin_diff.alloc(NB * EK); adj.lin_vj.alloc(NB * EK); adj.pvel_seed.alloc((size_t)4 * K * EK);
+    adj.lin_diff.alloc(NB1 * EK); adj.lin_vj.alloc(NB1 * EK); adj.pvel_seed.alloc((size_t)4 * K * EK);
     // seeds of the wall-flux probes are edge arrays like the wall velocity's
     for (DBuf<double>* b : {&adj.zero_e, &adj.lin_vort, &adj.lin_adv, &adj.pvbar}) b->alloc(EK);
     adj.lin_nvel.alloc(EK);
@@ -1952,12 +1948,17 @@ struct Solver {
     VelBatch vb;
     vb.psi = D; vb.trpsi = TR; vb.vel = 2 * D; vb.U = 2 * D; vb.trw = TR; vb.tru = TU; vb.vjump = EK; vb.diff = EK;
     for (int c = 0; c < adj.nc1; ++c) {
-      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, c, T, adj.seed, adj.seed_tr, stream));
+      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, c, 1, T, adj.seed, adj.seed_tr, stream));
       HIPCHK(launch_velocity_batch(K, N, T, G, adj.Bl, adj.seed, adj.seed_tr, adj.zero_d, adj.dvel, adj.dU, adj.dtrw,
                                    adj.dtru, 1. / (cfg.dt * re_inv), I, K2, vb, stream));
       HIPCHK(launch_adj_assemble_vel(N, E, K, adj.col1, c, d_nb, adj.own_el, adj.dU, adj.lin_diff, adj.Mv, adj.Md,
                                      stream));
     }
+    if (adj.seeds_kept) {
+      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, 0, adj.nc1, T, adj.seed, adj.seed_tr, stream));
+      HIPCHK(launch_adj_seed_u_batch(N, K, adj.col1, 0, 2 * adj.nc1, T, adj.dU, adj.dtru, stream));
+    }
+    if (E > 0) HIPCHK(launch_adj_edge_seed_batch(E, K, adj.own_f, adj.pvel_seed, stream));
     HIPCHK(hipStreamSynchronize(stream));
     adj.init = true;
   }
@@ -1991,7 +1992,7 @@ struct Solver {
   }
 
   // xbar = (dk_s/domega_s)^T lam for recorded stage st, adding (dk_s/dpvel)^T lam to adj.pvbar.
-  // The K^2 probes of a colour (and the 4K wall-velocity probes) run as one batched launch each.
+  // The probes of many colours (and the 4K wall-velocity probes) run as one batched launch each.
   void adj_stage(int st, const double* lam, double* xbar, double tau = std::nan("")) {
     const double idr = 1. / (cfg.dt * re_inv);
     const size_t TR = (size_t)4 * N * 2 * K, TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
@@ -2000,40 +2001,37 @@ struct Solver {
     so.bs_k = D;
     so.sig = adj.sig[st];
     // (1) omega and its face traces, with psi (so U and the wall flux) fixed
-    so.nbatch = K2;
     so.omega_adv = adj.seed; so.bs_wa = D;
     so.trw_adv = adj.seed_tr; so.bs_trwa = TR;
     so.bs_w = D; so.bs_trw = TR;
-    for (int c = 0; c < adj.nc1; ++c) {
-      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, c, T, adj.seed, adj.seed_tr, stream));
+    for (int u0 = 0; u0 < adj.nc1; u0 += adj.ub) {
+      const int nu = std::min(adj.ub, adj.nc1 - u0);
+      so.nbatch = nu * K2;
+      if (!adj.seeds_kept) HIPCHK(launch_adj_seed_batch(N, K, adj.col1, u0, nu, T, adj.seed, adj.seed_tr, stream));
       HIPCHK(launch_stage(K, 1, N, T, G, adj.Bz, adj.seed, adj.Us[st], adj.seed_tr, adj.trus[st], re_inv, cfg.dt, I,
                           so, stream, 2));
-      HIPCHK(launch_adj_dot_batch(N, K2, K2, lam, adj.y, adj.p, stream));
-      HIPCHK(launch_adj_gather_batch(N, K2, adj.moff[c + 1] - adj.moff[c], adj.members.p + adj.moff[c], adj.r1p,
-                                     adj.r1i, adj.p, xbar, K2, 0, stream));
+      HIPCHK(launch_adj_dot_batch(N, K2, so.nbatch, lam, adj.y, adj.p, stream));
+      HIPCHK(launch_adj_gather_batch(N, K2, 1, u0, nu, adj.col1, adj.r1p, adj.r1i, adj.p, xbar, stream));
     }
-    // (2) velocity: K^2 probes per colour and component (the stage depends on U over the face ring),
+    // (2) velocity: a unit per colour and component (the stage depends on U over the face ring),
     //     the stage advecting the recorded vorticity with the seeded velocity
     so.omega_adv = adj.ws[st]; so.bs_wa = 0;
     so.trw_adv = adj.trws[st]; so.bs_trwa = 0;
     so.bs_w = 0; so.bs_trw = 0; so.bs_U = 2 * D; so.bs_tru = TU; so.bs_diff = 0;
-    so.nbatch = K2;
     so.adv_only = 1;  // zero vorticity and wall flux for the diffusion term
-    for (int c = 0; c < adj.nc1; ++c)
-      for (int comp = 0; comp < 2; ++comp) {
-        HIPCHK(launch_adj_seed_u_batch(N, K, adj.col1, c, comp, T, adj.dU, adj.dtru, stream));
-        HIPCHK(launch_stage(K, 1, N, T, G, adj.Bz, adj.zero_d, adj.dU, adj.zero_tr, adj.dtru, re_inv, cfg.dt, I, so,
-                            stream, 2));
-        HIPCHK(launch_adj_dot_batch(N, K2, K2, lam, adj.y, adj.p, stream));
-        HIPCHK(launch_adj_gather_batch(N, K2, adj.moff[c + 1] - adj.moff[c], adj.members.p + adj.moff[c], adj.r1p,
-                                       adj.r1i, adj.p, adj.Ubar, 2 * K2, comp * K2,
-                                       stream));
-      }
+    for (int u0 = 0; u0 < 2 * adj.nc1; u0 += adj.ub) {
+      const int nu = std::min(adj.ub, 2 * adj.nc1 - u0);
+      so.nbatch = nu * K2;
+      if (!adj.seeds_kept) HIPCHK(launch_adj_seed_u_batch(N, K, adj.col1, u0, nu, T, adj.dU, adj.dtru, stream));
+      HIPCHK(launch_stage(K, 1, N, T, G, adj.Bz, adj.zero_d, adj.dU, adj.zero_tr, adj.dtru, re_inv, cfg.dt, I, so,
+                          stream, 2));
+      HIPCHK(launch_adj_dot_batch(N, K2, so.nbatch, lam, adj.y, adj.p, stream));
+      HIPCHK(launch_adj_gather_batch(N, K2, 2, u0, nu, adj.col1, adj.r1p, adj.r1i, adj.p, adj.Ubar, stream));
+    }
     // (3) wall flux: probe f K + j seeds edge flux point j of the edges owned through face f, which
     //     reaches only the owner elements; then the wall velocity's share of it
     HIPCHK(hipMemsetAsync(adj.diffbar.p, 0, EK * sizeof(double), stream));
     if (E > 0) {
-      HIPCHK(launch_adj_edge_seed_batch(E, K, adj.own_f, adj.pvel_seed, stream));
       so.omega_adv = adj.zero_d; so.trw_adv = adj.zero_tr;
       so.bs_U = 0; so.bs_tru = 0; so.bs_diff = EK;
       so.adv_only = 0;
