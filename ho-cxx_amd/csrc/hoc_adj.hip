@@ -19,24 +19,6 @@ __global__ void k_adj_seed(size_t D, int K2, const int32_t* __restrict__ color, 
   x[(size_t)b * D + i] = (color[e] == u0 + u && (int)(i - e * K2) == m) ? 1. : 0.;
 }
 
-// traces of the seeds (the traces of src/HO_2D.cpp:2695-2713 of a unit value at (j0, i0)):
-// faces 0/1 (xi = -1/+1) carry l_i0 and l_i0' at eta point j0, faces 2/3 l_j0 and l_j0' at xi point i0
-__global__ void k_adj_seed_tr(int N, int K, const int32_t* __restrict__ color, int u0, Tab T, double* __restrict__ tr) {
-  const size_t TR = (size_t)4 * N * 2 * K;
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // plane f, element e, slot kk
-  const int b = blockIdx.y;
-  if (q >= TR) return;
-  const int f = (int)(q / ((size_t)N * 2 * K));
-  const size_t rem = q - (size_t)f * N * 2 * K;
-  const int e = (int)(rem / (2 * K)), kk = (int)(rem - (size_t)e * 2 * K);
-  const int u = b / (K * K), m = b - u * K * K, j0 = m / K, i0 = m % K;
-  const int pos = f < 2 ? j0 : i0, idx = f < 2 ? i0 : j0, ib = f & 1;
-  const int k = kk < K ? kk : kk - K;
-  double v = 0.;
-  if (color[e] == u0 + u && k == pos) v = kk < K ? T.bb[idx][ib] : T.bgb[idx][ib];
-  tr[(size_t)b * TR + q] = v;
-}
-
 // 64 elements per block: the products are formed with coalesced reads into an LDS tile, then
 // each thread sums its element's row
 constexpr int kDotEl = 64;
@@ -214,14 +196,11 @@ __global__ void k_adj_wj(size_t D, int K, Wts W, const double* __restrict__ jac,
 
 }  // namespace
 
-hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* x,
-                                 double* tr, hipStream_t s) {
+hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, double* x, hipStream_t s) {
   const int K2 = K * K;
   const size_t D = (size_t)N * K2;
   if (D == 0) return hipSuccess;
-  if (K > kMaxKd) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_adj_seed, dim3(grid(D), nu * K2), dim3(kTB), 0, s, D, K2, color, u0, x);
-  hipLaunchKernelGGL(k_adj_seed_tr, dim3(grid((size_t)4 * N * 2 * K), nu * K2), dim3(kTB), 0, s, N, K, color, u0, T, tr);
   return hipGetLastError();
 }
 

@@ -17,10 +17,8 @@ namespace hoc {
 // unit 2 c + comp component comp of theirs.  A batch holds the units [u0, u0 + nu), probe m of unit u
 // at (u - u0) K^2 + m: one launch of the stage for many colours, where one colour's probes leave the
 // chip empty (24 x 24 elements, K = 4: 144 blocks and 14 us for a launch of 16 probes).
-// Vorticity: x[b] = unit seed at local dof m ([.][N][K2]) and tr[b] its face traces in the trace-plane
-// layout ([.][4][N][2K])
-hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, const Tab& T, double* x,
-                                 double* tr, hipStream_t s);
+// Vorticity: x[b] = unit seed at local dof m ([.][N][K2])
+hipError_t launch_adj_seed_batch(int N, int K, const int32_t* color, int u0, int nu, double* x, hipStream_t s);
 // p[b][e] = sum_r lam[e][r] y[b][e][r], b < nb
 hipError_t launch_adj_dot_batch(int N, int K2, int nb, const double* lam, const double* y, double* p, hipStream_t s);
 // out[i][comp K2 + m] (ncomp K2 values a row) = sum over e in ring(i) of p[b][e], for the elements i and

@@ -1,4 +1,4 @@
-// hoc_fr.hpp - launchers of the FR stage kernels (hoc_fr.hip).
+// hoc_fr.hpp - launchers of the stage kernels (hoc_stage.hip) and of the boundary values (hoc_fr.hip).
 #pragma once
 
 #include "hoc_kernels.hpp"
@@ -15,34 +15,30 @@ struct StageOut {
   const double *k1 = nullptr, *k2 = nullptr, *k3 = nullptr;
   // linearised stage (launch_stage mode 1 records, mode 2 reads the upwind switches)
   int8_t* sig = nullptr;               // [N][4][K] upwind switch of each interior flux point
-  const double* omega_adv = nullptr;   // mode 2: advected vorticity and its traces
-  const double* trw_adv = nullptr;
   // mode 2 batches: nbatch independent products in one launch, probe b reading/writing its
   // arrays at b * (stride in values); stride 0 shares an array between the probes
   int nbatch = 1;
   int adv_only = 0;  // mode 2: the diffusion inputs are zero (skip the diffusion term)
-  size_t bs_w = 0, bs_trw = 0, bs_U = 0, bs_tru = 0, bs_wa = 0, bs_trwa = 0, bs_k = 0, bs_diff = 0;
+  size_t bs_w = 0, bs_U = 0, bs_tru = 0, bs_k = 0, bs_diff = 0;
+  bool inner = false;  // an intermediate stage: the Cartesian velocity is not an output
 };
 
 // Batch strides (in values) of the batched velocity launch.
 struct VelBatch {
-  size_t psi = 0, trpsi = 0, omega = 0, vel = 0, U = 0, trw = 0, tru = 0, vjump = 0, diff = 0, pvel = 0;
+  size_t psi = 0, U = 0, tru = 0, vjump = 0, diff = 0, pvel = 0;
 };
 
-// Face traces of x (face-major, see hoc_fr.hip).
-hipError_t launch_trace(int K, int N, const Tab& T, const double* x, double* tr, hipStream_t s);
-hipError_t launch_rhs(int K, int N, const Tab& T, const Geo& G, const double* omega, const double* bcpsi, double* bs,
-                      double* part, hipStream_t s);
-hipError_t launch_velocity(int K, int N, const Tab& T, const Geo& G, const BCDev& B, const double* psi,
-                           const double* trpsi, const double* omega, double* vel, double* U, double* trw,
-                           double* tru, double inv_dt_re, const InstDev& I, hipStream_t s);
-// nbatch velocity evaluations in one launch (probe b offset by b * the strides of vb)
-hipError_t launch_velocity_batch(int K, int N, const Tab& T, const Geo& G, const BCDev& B, const double* psi,
-                                 const double* trpsi, const double* omega, double* vel, double* U, double* trw,
-                                 double* tru, double inv_dt_re, const InstDev& I, int nbatch, const VelBatch& vb,
-                                 hipStream_t s);
-hipError_t launch_stage(int K, int adv, int N, const Tab& T, const Geo& G, const BCDev& B, const double* omega,
-                        const double* U, const double* trw, const double* tru, double re_inv, double dt,
+// geo: GEO_ORTHO, GEO_AFFINE or GEO_POINT (hoc_poisson.hpp).  part: fine_blocks(K, N) sums.
+hipError_t launch_rhs(int K, int geo, int N, const Tab& T, const Geo& G, const double* omega, const double* bcpsi,
+                      double* bs, double* part, hipStream_t s);
+// vel may be null; tru: the normal traces of U, face-major [4][N][K].  nbatch velocity evaluations in one
+// launch: probe b offset by b * the strides of vb, vel null.
+hipError_t launch_velocity(int K, int geo, int N, const Tab& T, const Geo& G, const BCDev& B, const double* psi,
+                           double* vel, double* U, double* tru, double inv_dt_re, const InstDev& I, hipStream_t s,
+                           int nbatch = 1, const VelBatch& vb = VelBatch{});
+// omega may be none of the arrays that the launch writes.
+hipError_t launch_stage(int K, int geo, int adv, int N, const Tab& T, const Geo& G, const BCDev& B,
+                        const double* omega, const double* U, const double* tru, double re_inv, double dt,
                         const InstDev& I, const StageOut& so, hipStream_t s, int mode = 0);
 // n = E*K boundary values; tc = time factor (per instance through I.ramp when set)
 hipError_t launch_update_bcs(int n, int K, const BCDev& B, double tc, const InstDev& I, hipStream_t s);
@@ -51,6 +47,5 @@ hipError_t launch_update_bcs(int n, int K, const BCDev& B, double tc, const Inst
 hipError_t launch_update_bcs_hybrid(int n, int K, const BCDev& B, const HybridDev& H, double fac1, double fac2,
                                     hipStream_t s);
 hipError_t launch_hybrid_blend(size_t n, double* w, const HybridDev& H, double fac1, double fac2, hipStream_t s);
-int lap_blocks(int N);
 
 }  // namespace hoc

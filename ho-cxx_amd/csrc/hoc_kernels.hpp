@@ -58,6 +58,9 @@ struct GeoT {
   const int8_t* no_slip;                   // [E]
   const R* esign;                          // [E] 2*(ijp%2)-1 of the owner face
   const int32_t* inst;                     // [N] ensemble instance of each element, or null
+  const R* dcol;                           // [K][K]     l_d'(xi_k), k first
+  const R* wrow;                           // [K]        weights
+  const R* qn;                             // [E][K][K]  see FineGeo
 };
 using Geo = GeoT<double>;
 

@@ -22,88 +22,12 @@
 // a and c are the element's mean metrics.
 #include "hoc_poisson.hpp"
 
+#include "hoc_rowlane.hpp"
 #include "hoc_status.hpp"
 
 namespace hoc {
 
 namespace {
-
-// Blocks are dealt to the 8 XCDs in turn: block b works on part b % 8 of the elements, so the
-// elements an XCD works on at one time are neighbours and share its L2.
-__device__ __forceinline__ int xcd_block(int b, int nb) {
-  const int q = nb >> 3, r = nb & 7, x = b & 7, i = b >> 3;
-  return x * q + min(x, r) + i;
-}
-
-// Orders this wavefront's LDS writes before its reads (LDS serves one wavefront in order).
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-template <int K>
-struct Lay {
-  static constexpr int EPW = fine_epw(K);
-  static constexpr int RS = (K & 1) ? K : K + 1;  // row stride in LDS (odd: rows on distinct banks)
-  static constexpr int ES = K * RS;
-  static constexpr int TILE = EPW * ES;
-};
-
-// Two values at any address aligned to one of them (one 16- or 8-byte load).
-template <class R> struct Two;
-template <> struct Two<double> { typedef double t __attribute__((ext_vector_type(2), aligned(8))); };
-template <> struct Two<float> { typedef float t __attribute__((ext_vector_type(2), aligned(4))); };
-
-template <int K, class V, class R>
-__device__ __forceinline__ void load_row(const V* __restrict__ g, R (&v)[K]) {
-#pragma unroll
-  for (int i = 0; i + 1 < K; i += 2) {
-    const typename Two<V>::t t = *reinterpret_cast<const typename Two<V>::t*>(g + i);
-    v[i] = (R)t.x;
-    v[i + 1] = (R)t.y;
-  }
-  if (K & 1) v[K - 1] = (R)g[K - 1];
-}
-template <int K, class V, class R>
-__device__ __forceinline__ void store_row(V* __restrict__ g, const R (&v)[K]) {
-#pragma unroll
-  for (int i = 0; i + 1 < K; i += 2) {
-    typename Two<V>::t t;
-    t.x = (V)v[i];
-    t.y = (V)v[i + 1];
-    *reinterpret_cast<typename Two<V>::t*>(g + i) = t;
-  }
-  if (K & 1) g[K - 1] = (V)v[K - 1];
-}
-
-// rows -> columns (and columns -> rows) of the wavefront's elements through its LDS tile
-template <int K, class R>
-__device__ __forceinline__ void rows_to_cols(R* t, int k, const R (&row)[K], R (&col)[K]) {
-  constexpr int RS = Lay<K>::RS;
-  wave_fence();
-#pragma unroll
-  for (int i = 0; i < K; ++i) t[k * RS + i] = row[i];
-  wave_fence();
-#pragma unroll
-  for (int j = 0; j < K; ++j) col[j] = t[j * RS + k];
-}
-template <int K, class R>
-__device__ __forceinline__ void cols_to_rows(R* t, int k, const R (&col)[K], R (&row)[K]) {
-  constexpr int RS = Lay<K>::RS;
-  wave_fence();
-#pragma unroll
-  for (int j = 0; j < K; ++j) t[j * RS + k] = col[j];
-  wave_fence();
-#pragma unroll
-  for (int i = 0; i < K; ++i) row[i] = t[k * RS + i];
-}
 
 // Even and odd parts of a line, and back.
 template <int K, class R>
@@ -149,12 +73,6 @@ struct Face {
   int kk = 0;       // its point on that face
   bool neu = false;
 };
-
-// The neighbour's point on its face fn that meets this element's point k of face f.
-template <int K>
-__device__ __forceinline__ int face_point(int f, int fn, int k) {
-  return ((f + fn - f / 2 - fn / 2 + 1) & 1) ? K - 1 - k : k;
-}
 
 // As u on the lane's row (without the weights -w_k w_i).  u: rows; uc: columns.
 template <int K, int GEO, class R>
@@ -505,7 +423,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     check_block(A);
     return;
   }
-  constexpr int K2 = K * K, EPW = Lay<K>::EPW, ES = Lay<K>::ES;
+  constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES;
   constexpr int FS = GEO == GEO_ORTHO ? 0 : 4 * K;  // face values of one element
   __shared__ R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
   const int blk = xcd_block(blockIdx.x, nblk);
@@ -555,8 +473,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   }
   // The four neighbours' lines through the lane's face points, from the shared face inward: all
   // loads unconditional (a boundary face reads the element's own line and ignores it), so that
-  // their latencies overlap.  Where every neighbour of the wavefront across a face meets it with
-  // its opposite face (meshes numbered and oriented alike), the line's stride is a constant.
+  // their latencies overlap.
   Face<R> F[4];
   const int nbs[4] = {nbr.x, nbr.y, nbr.z, nbr.w};
   R l[4][K], pl[IN == IN_PUPD ? 4 : 1][K], cn[IN == IN_PROL ? 4 : 1][4];
@@ -567,45 +484,16 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
     const bool in = nbs[f] >= 0;
     const int nb = in ? nbs[f] : el, fn = in ? (nbf >> (8 * f)) & 3 : f ^ 1;
     F[f].nb = nbs[f];
-    if (__all(fn == (f ^ 1))) {
-      const size_t o = (size_t)nb * K2;
-      auto line = [&](const auto* g, R (&v)[K]) {
-        if (f < 2) {
-          R w[K];
-          load_row<K>(g + o + k * K, w);
-#pragma unroll
-          for (int m = 0; m < K; ++m) v[m] = f == 0 ? w[K - 1 - m] : w[m];
-        } else {
-#pragma unroll
-          for (int m = 0; m < K; ++m) v[m] = (R)g[o + k + (f == 2 ? (K - 1 - m) * K : m * K)];
-        }
-      };
-      if constexpr (IN == IN_PUPD) {
-        line(static_cast<const RZ*>(A.z), l[f]);
-        if (!first_dir) line(A.x, pl[f]);
-      } else {
-        line(A.x, l[f]);
-      }
-      F[f].fn = f ^ 1;
-      F[f].kk = k;
+    const bool opp = __all(fn == (f ^ 1));
+    const int kk = opp ? k : face_point<K>(f, fn, k);
+    if constexpr (IN == IN_PUPD) {
+      nbr_line<K>(static_cast<const RZ*>(A.z), nb, f, fn, kk, k, opp, l[f]);
+      if (!first_dir) nbr_line<K>(A.x, nb, f, fn, kk, k, opp, pl[f]);
     } else {
-      const int kk = face_point<K>(f, fn, k), up = fn & 1;
-      const int start = fn < 2 ? kk * K + (up ? K - 1 : 0) : (up ? (K - 1) * K : 0) + kk;
-      const int step = fn < 2 ? (up ? -1 : 1) : (up ? -K : K);
-      const size_t o = (size_t)nb * K2 + start;
-      if constexpr (IN == IN_PUPD) {
-#pragma unroll
-        for (int m = 0; m < K; ++m) l[f][m] = (R)(static_cast<const RZ*>(A.z) + o)[m * step];
-        if (!first_dir)
-#pragma unroll
-          for (int m = 0; m < K; ++m) pl[f][m] = (A.x + o)[m * step];
-      } else {
-#pragma unroll
-        for (int m = 0; m < K; ++m) l[f][m] = (A.x + o)[m * step];
-      }
-      F[f].fn = fn;
-      F[f].kk = kk;
+      nbr_line<K>(A.x, nb, f, fn, kk, k, opp, l[f]);
     }
+    F[f].fn = opp ? (f ^ 1) : fn;
+    F[f].kk = kk;
     if constexpr (IN == IN_PROL) {
       // vertex values at the corners of the shared face (along its parameter) and of the opposite one
       const int4 vn = *reinterpret_cast<const int4*>(G.ev + (size_t)nb * 4);

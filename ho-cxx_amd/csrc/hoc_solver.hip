@@ -97,8 +97,9 @@ struct Solver {
   DBuf<double> b_psi0, b_psi_r, b_diff0, b_diff_r, b_nvel0, b_nvel_r, b_pvel0, b_pvel_r;
   BCDev B{};
   // fields
-  DBuf<double> w, psi, vel, U, k1, k2, k3, k4, vort, kscratch, bs;
-  DBuf<double> trw, tru;
+  DBuf<double> w, psi, vel, U, k1, k2, k3, k4, vort, vort2, kscratch, bs;
+  DBuf<double> tru;      // normal traces of U
+  DBuf<double> d_dcol, d_wrow;
   // Poisson solver: FP64 state (the Krylov method, the initial residual, probing) and FP32
   // state (the mixed-precision V-cycle); S/F = scalars and flags of the Krylov solve.
   Prec<double> P64;
@@ -121,7 +122,6 @@ struct Solver {
   double lam_max = 0.;
   int geo_kind = GEO_POINT;          // what the fine-level kernels are instantiated for
   DBuf<uint16_t> d_ftype;            // kinds of each element's line ends
-  DBuf<double> d_traces;             // face traces of psi for the velocity kernel
   int krylov = HOC_KRYLOV_BICGSTAB;
   // live kernel timing (hoc_profile_*)
   struct Prof {
@@ -258,14 +258,21 @@ struct Solver {
           affine = std::fabs(fa[q0 + k] - fa[q0]) <= 1e-12 * fs && std::fabs(fb[q0 + k] - fb[q0]) <= 1e-12 * fs;
       }
     }
+    {
+      std::vector<double> dc((size_t)K2), wr(tab.wgt, tab.wgt + K);
+      for (int k = 0; k < K; ++k)
+        for (int d = 0; d < K; ++d) dc[(size_t)k * K + d] = tab.D[d][k];
+      d_dcol.upload(dc); d_wrow.upload(wr);
+    }
     if (affine) { d_gel.upload(gel); d_gface.upload(gface); d_gjm.upload(gjm); }
     G = Geo{N, E, d_jac, d_xxi, d_xeta, d_yxi, d_yeta, d_Ga, d_Gb, d_Gc, d_fa, d_fb, d_fA, d_fB, d_fjac, d_fAn,
             affine ? d_gel.p : nullptr, affine ? d_gface.p : nullptr, affine ? d_gjm.p : nullptr,
-            d_nb, d_nbf, d_swpsi, d_swdiff, d_noslip, d_esign, nullptr};
+            d_nb, d_nbf, d_swpsi, d_swdiff, d_noslip, d_esign, nullptr, d_dcol, d_wrow, nullptr};
     setup_instances();
     setup_hybrid();
     P64.prof_off = 0;
     setup_fine(P64, affine, Ga, Gb, Gc, fa, fb, gel, gface);
+    G.qn = P64.qn;
     const size_t EK = std::max<size_t>((size_t)E * K, 1);
     for (auto* b : {&b_psi, &b_diff, &b_nvel, &b_pvel, &b_vj, &b_vort, &b_adv}) b->alloc(EK);
     auto upl = [&](DBuf<double>& d, const std::vector<double>& h) { if (h.empty()) d.alloc(1); else d.upload(h); };
@@ -273,18 +280,17 @@ struct Solver {
     upl(b_nvel0, bch.nvel); upl(b_nvel_r, bch.nvel_ramp); upl(b_pvel0, bch.pvel); upl(b_pvel_r, bch.pvel_ramp);
     B = BCDev{b_psi, b_diff, b_nvel, b_pvel, b_vj, b_vort, b_adv, b_psi0, b_psi_r, b_diff0, b_diff_r, b_nvel0, b_nvel_r, b_pvel0, b_pvel_r};
     // fields
-    for (auto* f : {&w, &psi, &k1, &k2, &k3, &k4, &vort, &kscratch, &bs}) f->alloc(D);
+    for (auto* f : {&w, &psi, &k1, &k2, &k3, &k4, &vort, &vort2, &kscratch, &bs}) f->alloc(D);
     vel.alloc(2 * D); U.alloc(2 * D);
-    trw.alloc((size_t)N * 8 * K); tru.alloc((size_t)N * 4 * K);
+    tru.alloc((size_t)N * 4 * K);
     mixed = cfg.precision == HOC_MIXED;
-    d_traces.alloc((size_t)N * 8 * K);
     P64.alloc_vectors(D, N, true);
     if (mixed) {  // FP32 tables and metrics of the V-cycle's fine operator
       P32.prof_off = HOC_PROF_VARIANTS / 2;
       setup_fine(P32, affine, Ga, Gb, Gc, fa, fb, gel, gface);
       P32.alloc_vectors(D, N, false);
     }
-    nparts = std::max(std::max(lap_blocks(N), fine_blocks(K, N)), vec_grid(D));
+    nparts = std::max(fine_blocks(K, N), vec_grid(D));
     part.alloc(2 * (size_t)nparts);
     part2.alloc(2 * (size_t)nparts);
     S.alloc(S_COUNT); F.alloc(F_COUNT);
@@ -408,7 +414,7 @@ struct Solver {
     if (geo_kind != GEO_ORTHO) {
       qn.assign((size_t)std::max(E, 1) * K2, 0.);
       for (int e = 0; e < E; ++e) {
-        if (!bch.sw_psi[e]) continue;
+        if (!bch.sw_psi[e] && !bch.sw_diff[e]) continue;
         const int f = mesh.be_ijp[e];
         const size_t q = ((size_t)mesh.be_elem[e] * 4 + f) * K;
         const double gp = tab.gprime[f & 1];
@@ -1099,21 +1105,21 @@ struct Solver {
 
   // FP64 residual r = bs - As psi with the reference's unscaled norm, and the solve's
   // convergence state in (S, F).
-  // pbb (may be null): lap_blocks(N) partials of ||b||^2 for S[S_BB].
+  // pbb (may be null): fine_blocks(K, N) partials of ||b||^2 for S[S_BB].
   void outer_residual(const double* pbb) {
     const int lb = fine_blocks(K, N);
     residual_As(psi.p, bs.p, P64.r.p, part.p);
     if (ens_pcg()) {
       seg_norm2(stream, pseg, VA, P64.r.p, nullptr, ens_part.p, ens_rr.p);
       finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, ens_rr.p, ens_bb.p, pseg.nseg, pbb,
-               lap_blocks(N));
+               fine_blocks(K, N));
       if (ens_batched()) {
         EnsKry E = ensk();
         E.in = ens_rr.p;
         finalize_ens(stream, ENS_INIT, E, S, F, cfg.maxiter);
       }
     } else {
-      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, nullptr, nullptr, 0, pbb, lap_blocks(N));
+      finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, nullptr, nullptr, 0, pbb, fine_blocks(K, N));
     }
   }
 
@@ -1465,7 +1471,7 @@ struct Solver {
   void poisson(const double* omega) {
     guess_before_solve();
     const int maxit = cfg.maxiter;
-    HIPCHK(launch_rhs(K, N, T, G, omega, rhs_bc ? rhs_bc : b_psi.p, bs, part2, stream));
+    HIPCHK(launch_rhs(K, geo_kind, N, T, G, omega, rhs_bc ? rhs_bc : b_psi.p, bs, part2, stream));
     const bool proj = proj_on() && (!std::isnan(stage_tau) || proj_force);
     if (proj) proj_before(bs);
     bool have_bb = false;
@@ -1474,7 +1480,7 @@ struct Solver {
       ensure_segments();
       seg_norm2(stream, pseg, VA, bs, nullptr, ens_part.p, ens_bb.p);
     } else if (n_inst > 1) {
-      finalize(stream, PH_BB, part2, lap_blocks(N), S, F, maxit);
+      finalize(stream, PH_BB, part2, fine_blocks(K, N), S, F, maxit);
       have_bb = true;
       // BiCGSTAB: ||b - A psi|| <= tol min_i ||b_i|| bounds every instance's own relative residual
       // (instances with a zero right-hand side are left out of the minimum)
@@ -1555,8 +1561,7 @@ struct Solver {
   void refresh_fields() {
     update_bcs(0.);
     poisson(w);
-    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, w, vel, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
+    HIPCHK(launch_velocity(K, geo_kind, N, T, G, B, psi, vel, U, tru, 1. / (cfg.dt * re_inv), I, stream));
   }
   // Node-averaged vorticity, psi and velocity into d_nodeout (save_smooth_vtk,
   // src/HO_2D.cpp:3369-3531).
@@ -1646,12 +1651,11 @@ struct Solver {
   void stage_body(const double* win, const StageOut& so) {
     poisson(win);
     if (capture_psi && rk_stage >= 0) dcopy(capture_psi + (size_t)rk_stage * D, psi, D);
-    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
     // the Cartesian velocity is an output of the step's last stage only (what the getters and
     // writers read); intermediate RK stages need the contravariant fluxes U alone
-    double* v_out = (so.next && !so.final_mode) ? nullptr : vel.p;
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, win, v_out, U, trw, tru, 1. / (cfg.dt * re_inv), I, stream));
-    HIPCHK(launch_stage(K, cfg.advection_type, N, T, G, B, win, U, trw, tru, re_inv, cfg.dt, I, so, stream));
+    HIPCHK(launch_velocity(K, geo_kind, N, T, G, B, psi, so.inner ? nullptr : vel.p, U, tru, 1. / (cfg.dt * re_inv), I,
+                           stream));
+    HIPCHK(launch_stage(K, geo_kind, cfg.advection_type, N, T, G, B, win, U, tru, re_inv, cfg.dt, I, so, stream));
   }
   void stage(const double* win, double c, const StageOut& so) {
     update_bcs(c);
@@ -1673,11 +1677,13 @@ struct Solver {
   // solve_advection_diffusion (src/HO_2D.cpp:1465-1531)
   void rk_step() {
     StageOut so;
+    // a stage's input is none of its outputs: the inputs alternate between vort and vort2
     if (cfg.time_integration_type == 1) {
-      so.base = w; so.final_mode = 1;
+      so.next = vort; so.c = 1.; so.base = w;
       stage(w, 0., so);
+      dcopy(w, vort, D);
     } else if (cfg.time_integration_type == 2) {
-      so.k = k1; so.next = vort; so.c = 1.; so.base = w;
+      so.k = k1; so.next = vort; so.c = 1.; so.base = w; so.inner = true;
       stage(w, 0., so);
       StageOut s2; s2.base = w; s2.final_mode = 2; s2.k1 = k1;
       stage(vort, 1., s2);
@@ -1685,11 +1691,11 @@ struct Solver {
       const double c[4] = {0., 0.5, 0.5, 1.};
       double* ks[3] = {k1, k2, k3};
       rk_stage = 0;
-      stage_rk4(w, c[0], ks[0], 0.5);
+      stage_rk4(w, c[0], ks[0], 0.5, vort);
       rk_stage = 1;
-      stage_rk4(vort, c[1], ks[1], 0.5);
+      stage_rk4(vort, c[1], ks[1], 0.5, vort2);
       rk_stage = 2;
-      stage_rk4(vort, c[2], ks[2], 1.0);
+      stage_rk4(vort2, c[2], ks[2], 1.0, vort);
       StageOut s4; s4.base = w; s4.final_mode = 4; s4.k1 = k1; s4.k2 = k2; s4.k3 = k3;
       rk_stage = 3;
       stage(vort, c[3], s4);
@@ -1701,8 +1707,8 @@ struct Solver {
     ++step_count;
     for (int i = 0; i < n_inst && n_inst > 1; ++i) inst_time[i] += inst_dt[i];
   }
-  void stage_rk4(const double* win, double c, double* kout, double cnext) {
-    StageOut so; so.k = kout; so.next = vort; so.c = cnext; so.base = w;
+  void stage_rk4(const double* win, double c, double* kout, double cnext, double* next) {
+    StageOut so; so.k = kout; so.next = next; so.c = cnext; so.base = w; so.inner = true;
     stage(win, c, so);
   }
 
@@ -1783,7 +1789,7 @@ struct Solver {
   // ---- discrete adjoint of the RK4 trajectory -------------------------------------------
   // One stage maps omega_s to k_s = dt R(omega_s), with psi_s = A^-1 b(omega_s) and
   // b = -omega J - (boundary source).  Its transpose is applied as
-  //   omega_bar  = (dk/domega)^T lam                 (probes: omega and its face traces, 1-ring)
+  //   omega_bar  = (dk/domega)^T lam                 (probes: omega, 1-ring)
   //   U_bar      = (dk/dU)^T lam,  diff_bar = (dk/ddiff)^T lam   (probes: velocity, wall flux)
   //   pvel_bar  += sign idr diff_bar                 (no-slip walls: diff = (vjump + sign pvel) idr)
   //   psi_bar    = (dU/dpsi)^T U_bar + (ddiff/dpsi)^T diff_bar   (assembled once: the map is linear
@@ -1797,11 +1803,11 @@ struct Solver {
     int ub = 1;                       // probe units (hoc_adj.hpp) of a batch
     bool seeds_kept = false;          // every unit fits one batch: its seeds are written once, by the setup
     DBuf<int8_t> own_f;
-    DBuf<double> ws[4], Us[4], trws[4], trus[4];  // recorded stages of one step
+    DBuf<double> ws[4], Us[4], trus[4];  // recorded stages of one step
     DBuf<int8_t> sig[4];
-    // probe batches (ub K^2 probes, at least 4K): seeds and their traces, products, velocities
-    DBuf<double> seed, seed_tr, y, p, dU, dvel, dtrw, dtru, lin_diff, lin_vj, pvel_seed;
-    DBuf<double> zero_d, zero_tr, zero_e, lin_nvel, lin_vort, lin_adv;
+    // probe batches (ub K^2 probes, at least 4K): seeds, products, velocities and their traces
+    DBuf<double> seed, y, p, dU, dtru, lin_diff, lin_vj, pvel_seed;
+    DBuf<double> zero_d, zero_e, lin_nvel, lin_vort, lin_adv;
     DBuf<double> lam, xbar, psibar, z, fake, wbar, kbar[4], pvbar;
     DBuf<double> Mv, Md, Ubar, diffbar, zero_u, zero_tu;  // assembled velocity map and its adjoints
     // adjoint solves: the previous solution z (in z) and the one before (zprev) with their stage
@@ -1906,25 +1912,24 @@ struct Solver {
     std::vector<int8_t> of(std::max(E, 1), -1);
     for (int e = 0; e < E; ++e) { oe[e] = mesh.be_elem[e]; of[e] = mesh.be_ijp[e]; }
     adj.own_el.upload(oe); adj.own_f.upload(of);
-    const size_t TR = (size_t)4 * N * 2 * K, TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
+    const size_t TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
     // Units per batch: as many as 256 MiB hold (one, whatever it takes, on meshes whose single units
     // fill the chip): batches of all 14 take 24 x 24 elements, K = 4, from 95 launches a stage to 14.
-    const double unit = 8. * K2 * (4. * (double)D + (double)TR + (double)TU);
+    const double unit = 8. * K2 * (4. * (double)D + (double)TU);
     adj.ub = (int)std::min(std::max(268435456. / unit, 1.), 2. * adj.nc1);
     adj.seeds_kept = adj.ub == 2 * adj.nc1;
     const size_t NB1 = std::max(K2, 4 * K), NB = std::max<size_t>((size_t)adj.ub * K2, NB1);
     const size_t NBw = std::max<size_t>((size_t)std::min(adj.ub, adj.nc1) * K2, NB1);  // vorticity units alone
     for (int s4 = 0; s4 < 4; ++s4) {
-      adj.ws[s4].alloc(D); adj.Us[s4].alloc(2 * D); adj.trws[s4].alloc(TR); adj.trus[s4].alloc(TU);
+      adj.ws[s4].alloc(D); adj.Us[s4].alloc(2 * D); adj.trus[s4].alloc(TU);
       adj.sig[s4].alloc((size_t)4 * N * K); adj.kbar[s4].alloc(D);
     }
     for (DBuf<double>* b : {&adj.zero_d, &adj.lam, &adj.xbar, &adj.psibar, &adj.z, &adj.fake, &adj.wbar, &adj.save_w,
                             &adj.save_psi})
       b->alloc(D);
     adj.save_vel.alloc(2 * D);
-    adj.zero_tr.alloc(TR);
-    adj.seed.alloc(NBw * D); adj.y.alloc(NB * D); adj.seed_tr.alloc(NBw * TR); adj.dtrw.alloc(NB1 * TR);
-    adj.dU.alloc(NB * 2 * D); adj.dvel.alloc(NB1 * 2 * D); adj.dtru.alloc(NB * TU);
+    adj.seed.alloc(NBw * D); adj.y.alloc(NB * D);
+    adj.dU.alloc(NB * 2 * D); adj.dtru.alloc(NB * TU);
     adj.p.alloc(NB * std::max(N, 1));
     adj.lin_diff.alloc(NB1 * EK); adj.lin_vj.alloc(NB1 * EK); adj.pvel_seed.alloc((size_t)4 * K * EK);
     // seeds of the wall-flux probes are edge arrays like the wall velocity's
@@ -1946,16 +1951,16 @@ struct Solver {
     // the velocity map psi -> (U, wall flux): K^2 probes per colour of the distance-2 colouring
     // (U of an element depends on psi of its face ring), velocity with homogeneous boundary values
     VelBatch vb;
-    vb.psi = D; vb.trpsi = TR; vb.vel = 2 * D; vb.U = 2 * D; vb.trw = TR; vb.tru = TU; vb.vjump = EK; vb.diff = EK;
+    vb.psi = D; vb.U = 2 * D; vb.tru = TU; vb.vjump = EK; vb.diff = EK;
     for (int c = 0; c < adj.nc1; ++c) {
-      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, c, 1, T, adj.seed, adj.seed_tr, stream));
-      HIPCHK(launch_velocity_batch(K, N, T, G, adj.Bl, adj.seed, adj.seed_tr, adj.zero_d, adj.dvel, adj.dU, adj.dtrw,
-                                   adj.dtru, 1. / (cfg.dt * re_inv), I, K2, vb, stream));
+      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, c, 1, adj.seed, stream));
+      HIPCHK(launch_velocity(K, geo_kind, N, T, G, adj.Bl, adj.seed, nullptr, adj.dU, adj.dtru,
+                             1. / (cfg.dt * re_inv), I, stream, K2, vb));
       HIPCHK(launch_adj_assemble_vel(N, E, K, adj.col1, c, d_nb, adj.own_el, adj.dU, adj.lin_diff, adj.Mv, adj.Md,
                                      stream));
     }
     if (adj.seeds_kept) {
-      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, 0, adj.nc1, T, adj.seed, adj.seed_tr, stream));
+      HIPCHK(launch_adj_seed_batch(N, K, adj.col1, 0, adj.nc1, adj.seed, stream));
       HIPCHK(launch_adj_seed_u_batch(N, K, adj.col1, 0, 2 * adj.nc1, T, adj.dU, adj.dtru, stream));
     }
     if (E > 0) HIPCHK(launch_adj_edge_seed_batch(E, K, adj.own_f, adj.pvel_seed, stream));
@@ -1967,7 +1972,7 @@ struct Solver {
     HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
   }
 
-  // One RK4 step from w = omega_n recording every stage's input, velocity, traces and upwind
+  // One RK4 step from w = omega_n recording every stage's input, velocity and upwind
   // switches (w itself is not advanced).  stage_psi: the stage solutions of the same step kept by
   // the segment's recompute (their inputs are recomputed here by the same kernels), or null to
   // solve.
@@ -1979,15 +1984,14 @@ struct Solver {
       update_bcs(c[st]);
       if (stage_psi) dcopy(psi, stage_psi + (size_t)st * D, D);
       else poisson(adj.ws[st]);
-      HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
-      HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, adj.ws[st], vel, adj.Us[st], adj.trws[st], adj.trus[st],
-                             1. / (cfg.dt * re_inv), I, stream));
+      HIPCHK(launch_velocity(K, geo_kind, N, T, G, B, psi, vel, adj.Us[st], adj.trus[st], 1. / (cfg.dt * re_inv), I,
+                             stream));
       StageOut so;
       so.k = kscratch;
       so.sig = adj.sig[st];
       if (st < 3) { so.next = adj.ws[st + 1]; so.c = cn[st]; so.base = w; }
-      HIPCHK(launch_stage(K, 1, N, T, G, B, adj.ws[st], adj.Us[st], adj.trws[st], adj.trus[st], re_inv, cfg.dt, I, so,
-                          stream, 1));
+      HIPCHK(launch_stage(K, geo_kind, 1, N, T, G, B, adj.ws[st], adj.Us[st], adj.trus[st], re_inv, cfg.dt, I, so, stream,
+                          1));
     }
   }
 
@@ -1995,36 +1999,32 @@ struct Solver {
   // The probes of many colours (and the 4K wall-velocity probes) run as one batched launch each.
   void adj_stage(int st, const double* lam, double* xbar, double tau = std::nan("")) {
     const double idr = 1. / (cfg.dt * re_inv);
-    const size_t TR = (size_t)4 * N * 2 * K, TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
+    const size_t TU = (size_t)4 * N * K, EK = std::max<size_t>((size_t)E * K, 1);
     StageOut so;
     so.k = adj.y;
     so.bs_k = D;
     so.sig = adj.sig[st];
-    // (1) omega and its face traces, with psi (so U and the wall flux) fixed
-    so.omega_adv = adj.seed; so.bs_wa = D;
-    so.trw_adv = adj.seed_tr; so.bs_trwa = TR;
-    so.bs_w = D; so.bs_trw = TR;
+    // (1) omega, with psi (so U and the wall flux) fixed
+    so.bs_w = D;
     for (int u0 = 0; u0 < adj.nc1; u0 += adj.ub) {
       const int nu = std::min(adj.ub, adj.nc1 - u0);
       so.nbatch = nu * K2;
-      if (!adj.seeds_kept) HIPCHK(launch_adj_seed_batch(N, K, adj.col1, u0, nu, T, adj.seed, adj.seed_tr, stream));
-      HIPCHK(launch_stage(K, 1, N, T, G, adj.Bz, adj.seed, adj.Us[st], adj.seed_tr, adj.trus[st], re_inv, cfg.dt, I,
-                          so, stream, 2));
+      if (!adj.seeds_kept) HIPCHK(launch_adj_seed_batch(N, K, adj.col1, u0, nu, adj.seed, stream));
+      HIPCHK(launch_stage(K, geo_kind, 1, N, T, G, adj.Bz, adj.seed, adj.Us[st], adj.trus[st], re_inv, cfg.dt, I, so,
+                          stream, 2));
       HIPCHK(launch_adj_dot_batch(N, K2, so.nbatch, lam, adj.y, adj.p, stream));
       HIPCHK(launch_adj_gather_batch(N, K2, 1, u0, nu, adj.col1, adj.r1p, adj.r1i, adj.p, xbar, stream));
     }
     // (2) velocity: a unit per colour and component (the stage depends on U over the face ring),
     //     the stage advecting the recorded vorticity with the seeded velocity
-    so.omega_adv = adj.ws[st]; so.bs_wa = 0;
-    so.trw_adv = adj.trws[st]; so.bs_trwa = 0;
-    so.bs_w = 0; so.bs_trw = 0; so.bs_U = 2 * D; so.bs_tru = TU; so.bs_diff = 0;
+    so.bs_w = 0; so.bs_U = 2 * D; so.bs_tru = TU; so.bs_diff = 0;
     so.adv_only = 1;  // zero vorticity and wall flux for the diffusion term
     for (int u0 = 0; u0 < 2 * adj.nc1; u0 += adj.ub) {
       const int nu = std::min(adj.ub, 2 * adj.nc1 - u0);
       so.nbatch = nu * K2;
       if (!adj.seeds_kept) HIPCHK(launch_adj_seed_u_batch(N, K, adj.col1, u0, nu, T, adj.dU, adj.dtru, stream));
-      HIPCHK(launch_stage(K, 1, N, T, G, adj.Bz, adj.zero_d, adj.dU, adj.zero_tr, adj.dtru, re_inv, cfg.dt, I, so,
-                          stream, 2));
+      HIPCHK(launch_stage(K, geo_kind, 1, N, T, G, adj.Bz, adj.ws[st], adj.dU, adj.dtru, re_inv, cfg.dt, I, so, stream,
+                          2));
       HIPCHK(launch_adj_dot_batch(N, K2, so.nbatch, lam, adj.y, adj.p, stream));
       HIPCHK(launch_adj_gather_batch(N, K2, 2, u0, nu, adj.col1, adj.r1p, adj.r1i, adj.p, adj.Ubar, stream));
     }
@@ -2032,12 +2032,11 @@ struct Solver {
     //     reaches only the owner elements; then the wall velocity's share of it
     HIPCHK(hipMemsetAsync(adj.diffbar.p, 0, EK * sizeof(double), stream));
     if (E > 0) {
-      so.omega_adv = adj.zero_d; so.trw_adv = adj.zero_tr;
       so.bs_U = 0; so.bs_tru = 0; so.bs_diff = EK;
       so.adv_only = 0;
       so.nbatch = 4 * K;
-      HIPCHK(launch_stage(K, 1, N, T, G, adj.Bl_seed(), adj.zero_d, adj.zero_u, adj.zero_tr, adj.zero_tu, re_inv,
-                          cfg.dt, I, so, stream, 2));
+      HIPCHK(launch_stage(K, geo_kind, 1, N, T, G, adj.Bl_seed(), adj.zero_d, adj.zero_u, adj.zero_tu, re_inv, cfg.dt, I,
+                          so, stream, 2));
       HIPCHK(launch_adj_dot_batch(N, K2, 4 * K, lam, adj.y, adj.p, stream));
       HIPCHK(launch_adj_edge_gather_batch(N, E, K, adj.own_el, adj.own_f, adj.p, adj.diffbar, stream));
       HIPCHK(launch_adj_wall(E, K, d_noslip, d_esign, idr, adj.diffbar, adj.pvbar, stream));
@@ -2310,14 +2309,11 @@ struct Solver {
     h2d(adj.lam.p, lam_h, D * sizeof(double));
     update_bcs(0., t);
     poisson(adj.ws[0]);
-    HIPCHK(launch_trace(K, N, T, psi, d_traces.p, stream));
-    HIPCHK(launch_velocity(K, N, T, G, B, psi, d_traces, adj.ws[0], vel, adj.Us[0], adj.trws[0], adj.trus[0],
-                           1. / (cfg.dt * re_inv), I, stream));
+    HIPCHK(launch_velocity(K, geo_kind, N, T, G, B, psi, vel, adj.Us[0], adj.trus[0], 1. / (cfg.dt * re_inv), I, stream));
     StageOut so;
     so.k = kscratch;
     so.sig = adj.sig[0];
-    HIPCHK(launch_stage(K, 1, N, T, G, B, adj.ws[0], adj.Us[0], adj.trws[0], adj.trus[0], re_inv, cfg.dt, I, so,
-                        stream, 1));
+    HIPCHK(launch_stage(K, geo_kind, 1, N, T, G, B, adj.ws[0], adj.Us[0], adj.trus[0], re_inv, cfg.dt, I, so, stream, 1));
     HIPCHK(hipMemsetAsync(adj.pvbar.p, 0, EK * sizeof(double), stream));
     adj_stage(0, adj.lam, adj.xbar);
     d2h(out_h, adj.xbar.p, D * sizeof(double));
