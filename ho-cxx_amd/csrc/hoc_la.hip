@@ -174,16 +174,7 @@ __device__ void finalize_phase(int phase, double a, double b, double* __restrict
   }
   switch (phase) {
     case PH_BB: S[S_BB] = a; break;
-    case PH_INIT: {
-      S[S_RR] = S[S_RRL] = S[S_PRED] = b;
-      const double tiny = 2. * 2.220446049250313e-16;
-      const bool zero = S[S_BB] < tiny * tiny;
-      F[F_ZERO] = zero;
-      F[F_ITER] = 0;
-      F[F_HALF] = 0;
-      F[F_ACTIVE] = (!zero && above && maxiter > 0) ? 1 : 0;
-      S[S_RZ] = 0.; S[S_RHO] = S[S_RHON] = a; S[S_ALPHA] = 1.; S[S_OMEGA] = 1.; S[S_BETA] = 0.;
-    } break;
+    case PH_INIT: init_phase(a, b, above, S, F, maxiter); break;
     case PH_RZ: {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
       if (!(a > 0.) || !isfinite(a)) { F[F_ACTIVE] = 0; break; }
       S[S_BETA] = F[F_ITER] > 0 ? a / S[S_RZ] : 0.;
@@ -643,9 +634,10 @@ void proj_seg_layout(const std::vector<int64_t>& sbeg, std::vector<int32_t>& bbe
   const int nseg = (int)sbeg.size() - 1;
   bbeg.assign(nseg + 1, 0);
   blk_seg.clear();
-  for (int s = 0; s < nseg; ++s) {  // about 8 dofs per thread, at least one block per segment
+  const int64_t per = 256 * std::min<int64_t>(std::max<int64_t>((sbeg[nseg] - sbeg[0]) / (256 * 256), 1), 8);
+  for (int s = 0; s < nseg; ++s) {  // at least one block per segment
     const int64_t n = sbeg[s + 1] - sbeg[s];
-    const int nb = (int)std::max<int64_t>(1, (n + 2047) / 2048);
+    const int nb = (int)std::max<int64_t>(1, (n + per - 1) / per);
     bbeg[s + 1] = bbeg[s] + nb;
     for (int k = 0; k < nb; ++k) blk_seg.push_back(s);
   }
@@ -664,21 +656,35 @@ void proj_dispatch_impl(int m, Fn& fn) {
 template <int LO, class Fn>
 void proj_dispatch(int m, Fn fn) { proj_dispatch_impl<kProjMax, LO>(m, fn); }
 
+// Sums over a wavefront of N values a lane: at every step a lane gives half of its values to the lane
+// whose bit differs and adds the other's to the half it keeps, so that it ends with a few complete sums
+// (N = 72: 73 exchanges; a tree per value takes 432).  The lane's first n values are those from idx on of
+// the N, the rest is padding of halves of odd length.
+template <int OFF, int N>
+__device__ __forceinline__ void scatter_sums(double (&v)[N], int idx, int n, double* __restrict__ red) {
+  if constexpr (OFF == 0) {
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+      if (q < n) red[idx + q] = v[q];
+  } else {
+    constexpr int H = (N + 1) / 2;
+    const bool up = (threadIdx.x & OFF) != 0;
+    double h[H];
+#pragma unroll
+    for (int q = 0; q < H; ++q) {
+      const double a = v[q], b = H + q < N ? v[H + q] : 0.;
+      h[q] = (up ? b : a) + __shfl_xor(up ? a : b, OFF, 64);
+    }
+    scatter_sums<OFF / 2, H>(h, idx + (up ? H : 0), up ? n - H : min(n, H), red);
+  }
+}
 // Sum over the block (256 threads) of NV per-thread values; thread k < NV writes sum k to out[k].
 template <int NV>
 __device__ __forceinline__ void block_sums(double (&v)[NV], double* __restrict__ out) {
   __shared__ double red[4][NV];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const double w = wsum(v[k]);
-    if (lane == 0) red[wv][k] = w;
-  }
+  scatter_sums<32, NV>(v, 0, NV, red[threadIdx.x >> 6]);
   __syncthreads();
-  if (threadIdx.x < NV) {
-    const int k = threadIdx.x;
-    out[k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
-  }
+  for (int k = threadIdx.x; k < NV; k += 256) out[k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
 }
 // part[block][0, M) = Y_j . t,  part[block][M, 2M) = Y_j . b over the block's segment
 template <int M>
@@ -781,7 +787,8 @@ __global__ __launch_bounds__(256) void k_proj_append(size_t n, ProjSeg S, int m,
                                                      const double* __restrict__ e, int estride,
                                                      const double* __restrict__ psi, const double* __restrict__ b,
                                                      double* __restrict__ x, double* __restrict__ part,
-                                                     double* __restrict__ wcol, int wstride, int ldw) {
+                                                     double* __restrict__ wcol, int wstride, int ldw,
+                                                     double* __restrict__ save) {
   const SegRange R = seg_range(S);
   double s[1] = {0.};
   if (R.lb == 0 && (int)threadIdx.x < ldw) {
@@ -791,6 +798,7 @@ __global__ __launch_bounds__(256) void k_proj_append(size_t n, ProjSeg S, int m,
   for (size_t i = R.i0; i < R.i1; i += R.step) {
     const double p = psi[i], bv = b[i];
     x[i] = p + x[i];
+    if (save) save[i] = p;
     s[0] += (mr ? bv : p) * bv;
   }
   block_sums<1>(s, part + blockIdx.x);
@@ -872,52 +880,118 @@ __global__ __launch_bounds__(256) void k_proj_reseed(size_t n, ProjSeg S, int kk
     }
   }
 }
-// The small system of a basis of m vectors, one per segment (grid: nseg; G + s gstride,
-// v + s vstride): column j of G (at G + j ldg) holds G_ij (i < j), G_jj, and in row j + 1 the
-// squared norm of the solution the vector came from.  A vector with G_jj <= 1e-24 of that norm
-// (left in the span of the others), or whose Cholesky pivot falls below 1e-8 G_jj, is left out.
-// v[0, m) and v[m, 2m) become G^-1 v on the kept vectors and 0 on the others: Cholesky by one
-// wavefront, lane i holding row i of L in registers (m <= kProjMax <= 64); each column of L is
-// broadcast by lane reads (scalar registers; shuffles through the LDS unit took 25 us at m = 24), and
-// L goes to LDS once for the back substitution, which reads it by columns.
 __device__ __forceinline__ double lane_bcast(double v, int lane) {  // lane: a compile-time constant
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
   return __hiloint2double(hi, lo);
 }
-__global__ __launch_bounds__(64) void k_proj_solve(int m, const double* __restrict__ Gall, int ldg, int gstride,
-                                                   double* __restrict__ vall, int vstride) {
-  constexpr int MX = kProjMax;
+// v <- G^-1 v for the two right-hand sides in v, by the Cholesky factor of G in one wavefront (lane i:
+// row i).  Rows before `done` were factored by an earlier call and are read from L ([row][kProjMax + 2]:
+// the row, 1 / L_ii, kept or not), since a basis grows by a vector at a time: a new row is one forward
+// substitution, 24 dependent steps, against the 300 of the whole factor (m = 24: 22 us a call).  A
+// vector within rounding of the span of those before it (its pivot below 1e-8 of its norm, itself below
+// 1e-24 of the solution's) is left out: zero coefficients.
+// With part set (np values per block, k_proj_dots3; few blocks), the block first sums what is there:
+// [0, 2m) right-hand sides, [2m, 3m) the newest Gram column, and part0, the newest solution's norm.
+__global__ void k_proj_solve(ProjSeg S, int m, int done, double* __restrict__ Gall, int ldg, int gstride,
+                             double* __restrict__ Lall, double* __restrict__ vall, int vstride,
+                             const double* __restrict__ part, const double* __restrict__ part0) {
+  constexpr int MX = kProjMax, LD = MX + 2;
   static_assert(MX <= 64, "one lane per row");
-  const double* G = Gall + (size_t)blockIdx.x * gstride;
-  double* v = vall + (size_t)blockIdx.x * vstride;
+  const int sg = blockIdx.x;
+  double* G = Gall + (size_t)sg * gstride;
+  double* L = Lall + (size_t)sg * kProjL;
+  double* v = vall + (size_t)sg * vstride;
   __shared__ double Ls[MX][MX + 1];
-  const int i = threadIdx.x;
+  __shared__ double acc[1024], sums[3 * MX + 1];
+  const int t = threadIdx.x;
+  if (part) {
+    const int np = 3 * m, ng = blockDim.x / np, k = t % np, g = t / np, b0 = S.bbeg[sg], b1 = S.bbeg[sg + 1];
+    double s = 0.;
+    if (g < ng)
+#pragma unroll 8
+      for (int b = b0 + g; b < b1; b += ng) s += part[(size_t)b * np + k];
+    acc[t] = s;
+    if (t >= (int)blockDim.x - 64) {
+      double q = 0.;
+      for (int b = b0 + (t & 63); b < b1; b += 64) q += part0[b];
+      q = wsum(q);
+      if ((t & 63) == 0) sums[np] = q;
+    }
+    __syncthreads();
+    if (t < np) {
+      double q = 0.;
+      for (int i = 0; i < ng; ++i) q += acc[i * np + t];
+      sums[t] = q;
+      if (t >= 2 * m) G[(size_t)(m - 1) * ldg + t - 2 * m] = q;
+    }
+    if (t == 0) G[(size_t)(m - 1) * ldg + m] = sums[np];
+    __syncthreads();
+  }
+  if (t >= 64) return;
+  const int i = t;
+  double a[MX], il = 0.;  // lane i: row i, and 1 / L_ii
+  int ok = 0;
+#pragma unroll
+  for (int k = 0; k < MX; ++k) a[k] = i < done ? L[i * LD + k] : 0.;
+  if (i < done) {
+    il = L[i * LD + MX];
+    ok = L[i * LD + MX + 1] != 0.;
+  }
   const bool row = i < m;
-  double a[MX];  // row i of the lower triangle: G_ik (k <= i), the upper half of column i
+  double y0 = 0., y1 = 0.;
+  if (row) {
+    y0 = part ? sums[i] : v[i];
+    y1 = part ? sums[m + i] : v[m + i];
+  }
+  // row r: lane k works on L_rk, lane r on the pivot; with the last row goes the sweep L y = v
+  for (int r = done; r < m; ++r) {
+    const bool last = r == m - 1;
+    const double* col = G + (size_t)r * ldg;
+    double x = i <= r ? (part && last ? sums[2 * m + i] : col[i]) : 0.;
+    const double n0 = part && last ? sums[3 * m] : col[r + 1], gd = __shfl(x, r, 64);
+    const bool okr = gd > 1e-24 * fabs(n0) && gd > 0.;
 #pragma unroll
-  for (int k = 0; k < MX; ++k) a[k] = (row && k <= i) ? G[(size_t)i * ldg + k] : 0.;
-  const double gd = row ? G[(size_t)i * ldg + i] : 0.;
-  int ok = row && gd > 1e-24 * fabs(G[(size_t)i * ldg + i + 1]) && gd > 0.;
-  double y0 = row ? v[i] : 0., y1 = row ? v[m + i] : 0.;
-  double il = 0.;  // lane j: 1 / L_jj
-#pragma unroll
-  for (int j = 0; j < MX; ++j) {  // right-looking: column j, then the trailing rows
-    if (j < m) {                  // uniform
-      const double d = lane_bcast(a[j], j);
-      const bool okj = __builtin_amdgcn_readlane(ok, j) && d > 1e-8 * lane_bcast(gd, j);  // the same on every lane
-      if (okj) {
-        const double ij = 1. / sqrt(d);
-        if (i == j) il = ij;
-        else if (i > j && ok) a[j] *= ij;
-#pragma unroll
-        for (int k = j + 1; k < MX; ++k) {
-          const double lkj = lane_bcast(a[j], k);
-          const int okk = __builtin_amdgcn_readlane(ok, k);
-          if (k < m && k <= i && i > j && ok && okk) a[k] -= a[j] * lkj;
-        }
-        // L y = v, column j
+    for (int j = 0; j < MX; ++j)
+      if (j < r && __builtin_amdgcn_readlane(ok, j)) {  // uniform
+        const double ij = lane_bcast(il, j), xj = lane_bcast(x, j) * ij;
         const double y0j = lane_bcast(y0, j) * ij, y1j = lane_bcast(y1, j) * ij;
+        if (i == j) {
+          x = xj;
+          if (last) {
+            y0 = y0j;
+            y1 = y1j;
+          }
+        } else if (i == r) {
+          a[j] = xj;
+          x -= xj * xj;
+        } else if (i > j && i < r && ok) {
+          x -= a[j] * xj;
+        }
+        if (last && i > j && (ok || i == r)) {
+          y0 -= a[j] * y0j;
+          y1 -= a[j] * y1j;
+        }
+      }
+    const double d = __shfl(x, r, 64);
+    const bool okd = okr && d > 1e-8 * gd;
+    if (i < r) L[r * LD + i] = x;
+    if (i == r) {
+      ok = okd;
+      il = okd ? 1. / sqrt(d) : 0.;
+      L[r * LD + MX] = il;
+      L[r * LD + MX + 1] = okd ? 1. : 0.;
+      if (last) {
+        y0 *= il;
+        y1 *= il;
+      }
+    }
+  }
+  if (done >= m) {
+#pragma unroll
+    for (int j = 0; j < MX; ++j)  // L y = v
+      if (j < m && __builtin_amdgcn_readlane(ok, j)) {
+        const double ij = lane_bcast(il, j), y0j = lane_bcast(y0, j) * ij, y1j = lane_bcast(y1, j) * ij;
         if (i == j) {
           y0 = y0j;
           y1 = y1j;
@@ -925,16 +999,15 @@ __global__ __launch_bounds__(64) void k_proj_solve(int m, const double* __restri
           y0 -= a[j] * y0j;
           y1 -= a[j] * y1j;
         }
-      } else if (i == j) {
-        ok = 0;
       }
-    }
   }
   if (row) {
 #pragma unroll
     for (int k = 0; k < MX; ++k) Ls[i][k] = a[k];
   }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int j = MX - 1; j >= 0; --j) {  // L^T x = y
     if (j < m && __builtin_amdgcn_readlane(ok, j)) {
@@ -1001,6 +1074,9 @@ void proj_dots2(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* 
   });
   hipLaunchKernelGGL(k_proj_fin, dim3(2 * m, S.nseg), dim3(256), 0, s, S, 2 * m, part, out, ostride, 2 * m, nullptr, 0);
 }
+// Up to this many blocks a segment, one block sums their partials faster than a launch does (256 blocks of
+// 72 values: 3 us).
+bool proj_inline(const ProjSeg& S) { return S.maxb <= 320; }
 void proj_dots3(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* ax, const double* t,
                 const double* b, double* part, double* out, int ostride, double* gcol, int gstride) {
   if (m <= 0 || m > kProjMax || n == 0) return;
@@ -1008,12 +1084,17 @@ void proj_dots3(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* 
     constexpr int M = decltype(Mc)::value;
     hipLaunchKernelGGL(k_proj_dots3<M>, dim3(S.nb), dim3(256), 0, s, n, S, Y, ax, t, b, part);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(3 * m, S.nseg), dim3(256), 0, s, S, 3 * m, part, out, ostride, 2 * m, gcol, gstride);
+  if (!proj_inline(S))
+    hipLaunchKernelGGL(k_proj_fin, dim3(3 * m, S.nseg), dim3(256), 0, s, S, 3 * m, part, out, ostride, 2 * m, gcol, gstride);
 }
-void proj_solve(hipStream_t s, const ProjSeg& S, int m, const double* G, int ldg, int gstride, double* v,
-                int vstride) {
+void proj_sum(hipStream_t s, const ProjSeg& S, const double* part, double* out, int ostride) {
+  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, out, ostride, 1, nullptr, 0);
+}
+void proj_solve(hipStream_t s, const ProjSeg& S, int m, int done, double* G, int ldg, int gstride, double* L, double* v,
+                int vstride, const double* part, const double* part0) {
   if (m <= 0 || m > kProjMax) return;
-  hipLaunchKernelGGL(k_proj_solve, dim3(S.nseg), dim3(64), 0, s, m, G, ldg, gstride, v, vstride);
+  hipLaunchKernelGGL(k_proj_solve, dim3(S.nseg), dim3(part ? 1024 : 64), 0, s, S, m, std::min(done, m), G, ldg, gstride,
+                     L, v, vstride, part, part0);
 }
 void proj_combine(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* X, const double* c, int cstride,
                   double* out, double* v) {
@@ -1024,23 +1105,21 @@ void proj_combine(hipStream_t s, size_t n, const ProjSeg& S, int m, const double
   });
 }
 void proj_append(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* e, int estride,
-                 const double* psi, const double* b, double* x, double* part, double* n0, int n0stride,
-                 double* wcol, int wstride, int ldw) {
+                 const double* psi, const double* b, double* x, double* part0, double* wcol, int wstride, int ldw,
+                 double* save) {
   if (m < 0 || m > kProjMax || n == 0 || ldw > 256) return;
-  hipLaunchKernelGGL(k_proj_append, dim3(S.nb), dim3(256), 0, s, n, S, m, mr, e, estride, psi, b, x, part, wcol,
-                     wstride, ldw);
-  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride, 1, nullptr, 0);
+  hipLaunchKernelGGL(k_proj_append, dim3(S.nb), dim3(256), 0, s, n, S, m, mr, e, estride, psi, b, x, part0, wcol,
+                     wstride, ldw, save);
 }
 void proj_ortho(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* X, const double* e,
-                int estride, const double* psi, const double* b, double* x, double* part, double* n0, int n0stride,
-                double* wcol, int wstride, int ldw) {
+                int estride, const double* psi, const double* b, double* x, double* part0, double* wcol, int wstride,
+                int ldw) {
   if (m < 0 || m > kProjMax || n == 0 || ldw > 256) return;
   proj_dispatch<0>(m, [&](auto Mc) {
     constexpr int M = decltype(Mc)::value;
-    hipLaunchKernelGGL(k_proj_ortho<M>, dim3(S.nb), dim3(256), 0, s, n, S, mr, X, e, estride, psi, b, x, part, wcol,
+    hipLaunchKernelGGL(k_proj_ortho<M>, dim3(S.nb), dim3(256), 0, s, n, S, mr, X, e, estride, psi, b, x, part0, wcol,
                        wstride, ldw);
   });
-  hipLaunchKernelGGL(k_proj_fin, dim3(1, S.nseg), dim3(256), 0, s, S, 1, part, n0, n0stride, 1, nullptr, 0);
 }
 void proj_gcol(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* Y, const double* x,
                const double* ax, double* part, double* gcol, int gstride) {
@@ -1068,19 +1147,22 @@ void proj_reseed(hipStream_t s, size_t n, const ProjSeg& S, int m, int kk, const
     hipLaunchKernelGGL(k_proj_reseed<M>, dim3(S.nb), dim3(256), 0, s, n, S, kk, C, cstride, X, AX);
   });
 }
-// The per-segment sum of one partial per block (k_proj_fin with nv = 1), leaving out[s] as it is
-// for a segment whose flag in iact (may be null) is 0.
-__global__ __launch_bounds__(256) void k_seg_fin(ProjSeg S, const double* __restrict__ part, double* __restrict__ out,
-                                                 const int* __restrict__ iact) {
-  const int sg = blockIdx.y;
+// out[s] = sum of part[beg[s], beg[s + 1]); left as it is for a segment whose flag in iact (may be null) is 0.
+__global__ __launch_bounds__(256) void k_seg_fin(const int32_t* __restrict__ beg, const double* __restrict__ part,
+                                                 double* __restrict__ out, const int* __restrict__ iact) {
+  const int sg = blockIdx.x;
   if (iact && !iact[sg]) return;
   double s = 0.;
-  for (int b = S.bbeg[sg] + threadIdx.x; b < S.bbeg[sg + 1]; b += 256) s += part[b];
+#pragma unroll 4
+  for (int b = beg[sg] + threadIdx.x; b < beg[sg + 1]; b += 256) s += part[b];
   s = wsum(s);
   __shared__ double red[4];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) out[sg] = red[0] + red[1] + red[2] + red[3];
+}
+void seg_sum(hipStream_t s, int nseg, const int32_t* beg, const double* part, double* out, const int* iact) {
+  hipLaunchKernelGGL(k_seg_fin, dim3(nseg), dim3(256), 0, s, beg, part, out, iact);
 }
 __global__ __launch_bounds__(256) void k_seg_norm2(ProjSeg S, VecArgs A, const double* __restrict__ r,
                                                    const int* __restrict__ F, double* __restrict__ part,
@@ -1099,40 +1181,30 @@ __global__ __launch_bounds__(256) void k_seg_norm2(ProjSeg S, VecArgs A, const d
 void seg_norm2(hipStream_t s, const ProjSeg& S, const VecArgs& A, const double* r, const int* F, double* part,
                double* out, const int* iact) {
   hipLaunchKernelGGL(k_seg_norm2, dim3(S.nb), dim3(256), 0, s, S, A, r, F, part, iact);
-  hipLaunchKernelGGL(k_seg_fin, dim3(1, S.nseg), dim3(256), 0, s, S, part, out, iact);
+  seg_sum(s, S.nseg, S.bbeg, part, out, iact);
 }
-template <class RB>
-__global__ __launch_bounds__(256) void k_seg_dot(ProjSeg S, const double* __restrict__ a, const RB* __restrict__ b,
-                                                 const int* __restrict__ F, double* __restrict__ part,
-                                                 const int* __restrict__ iact) {
-  if (F && !F[F_ACTIVE]) return;
-  const SegRange R = seg_range(S);
-  if (iact && !iact[R.s]) return;
-  double p[1] = {0.};
-  for (size_t v = R.i0; v < R.i1; v += R.step) p[0] += a[v] * (double)b[v];
-  block_sums<1>(p, part + blockIdx.x);
-}
-template <class RB>
-void seg_dot(hipStream_t s, const ProjSeg& S, const double* a, const RB* b, const int* F, double* part, double* out,
-             const int* iact) {
-  hipLaunchKernelGGL(k_seg_dot<RB>, dim3(S.nb), dim3(256), 0, s, S, a, b, F, part, iact);
-  hipLaunchKernelGGL(k_seg_fin, dim3(1, S.nseg), dim3(256), 0, s, S, part, out, iact);
-}
-template void seg_dot<double>(hipStream_t, const ProjSeg&, const double*, const double*, const int*, double*, double*,
-                              const int*);
-template void seg_dot<float>(hipStream_t, const ProjSeg&, const double*, const float*, const int*, double*, double*,
-                             const int*);
-
-// One block: thread t handles instances t, t + 256, ..; the block then reduces "any active", the
+// One block: thread t handles instances t, t + kEnsThreads, ..; the block then reduces "any active", the
 // largest residual ratio of the active instances and the sum of the residual norms.
-__global__ __launch_bounds__(256) void k_finalize_ens(int phase, EnsKry E, double* __restrict__ S,
+constexpr int kEnsThreads = 1024;
+__global__ __launch_bounds__(kEnsThreads) void k_finalize_ens(int phase, EnsKry E, double* __restrict__ S,
                                                       int* __restrict__ F, int maxiter,
                                                       MirrorState* __restrict__ mirror, int seq) {
   const bool live = phase == ENS_INIT || F[F_ACTIVE];
-  __shared__ int sany[256];
-  __shared__ double smax[256], ssum[256];
+  __shared__ int sany[kEnsThreads];
+  __shared__ double smax[kEnsThreads], ssum[kEnsThreads];
   int any = 0;
   double rmax = 0., rsum = 0.;
+  if (live && E.part) {  // a wavefront sums an instance's partials
+    for (int i = threadIdx.x >> 6; i < E.n; i += kEnsThreads / 64) {
+      if (!E.act[i]) continue;  // a stopped instance keeps its last value
+      double s = 0.;
+#pragma unroll 8
+      for (int b = E.beg[i] + (threadIdx.x & 63); b < E.beg[i + 1]; b += 64) s += E.part[b];
+      s = wsum(s);
+      if ((threadIdx.x & 63) == 0) E.in[i] = s;
+    }
+    __syncthreads();
+  }
   if (live) {
     const double tol2 = S[S_TOL2];
     double bmax = 0.;
@@ -1210,7 +1282,7 @@ __global__ __launch_bounds__(256) void k_finalize_ens(int phase, EnsKry E, doubl
 }
 void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter, MirrorState* mirror,
                   int seq) {
-  hipLaunchKernelGGL(k_finalize_ens, dim3(1), dim3(256), 0, s, phase, E, S, F, maxiter, mirror, seq);
+  hipLaunchKernelGGL(k_finalize_ens, dim3(1), dim3(kEnsThreads), 0, s, phase, E, S, F, maxiter, mirror, seq);
 }
 void psi_predict(hipStream_t s, size_t n, double f, int extrap, double* psi, double* prev) {
   if (n == 0) return;

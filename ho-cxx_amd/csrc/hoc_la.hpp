@@ -100,14 +100,16 @@ void psi_predict(hipStream_t s, size_t n, double f, int extrap, double* psi, dou
 //   proj_dots3:   proj_dots2 and, from the same pass over Y, gcol[j] = Y_j . ax (j < m; ax the
 //                 image of the newest vector Y_{m-1}: its Gram column, as proj_gcol gives it);
 //                 part: S.nb * 3m
-//   proj_solve:   v[0, m) and v[m, 2m) <- G^-1 v (G in columns of ldg values, see k_proj_solve)
+//   proj_solve:   v[0, m) and v[m, 2m) <- G^-1 v (G in columns of ldg values) by the Cholesky factor of
+//                 the rows before `done`, kept in L, extended to m rows (see k_proj_solve); with part
+//                 set, what proj_dots3 left there (and n0's partials in part0) is summed first
 //   proj_combine: out += sum_j c[j] X_j; with v set, also v = -sum_j c[m + j] X_j (the e of a
 //                 later append, from the same pass over X)
 //   proj_append:  proj_ortho's append when proj_combine has left v = -X e in x: x = psi + x,
-//                 with n0 and wcol as proj_ortho writes them
+//                 with n0's partials and wcol as proj_ortho writes them; save (may be null) receives psi
 //   proj_ortho:   appends a new solution psi: x = psi - sum_j e[j] X_j (e = G^-1 Y . b from
 //                 before the solve: Y . As psi = Y . b up to the solve's residual), psi's
-//                 squared norm (mr ? b . b : psi . b) into n0 (the scale of the in-span test),
+//                 squared norm (mr ? b . b : psi . b; the scale of the in-span test) as partials in part0,
 //                 and wcol[0, ldw): psi's coefficients in the basis with x appended; part: S.nb
 //   proj_gcol:    the Gram column of the appended x from its image ax = As x (applied by the
 //                 operator, not inferred from the solve's recursive residual): Y_j . ax (j < m)
@@ -117,27 +119,34 @@ void psi_predict(hipStream_t s, size_t n, double f, int extrap, double* psi, dou
 constexpr int kProjMax = 24;
 struct ProjSeg {
   int nseg = 0, nb = 0;              // segments; blocks of 256 threads over all of them
+  int maxb = 0;                      // most blocks of one segment
   const int32_t* blk_seg = nullptr;  // [nb] the segment of each block (device)
   const int32_t* bbeg = nullptr;     // [nseg + 1] first block of each segment (device)
   const int64_t* sbeg = nullptr;     // [nseg + 1] first dof of each segment (device)
 };
-// Host side of a ProjSeg: blocks per segment (about 8 dofs per thread, at least one) from the
-// segments' first dofs.
+// Host side of a ProjSeg: blocks per segment from the segments' first dofs: 8 dofs a thread where that
+// still makes 256 blocks, fewer on smaller problems (16384 dofs and 15 vectors in 8 blocks: proj_dots3
+// 18 us).
 void proj_seg_layout(const std::vector<int64_t>& sbeg, std::vector<int32_t>& bbeg, std::vector<int32_t>& blk_seg);
 void proj_dots2(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* t, const double* b,
                 double* part, double* out, int ostride);
+// With few enough blocks (proj_inline) the sums are left to proj_solve, and gcol and n0 are not used.
+bool proj_inline(const ProjSeg& S);
 void proj_dots3(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* ax, const double* t,
                 const double* b, double* part, double* out, int ostride, double* gcol, int gstride);
-void proj_solve(hipStream_t s, const ProjSeg& S, int m, const double* G, int ldg, int gstride, double* v,
-                int vstride);
+// out[sg ostride] = the sum of one partial per block of segment sg
+void proj_sum(hipStream_t s, const ProjSeg& S, const double* part, double* out, int ostride);
+constexpr int kProjL = kProjMax * (kProjMax + 2);  // values of a segment's factor
+void proj_solve(hipStream_t s, const ProjSeg& S, int m, int done, double* G, int ldg, int gstride, double* L, double* v,
+                int vstride, const double* part = nullptr, const double* part0 = nullptr);
 void proj_combine(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* X, const double* c, int cstride,
                   double* out, double* v = nullptr);
 void proj_append(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* e, int estride,
-                 const double* psi, const double* b, double* x, double* part, double* n0, int n0stride,
-                 double* wcol, int wstride, int ldw);
+                 const double* psi, const double* b, double* x, double* part0, double* wcol, int wstride, int ldw,
+                 double* save);
 void proj_ortho(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const double* X, const double* e,
-                int estride, const double* psi, const double* b, double* x, double* part, double* n0, int n0stride,
-                double* wcol, int wstride, int ldw);
+                int estride, const double* psi, const double* b, double* x, double* part0, double* wcol, int wstride,
+                int ldw);
 void proj_gram(hipStream_t s, size_t n, const ProjSeg& S, int m, const double* Y, const double* AX, double* part,
                double* out);
 void proj_reseed(hipStream_t s, size_t n, const ProjSeg& S, int m, int kk, const double* C, int cstride, double* X,
@@ -149,13 +158,16 @@ void proj_gcol(hipStream_t s, size_t n, const ProjSeg& S, int m, int mr, const d
 // kernels run while any instance is active, and an instance that has stopped takes alpha =
 // beta = 0, so its x and r stay as they are (its Poisson-operator blocks return at once).
 struct EnsKry {
-  double* in;        // the per-instance sums of the phase (r.z, p.q or the weighted ||r||^2)
+  double* in;        // the per-instance sums of the phase (r.z, p.q or the weighted ||r||^2): given, or formed
+                     // for the active instances i from part[beg[i], beg[i + 1]) when that is set
   double* rz;        // r.z of the last direction update
   double* alpha;     // step lengths
   double* beta;      // direction-update coefficients
   const double* bb;  // weighted ||b_i||^2
   int* act;          // per-instance active flags
   int n;
+  const double* part = nullptr;
+  const int32_t* beg = nullptr;
 };
 enum { ENS_INIT = 0, ENS_RZ, ENS_PQ, ENS_UPD };
 // ENS_INIT after the joint PH_INIT finalize (E.in = ||r_i||^2): each instance active when the
@@ -165,15 +177,10 @@ enum { ENS_INIT = 0, ENS_RZ, ENS_PQ, ENS_UPD };
 // finalize publishes it.  An instance with bb_i = 0 is held to the largest bb.
 void finalize_ens(hipStream_t s, int phase, const EnsKry& E, double* S, int* F, int maxiter,
                   MirrorState* mirror = nullptr, int seq = 0);
-// out[s] = sum over segment s of a . b (a FP64, b FP64 or FP32); skipped when F's active flag is
-// clear (F may be null), and out[s] left as it is for a segment whose flag in iact (may be null)
-// is 0.  part: S.nb values.
-template <class RB>
-void seg_dot(hipStream_t s, const ProjSeg& S, const double* a, const RB* b, const int* F, double* part, double* out,
-             const int* iact = nullptr);
-// out[s] = sum over segment s of (r winv)^2 (weighted squared norms per ensemble instance);
-// skipped when F (may be null) has its active flag clear, and out[s] left as it is for a segment
-// whose flag in iact (may be null) is 0.  part: S.nb values.
+// out[s] = sum of part[beg[s], beg[s + 1]); left as it is for a segment whose flag in iact (may be null) is 0.
+void seg_sum(hipStream_t s, int nseg, const int32_t* beg, const double* part, double* out, const int* iact);
+// out[s] = sum over segment s of (r winv)^2 (weighted squared norms per ensemble instance); skipped when F
+// (may be null) has its active flag clear, and as seg_sum for iact.  part: S.nb values.
 void seg_norm2(hipStream_t s, const ProjSeg& S, const VecArgs& A, const double* r, const int* F, double* part,
                double* out, const int* iact = nullptr);
 // The RK4 guess and stage-difference history at the first stage of a step, in one pass: psi (the

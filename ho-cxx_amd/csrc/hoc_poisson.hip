@@ -377,6 +377,22 @@ __device__ __forceinline__ double sum_parts(const double* __restrict__ part, int
   return sp[0] + sp[1] + sp[2] + sp[3];
 }
 
+// Sum of a per-lane value over the K lanes of each element, into part[el]; through the LDS that the
+// block has done with.
+template <int K>
+__device__ __forceinline__ void element_part(double a, double* lds, int wv, int le, int k, bool live,
+                                             double* __restrict__ part, int el) {
+  double* s = lds + (wv * Lay<K>::EPW + le) * K;
+  __syncthreads();
+  s[k] = a;
+  wave_fence();
+  if (k != 0 || !live) return;
+  double r = 0.;
+#pragma unroll
+  for (int i = 0; i < K; ++i) r += s[i];
+  part[el] = r;
+}
+
 // sums of the first and of the second halves of 2 np partials, for thread 0 of the block
 __device__ __forceinline__ void sum_pairs(const double* __restrict__ part, int np, double& a, double& b) {
   __shared__ double sa[kFineThreads / 64], sb[kFineThreads / 64];
@@ -399,21 +415,25 @@ __device__ __forceinline__ void sum_pairs(const double* __restrict__ part, int n
 // that it clears: what they write is not used then.
 template <class A>
 __device__ void check_block(const A& a) {
-  int* F = a.active;
-  const bool live = F[F_ACTIVE] != 0;  // uniform over the block
-  double u = 0., v = 0.;
-  if (live) sum_pairs(a.chk_part, a.chk_np, u, v);
-  if (threadIdx.x) return;
+  int* F = a.chk_F;
   double* S = a.scal;
-  if (live) check_phase(a.chk_phase, u, v, S, F, a.chk_maxit >= 0 ? a.chk_maxit : F[F_MAXIT]);
+  const bool init = a.chk_phase == PH_INIT;
+  const bool live = init || F[F_ACTIVE] != 0;  // uniform over the block
+  double u = 0., v = 0., bb = 0.;
+  if (live) sum_pairs(a.chk_part, a.chk_np, u, v);
+  if (a.chk_bb) bb = sum_parts(a.chk_bb, a.chk_nbb);
+  if (threadIdx.x) return;
+  const int maxit = a.chk_maxit >= 0 ? a.chk_maxit : F[F_MAXIT];
+  if (init) {
+    if (a.chk_bb) S[S_BB] = bb;
+    init_phase(u, v, v > S[S_TOL2] * S[S_BB], S, F, maxit);
+  } else if (live) {
+    check_phase(a.chk_phase, u, v, S, F, maxit);
+  }
   if (!a.chk_mirror) return;
   const int seq = a.chk_seq >= 0 ? a.chk_seq : ++F[F_SEQ];
   publish(a.chk_mirror, seq, F[F_ACTIVE] && likely_last(S), S, F);
 }
-
-// Makes a loaded value due here, so that its load is issued before the branch that follows (on the
-// flag of the solve, loaded at the same time) and not after it.
-__device__ __forceinline__ void due(int v) { asm volatile("" ::"v"(v)); }
 
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> G, FineArgs<R> A) {
@@ -425,7 +445,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   }
   constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES;
   constexpr int FS = GEO == GEO_ORTHO ? 0 : 4 * K;  // face values of one element
-  __shared__ R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
+  __shared__ __align__(16) R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
   const int blk = xcd_block(blockIdx.x, nblk);
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int EPB = EPW * (kFineThreads / 64);
@@ -436,10 +456,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   // lanes past the mesh follow its last element in a slot of their own, and the lanes past the last
   // slot its last row: the same reads, so the same values in LDS; neither writes to memory
   const int el = min(el0, G.N - 1);
-  const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
-  const int nbf = G.nbf[el];
   const bool go = !A.active || A.active[F_ACTIVE];
-  due(nbr.x); due(nbr.y); due(nbr.z); due(nbr.w); due(nbf);
   if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
   if (!go) return;
   if (G.iact) {  // a block inside one stopped ensemble instance
@@ -454,6 +471,8 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   (void)xk;
   (void)lamk;
 
+  const int4 nbr = *reinterpret_cast<const int4*>(G.nb + (size_t)el * 4);
+  const int nbf = G.nbf[el];
   // every global read of the kernel, issued before the arithmetic
   R u[K], z[K], b[K];
   (void)z;
@@ -618,13 +637,22 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
       block_inverse<K>(T, G, el, k, lamk, t, res);
       const R om = (R)A.omega;
 #pragma unroll
-      for (int i = 0; i < K; ++i) {
-        u[i] += om * res[i];
-        p0 += (double)b[i] * (double)u[i];
+      for (int i = 0; i < K; ++i) u[i] += om * res[i];
+      if (A.part || A.elpart) {
+        double bd[K];
+        if constexpr (sizeof(R) == 4) {
+          load_row<K>(A.b64 + row, bd);
+        } else {
+#pragma unroll
+          for (int i = 0; i < K; ++i) bd[i] = b[i];
+        }
+#pragma unroll
+        for (int i = 0; i < K; ++i) p0 += bd[i] * (double)u[i];
       }
       if (live) store_row<K>(A.y + row, u);
     }
   }
+  if (A.elpart) element_part<K>(p0, reinterpret_cast<double*>(lds), wv, le, k, live, A.elpart, el);
   if (A.part) {
     if (!live) p0 = p1 = 0.;
     block_part(p0, p1, A.part, blk, nblk);
@@ -633,10 +661,10 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
 
 template <int K, int UPD, class R>
 __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G, PreArgs<R> A) {
-  constexpr bool XR = UPD == PRE_XR, ZERO = UPD == PRE_NONE || UPD == PRE_BICG0;
-  if (!(ZERO && A.zero) && A.active && !A.active[F_ACTIVE]) return;
+  constexpr bool XR = UPD == PRE_XR;
+  if (A.active && !A.active[F_ACTIVE]) return;
   constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES, EPB = EPW * (kFineThreads / 64);
-  __shared__ R lds[(kFineThreads / 64) * Lay<K>::TILE];
+  __shared__ __align__(16) R lds[(kFineThreads / 64) * Lay<K>::TILE];
   const int blk = xcd_block(blockIdx.x, gridDim.x);
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (G.iact) {
@@ -650,13 +678,6 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
   const int el = min(el0, G.N - 1);
   R* t = lds + wv * Lay<K>::TILE + le * ES;
   const size_t row = ((size_t)el * K + k) * K;
-  if (ZERO && A.zero) {  // a zero right-hand side: x = 0, as the reference's solver returns
-    if (*A.zero && live) {
-      const double z[K] = {};
-      store_row<K>(A.x + row, z);
-    }
-    if (A.active && !A.active[F_ACTIVE]) return;
-  }
   double r[K];
   load_row<K>(A.r + row, r);
   double p0 = 0., p1 = 0.;
@@ -738,6 +759,7 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
 #pragma unroll
   for (int i = 0; i < K; ++i) v[i] *= om;
   if (live) store_row<K>(A.z + row, v);
+  if (XR && A.elpart) element_part<K>(p1, reinterpret_cast<double*>(lds), wv, le, k, live, A.elpart, el);
   if (XR && A.part) {
     if (!live) p0 = p1 = 0.;
     block_part(p0, p1, A.part, blk, gridDim.x);

@@ -90,10 +90,16 @@ struct FineArgs {
   const double* rz = nullptr;
   int np = 0;
   double* part = nullptr;    // [fine_blocks] sums, then [fine_blocks] second sums
+  double* elpart = nullptr;  // instead: the first sum's share of every element [N]
+  const double* b64 = nullptr;  // EPI_SMOOTH in FP32: b in FP64 for the sums of b.y
   int* active = nullptr;     // the Krylov flags F (may be null)
   int* ran = nullptr;        // set to 1 when the launch worked, 0 when active made it return at once
   // EPI_SMOOTH of IN_X: one block more, which tests np pairs of partial norms that an earlier kernel
-  // left (phase: check_phase) and publishes the state; the other blocks do not wait for it
+  // left (phase: check_phase, or PH_INIT) on the flags chk_F and publishes the state; the other blocks
+  // do not wait for it.  chk_bb: chk_nbb partials of ||b||^2 for scal[S_BB] (PH_INIT; may be null)
+  int* chk_F = nullptr;
+  const double* chk_bb = nullptr;
+  int chk_nbb = 0;
   const double* chk_part = nullptr;
   int chk_np = 0, chk_phase = 0, chk_maxit = 0, chk_seq = 0;
   MirrorState* chk_mirror = nullptr;  // null: tested, not published
@@ -134,8 +140,8 @@ struct PreArgs {
   int np = 0, num = 0, keep = 0;
   bool spd = true;
   double* part = nullptr;
+  double* elpart = nullptr;  // instead: every element's share of (r/W).(r/W) [N]
   int* active = nullptr;     // the Krylov flags F (may be null)
-  const int* zero = nullptr; // PRE_NONE, PRE_BICG0: x is set to zero where this flag is set
   double iw[6] = {0., 0., 0., 0., 0., 0.};  // 1 / w_k
   const double* iwl = nullptr;              // the same on the device, for the lane's own
 };

@@ -473,7 +473,8 @@ struct Solver {
                        double* scal, int scal_idx, const double* rz, double* partp,
                        int* active) {
     FineArgs<double> A;
-    A.x = p; A.z = z; A.pn = pn; A.y = q; A.scal = scal; A.scal_idx = scal_idx; A.part = partp; A.active = active;
+    A.x = p; A.z = z; A.pn = pn; A.y = q; A.scal = scal; A.scal_idx = scal_idx; A.active = active;
+    (P.iact ? A.elpart : A.part) = partp;
     A.rz = rz; A.np = rz ? fine_blocks(K, N) : 0;
     if (!z32) { fine(P, IN_PUPD, EPI_STORE, A); return; }
     const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
@@ -739,31 +740,38 @@ struct Solver {
     int np, phase, maxit, seq;
     MirrorState* mirror;
     double* S;
+    int* F;
+    const double* bb;  // PH_INIT: partials of ||b||^2 (fine_blocks), or null
   };
   enum { WHOLE = 0, HEAD, REST };
   // The rest of the V-cycle for the residual rr after its first smoothing step has left the first
   // iterate in P.t: the iterate ping-pongs between P.t and zout and ends in zout; if partp != nullptr,
-  // partials of rr.zout are left there.  HEAD: the second smoothing step only; REST: what follows it.
+  // partials of r64.zout (r64: the residual in FP64) are left there, per element while an ensemble's masks
+  // are set.  HEAD: the second smoothing step only; REST: what follows it.
   template <class R>
-  void vcycle_rest(Prec<R>& P, const R* rr, R* zout, double* partp, int* Fp, int part_of = WHOLE,
+  void vcycle_rest(Prec<R>& P, const R* rr, const double* r64, R* zout, double* partp, int* Fp, int part_of = WHOLE,
                    const Check* chk = nullptr) {
     R *cur = P.t.p, *nxt = zout;
     FineArgs<R> A;
     A.b = rr;
     A.active = Fp;
+    if constexpr (std::is_same<R, float>::value) A.b64 = r64;
     auto smooth = [&](int in, double omega, double* pp) {
-      A.x = cur; A.y = nxt; A.omega = omega; A.part = pp;
+      A.x = cur; A.y = nxt; A.omega = omega; (P.iact ? A.elpart : A.part) = pp;
       fine(P, in, EPI_SMOOTH, A);
       std::swap(cur, nxt);
     };
     for (int k = 1; k < cheb_m; ++k) {
       if (k == 1 && chk) {
         A.chk_part = chk->part; A.chk_np = chk->np; A.chk_phase = chk->phase; A.chk_maxit = chk->maxit;
-        A.chk_seq = chk->seq; A.chk_mirror = chk->mirror; A.scal = chk->S;
+        A.chk_seq = chk->seq; A.chk_mirror = chk->mirror; A.scal = chk->S; A.chk_F = chk->F;
+        A.chk_bb = chk->bb; A.chk_nbb = chk->bb ? fine_blocks(K, N) : 0;
+        if (chk->phase == PH_INIT) A.active = nullptr;  // the flags are of an earlier solve
       }
       if (k > 1 || part_of != REST) smooth(IN_X, cheb_w[k], nullptr);
       else std::swap(cur, nxt);
       A.chk_part = nullptr;
+      A.active = Fp;
       if (part_of == HEAD) return;
     }
     // restrict the residual to the corner vertices
@@ -785,10 +793,10 @@ struct Solver {
   // its precision, for a mixed-precision handle with a promotion of z at the end.
   void precond_rest(const double* rin, double* zout, int* Fp, int part_of, const Check* chk) {
     if (mixed) {
-      vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, nullptr, Fp, part_of, chk);
+      vcycle_rest(P32, (const float*)P32.r.p, rin, P32.z.p, nullptr, Fp, part_of, chk);
       if (part_of != HEAD) promote_dot(stream, D, P32.z.p, zout, rin, nullptr, Fp);
     } else {
-      vcycle_rest(P64, rin, zout, nullptr, Fp, part_of, chk);
+      vcycle_rest(P64, rin, rin, zout, nullptr, Fp, part_of, chk);
     }
   }
 
@@ -876,17 +884,18 @@ struct Solver {
     if (mixed) go(P32);
     else go(P64);
   }
-  // Before the first iteration: its V-cycle (an iteration ends with the next one's).  The first
+  // Before the first iteration, from the residual r with its norms' partials in part: its V-cycle (an
+  // iteration ends with the next one's), and the start of the solve's state where that is not a launch of
+  // its own (outer_residual).  The first
   // direction needs no clearing, beta = 0 leaves the old one out.
-  void krylov_begin(double* x, double* r, double* Sp, int* Fp, int maxit) {
-    if (krylov == HOC_KRYLOV_PCG) {
-      krylov_pre(r, [&](auto& A) { A.x = x; A.zero = Fp + F_ZERO; A.active = Fp; });
-    } else {
-      krylov_pre(r, [&](auto& A) {
-        A.up = PRE_BICG0; A.x = x; A.zero = Fp + F_ZERO; A.pw = P64.p; A.rh = P64.rh; A.active = Fp;
-      });
-    }
-    krylov_vcycle(r, Sp, Fp, maxit, WHOLE, nullptr);
+  // pbb: partials of ||b||^2 for S[S_BB] (null: it is set).
+  void krylov_begin(double* r, const double* pbb, double* Sp, int* Fp, int maxit) {
+    krylov_pre(r, [&](auto& A) {
+      if (krylov != HOC_KRYLOV_PCG) { A.up = PRE_BICG0; A.pw = P64.p; A.rh = P64.rh; }
+      A.active = inline_check() ? nullptr : Fp;
+    });
+    const Check init{part.p, fine_blocks(K, N), PH_INIT, maxit, 0, nullptr, Sp, Fp, pbb};
+    krylov_vcycle(r, Sp, Fp, maxit, WHOLE, inline_check() ? &init : nullptr);
   }
   // The V-cycle of the next iteration, or a part of it, after its first smoothing step.
   void krylov_vcycle(double* r, double* Sp, int* Fp, int maxit, int part_of, const Check* chk) {
@@ -897,11 +906,8 @@ struct Solver {
     }
     if (ens_batched()) {
       EnsMask mask(*this);
-      vcycle_pcg(r, nullptr, Fp, part_of, chk);
-      if (part_of == HEAD) return;
-      if (mixed) seg_dot<float>(stream, pseg, r, P32.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-      else seg_dot<double>(stream, pseg, r, P.z.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-      finalize_ens(stream, ENS_RZ, ensk(), Sp, Fp, maxit);
+      vcycle_pcg(r, ens_part.p, Fp, part_of, chk);
+      ens_finalize(ENS_RZ, Sp, Fp, maxit);
       return;
     }
     // r.z from the V-cycle's last sweep; in mixed precision the direction update reads z in FP32
@@ -909,8 +915,8 @@ struct Solver {
     if (part_of != HEAD && !inline_sums()) finalize(stream, PH_RZ, part, fine_blocks(K, N), Sp, Fp, maxit);
   }
   void vcycle_pcg(double* r, double* partp, int* Fp, int part_of, const Check* chk) {
-    if (mixed) vcycle_rest(P32, (const float*)P32.r.p, P32.z.p, partp, Fp, part_of, chk);
-    else vcycle_rest(P64, r, P64.z.p, partp, Fp, part_of, chk);
+    if (mixed) vcycle_rest(P32, (const float*)P32.r.p, r, P32.z.p, partp, Fp, part_of, chk);
+    else vcycle_rest(P64, r, r, P64.z.p, partp, Fp, part_of, chk);
   }
   // One iteration up to its test and the publication of its status (seq >= 0: as seq; seq < 0: as the
   // next number of F[F_SEQ]); with inline_check() that takes the second smoothing step of the next
@@ -926,7 +932,7 @@ struct Solver {
       ens_iter(x, r, pold, pnew, Sp, Fp, maxit, seq);
       return;
     }
-    Check chk{part.p, fb, PH_UPD, maxit, seq, mirror_dev, Sp};
+    Check chk{part.p, fb, PH_UPD, maxit, seq, mirror_dev, Sp, Fp, nullptr};
     if (krylov == HOC_KRYLOV_PCG) {
       direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, Sp, S_BETA,
                       inl ? part.p : nullptr, part2.p, Fp);
@@ -954,7 +960,7 @@ struct Solver {
         B.spd = false;
         if (inl) { B.pq = part2; B.np = fb; B.num = S_RHON; B.keep = S_RHO; }
       });
-      const Check half{part.p, fb, PH_BHALF, maxit, 0, nullptr, Sp};
+      const Check half{part.p, fb, PH_BHALF, maxit, 0, nullptr, Sp, Fp, nullptr};
       if (!ichk) finalize(stream, PH_BHALF, part, fb, Sp, Fp, maxit);
       precond_rest(r, P.sh.p, Fp, WHOLE, ichk ? &half : nullptr);
       A.x = P.sh.p; A.y = P.q.p; A.b = r; A.part = part2;
@@ -983,6 +989,19 @@ struct Solver {
     explicit EnsMask(Solver& so) : s(so) { s.P64.iact = s.P32.iact = s.ens_act.p; }
     ~EnsMask() { s.P64.iact = s.P32.iact = nullptr; }
   };
+  // A phase of the batched ensemble PCG from the elements' sums in ens_part.  Up to kEnsInline elements the
+  // phase's own block sums them, past that one block per instance does first (35152 elements, a pass of 12
+  // solves: 18.4 ms without that launch, 17.7 with it).
+  static constexpr int kEnsInline = 16384;
+  void ens_finalize(int phase, double* Sp, int* Fp, int maxit, MirrorState* mir = nullptr, int seq = 0) {
+    EnsKry E = ensk();
+    if (phase == ENS_UPD) E.in = ens_rr.p;
+    if (N > kEnsInline) {
+      seg_sum(stream, pseg.nseg, d_ioff, ens_part, E.in, ens_act);
+      E.part = nullptr;
+    }
+    finalize_ens(stream, phase, E, Sp, Fp, maxit, mir, seq);
+  }
   // One iteration of the batched ensemble PCG (ens_batched): PCG with a step length and a
   // direction coefficient per instance (r_i.z_i, p_i.q_i and ||r_i|| by segment), each instance
   // stopping on its own test; while an instance is stopped, the fine-level kernels skip the
@@ -991,19 +1010,15 @@ struct Solver {
   void ens_iter(double* x, double* r, const double* pold, double* pnew, double* Sp, int* Fp, int maxit, int seq) {
     EnsMask mask(*this);
     Prec<double>& P = P64;
-    const EnsKry E = ensk();
-    direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr, nullptr,
-                    Fp);
-    seg_dot<double>(stream, pseg, pnew, P.q.p, Fp, ens_part.p, ens_in.p, ens_act.p);
-    finalize_ens(stream, ENS_PQ, E, Sp, Fp, maxit);
+    direction_apply(P, mixed ? (const void*)P32.z.p : P.z.p, mixed, pold, pnew, P.q.p, ens_beta.p, -1, nullptr,
+                    ens_part.p, Fp);
+    ens_finalize(ENS_PQ, Sp, Fp, maxit);
     krylov_pre(r, [&](auto& A) {
       A.up = PRE_XR; A.x = x; A.p = pnew; A.q = P.q; A.scal = ens_alpha; A.scal_idx = -1; A.active = Fp;
+      A.elpart = ens_part;
     });
     // ||r_i||^2 into ens_rr, where a stopped instance keeps its last value (its r no longer changes)
-    seg_norm2(stream, pseg, VA, r, Fp, ens_part.p, ens_rr.p, ens_act.p);
-    EnsKry Eu = E;
-    Eu.in = ens_rr.p;
-    finalize_ens(stream, ENS_UPD, Eu, Sp, Fp, maxit, mirror_dev, seq);
+    ens_finalize(ENS_UPD, Sp, Fp, maxit, mirror_dev, seq);
   }
   // The instantiated graph of a piece of an iteration on these buffers (captured on first use).
   hipGraphExec_t krylov_graph(double* x, double* r, double* Sp, int* Fp, int maxit, int piece) {
@@ -1029,10 +1044,10 @@ struct Solver {
     kgraphs.push_back(kg);
     return kg.e;
   }
-  void krylov_solve(double* x, double* r, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
+  void krylov_solve(double* x, double* r, const double* pbb, double* Sp, int* Fp, int maxit_host, int maxit_dev) {
     const int maxit = maxit_dev;
     const int seq0 = seq_next;
-    krylov_begin(x, r, Sp, Fp, maxit);
+    krylov_begin(r, pbb, Sp, Fp, maxit);
     const bool graphs = use_graphs && !prof.on;
     hipGraphExec_t ge[3] = {nullptr, nullptr, nullptr};
     if (graphs) {
@@ -1074,7 +1089,7 @@ struct Solver {
     auto run = [&](bool graph) {
       HIPCHK(hipMemsetAsync(psi.p, 0, D * sizeof(double), stream));
       outer_residual(nullptr);
-      krylov_begin(psi.p, P64.r.p, S.p, F.p, maxit);
+      krylov_begin(P64.r.p, nullptr, S.p, F.p, maxit);
       hipGraphExec_t ge[3] = {nullptr, nullptr, nullptr};
       for (int k = 0; k < 3 && graph; ++k) ge[k] = krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit, k);
       HIPCHK(hipStreamSynchronize(stream));
@@ -1116,9 +1131,10 @@ struct Solver {
       if (ens_batched()) {
         EnsKry E = ensk();
         E.in = ens_rr.p;
+        E.part = nullptr;
         finalize_ens(stream, ENS_INIT, E, S, F, cfg.maxiter);
       }
-    } else {
+    } else if (!inline_check()) {
       finalize(stream, PH_INIT, part, lb, S, F, cfg.maxiter, nullptr, 0, nullptr, nullptr, 0, pbb, fine_blocks(K, N));
     }
   }
@@ -1209,10 +1225,15 @@ struct Solver {
       psi_combine(stream, D, 2, a, x, psi, nullptr);
     }
   }
-  void rk_guess_after() {
+  // Whether the stage solution in psi continues the history, and where its copy goes (null: nowhere).
+  bool rk_continues() const { return !(rk_stage != rk_cur % 4 || (rk_stage > 0 && rk_cur != rk_stage)); }
+  double* rk_copy() {
+    return guess_mode() >= 3 && rk_stage >= 1 && !std::isnan(stage_tau) && rk_continues() ? rkS[rk_stage].p : nullptr;
+  }
+  void rk_guess_after(bool copied) {
     const int st = rk_stage;
-    if (st != rk_cur % 4 || (st > 0 && rk_cur != st)) { rk_full = false; rk_qok = false; rk_cur = 0; return; }
-    if (st >= 1) dcopy(rkS[st], psi, D);
+    if (!rk_continues()) { rk_full = false; rk_qok = false; rk_cur = 0; return; }
+    if (st >= 1 && !copied) dcopy(rkS[st], psi, D);
     rk_cur = st + 1;
     if (st == 3) { rk_full = true; rk_cur = 0; }
   }
@@ -1248,10 +1269,14 @@ struct Solver {
     // per segment: Gram columns (M x kProjLdg), solution coefficients (M x M), restart combination
     // or measured Gram matrix (M x M)
     DBuf<double> G, W, C;
+    DBuf<double> L;  // per segment: the Gram matrix's Cholesky factor (k_proj_solve)
+    int fact = 0;    // its rows
     int m = 0;       // vectors held
     int e_m = -1;    // basis size the coefficients e of the solve in progress were formed for
     int v_slot = -1; // the slot holding -X e for the append after the solve in progress (or -1)
-    int gcol_pending = -1;  // the newest slot, whose Gram column the next projected solve forms
+    // the newest slot, whose Gram column and solution norm (partials in pnorm) the next projected solve forms
+    int gcol_pending = -1;
+    DBuf<double> pnorm;
     int nseg = 0;    // segments the per-segment arrays were sized for
     int restarts = 0;
   };
@@ -1278,7 +1303,7 @@ struct Solver {
   DBuf<double> ens_in, ens_rz, ens_alpha, ens_beta;
   DBuf<int> ens_act;
   EnsKry ensk() {
-    return EnsKry{ens_in.p, ens_rz.p, ens_alpha.p, ens_beta.p, ens_bb.p, ens_act.p, pseg.nseg};
+    return EnsKry{ens_in.p, ens_rz.p, ens_alpha.p, ens_beta.p, ens_bb.p, ens_act.p, pseg.nseg, ens_part.p, d_ioff.p};
   }
   void ensure_segments() {
     std::vector<int64_t> sb;
@@ -1292,10 +1317,12 @@ struct Solver {
     pseg_sbeg.upload(sb); pseg_bbeg.upload(bbeg); pseg_blk.upload(blk);
     pseg.nseg = (int)sb.size() - 1;
     pseg.nb = (int)blk.size();
+    pseg.maxb = 0;
+    for (int i = 0; i < pseg.nseg; ++i) pseg.maxb = std::max(pseg.maxb, bbeg[i + 1] - bbeg[i]);
     pseg.blk_seg = pseg_blk.p; pseg.bbeg = pseg_bbeg.p; pseg.sbeg = pseg_sbeg.p;
     pseg_key = sb;
     ptmp.alloc(0);
-    ens_part.alloc(pseg.nb); ens_rr.alloc(pseg.nseg); ens_bb.alloc(pseg.nseg);
+    ens_part.alloc(std::max(N, pseg.nb)); ens_rr.alloc(pseg.nseg); ens_bb.alloc(pseg.nseg);
     for (auto* b : {&ens_in, &ens_rz, &ens_alpha, &ens_beta}) b->alloc(pseg.nseg);
     ens_act.alloc(pseg.nseg);
     HIPCHK(hipMemsetAsync(ens_alpha.p, 0, pseg.nseg * sizeof(double), stream));
@@ -1309,6 +1336,12 @@ struct Solver {
       ppart.alloc((size_t)pseg.nb * std::max(2 * kProjMax + 2, kProjVectors * kProjVectors));
     }
   }
+  // c, e: the coefficients of the first m vectors; sums: proj_dots3's are still to be formed
+  void proj_coefs(ProjBasis& P, int m, bool sums) {
+    proj_solve(stream, pseg, m, P.fact, P.G.p, kProjLdg, kProjVectors * kProjLdg, P.L, pcoef, kProjCoef,
+               sums ? ppart.p : nullptr, sums ? P.pnorm.p : nullptr);
+    P.fact = m;
+  }
   void proj_before(const double* b) {
     ProjBasis& P = *proj_cur;
     P.e_m = -1;
@@ -1321,13 +1354,17 @@ struct Solver {
     const double* Y = proj_mr() ? P.AX.p : P.X.p;
     if (P.gcol_pending >= 0 && P.gcol_pending == P.m - 1) {  // Y^T t, Y^T b and the newest Gram column
       const int j = P.m - 1;
-      proj_dots3(stream, D, pseg, P.m, Y, P.AX.p + (size_t)j * D, t, b, ppart, pcoef, kProjCoef,
-                 P.G.p + (size_t)j * kProjLdg, kProjVectors * kProjLdg);
+      double* gcol = P.G.p + (size_t)j * kProjLdg;
+      proj_dots3(stream, D, pseg, P.m, Y, P.AX.p + (size_t)j * D, t, b, ppart, pcoef, kProjCoef, gcol,
+                 kProjVectors * kProjLdg);
+      const bool inl = proj_inline(pseg);  // the solve sums what the dots left
+      if (!inl) proj_sum(stream, pseg, P.pnorm, gcol + P.m, kProjVectors * kProjLdg);
+      proj_coefs(P, P.m, inl);
     } else {
       proj_dots2(stream, D, pseg, P.m, Y, t, b, ppart, pcoef, kProjCoef);  // Y^T t, Y^T b
+      proj_coefs(P, P.m, false);
     }
     P.gcol_pending = -1;
-    proj_solve(stream, pseg, P.m, P.G.p, kProjLdg, kProjVectors * kProjLdg, pcoef, kProjCoef);    // c, e
     // with a free slot, the same pass leaves -X e there for the append after this solve
     const bool pre = P.m < kProjVectors;
     proj_combine(stream, D, pseg, P.m, P.X.p, pcoef, kProjCoef, psi, pre ? P.X.p + (size_t)P.m * D : nullptr);
@@ -1347,6 +1384,7 @@ struct Solver {
     P.e_m = -1;
     P.v_slot = -1;
     P.gcol_pending = -1;
+    P.fact = 0;
     ++P.restarts;
     if (KP == 0) return;
     std::vector<double> w((size_t)ns * M * M), gc((size_t)ns * M * LG), gm((size_t)M * M);
@@ -1384,34 +1422,40 @@ struct Solver {
     HIPCHK(hipStreamSynchronize(stream));  // (gi is a local)
     P.m = kk;
   }
-  void proj_after(const double* b) {
+  // save (may be null): where a copy of psi is wanted; true when the append's pass has made it.
+  bool proj_after(const double* b, double* save) {
     constexpr int M = kProjVectors;
+    bool saved = false;
     ProjBasis& P = *proj_cur;
     proj_alloc();
     if (P.X.n < (size_t)M * D || P.nseg != pseg.nseg) {
       P.X.alloc((size_t)M * D); P.AX.alloc((size_t)M * D);
       const size_t ns = pseg.nseg;
       P.G.alloc(ns * M * kProjLdg); P.W.alloc(ns * M * M); P.C.alloc(ns * M * M);
+      P.L.alloc(ns * kProjL);
       P.nseg = pseg.nseg;
       P.m = 0;
     }
+    if (P.pnorm.n < (size_t)pseg.nb) P.pnorm.alloc(pseg.nb);
     proj_flush_gcol(P);
     if (P.m >= M) proj_restart(P);
     const int j = P.m;
+    P.fact = std::min(P.fact, j);
     if (j > 0 && P.e_m != j) {  // e = G^-1 Y^T b
       proj_dots2(stream, D, pseg, j, proj_mr() ? P.AX.p : P.X.p, b, b, ppart, pcoef, kProjCoef);
-      proj_solve(stream, pseg, j, P.G.p, kProjLdg, M * kProjLdg, pcoef, kProjCoef);
+      proj_coefs(P, j, false);
     }
     // x = psi - X e into slot j, its exact image As x, and its Gram column
     double* xj = P.X.p + (size_t)j * D;
     double* axj = P.AX.p + (size_t)j * D;
-    double* gcol = P.G.p + (size_t)j * kProjLdg;
-    if (P.v_slot == j && P.e_m == j)  // slot j holds -X e from proj_before's pass
-      proj_append(stream, D, pseg, j, proj_mr() ? 1 : 0, pcoef.p + j, kProjCoef, psi, b, xj, ppart, gcol + j + 1,
-                  M * kProjLdg, P.W.p + (size_t)j * M, M * M, M);
-    else
-      proj_ortho(stream, D, pseg, j, proj_mr() ? 1 : 0, P.X.p, pcoef.p + j, kProjCoef, psi, b, xj, ppart,
-                 gcol + j + 1, M * kProjLdg, P.W.p + (size_t)j * M, M * M, M);
+    if (P.v_slot == j && P.e_m == j) {  // slot j holds -X e from proj_before's pass
+      proj_append(stream, D, pseg, j, proj_mr() ? 1 : 0, pcoef.p + j, kProjCoef, psi, b, xj, P.pnorm,
+                  P.W.p + (size_t)j * M, M * M, M, save);
+      saved = save != nullptr;
+    } else {
+      proj_ortho(stream, D, pseg, j, proj_mr() ? 1 : 0, P.X.p, pcoef.p + j, kProjCoef, psi, b, xj, P.pnorm,
+                 P.W.p + (size_t)j * M, M * M, M);
+    }
     apply_As(xj, axj);
     // its Gram column (Y_i . axj, i <= j) comes from the next projected solve's pass over Y
     // (proj_dots3), or from proj_flush_gcol when the basis is used otherwise first
@@ -1419,6 +1463,7 @@ struct Solver {
     P.e_m = -1;
     P.v_slot = -1;
     P.gcol_pending = j;
+    return saved;
   }
   // The Gram column of the newest vector when it is still pending (its vector and image are in
   // their slots); a pending column of a basis since reset is dropped.
@@ -1429,6 +1474,7 @@ struct Solver {
     constexpr int M = kProjVectors;
     proj_gcol(stream, D, pseg, j, proj_mr() ? 1 : 0, proj_mr() ? P.AX.p : P.X.p, P.X.p + (size_t)j * D,
               P.AX.p + (size_t)j * D, ppart, P.G.p + (size_t)j * kProjLdg, M * kProjLdg);
+    proj_sum(stream, pseg, P.pnorm, P.G.p + (size_t)j * kProjLdg + j + 1, M * kProjLdg);
   }
   // The adjoint's colouring, velocity map, buffers and recorded trajectory belong to one mesh and
   // one set-up: a new mesh or set-up rebuilds them on the next adjoint call.
@@ -1455,8 +1501,9 @@ struct Solver {
     const bool ok = n_hist == 2 && tau > tau_a && tau - tau_a <= 1. && tau_a > tau_b && tau_a - tau_b <= 1.;
     psi_predict(stream, D, ok ? (tau - tau_a) / (tau_a - tau_b) : 0., ok ? 1 : 0, psi, psi_prev);
   }
-  void guess_after_solve() {
-    if (guess_mode() >= 3 && rk_stage >= 0 && !std::isnan(stage_tau)) { rk_guess_after(); return; }
+  // copied: rk_copy's copy has been made
+  void guess_after_solve(bool copied) {
+    if (guess_mode() >= 3 && rk_stage >= 0 && !std::isnan(stage_tau)) { rk_guess_after(copied); return; }
     rk_full = false;
     rk_qok = false;
     rk_cur = 0;
@@ -1498,12 +1545,15 @@ struct Solver {
       HIPCHK(hipMemcpyAsync(S.p + S_TOL2, &t2, sizeof(double), hipMemcpyHostToDevice, stream));
       HIPCHK(hipStreamSynchronize(stream));
     }
-    outer_residual(have_bb ? nullptr : part2.p);
+    const double* pbb = have_bb ? nullptr : part2.p;
+    outer_residual(pbb);
     // FP64: the FP64 V-cycle; mixed: the FP32 V-cycle (precond), the Krylov vectors, the operator
     // application and the stopping test in FP64 either way.  The results arrive with the status of
     // the last iteration, so the stream goes on without a copy or a wait for it to drain.
-    krylov_solve(psi.p, P64.r.p, S.p, F.p, maxit, maxit);
+    krylov_solve(psi.p, P64.r.p, pbb, S.p, F.p, maxit, maxit);
     const MirrorState res = *mirror;
+    // a zero right-hand side: psi = 0, as the reference's solver returns
+    if (res.zero) HIPCHK(hipMemsetAsync(psi.p, 0, D * sizeof(double), stream));
     // statistics
     last_iters = res.iter;
     last_outer = 0;
@@ -1515,8 +1565,9 @@ struct Solver {
     if (res.zero) last_rel = 0.;
     total_iters += last_iters;
     ++n_solves;
-    if (proj && !res.zero) proj_after(bs);
-    guess_after_solve();
+    bool copied = false;
+    if (proj && !res.zero) copied = proj_after(bs, rk_copy());
+    guess_after_solve(copied);
     if (!std::isfinite(last_rel)) throw StatusError(HOC_ENAN, "NaN/Inf in the Poisson solve");
     if (cfg.fail_on_noconv && last_rel > cfg.tol)
       throw StatusError(HOC_ENOCONV, "Poisson solve did not converge: rel residual " + std::to_string(last_rel));

@@ -28,6 +28,19 @@ __device__ __forceinline__ bool likely_last(const double* __restrict__ S) {
   return S[S_PRED] <= 4. * S[S_TOL2] * S[S_BB];
 }
 
+// Start of a solve, from its first residual: a = r.r, b = ||r||^2 (unscaled), above: over the tolerance.
+__device__ __forceinline__ void init_phase(double a, double b, bool above, double* __restrict__ S,
+                                           int* __restrict__ F, int maxiter) {
+  S[S_RR] = S[S_RRL] = S[S_PRED] = b;
+  const double tiny = 2. * 2.220446049250313e-16;
+  const bool zero = S[S_BB] < tiny * tiny;
+  F[F_ZERO] = zero;
+  F[F_ITER] = 0;
+  F[F_HALF] = 0;
+  F[F_ACTIVE] = (!zero && above && maxiter > 0) ? 1 : 0;
+  S[S_RZ] = 0.; S[S_RHO] = S[S_RHON] = a; S[S_ALPHA] = 1.; S[S_OMEGA] = 1.; S[S_BETA] = 0.;
+}
+
 // b = ||r||^2 (unscaled) against the tolerance.  PH_UPD: end of a PCG iteration.  PH_BHALF: BiCGSTAB
 // at its half step (x already holds alpha ph).  PH_BNEXT: end of a BiCGSTAB iteration, a = rh . r of
 // the next; rho = 0 or not finite is a breakdown.
