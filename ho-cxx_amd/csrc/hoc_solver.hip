@@ -693,8 +693,11 @@ struct Solver {
 
   // ---------------------------------------------------------------------------------------
   // Coarsening stops at this many unknowns, solved by their dense inverse: one launch in place of
-  // two per level below.
-  static constexpr int kCoarseDense = 1200;
+  // two per level below.  1200, 1700 and 2450: cavity 127 x 127, K = 5 (coarsest 258, or 1213) 23.0, 22.0
+  // and 21.9 ms a pass, step 384 x 64 (294, or 1209) 21.3, 20.3 and 20.5, cylinder 96 x 96 (288, or 1235)
+  // 7.3, 7.0 and 7.2; where 2450 takes one of 2401 instead of 695 (hybrid 48 x 48) 5.0 ms stay 5.0 and
+  // the setup doubles.
+  static constexpr int kCoarseDense = 1700;
   // The dense inverse of the coarsest matrix, by the GPU's unpivoted elimination; a result that does
   // not reproduce a vector to 1e-6 is replaced by the host's pivoted one.
   void coarse_inverse(const CSR& A, std::vector<double>& ci) {

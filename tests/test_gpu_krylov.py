@@ -28,7 +28,7 @@ def jacobian(g, K):
 @pytest.mark.parametrize("precision", [hoc.HOC_FP64, hoc.HOC_MIXED])
 @pytest.mark.parametrize("n,K,curved,cheb", [
     (16, 3, False, 0), (17, 3, False, 0),    # 289 and 324 vertices: the two register counts of the product
-    (33, 2, False, 0), (34, 2, False, 0),    # 1156 vertices, and 1225: a sparse level in between
+    (33, 2, False, 0), (34, 2, False, 0),    # 1156 vertices, and 1225: past the size of the fused product
     (6, 4, False, 1), (6, 4, True, 1),       # one smoothing step
     (9, 5, True, 3), (16, 2, True, 0),
     (203, 6, False, 0), (203, 6, True, 0),   # 1031 partial sums
