@@ -438,15 +438,17 @@ __device__ void check_block(const A& a) {
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> G, FineArgs<R> A) {
   constexpr bool CHK = IN == IN_X && EPI == EPI_SMOOTH;
-  const int nblk = CHK && A.chk_part ? (int)gridDim.x - 1 : (int)gridDim.x;
-  if (CHK && (int)blockIdx.x == nblk) {
-    check_block(A);
+  // the test goes first, so that it ends in the shadow of the others; eight blocks, so that these keep
+  // their XCDs
+  const int nchk = CHK && A.chk_part ? 8 : 0, nblk = (int)gridDim.x - nchk;
+  if (CHK && (int)blockIdx.x < nchk) {
+    if (blockIdx.x == 0) check_block(A);
     return;
   }
   constexpr int EPW = Lay<K>::EPW, ES = Lay<K>::ES;
   constexpr int FS = GEO == GEO_ORTHO ? 0 : 4 * K;  // face values of one element
   __shared__ __align__(16) R lds[(kFineThreads / 64) * (Lay<K>::TILE + EPW * FS)];
-  const int blk = xcd_block(blockIdx.x, nblk);
+  const int blk = xcd_block(blockIdx.x - nchk, nblk);
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int EPB = EPW * (kFineThreads / 64);
   const int le = lane < EPW * K ? lane / K : EPW - 1;
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   // slot its last row: the same reads, so the same values in LDS; neither writes to memory
   const int el = min(el0, G.N - 1);
   const bool go = !A.active || A.active[F_ACTIVE];
-  if (A.ran && blockIdx.x == 0 && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
+  if (A.ran && (int)blockIdx.x == nchk && threadIdx.x == 0) *A.ran = go ? 1 : 0;  // timed launches: did it work?
   if (!go) return;
   if (G.iact) {  // a block inside one stopped ensemble instance
     const int i0 = G.inst[blk * EPB];
@@ -832,7 +834,7 @@ __global__ __launch_bounds__(kFineThreads) void k_bicg_x(int N, BicgArgs A) {
 
 template <int K, int GEO, int IN, int EPI, class R, class RZ>
 static void go_fine(const FineTab<R>& T, const FineGeo<R>& G, const FineArgs<R>& A, hipStream_t s) {
-  hipLaunchKernelGGL((k_fine<K, GEO, IN, EPI, R, RZ>), dim3(fine_blocks(K, G.N) + (A.chk_part ? 1 : 0)),
+  hipLaunchKernelGGL((k_fine<K, GEO, IN, EPI, R, RZ>), dim3(fine_blocks(K, G.N) + (A.chk_part ? 8 : 0)),
                      dim3(kFineThreads), 0, s, T, G, A);
 }
 

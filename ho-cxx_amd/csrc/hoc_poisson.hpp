@@ -94,7 +94,7 @@ struct FineArgs {
   const double* b64 = nullptr;  // EPI_SMOOTH in FP32: b in FP64 for the sums of b.y
   int* active = nullptr;     // the Krylov flags F (may be null)
   int* ran = nullptr;        // set to 1 when the launch worked, 0 when active made it return at once
-  // EPI_SMOOTH of IN_X: one block more, which tests np pairs of partial norms that an earlier kernel
+  // EPI_SMOOTH of IN_X: a block more, which tests np pairs of partial norms that an earlier kernel
   // left (phase: check_phase, or PH_INIT) on the flags chk_F and publishes the state; the other blocks
   // do not wait for it.  chk_bb: chk_nbb partials of ||b||^2 for scal[S_BB] (PH_INIT; may be null)
   int* chk_F = nullptr;
