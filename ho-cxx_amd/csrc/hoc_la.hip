@@ -493,21 +493,12 @@ __global__ void k_q1_probe_accum(int N, int K, Tab T, int rs, const double* __re
 }
 
 // ---- mixed precision ---------------------------------------------------------------------------
-// FP64 Krylov method with the FP32 V-cycle as its preconditioner: the V-cycle's output
-// z64 = (double) z32 with partials of r64 . z64 (slot 0; slot 1 zero) when part is set.
-__global__ void k_promote_dot(size_t n, const float* __restrict__ z32, double* __restrict__ z64,
-                              const double* __restrict__ r64, double* __restrict__ part, const int* __restrict__ F) {
+// BiCGSTAB with the FP32 V-cycle as its preconditioner: the V-cycle's output z64 = (double) z32.
+__global__ void k_promote(size_t n, const float* __restrict__ z32, double* __restrict__ z64,
+                          const int* __restrict__ F) {
   if (F && !F[F_ACTIVE]) return;
-  double p0 = 0., p1 = 0.;
-  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x) {
-    const double z = (double)z32[v];
-    z64[v] = z;
-    if (part) p0 += r64[v] * z;
-  }
-  if (part) {
-    block_sum2(p0, p1);
-    if (threadIdx.x == 0) { part[blockIdx.x] = p0; part[gridDim.x + blockIdx.x] = p1; }
-  }
+  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x)
+    z64[v] = (double)z32[v];
 }
 
 // ---- ensembles ---------------------------------------------------------------------------------
@@ -1362,9 +1353,8 @@ void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc
   if (n <= 320) hipLaunchKernelGGL((k_dense_gather<5, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
   else hipLaunchKernelGGL((k_dense_gather<kDenseGather / 64, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
 }
-void promote_dot(hipStream_t s, size_t n, const float* z32, double* z64, const double* r64, double* part,
-                 const int* F) {
-  hipLaunchKernelGGL(k_promote_dot, dim3(vec_grid(n)), dim3(256), 0, s, n, z32, z64, r64, part, F);
+void promote(hipStream_t s, size_t n, const float* z32, double* z64, const int* F) {
+  hipLaunchKernelGGL(k_promote, dim3(vec_grid(n)), dim3(256), 0, s, n, z32, z64, F);
 }
 void inst_norms(hipStream_t s, const VecArgs& A, int n_inst, const int32_t* off, int K2, const double* b, double* out) {
   hipLaunchKernelGGL(k_inst_norms, dim3(n_inst), dim3(256), 0, s, A, off, K2, b, out);
@@ -1380,15 +1370,15 @@ void q1_probe_accum(hipStream_t s, int N, int K, const Tab& T, int rs, const dou
   hipLaunchKernelGGL(k_q1_probe_accum, dim3((N + 255) / 256), dim3(256), 0, s, N, K, T, rs, y, M);
 }
 
+template void vec<double>(hipStream_t, int, const VecArgs&, size_t, double*, double*, const double*, const double*,
+                          double*, const double*, const int*, double*);
+template void bicg_half<double>(hipStream_t, size_t, double*, const double*, const double*, int*);
+template void zero_if_flag<double>(hipStream_t, size_t, double*, const int*);
+template void csr<double>(hipStream_t, int, int, const int32_t*, const int32_t*, const double*, const double*,
+                          const double*, double*, const double*, double*, const int*, int);
+template void ell<double>(hipStream_t, int, int, int, int, const int32_t*, const double*, const double*, const double*,
+                          double*, const double*, double*, const int*);
 #define HOC_LA_INST(R)                                                                                                 \
-  template void vec<R>(hipStream_t, int, const VecArgs&, size_t, R*, R*, const R*, const R*, R*, const double*,        \
-                       const int*, double*);                                                                           \
-  template void bicg_half<R>(hipStream_t, size_t, R*, const R*, const double*, int*);                                 \
-  template void zero_if_flag<R>(hipStream_t, size_t, R*, const int*);                                                 \
-  template void csr<R>(hipStream_t, int, int, const int32_t*, const int32_t*, const R*, const R*, const R*, R*,        \
-                       const R*, R*, const int*, int);                                                                 \
-  template void ell<R>(hipStream_t, int, int, int, int, const int32_t*, const R*, const R*, const R*, R*, const R*,  \
-                       R*, const int*);                                                                        \
   template void sell<R>(hipStream_t, int, int, const int32_t*, const int32_t*, const R*, const R*, R*, const int*);    \
   template void dense<R>(hipStream_t, int, const R*, const R*, R*, const int*);                                       \
   template void q1_gather<R>(hipStream_t, int, int, const int32_t*, const R*, R*, const int*);                          \

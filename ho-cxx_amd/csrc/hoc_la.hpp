@@ -1,7 +1,7 @@
 // hoc_la.hpp - vector/reduction/CSR/probing kernels of the Poisson solver (hoc_la.hip).
 //
-// Vector and level kernels are instantiated for double (FP64 solve) and float (the
-// mixed-precision inner solve); scalars, partial sums and flags are always double/int.
+// Level kernels are instantiated for double and float (the mixed-precision V-cycle); scalars, partial
+// sums and flags are always double/int.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -81,10 +81,8 @@ constexpr int kDenseGather = 1216;
 template <class R>
 void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc, const R* ec, R* x, const int* F);
 
-// The FP32 V-cycle inside the FP64 Krylov method: z64 = (double) z32 with partials of r64 . z64 in
-// part (vec_grid(n) blocks; may be null).
-void promote_dot(hipStream_t s, size_t n, const float* z32, double* z64, const double* r64, double* part,
-                 const int* F);
+// The FP32 V-cycle inside the FP64 BiCGSTAB: z64 = (double) z32.
+void promote(hipStream_t s, size_t n, const float* z32, double* z64, const int* F);
 
 // Initial guess of a stage solve from the solutions at the last two distinct stage times:
 // extrap = 0: prev = psi (history shift, psi kept);  extrap = 1: psi' = psi + f (psi - prev)

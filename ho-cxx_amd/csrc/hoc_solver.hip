@@ -169,7 +169,7 @@ struct Solver {
   bool mixed = false;
 
   // device: geometry and connectivity
-  DBuf<double> d_jac, d_xxi, d_xeta, d_yxi, d_yeta, d_Ga, d_Gb, d_Gc, d_fa, d_fb, d_fA, d_fB, d_fjac, d_fAn;
+  DBuf<double> d_jac, d_xxi, d_xeta, d_yxi, d_yeta, d_Ga, d_Gb, d_Gc, d_fa, d_fb, d_fA, d_fjac, d_fAn;
   DBuf<int32_t> d_nb;
   DBuf<int8_t> d_nbf, d_swpsi, d_swdiff, d_noslip;
   DBuf<double> d_esign, d_gel, d_gface, d_gjm;
@@ -306,7 +306,7 @@ struct Solver {
     for (size_t i = 0; i < fa.size(); ++i) { fa[i] = geo.fA[i] / geo.fjac[i]; fb[i] = geo.fB[i] / geo.fjac[i]; }
     d_jac.upload(geo.jac); d_xxi.upload(geo.xxi); d_xeta.upload(geo.xeta); d_yxi.upload(geo.yxi); d_yeta.upload(geo.yeta);
     d_Ga.upload(Ga); d_Gb.upload(Gb); d_Gc.upload(Gc);
-    d_fa.upload(fa); d_fb.upload(fb); d_fA.upload(geo.fA); d_fB.upload(geo.fB); d_fjac.upload(geo.fjac); d_fAn.upload(geo.fAn);
+    d_fa.upload(fa); d_fb.upload(fb); d_fA.upload(geo.fA); d_fjac.upload(geo.fjac); d_fAn.upload(geo.fAn);
     d_nb.upload(mesh.nb);
     d_nbf.upload(mesh.nb_face);
     std::vector<int8_t> swp(E), swd(E), ns(E);
@@ -347,7 +347,7 @@ struct Solver {
       d_dcol.upload(dc); d_wrow.upload(wr);
     }
     if (affine) { d_gel.upload(gel); d_gface.upload(gface); d_gjm.upload(gjm); }
-    G = Geo{N, E, d_jac, d_xxi, d_xeta, d_yxi, d_yeta, d_Ga, d_Gb, d_Gc, d_fa, d_fb, d_fA, d_fB, d_fjac, d_fAn,
+    G = Geo{N, E, d_jac, d_xxi, d_xeta, d_yxi, d_yeta, d_Ga, d_Gb, d_Gc, d_fa, d_fb, d_fA, d_fjac, d_fAn,
             affine ? d_gel.p : nullptr, affine ? d_gface.p : nullptr, affine ? d_gjm.p : nullptr,
             d_nb, d_nbf, d_swpsi, d_swdiff, d_noslip, d_esign, nullptr, d_dcol, d_wrow, nullptr};
     setup_instances();
@@ -537,7 +537,8 @@ struct Solver {
     P.G.iact = P.iact;
     A.ran = rec ? prof.ran.p + prof.n : nullptr;
     HIPCHK(launch_fine(K, geo_kind, in, epi, P.T, P.G, A, stream));
-    if (rec) prof_mark(P.prof_off + prof_variant(in, epi), lap_bytes(in, epi, (double)sizeof(R), (double)sizeof(R)));
+    const double b64 = epi == EPI_SMOOTH && A.b64 && (A.part || A.elpart) ? 8. * D : 0.;  // FP32: b in FP64 too
+    if (rec) prof_mark(P.prof_off + prof_variant(in, epi), lap_bytes(in, epi, (double)sizeof(R), (double)sizeof(R)) + b64);
   }
   void prof_mark(int variant, double bytes) {
     HIPCHK(hipEventRecord(prof.e1[prof.n], stream));
@@ -882,7 +883,7 @@ struct Solver {
   void precond_rest(const double* rin, double* zout, int* Fp, int part_of, const Check* chk) {
     if (mixed) {
       vcycle_rest(P32, (const float*)P32.r.p, rin, P32.z.p, nullptr, Fp, part_of, chk);
-      if (part_of != HEAD) promote_dot(stream, D, P32.z.p, zout, rin, nullptr, Fp);
+      if (part_of != HEAD) promote(stream, D, P32.z.p, zout, Fp);
     } else {
       vcycle_rest(P64, rin, rin, zout, nullptr, Fp, part_of, chk);
     }
