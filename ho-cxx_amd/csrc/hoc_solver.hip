@@ -1155,7 +1155,8 @@ struct Solver {
       else krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
       bool near = false;
       if (!poll(seq, seq0, it > maxit_host + 2, 1, &near) || it > maxit_host + 4) break;
-      if (near && !poll(seq, seq0, true)) break;
+      // (before the first iteration there is no status to go by: as the solve before, which ended there)
+      if ((near || (it == 0 && last_iters == 1)) && !poll(seq, seq0, true)) break;
       if (graphs) HIPCHK(hipGraphLaunch(ge[2], stream));
       else krylov_tail(r, Sp, Fp, maxit);
     }
