@@ -200,6 +200,47 @@ struct Solver {
   // Chebyshev smoother of degree cheb_m in B As (B: the element blocks' inverse) as damped
   // Richardson steps x += cheb_w[k] B (r - As x)
   int cheb_m = 2;
+  // Lower end of the smoothing interval over 1.1 lambda_max(B As).
+  double cheb_lo = .1;
+  // Degree and interval by order and shape of the elements: what the bilinear functions leave to the
+  // smoother reaches down to a part of the spectrum that shrinks with the order and, far more, with the
+  // elements' aspect ratio, where three steps down to 1/20 (order 6: 0.06) save a third of the iterations
+  // for 4 of about 29 launches each.  ms per solve to 1e-11 (iterations), degree 2 at 1/10 | degree 2 at the
+  // table's end (order 6: 0.08) | degree 3.  Squares: 48x48 K=2 0.52 (10) | 0.46 (9) | 0.63 (10), K=4 0.58 (11) | 0.56 (11) | 0.70 (11),
+  // K=5 0.72 (12) | same | 0.77 (11), K=6 0.90 (15) | 0.92 (15) | 0.82 (11); jittered 128x128 K=5 1.98 (9)
+  // | same | 2.19 (9).  Ratio 1.9, 128x16: K=2 0.53 | 0.44 | 0.64, K=3 0.65 | 0.67 | 0.64, K=4 0.83 | 0.93
+  // | 0.74, K=5 1.12 | same | 0.98.  Ratio 3.8, 96x24: K=2 0.70 | 0.77 | 0.68, K=3 1.17 | 1.29 | 0.93, K=5
+  // 2.2 (39) | same | 1.8 (27); jittered 2.97 (25) | same | 2.78 (17); ratio 7.5, 96x48: K=5 4.6 (78) |
+  // same | 3.8 (53).  Degree 1 takes about twice the iterations of degree 2 throughout.
+  void choose_smoother(double aspect) {
+    static const double two[4] = {.15, .15, .12, .1};
+    if (cfg.cheb_degree > 0) {
+      cheb_m = cfg.cheb_degree;
+      cheb_lo = .1;
+    } else if (K == 6 || aspect > (K == 2 ? 3. : 1.5)) {
+      cheb_m = 3;
+      cheb_lo = K == 6 ? .06 : .05;
+    } else {
+      cheb_m = 2;
+      cheb_lo = two[K - 2];
+    }
+    if (cfg.cheb_lower > 0.) cheb_lo = cfg.cheb_lower;
+  }
+  // Mean ratio of the elements' sides: the longer to the shorter pair's sum.
+  double mean_aspect() const {
+    double sum = 0.;
+    for (int e = 0; e < N; ++e) {
+      const int32_t* nd = &mesh.elem[(size_t)e * mesh.lnod * mesh.lnod];
+      double side[4];
+      for (int k = 0; k < 4; ++k) {
+        const double *p = &mesh.xy[2 * (size_t)nd[k]], *q = &mesh.xy[2 * (size_t)nd[(k + 1) & 3]];
+        side[k] = std::hypot(q[0] - p[0], q[1] - p[1]);
+      }
+      const double a = side[0] + side[2], b = side[1] + side[3];
+      sum += std::max(a, b) / std::max(std::min(a, b), 1e-300);
+    }
+    return sum / N;
+  }
   double cheb_w[kMaxCheb] = {0};
   double lam_max = 0.;
   int geo_kind = GEO_POINT;          // what the fine-level kernels are instantiated for
@@ -764,12 +805,11 @@ struct Solver {
       for (size_t i = 0; i < D; ++i) { a += hx2[i] * hAx[i]; b += hx[i] * hAy[i]; na += std::fabs(hx2[i] * hAx[i]); nb += std::fabs(hx[i] * hAy[i]); }
       krylov = std::fabs(a - b) <= 1e-12 * std::max(na, nb) ? HOC_KRYLOV_PCG : HOC_KRYLOV_BICGSTAB;
     }
-    const double lmax = 1.1 * lam, lmin = lmax * (cfg.cheb_lower > 0. ? cfg.cheb_lower : 1. / 10.);
+    choose_smoother(mean_aspect());
+    const double lmax = 1.1 * lam, lmin = lmax * cheb_lo;
     const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
-    // Degree 2 by default: on the cavity (K = 5) degree 1 takes about twice the iterations and
-    // degree 3 no fewer, the coarse space limiting them from there on.  The dampings are the
-    // inverse roots of the Chebyshev polynomial on [lmin, lmax], large and small in turn.
-    cheb_m = cfg.cheb_degree > 0 ? cfg.cheb_degree : 2;
+    // The dampings are the inverse roots of the Chebyshev polynomial on [lmin, lmax], large and small in
+    // turn.
     std::vector<double> root(cheb_m);
     for (int k = 0; k < cheb_m; ++k) root[k] = theta + delta * std::cos(M_PI * (k + 0.5) / cheb_m);
     for (int k = 0; k < cheb_m; ++k) cheb_w[k] = 1. / ((k & 1) ? root[cheb_m - 1 - k / 2] : root[k / 2]);

@@ -55,7 +55,8 @@ typedef struct {
   int32_t fail_on_noconv;         /* nonzero: return HOC_ENOCONV when tol is not met     */
   double mixed_inner_tol;         /* unused (kept for layout); must lie in [0, 1)       */
   int32_t cheb_degree;            /* degree of the fine-level Chebyshev smoother in B As, pre and
-                                     post (B: the element blocks' inverse; 0 = 2; at most 8) */
+                                     post (B: the element blocks' inverse; at most 8;
+                                     0 = 3 at order 6 and for stretched elements, else 2) */
   int32_t psi_guess;              /* initial guess of the stage Poisson solves: 1 = the
                                      previous solution (the reference's warm start),
                                      2 = linear extrapolation in the stage time from the
@@ -70,7 +71,8 @@ typedef struct {
                                      solutions: in the As-norm for a symmetric operator,
                                      least-squares residual otherwise  (0 = 5)            */
   double cheb_lower;              /* smoothing interval [cheb_lower, 1.1] x lambda_max(B As)
-                                     (0 = 1/10)                                          */
+                                     (0 = chosen with the degree; 1/10 where cheb_degree
+                                     is given)                                           */
   int32_t launch_mode;            /* Krylov iterations: 0 = chosen at hoc_setup by timing
                                      both, 1 = kernels queued one by one, 2 = replays of a
                                      captured hipGraph of an iteration (same iterates)   */
