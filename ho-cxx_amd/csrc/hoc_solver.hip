@@ -212,11 +212,19 @@ struct Solver {
   // | 0.74, K=5 1.12 | same | 0.98.  Ratio 3.8, 96x24: K=2 0.70 | 0.77 | 0.68, K=3 1.17 | 1.29 | 0.93, K=5
   // 2.2 (39) | same | 1.8 (27); jittered 2.97 (25) | same | 2.78 (17); ratio 7.5, 96x48: K=5 4.6 (78) |
   // same | 3.8 (53).  Degree 1 takes about twice the iterations of degree 2 throughout.
+  // Further out degree 4 at 0.03 gains on degree 3: ratio 1.9, 128x16: K=3 0.64 -> 0.74, K=4 0.74 -> 0.79,
+  // K=5 0.98 -> 0.92, K=6 1.36 -> 1.16; jittered K=5 1.38 -> 1.26, K=6 1.87 -> 1.53.  Ratio 2.5, 256x42: K=3
+  // 0.96 -> 1.02, K=4 1.23 -> 1.19, K=5 1.75 -> 1.49, K=6 2.34 -> 2.03; jittered K=3 1.06 -> 1.21, K=4 1.59 ->
+  // 1.60, K=5 2.22 -> 1.93, K=6 3.11 -> 2.52.  Ratio 3.8, 96x24: K=2 0.68 -> 0.72, K=3 0.93 -> 0.88, K=4 1.31
+  // -> 1.17, K=5 1.82 -> 1.56, K=6 2.36 -> 2.04.
   void choose_smoother(double aspect) {
     static const double two[4] = {.15, .15, .12, .1};
     if (cfg.cheb_degree > 0) {
       cheb_m = cfg.cheb_degree;
       cheb_lo = .1;
+    } else if (K > 2 && aspect > (K < 5 ? 3. : 1.8)) {
+      cheb_m = 4;
+      cheb_lo = .03;
     } else if (K == 6 || aspect > (K == 2 ? 3. : 1.5)) {
       cheb_m = 3;
       cheb_lo = K == 6 ? .06 : .05;

@@ -56,7 +56,7 @@ typedef struct {
   double mixed_inner_tol;         /* unused (kept for layout); must lie in [0, 1)       */
   int32_t cheb_degree;            /* degree of the fine-level Chebyshev smoother in B As, pre and
                                      post (B: the element blocks' inverse; at most 8;
-                                     0 = 3 at order 6 and for stretched elements, else 2) */
+                                     0 = 2, more at order 6 and for stretched elements) */
   int32_t psi_guess;              /* initial guess of the stage Poisson solves: 1 = the
                                      previous solution (the reference's warm start),
                                      2 = linear extrapolation in the stage time from the

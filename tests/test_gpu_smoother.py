@@ -27,7 +27,9 @@ def solve(m, K, w, **options):
 @pytest.mark.parametrize("jitter", [0.0, 0.1])
 @pytest.mark.parametrize("K,ratio,degree,lower", [
     (2, 2.8, 2, 0.15), (2, 3.2, 3, 0.05), (3, 1.4, 2, 0.15), (3, 1.6, 3, 0.05), (4, 1.4, 2, 0.12),
-    (5, 1.4, 2, 0.1), (5, 1.6, 3, 0.05), (6, 1.0, 3, 0.06), (6, 20.0, 3, 0.06),
+    (5, 1.4, 2, 0.1), (5, 1.6, 3, 0.05), (6, 1.0, 3, 0.06), (6, 20.0, 4, 0.03),
+    (2, 5.0, 3, 0.05), (3, 2.8, 3, 0.05), (3, 3.2, 4, 0.03), (4, 2.8, 3, 0.05), (4, 3.2, 4, 0.03), (5, 2.0, 4, 0.03),
+    (6, 1.6, 3, 0.06), (6, 2.0, 4, 0.03),
 ])
 def test_choice(gpu_available, K, ratio, degree, lower, jitter):
     m = meshes.cavity(11, 2, seed=3, jitter=jitter * min(1.0, 2.0 / ratio) if ratio < 10 else 0.0)
