@@ -56,8 +56,15 @@ struct Prec {
   DevVHierarchy<R> lv;  // Q1 vertex level and below
   int prof_off = 0;  // offset of this precision's entries in the live kernel profile
   // set only while the iterations of a batched ensemble PCG are queued: the instances' live flags;
-  // fine-level blocks of a stopped instance then return at once
+  // fine-level blocks of a stopped instance then return at once.  They go with a launch's copy of G
+  // (masked): G itself has none, so that an operator application beside or after a solve works on every
+  // instance.
   const int* iact = nullptr;
+  FineGeo<R> masked() const {
+    FineGeo<R> g = G;
+    g.iact = iact;
+    return g;
+  }
   // vectors of the Krylov method (krylov) and of the V-cycle alone (the FP32 state)
   void alloc_vectors(size_t D, int N, bool krylov) {
     for (auto* f : {&r, &z, &t}) f->alloc(D);
@@ -583,9 +590,8 @@ struct Solver {
   void fine(Prec<R>& P, int in, int epi, FineArgs<R> A) {
     const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
     if (rec) HIPCHK(hipEventRecord(prof.e0[prof.n], stream));
-    P.G.iact = P.iact;
     A.ran = rec ? prof.ran.p + prof.n : nullptr;
-    HIPCHK(launch_fine(K, geo_kind, in, epi, P.T, P.G, A, stream));
+    HIPCHK(launch_fine(K, geo_kind, in, epi, P.T, P.masked(), A, stream));
     const double b64 = epi == EPI_SMOOTH && A.b64 && (A.part || A.elpart) ? 8. * D : 0.;  // FP32: b in FP64 too
     if (rec) prof_mark(P.prof_off + prof_variant(in, epi), lap_bytes(in, epi, (double)sizeof(R), (double)sizeof(R)) + b64);
   }
@@ -611,9 +617,8 @@ struct Solver {
     if (!z32) { fine(P, IN_PUPD, EPI_STORE, A); return; }
     const bool rec = prof.on && (prof.seen++ % prof.every) == 0;
     if (rec) HIPCHK(hipEventRecord(prof.e0[prof.n], stream));
-    P.G.iact = P.iact;
     A.ran = rec ? prof.ran.p + prof.n : nullptr;
-    HIPCHK(launch_fine_pupd_f32z(K, geo_kind, P.T, P.G, A, stream));
+    HIPCHK(launch_fine_pupd_f32z(K, geo_kind, P.T, P.masked(), A, stream));
     if (rec) prof_mark(0, lap_bytes(IN_PUPD, EPI_STORE, 8., 4.));
   }
   // Only launches that worked count: a launch predicated off after convergence returns at once
@@ -1017,8 +1022,7 @@ struct Solver {
       PreArgs<R> A = pre_args<R>(r, P.t.p, cheb_w[0]);
       if constexpr (std::is_same<R, float>::value) A.r32 = P.r.p;
       set(A);
-      P.G.iact = P.iact;
-      HIPCHK(launch_pre(K, P.T, P.G, A, stream));
+      HIPCHK(launch_pre(K, P.T, P.masked(), A, stream));
     };
     if (mixed) go(P32);
     else go(P64);
