@@ -65,7 +65,8 @@ template <class R>
 struct FineTab {
   R lv[6], ld[6];  // l_m(-1), l_m'(-1) (the upper end by reflection)
   R lvE[3], lvO[3], ldE[3], ldO[3];      // the same on the even and odd parts
-  R DDE[3][3], DDO[3][3];                // second derivative: [in][out]
+  R DDE[3][3], DDO[3][3];                // second derivative: [in][out] (V-cycle)
+  R DE[3][3], DO[3][3];                  // derivative: the odd part of an even line's, and vice versa
   R gdE[3], gdO[3], DgE[3], DgO[3];      // lower Radau correction's derivative, and its derivative
   R m0, m1;        // that correction's derivative extrapolated to -1 and +1
   R g0, ig0;       // -g'(-1), the interface coefficient, and its inverse

@@ -485,10 +485,12 @@ struct Solver {
     for (int i = 0; i < HE; ++i) {
       F.lvE[i] = (R)even(lv, i); F.ldE[i] = (R)even(ld, i); F.gdE[i] = (R)even(gd, i); F.DgE[i] = (R)even(ft.Dg, i);
       for (int d = 0; d < HE; ++d) F.DDE[d][i] = (R)even(ft.DD[d], i);
+      for (int d = 0; d < HO; ++d) F.DO[d][i] = (R)even(tab.D[d], i);
     }
     for (int i = 0; i < HO; ++i) {
       F.lvO[i] = (R)odd(lv, i); F.ldO[i] = (R)odd(ld, i); F.gdO[i] = (R)odd(gd, i); F.DgO[i] = (R)odd(ft.Dg, i);
       for (int d = 0; d < HO; ++d) F.DDO[d][i] = (R)odd(ft.DD[d], i);
+      for (int d = 0; d < HE; ++d) F.DE[d][i] = (R)odd(tab.D[d], i);
     }
     // interior eigenvectors, even ones first (the line operator commutes with the reflection)
     for (int q = 0, ne = 0, no = 0; q < K; ++q) {
