@@ -187,6 +187,7 @@ __device__ void finalize_phase(int phase, double a, double b, double* __restrict
       S[S_ALPHA] = al;
     } break;
     case PH_UPD: {
+      if (F[F_BREAK]) { F[F_ACTIVE] = 0; break; }
       S[S_RR] = b;
       F[F_ITER] += 1;
       F[F_ACTIVE] = (above && F[F_ITER] < maxiter && isfinite(b)) ? 1 : 0;

@@ -15,8 +15,10 @@ namespace hoc {
 
 // Device scalar slots (double) and flags (int) of the Krylov solvers.
 // F_MAXIT: iteration budget read by finalize kernels launched with maxiter < 0.
+// F_BREAK: a breakdown seen by the blocks of a kernel that F_ACTIVE predicates, which therefore may not
+// clear F_ACTIVE themselves (a block that starts late would leave in part); the next test does.
 enum { S_BB = 0, S_RR, S_RZ, S_PQ, S_ALPHA, S_BETA, S_OMEGA, S_RHO, S_TOL2, S_IMAX, S_RZN, S_RHON, S_RRL, S_PRED, S_COUNT = 16 };
-enum { F_ACTIVE = 0, F_ITER, F_ZERO, F_HALF, F_MAXIT, F_SEQ, F_COUNT = 8 };
+enum { F_ACTIVE = 0, F_ITER, F_ZERO, F_HALF, F_MAXIT, F_SEQ, F_BREAK, F_COUNT = 8 };
 enum { PH_BB = 0, PH_INIT, PH_RZ, PH_PQ, PH_UPD, PH_RHO, PH_ALPHA, PH_SNORM, PH_OMEGA, PH_RNORM, PH_BHALF, PH_BNEXT };
 enum { VOP_BICG_P = 0, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
 

@@ -609,15 +609,12 @@ __global__ __launch_bounds__(kFineThreads) void k_fine(FineTab<R> T, FineGeo<R> 
   if constexpr (IN == IN_PUPD) {
     if (A.rz) {  // behind the loads: the sum takes longer than they do
       const double rz = sum_parts(A.rz, A.np), be = A.active[F_ITER] > 0 ? rz / A.scal[S_RZ] : 0.;
-      const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-      if (!(rz > 0.) || !isfinite(rz)) {  // breakdown (z = 0 or an indefinite preconditioner) ends the solve
-        if (first) A.active[F_ACTIVE] = 0;
-        return;
-      }
-      if (first) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
         A.scal[S_RZN] = rz;
         A.scal[S_BETA] = be;
       }
+      // breakdown (z = 0 or an indefinite preconditioner): PRE_XR sees it by S_RZN
+      if (!(rz > 0.) || !isfinite(rz)) return;
       beta = (R)be;
     }
   }
@@ -772,8 +769,9 @@ __global__ __launch_bounds__(kFineThreads) void k_pre(FineTab<R> T, FineGeo<R> G
       const double pq = sum_parts(A.pq, A.np), num = A.scal[A.num];
       al = num / pq;
       const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-      if (pq == 0. || (A.spd && !(pq > 0.)) || !isfinite(al)) {
-        if (first) A.active[F_ACTIVE] = 0;
+      // the same in every wavefront of every block, as F_ACTIVE at entry is: none clears it here
+      if (pq == 0. || (A.spd && !(pq > 0. && num > 0.)) || !isfinite(al)) {
+        if (first) A.active[F_BREAK] = 1;
         return;
       }
       if (first) {

@@ -87,7 +87,7 @@ struct FineArgs {
   double* scal = nullptr;  // IN_PUPD: beta = scal[scal_idx], scal_idx < 0: scal[inst[el]]
   int scal_idx = 0;
   // IN_PUPD, small meshes: r.z as np partials, summed by every block; block 0 leaves the new r.z and
-  // beta in scal (S_RZN, S_BETA) and clears active on a breakdown
+  // beta in scal (S_RZN, S_BETA).  On a breakdown (r.z not positive) nothing else is written
   const double* rz = nullptr;
   int np = 0;
   double* part = nullptr;    // [fine_blocks] sums, then [fine_blocks] second sums
@@ -134,8 +134,9 @@ struct PreArgs {
   int up = PRE_NONE;
   double *pw = nullptr, *rh = nullptr;  // PRE_BICGP, PRE_BICG0: the direction, the shadow residual
   // small meshes: a dot product as np partials, summed by every block.  PRE_XR: the denominator of
-  // alpha (numerator scal[num]); block 0 leaves alpha and the numerator (in scal[keep]) behind and
-  // clears active on a breakdown (spd: also where the sum is negative).  PRE_BICGP: rh.r, from which
+  // alpha (numerator scal[num]); block 0 leaves alpha and the numerator (in scal[keep]) behind.  On a
+  // breakdown (spd: also where either is not positive) no block writes x or r, and block 0 sets F_BREAK
+  // for the test of the iteration.  PRE_BICGP: rh.r, from which
   // block 0 leaves beta and scal[S_RHON]; a breakdown is left to the test of the iteration.
   const double* pq = nullptr;
   int np = 0, num = 0, keep = 0;
