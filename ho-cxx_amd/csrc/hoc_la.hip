@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(int phase, const doubl
     F[F_ACTIVE] = 0;
   }
   if (mirror && threadIdx.x == 0) {
-    const int sq = seq >= 0 ? seq : ++F[F_SEQ];
+    const int sq = take_seq(seq, F);
     const bool near = F[F_ACTIVE] && (irr ? S[S_IMAX] <= 64. : likely_last(S));
     publish(mirror, sq, near, S, F);
   }
@@ -1268,7 +1268,7 @@ __global__ __launch_bounds__(kEnsThreads) void k_finalize_ens(int phase, EnsKry 
     }
   }
   if (mirror) {
-    const int sq = seq >= 0 ? seq : ++F[F_SEQ];
+    const int sq = take_seq(seq, F);
     publish(mirror, sq, F[F_ACTIVE] && S[S_IMAX] <= 64., S, F);
   }
 }

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "hoc_kernels.hpp"
+#include "hoc_seq.hpp"
 
 namespace hoc {
 
@@ -25,7 +26,7 @@ enum { VOP_BICG_P = 0, VOP_BICG_S, VOP_DOT2, VOP_COPY, VOP_BICG_X };
 // What a solve's finalize kernels leave in pinned host memory: the status word, and the results of
 // the solve so far (stored before the status, ordered by a system-scope fence).
 struct MirrorState {
-  int status;
+  uint32_t status;  // status_word
   int iter, zero;
   double bb, rr;
 };
@@ -46,7 +47,7 @@ void bicg_half(hipStream_t s, size_t n, R* x, const R* ph, const double* S, int*
 template <class R>
 void zero_if_flag(hipStream_t s, size_t n, R* x, const int* F);
 // mirror (optional): pinned host state that receives the solve's results and the status word
-// seq * 4 + near * 2 + (active flag) when the kernel ends (near: likely_last);
+// status_word(seq, near, active) when the kernel ends (near: likely_last);
 // seq < 0: the next number of the device counter F[F_SEQ] (incremented) instead of seq.
 // pbb (PH_INIT): npbb partials of ||b||^2 for S[S_BB], which PH_BB would otherwise have set.
 // maxiter < 0: the budget is read from F[F_MAXIT].

@@ -510,7 +510,7 @@ __device__ void check_block(const A& a) {
     check_phase(a.chk_phase, u, v, S, F, maxit);
   }
   if (!a.chk_mirror) return;
-  const int seq = a.chk_seq >= 0 ? a.chk_seq : ++F[F_SEQ];
+  const int seq = take_seq(a.chk_seq, F);
   publish(a.chk_mirror, seq, F[F_ACTIVE] && likely_last(S), S, F);
 }
 

@@ -196,10 +196,10 @@ struct Solver {
   DBuf<double> part, part2, S;  // part2: p.q partials, and ||b||^2's before the first residual
   DBuf<int> F;
   // Krylov progress and results published by the end-of-iteration finalize kernel, in pinned coherent
-  // host memory; the status' sequence number counts iterations over the handle's lifetime.
+  // host memory; the status' number counts iterations over the handle's lifetime (hoc_seq.hpp).
   MirrorState* mirror = nullptr;
   MirrorState* mirror_dev = nullptr;
-  int seq_next = 0;
+  int seq_next = kSeqStart;
   int nparts = 0;
   int nv = 0;                             // Q1 coarse space: element-corner vertices
   DBuf<int32_t> d_ev, d_vinc;             // element -> 4 vertices; vertex -> (element*4+corner), k_q1_gather
@@ -434,7 +434,7 @@ struct Solver {
     S.alloc(S_COUNT); F.alloc(F_COUNT);
     if (!mirror) {
       HIPCHK(hipHostMalloc((void**)&mirror, sizeof(MirrorState), hipHostMallocCoherent | hipHostMallocMapped));
-      __atomic_store_n(&mirror->status, -2, __ATOMIC_RELEASE);
+      __atomic_store_n(&mirror->status, status_word(seq_add(seq_next, -1), false, false), __ATOMIC_RELEASE);
       HIPCHK(hipHostGetDevicePointer((void**)&mirror_dev, mirror, 0));
     }
     build_hierarchy();
@@ -950,22 +950,22 @@ struct Solver {
   // on the pinned word and checks the stream every 4096 reads, so an idle stream without the
   // expected status (or a device error) ends it with an error instead of a hang.
   bool poll(int seq, int seq_first, bool final_wait, int lag = 1, bool* near = nullptr) {
-    const int target = final_wait ? seq : seq - lag;
+    const int target = final_wait ? seq : seq_add(seq, -lag);
     if (near) *near = false;
-    if (target < seq_first) return true;
+    if (!seq_reached(target, seq_first)) return true;
     for (unsigned spin = 1;; ++spin) {
-      const int v = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
-      if ((v >> 2) >= target) {
-        if (near) *near = (v & 2) != 0;
-        return (v & 1) != 0;
+      const uint32_t v = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
+      if (seq_reached(status_seq(v), target)) {
+        if (near) *near = status_near(v);
+        return status_active(v);
       }
       if ((spin & 4095) == 0) {
         const hipError_t q = hipStreamQuery(stream);
         if (q == hipSuccess) {
-          const int v2 = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
-          if ((v2 >> 2) >= target) {
-            if (near) *near = (v2 & 2) != 0;
-            return (v2 & 1) != 0;
+          const uint32_t v2 = __atomic_load_n(&mirror->status, __ATOMIC_ACQUIRE);
+          if (seq_reached(status_seq(v2), target)) {
+            if (near) *near = status_near(v2);
+            return status_active(v2);
           }
           throw HipError("Krylov status of an iteration was not published");
         }
@@ -1197,14 +1197,15 @@ struct Solver {
     hipGraphExec_t ge[3] = {nullptr, nullptr, nullptr};
     if (graphs) {
       for (int k = 0; k < 3; ++k) ge[k] = krylov_graph(x, r, Sp, Fp, maxit, k);
-      set_int(stream, Fp + F_SEQ, seq_next - 1);
+      set_int(stream, Fp + F_SEQ, seq_add(seq_next, -1));
     }
     // The host runs ahead by an iteration up to its test: while it waits for the status of the one
     // before, the rest of a V-cycle and that iteration are queued.  Where that status says that the
     // iteration is likely the last (near), its own is waited for before the next V-cycle is queued,
     // which would run predicated off.
     for (int it = 0;; ++it) {
-      const int seq = seq_next++;
+      const int seq = seq_next;
+      seq_next = seq_add(seq_next, 1);
       if (graphs) HIPCHK(hipGraphLaunch(ge[it & 1], stream));
       else krylov_iter(x, r, Sp, Fp, maxit, seq, it & 1);
       bool near = false;
@@ -1240,8 +1241,8 @@ struct Solver {
       for (int k = 0; k < 3 && graph; ++k) ge[k] = krylov_graph(psi.p, P64.r.p, S.p, F.p, maxit, k);
       HIPCHK(hipStreamSynchronize(stream));
       const auto t0 = std::chrono::steady_clock::now();
-      if (graph) set_int(stream, F.p + F_SEQ, seq_next - 1);
-      for (int i = 0; i < kTuneIters; ++i, ++seq_next) {
+      if (graph) set_int(stream, F.p + F_SEQ, seq_add(seq_next, -1));
+      for (int i = 0; i < kTuneIters; ++i, seq_next = seq_add(seq_next, 1)) {
         if (graph) {
           HIPCHK(hipGraphLaunch(ge[i & 1], stream));
           HIPCHK(hipGraphLaunch(ge[2], stream));

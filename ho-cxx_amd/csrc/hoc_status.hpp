@@ -8,8 +8,8 @@
 
 namespace hoc {
 
-// The solve's results, then, after a system-scope fence, the status word seq * 4 + near * 2 +
-// (active flag): the host follows the iterations and takes the results without a copy.
+// The solve's results, then, after a system-scope fence, the status word: the host follows
+// the iterations and takes the results without a copy.
 __device__ __forceinline__ void publish(MirrorState* __restrict__ mirror, int seq, bool near,
                                         const double* __restrict__ S, const int* __restrict__ F) {
   mirror->bb = S[S_BB];
@@ -17,8 +17,13 @@ __device__ __forceinline__ void publish(MirrorState* __restrict__ mirror, int se
   mirror->iter = F[F_ITER];
   mirror->zero = F[F_ZERO];
   __threadfence_system();
-  __hip_atomic_store(&mirror->status, seq * 4 + (near ? 2 : 0) + (F[F_ACTIVE] ? 1 : 0), __ATOMIC_RELAXED,
+  __hip_atomic_store(&mirror->status, status_word(seq, near, F[F_ACTIVE] != 0), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The number that a status goes out with: seq, or the next of the device's counter for seq < 0.
+__device__ __forceinline__ int take_seq(int seq, int* __restrict__ F) {
+  return seq >= 0 ? seq : (F[F_SEQ] = seq_add(F[F_SEQ], 1));
 }
 
 // Whether the next iteration is likely the last, if it reduces the residual as the one before did
