@@ -1888,7 +1888,7 @@ struct Solver {
     if (cfg.time_integration_type == 1) {
       so.next = vort; so.c = 1.; so.base = w;
       stage(w, 0., so);
-      dcopy(w, vort, D);
+      std::swap(w.p, vort.p);  // nothing keeps either address from one launch to the next
     } else if (cfg.time_integration_type == 2) {
       so.k = k1; so.next = vort; so.c = 1.; so.base = w; so.inner = true;
       stage(w, 0., so);
