@@ -11,7 +11,7 @@ struct StageOut {
   double* next = nullptr;    // base + c k_s (next stage input), or nullptr
   double c = 0.;
   double* base = nullptr;    // omega_n (read for next; updated for final_mode)
-  int final_mode = 0;        // 0 none, 1 Euler, 2 RK2 (needs k1), 4 RK4 (needs k1..k3)
+  int final_mode = 0;        // 0 none, 2 RK2 (needs k1), 4 RK4 (needs k1..k3)
   const double *k1 = nullptr, *k2 = nullptr, *k3 = nullptr;
   // linearised stage (launch_stage mode 1 records, mode 2 reads the upwind switches)
   int8_t* sig = nullptr;               // [N][4][K] upwind switch of each interior flux point

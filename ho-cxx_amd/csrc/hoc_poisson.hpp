@@ -24,8 +24,8 @@ enum { IN_X = 0, IN_PROL = 1, IN_PUPD = 2 };
 enum { GEO_ORTHO = 0, GEO_AFFINE = 1, GEO_POINT = 2 };
 
 constexpr int kFineThreads = 256;
-// Elements per wavefront: K lanes each, and a multiple of 4 so that a block's elements start on
-// a 16-byte boundary in every field.
+// Elements per wavefront: K lanes each.  A block's four wavefronts hold a multiple of 4, so that its
+// elements start on a 16-byte boundary in every field.
 constexpr int fine_epw(int K) { return K == 2 ? 32 : K == 3 ? 20 : K == 4 ? 16 : K == 5 ? 12 : 10; }
 // Up to this many partials every block of the next kernel sums them itself, which saves a launch
 // (4.4 us in a chain of dependent kernels) for about 1 us; above, a finalize kernel does.

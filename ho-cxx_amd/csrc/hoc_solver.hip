@@ -4,11 +4,11 @@
 //   update_BCs(t)            k_update_bcs
 //   solve_Poisson            k_rhs, then PCG or BiCGSTAB on As = -W A (W = Gauss weights
 //                            w_i w_j, which makes As symmetric on affine meshes) with a
-//                            V-cycle: matrix-free fine level + Chebyshev(2) element-block
-//                            smoothing, continuous bilinear coarse space on the element
-//                            corners (Ac = Pc^T As Pc assembled from probes of As), then
-//                            Ruge-Stueben coarsening below
-//   velocity, wall vorticity k_trace + k_velocity
+//                            V-cycle: matrix-free fine level + Chebyshev smoothing with the
+//                            element blocks' inverse (degree by order and shape), continuous
+//                            bilinear coarse space on the element corners (Ac = Pc^T As Pc
+//                            assembled from probes of As), then Ruge-Stueben coarsening below
+//   velocity, wall vorticity k_velocity
 //   diffusion + advection    k_stage (fused with k = dt (adv + diff) and the RK update)
 #include <hip/hip_runtime.h>
 
@@ -1300,8 +1300,8 @@ struct Solver {
   //         reference's ||b - A psi|| <= tol ||b||.
   //  mixed: the same FP64 Krylov method, the same operator and the same stopping test, with
   //         the V-cycle in FP32 as its preconditioner: the residual is demoted at the cycle's
-  //         entry and the cycle's output enters the FP64 direction update (precond, and the
-  //         PCG loop's FP32-input direction update).
+  //         entry and the cycle's output enters the FP64 direction update (PCG's reads it in FP32,
+  //         BiCGSTAB's after a promotion, precond_rest).
   const double* rhs_bc = nullptr;  // boundary stream-function values of the next solve (null: b_psi)
 
   // Initial guess of the stage solves.  Mode 1: the previous solution, as the reference
@@ -1703,7 +1703,7 @@ struct Solver {
     }
     const double* pbb = have_bb ? nullptr : part2.p;
     outer_residual(pbb);
-    // FP64: the FP64 V-cycle; mixed: the FP32 V-cycle (precond), the Krylov vectors, the operator
+    // FP64: the FP64 V-cycle; mixed: the FP32 V-cycle; the Krylov vectors, the operator
     // application and the stopping test in FP64 either way.  The results arrive with the status of
     // the last iteration, so the stream goes on without a copy or a wait for it to drain.
     krylov_solve(psi.p, P64.r.p, pbb, S.p, F.p, maxit, maxit);

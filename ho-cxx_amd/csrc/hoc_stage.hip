@@ -572,15 +572,14 @@ __global__ __launch_bounds__(kFineThreads) void k_stage(int N, Tab T, Geo G, BCD
   }
   if (so.final_mode) {  // vorticity update
     double k1[K], k2[K], k3[K];
-    if (so.final_mode >= 2) load_row<K>(so.k1 + row, k1);
+    load_row<K>(so.k1 + row, k1);
     if (so.final_mode == 4) {
       load_row<K>(so.k2 + row, k2);
       load_row<K>(so.k3 + row, k3);
     }
 #pragma unroll
     for (int i = 0; i < K; ++i) {
-      if (so.final_mode == 1) o[i] = b[i] + kk[i];
-      else if (so.final_mode == 2) o[i] = b[i] + 0.5 * (k1[i] + kk[i]);
+      if (so.final_mode == 2) o[i] = b[i] + 0.5 * (k1[i] + kk[i]);
       else o[i] = b[i] + (k1[i] + 2. * k2[i] + 2. * k3[i] + kk[i]) / 6.;
     }
     store_row<K>(so.base + row, o);
