@@ -847,6 +847,26 @@ void sell_pack(const CSR& A, int lanes, std::vector<int32_t>& off, std::vector<i
     }
 }
 
+void gather_pack(const std::vector<int32_t>& vptr, const std::vector<int32_t>& vinc, int pad, int& w,
+                 std::vector<int32_t>& off, std::vector<int32_t>& inc) {
+  const int nv = (int)vptr.size() - 1, ns = (nv + 63) / 64;
+  off.assign(ns + 1, 0);
+  w = 0;
+  for (int s = 0; s < ns; ++s) {
+    int ws = 0;
+    for (int v = 64 * s; v < std::min(nv, 64 * (s + 1)); ++v) ws = std::max(ws, vptr[v + 1] - vptr[v]);
+    off[s + 1] = off[s] + 64 * ws;
+    w = std::max(w, ws);
+  }
+  const bool same = (int64_t)64 * w * ns <= 2 * (int64_t)off[ns];
+  inc.assign(same ? (size_t)64 * w * ns : (size_t)off[ns], pad);
+  for (int v = 0; v < nv; ++v) {
+    const size_t q = (same ? (size_t)64 * w * (v / 64) : (size_t)off[v / 64]) + v % 64;
+    for (int k = vptr[v]; k < vptr[v + 1]; ++k) inc[q + (size_t)64 * (k - vptr[v])] = vinc[k];
+  }
+  if (same) off.clear();
+}
+
 void csr_check(const CSR& A) {
   if (A.n < 0 || A.m < 0 || (int64_t)A.ptr.size() != (int64_t)A.n + 1 || A.ptr[0] != 0 ||
       (size_t)A.ptr[A.n] != A.col.size() || A.col.size() != A.val.size())

@@ -192,6 +192,12 @@ void build_vhierarchy(const CSR& A, int coarse_enough, VHierarchy& h);
 void sell_pack(const CSR& A, int lanes, std::vector<int32_t>& off, std::vector<int32_t>& col, std::vector<double>& val);
 // Lanes per row: enough to fill the device with a level's rows, at most about a row's length.
 int sell_lanes(const CSR& A);
+// The corners that meet at each vertex (CSR vptr, vinc), for a gather by 64 vertices a wavefront: entry c of
+// vertex v at off[v / 64] + 64 c + v % 64, as many as the slice's vertices have at most, padding = pad.
+// off empty: every slice takes the same w entries (off[s] = 64 w s), where that padding costs less than the
+// slices' own widths' again; off's extra load is for meshes with vertices of many elements.
+void gather_pack(const std::vector<int32_t>& vptr, const std::vector<int32_t>& vinc, int pad, int& w,
+                 std::vector<int32_t>& off, std::vector<int32_t>& inc);
 // Dense inverse (row-major) by Gauss-Jordan with partial pivoting; a singular direction is left out.
 void dense_inverse(const CSR& A, std::vector<double>& inv);
 

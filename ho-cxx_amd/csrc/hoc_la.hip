@@ -433,16 +433,29 @@ __global__ void k_probe_diag(int N, int K2, const int32_t* __restrict__ color, i
   diag[(size_t)el * K2 + rs] = y[(size_t)el * K2 + rs];
 }
 // ---- Q1 coarse space ---------------------------------------------------------------------------
-// rc[v] = sum over the (element, corner) incidences of vertex v of ec[element][corner]
+// sum over the (element, corner) incidences of vertex v of ec[element][corner]; v / 64 is the same in the
+// whole wavefront
 template <class R>
-__global__ void k_q1_gather(int nv, int w, const int32_t* __restrict__ inc, const R* __restrict__ ec,
-                            R* __restrict__ rc, const int* __restrict__ F) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if ((F && !F[F_ACTIVE]) || v >= nv) return;
+__device__ __forceinline__ R corner_sum(const Corners& C, int v, const R* __restrict__ ec) {
+  const int sl = __builtin_amdgcn_readfirstlane(v >> 6);
+  size_t q = (size_t)sl * 64 * C.w;
+  int n = C.w;
+  if (C.off) {
+    q = C.off[sl];
+    n = (C.off[sl + 1] - C.off[sl]) >> 6;
+  }
+  q += v & 63;
   R s = 0;
 #pragma unroll 4
-  for (int c = 0; c < w; ++c) s += ec[inc[(size_t)c * nv + v]];
-  rc[v] = s;
+  for (int c = 0; c < n; ++c) s += ec[C.inc[q + (size_t)64 * c]];
+  return s;
+}
+template <class R>
+__global__ void k_q1_gather(int nv, Corners C, const R* __restrict__ ec, R* __restrict__ rc,
+                            const int* __restrict__ F) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if ((F && !F[F_ACTIVE]) || v >= nv) return;
+  rc[v] = corner_sum(C, v, ec);
 }
 
 // The coarsest level where it is the vertex space itself: the gather of the corner sums and the
@@ -450,9 +463,9 @@ __global__ void k_q1_gather(int nv, int w, const int32_t* __restrict__ inc, cons
 // before the block has gathered the right-hand side into LDS, so the row is in flight meanwhile.
 // Every block gathers the whole right-hand side (4 n values from the L2); a launch costs more.
 template <int C, class R>
-__global__ __launch_bounds__(256) void k_dense_gather(int n, const R* __restrict__ Ainv, int w,
-                                                      const int32_t* __restrict__ inc, const R* __restrict__ ec,
-                                                      R* __restrict__ x, const int* __restrict__ F) {
+__global__ __launch_bounds__(256) void k_dense_gather(int n, const R* __restrict__ Ainv, Corners V,
+                                                      const R* __restrict__ ec, R* __restrict__ x,
+                                                      const int* __restrict__ F) {
   __shared__ R f[64 * C];
   const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const R* a = Ainv + (size_t)min(row, n - 1) * n;
@@ -464,9 +477,7 @@ __global__ __launch_bounds__(256) void k_dense_gather(int n, const R* __restrict
   for (int q = 0; q < (64 * C + 255) / 256; ++q) {
     const int i = threadIdx.x + 256 * q;
     R s = 0;
-    if (i < n)
-#pragma unroll 4
-      for (int c = 0; c < w; ++c) s += ec[inc[(size_t)c * n + i]];
+    if (i < n) s = corner_sum(V, i, ec);
     if (i < 64 * C) f[i] = s;
   }
   __syncthreads();
@@ -1345,14 +1356,14 @@ void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F) 
   else hipLaunchKernelGGL((k_dense<256, R>), dim3(n), dim3(256), 0, s, n, Ainv, f, x, F);
 }
 template <class R>
-void q1_gather(hipStream_t s, int nv, int w, const int32_t* inc, const R* ec, R* rc, const int* F) {
-  hipLaunchKernelGGL(k_q1_gather<R>, dim3((nv + 255) / 256), dim3(256), 0, s, nv, w, inc, ec, rc, F);
+void q1_gather(hipStream_t s, int nv, const Corners& C, const R* ec, R* rc, const int* F) {
+  hipLaunchKernelGGL(k_q1_gather<R>, dim3((nv + 255) / 256), dim3(256), 0, s, nv, C, ec, rc, F);
 }
 template <class R>
-void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc, const R* ec, R* x, const int* F) {
+void dense_gather(hipStream_t s, int n, const R* Ainv, const Corners& C, const R* ec, R* x, const int* F) {
   const dim3 grid((n + 3) / 4), block(256);
-  if (n <= 320) hipLaunchKernelGGL((k_dense_gather<5, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
-  else hipLaunchKernelGGL((k_dense_gather<kDenseGather / 64, R>), grid, block, 0, s, n, Ainv, w, inc, ec, x, F);
+  if (n <= 320) hipLaunchKernelGGL((k_dense_gather<5, R>), grid, block, 0, s, n, Ainv, C, ec, x, F);
+  else hipLaunchKernelGGL((k_dense_gather<kDenseGather / 64, R>), grid, block, 0, s, n, Ainv, C, ec, x, F);
 }
 void promote(hipStream_t s, size_t n, const float* z32, double* z64, const int* F) {
   hipLaunchKernelGGL(k_promote, dim3(vec_grid(n)), dim3(256), 0, s, n, z32, z64, F);
@@ -1382,8 +1393,8 @@ template void ell<double>(hipStream_t, int, int, int, int, const int32_t*, const
 #define HOC_LA_INST(R)                                                                                                 \
   template void sell<R>(hipStream_t, int, int, const int32_t*, const int32_t*, const R*, const R*, R*, const int*);    \
   template void dense<R>(hipStream_t, int, const R*, const R*, R*, const int*);                                       \
-  template void q1_gather<R>(hipStream_t, int, int, const int32_t*, const R*, R*, const int*);                          \
-  template void dense_gather<R>(hipStream_t, int, const R*, int, const int32_t*, const R*, R*, const int*);
+  template void q1_gather<R>(hipStream_t, int, const Corners&, const R*, R*, const int*);                               \
+  template void dense_gather<R>(hipStream_t, int, const R*, const Corners&, const R*, R*, const int*);
 HOC_LA_INST(double)
 HOC_LA_INST(float)
 #undef HOC_LA_INST

@@ -76,13 +76,18 @@ size_t dense_invert_work(int n);
 void dense_invert(hipStream_t s, int n, double* A, double* work);
 template <class R>
 void dense(hipStream_t s, int n, const R* Ainv, const R* f, R* x, const int* F);
-// rc[v] = sum of the element corners at vertex v: ec[inc[c nv + v]], c < w (padding names a zero).
+// The corners at each vertex as gather_pack lays them out (off null: w entries a vertex; padding names a zero).
+struct Corners {
+  int w;
+  const int32_t *off, *inc;
+};
+// rc[v] = sum of ec over the element corners at vertex v.
 template <class R>
-void q1_gather(hipStream_t s, int nv, int w, const int32_t* inc, const R* ec, R* rc, const int* F);
+void q1_gather(hipStream_t s, int nv, const Corners& C, const R* ec, R* rc, const int* F);
 // x = Ainv q1_gather(ec) in one launch (n = nv <= kDenseGather).
 constexpr int kDenseGather = 1216;
 template <class R>
-void dense_gather(hipStream_t s, int n, const R* Ainv, int w, const int32_t* inc, const R* ec, R* x, const int* F);
+void dense_gather(hipStream_t s, int n, const R* Ainv, const Corners& C, const R* ec, R* x, const int* F);
 
 // The FP32 V-cycle inside the FP64 BiCGSTAB: z64 = (double) z32.
 void promote(hipStream_t s, size_t n, const float* z32, double* z64, const int* F);

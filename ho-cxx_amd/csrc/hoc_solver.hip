@@ -211,8 +211,8 @@ struct Solver {
   int seq_next = kSeqStart;
   int nparts = 0;
   int nv = 0;                             // Q1 coarse space: element-corner vertices
-  DBuf<int32_t> d_ev, d_vinc;             // element -> 4 vertices; vertex -> (element*4+corner), k_q1_gather
-  int vdeg = 0;                           // largest number of elements at a vertex
+  DBuf<int32_t> d_ev, d_vinc, d_voff;     // element -> 4 vertices; vertex -> (element*4+corner), gather_pack
+  Corners corners{};
   // Chebyshev smoother of degree cheb_m in B As (B: the element blocks' inverse) as damped
   // Richardson steps x += cheb_w[k] B (r - As x)
   int cheb_m = 2;
@@ -724,12 +724,11 @@ struct Solver {
       for (int e = 0; e < N; ++e)
         for (int a = 0; a < 4; ++a) vinc[pos[ev[(size_t)e * 4 + a]]++] = e * 4 + a;
     }
-    vdeg = 0;
-    for (int v = 0; v < nv; ++v) vdeg = std::max(vdeg, vptr[v + 1] - vptr[v]);
-    std::vector<int32_t> inc((size_t)vdeg * nv, N * 4);
-    for (int v = 0; v < nv; ++v)
-      for (int k = vptr[v]; k < vptr[v + 1]; ++k) inc[(size_t)(k - vptr[v]) * nv + v] = vinc[k];
-    d_ev.upload(ev); d_vinc.upload(inc);
+    std::vector<int32_t> voff, inc;
+    gather_pack(vptr, vinc, N * 4, corners.w, voff, inc);
+    d_ev.upload(ev); d_vinc.upload(inc); d_voff.upload(voff);
+    corners.off = d_voff;
+    corners.inc = d_vinc;
     P64.G.ev = d_ev;
     P32.G.ev = d_ev;
     inst_coupled = false;  // an ensemble whose instances share a corner vertex
@@ -931,9 +930,9 @@ struct Solver {
     A.x = cur; A.y = P.ec.p; A.part = nullptr;
     fine(P, IN_X, EPI_RESTRICT, A);
     if (P.lv.dense_only() && nv <= kDenseGather) {
-      dense_gather<R>(stream, nv, P.lv.inv, vdeg, d_vinc, P.ec, P.xc.p, Fp);
+      dense_gather<R>(stream, nv, P.lv.inv, corners, P.ec, P.xc.p, Fp);
     } else {
-      q1_gather<R>(stream, nv, vdeg, d_vinc, P.ec, P.lv.rhs(), Fp);
+      q1_gather<R>(stream, nv, corners, P.ec, P.lv.rhs(), Fp);
       P.lv.cycle(stream, P.xc.p, Fp);
     }
     // prolongate and post-smooth, the dampings in reverse: the cycle stays symmetric
