@@ -724,8 +724,9 @@ void build_vhierarchy(const CSR& A0, int coarse_enough, VHierarchy& h) {
     rs_colour(n, sp, si, state);
     std::vector<int32_t> cid(n, -1);
     int nc = 0;
+    // nc < n: the first row made coarse makes the rows that depend on it fine, of which it has some, and
+    // without strong couplings every row is fine
     for (int i = 0; i < n; ++i) if (state[i] == 1) cid[i] = nc++;
-    if (nc >= n) break;
     std::vector<double> dia(n, 0.), M(n, 0.);
     for (int i = 0; i < n; ++i) {
       double s2 = 0.;
