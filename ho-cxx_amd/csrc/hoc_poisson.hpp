@@ -61,18 +61,20 @@ struct FineGeo {
 // line operators are applied to a line's even and odd parts, e_i = u_i + u_{K-1-i} (the middle value
 // itself) and o_i = u_i - u_{K-1-i}: about half the products and half the constants, which then
 // stay in scalar registers.
+// Aligned to the scalar cache's lines, so that the arguments behind it keep their places in them.
 template <class R>
-struct FineTab {
+struct alignas(64) FineTab {
   R lv[6], ld[6];  // l_m(-1), l_m'(-1) (the upper end by reflection)
   R lvE[3], lvO[3], ldE[3], ldO[3];      // the same on the even and odd parts
   R DDE[3][3], DDO[3][3];                // second derivative: [in][out] (V-cycle)
-  R DE[3][3], DO[3][3];                  // derivative: the odd part of an even line's, and vice versa
   R gdE[3], gdO[3], DgE[3], DgO[3];      // lower Radau correction's derivative, and its derivative
   R m0, m1;        // that correction's derivative extrapolated to -1 and +1
   R g0, ig0;       // -g'(-1), the interface coefficient, and its inverse
   R w[6], x[6];    // Gauss weights and points
   R SE[3][3], SO[3][3], lam[6];  // eigenpairs of an interior element's line operator, even ones first
   R D[6][6], gd[6];  // l_m'(xi_k), the correction's derivative (elements with tangential metrics)
+  R DE[3][3], DO[3][3];  // derivative: the odd part of an even line's, and vice versa (behind what the
+                         // V-cycle's kernels load: in front, 0.3 us more for each of them, FP32, 121 x 121, K = 3)
 };
 
 template <class R>
