@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(int phase, const doubl
                                                           MirrorState* __restrict__ mirror, int seq,
                                                           const double* __restrict__ irr,
                                                           const double* __restrict__ ibb, int ninst) {
-  const bool live = phase == PH_INIT || phase == PH_BB || F[F_ACTIVE];
+  const bool live = phase == PH_INIT || phase == PH_BB || solve_live(F);
   const bool half = live && phase >= PH_OMEGA && F[F_HALF];  // BiCGSTAB converged at the half step
   if (live && !half) {  // uniform over the block
     double a = 0., b = 0., c = 0.;
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(int phase, const doubl
       if (pbb) S[S_BB] = c;
       finalize_phase(phase, a, b, S, F, maxiter >= 0 ? maxiter : F[F_MAXIT], irr, ibb, ninst);
     }
-  } else if (half && phase == PH_RNORM && threadIdx.x == 0) {
+  } else if ((!live || phase == PH_RNORM) && threadIdx.x == 0) {
     F[F_ACTIVE] = 0;
   }
   if (mirror && threadIdx.x == 0) {
@@ -187,7 +187,6 @@ __device__ void finalize_phase(int phase, double a, double b, double* __restrict
       S[S_ALPHA] = al;
     } break;
     case PH_UPD: {
-      if (F[F_BREAK]) { F[F_ACTIVE] = 0; break; }
       S[S_RR] = b;
       F[F_ITER] += 1;
       F[F_ACTIVE] = (above && F[F_ITER] < maxiter && isfinite(b)) ? 1 : 0;

@@ -497,7 +497,7 @@ __device__ void check_block(const A& a) {
   int* F = a.chk_F;
   double* S = a.scal;
   const bool init = a.chk_phase == PH_INIT;
-  const bool live = init || F[F_ACTIVE] != 0;  // uniform over the block
+  const bool live = init || solve_live(F);  // uniform over the block
   double u = 0., v = 0., bb = 0.;
   if (live) sum_pairs(a.chk_part, a.chk_np, u, v);
   if (a.chk_bb) bb = sum_parts(a.chk_bb, a.chk_nbb);
@@ -508,6 +508,8 @@ __device__ void check_block(const A& a) {
     init_phase(u, v, v > S[S_TOL2] * S[S_BB], S, F, maxit);
   } else if (live) {
     check_phase(a.chk_phase, u, v, S, F, maxit);
+  } else {
+    F[F_ACTIVE] = 0;
   }
   if (!a.chk_mirror) return;
   const int seq = take_seq(a.chk_seq, F);

@@ -47,13 +47,18 @@ __device__ __forceinline__ void init_phase(double a, double b, bool above, doubl
   S[S_RZ] = 0.; S[S_RHO] = S[S_RHON] = a; S[S_ALPHA] = 1.; S[S_OMEGA] = 1.; S[S_BETA] = 0.;
 }
 
+// Whether a test has a solve to test.  After a breakdown that the update in front of it has seen (F_BREAK) it
+// has none: x and r are those of the iteration before, and the norms are not this one's.
+__device__ __forceinline__ bool solve_live(const int* __restrict__ F) {
+  const int a = F[F_ACTIVE], b = F[F_BREAK];  // (both loads under way before either is looked at)
+  return (a != 0) & (b == 0);
+}
+
 // b = ||r||^2 (unscaled) against the tolerance.  PH_UPD: end of a PCG iteration.  PH_BHALF: BiCGSTAB
 // at its half step (x already holds alpha ph).  PH_BNEXT: end of a BiCGSTAB iteration, a = rh . r of
-// the next; rho = 0 or not finite is a breakdown.  After one that the update in front of the test has seen
-// (F_BREAK), x and r are those of the iteration before and the norms are not this one's.
+// the next; rho = 0 or not finite is a breakdown.
 __device__ __forceinline__ void check_phase(int phase, double a, double b, double* __restrict__ S,
                                             int* __restrict__ F, int maxiter) {
-  if (F[F_BREAK]) { F[F_ACTIVE] = 0; return; }
   const double tol2bb = S[S_TOL2] * S[S_BB];
   S[S_RR] = b;
   if (phase == PH_BHALF) {
