@@ -95,16 +95,9 @@ class HostCopy {
       if (e) (void)hipEventDestroy(e);
     if (pin_) (void)hipHostFree(pin_);
   }
-  // false: no pinned memory or no threads to be had, and nothing copied
+  // false: no events, pinned memory or threads to be had, and nothing copied
   bool d2h(int device, hipStream_t s, char* dst, const char* src, size_t bytes) {
-    if (!pin_) {
-      if (hipHostMalloc(reinterpret_cast<void**>(&pin_), kSlots * kChunk) != hipSuccess) {
-        (void)hipGetLastError();
-        pin_ = nullptr;
-        return false;
-      }
-      for (auto& e : ev_) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    if (!ring()) return false;
     const size_t n = (bytes + kChunk - 1) / kChunk;
     std::atomic<size_t> issued{0};
     std::atomic<int> err{hipSuccess};
@@ -156,6 +149,21 @@ class HostCopy {
 
  private:
   static constexpr size_t kChunk = size_t(1) << 20, kSlots = 16, kThreads = 4;
+  // The events and then the slots; what a failed call has made, the next one keeps.
+  bool ring() {
+    for (auto& e : ev_)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        e = nullptr;
+        return false;
+      }
+    if (!pin_ && hipHostMalloc(reinterpret_cast<void**>(&pin_), kSlots * kChunk) != hipSuccess) {
+      (void)hipGetLastError();
+      pin_ = nullptr;
+      return false;
+    }
+    return true;
+  }
   char* pin_ = nullptr;
   hipEvent_t ev_[kSlots] = {};
 };
